@@ -288,8 +288,8 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     L.l_k = nm <= 16 ? lds(2L * nm * nm * 8) : -1;
     L.l_strip = nm > 16 ? lds(128L * 16 * 8) : -1;
     L.l_legc = lds(2L * std::max(h->nleg, 1) * 8);
-    // blocks of up to 4 states: quad-walk chunk buffers (16 operators)
-    if (nm <= 4) {
+    // chunk buffers of the register walks (16 operators)
+    if (nm <= 16) {
         L.l_qa = lds(16L * 16 * 8);
         L.l_qlc = lds(16L * 8);
         L.l_qrec = lds(16L * 16);
@@ -308,13 +308,10 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     } else {
         L.l_rk = L.l_lb = L.l_rkx = L.l_lbx = L.l_rks = L.l_lbs = -1;
     }
-    const long opsb = (long)m.ops.size() * 8;
-    // blocks of up to 4 states: the kernels read operator blocks from LDS only
-    // operator blocks join LDS when the total stays within 64 KB (more would
-    // cut the number of chains resident per CU); blocks of up to 4 states always
-    // (above 16 states they stay in global memory: the MFMA walks read them
-    // with global instructions)
-    L.l_ops = (nm <= 4 || (nm <= 16 && q + opsb <= 64 * 1024)) ? lds(opsb) : -1;
+    // operator blocks: in LDS for blocks of up to 4 states; above, the matrix-
+    // core walks read them from global memory (the table is shared by all
+    // chains and prefetched, and LDS buys chains per CU)
+    L.l_ops = nm <= 4 ? lds((long)m.ops.size() * 8) : -1;
     L.lds_bytes = q;
     if (L.lds_bytes > h->lds_max) return W2D_ERR_CAPACITY;
     L.hdrs = L.stride * h->nchains;

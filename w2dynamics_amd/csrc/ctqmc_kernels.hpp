@@ -426,154 +426,10 @@ struct Work {
     }
 };
 
-// exp(-(E_k - E0) dt) of superstate s into LDS dvec; returns the log factor
-// -(E0 - Egs) dt.  Ends with a barrier.  (Blocks above 16 states.)
-DEV double prop_factors(Ctx &c, int s, double dt)
-{
-    const int ns = c.sz[s];
-    const double *E = c.ev + c.off[s];
-    const double e0 = E[0];
-    for (int k = lane_id(); k < ns; k += WAVE) c.dvec[k] = (ns > 1) ? exp(-(E[k] - e0) * dt) : 1.0;
-    wsync();
-    return -(e0 - c.M.egs) * dt;
-}
-
-// Lane k's propagator factor exp(-(E_k - E0) dt) of superstate s (1 beyond the
-// block); the common log factor -(E0 - Egs) dt is added to lg.  No LDS traffic:
-// the factors are broadcast by readlane inside apply_small.
-DEV double prop_lane(const Ctx &c, int s, double dt, double &lg)
-{
-    const int ns = c.sz[s];
-    const double *E = c.ev + c.off[s];
-    const double e0 = E[0];
-    lg += -(e0 - c.M.egs) * dt;
-    const int k = lane_id();
-    const double ek = k < ns ? E[k] : e0;
-    return exp(-(ek - e0) * dt);   // exactly 1 beyond the block and for 1-state blocks
-}
-
-// prop_lane for a block given by its energies E and size ns
-DEV double prop_e(const Ctx &c, const double *E, int ns, double dt, double &lg)
-{
-    const double e0 = E[0];
-    lg += -(e0 - c.M.egs) * dt;
-    const int k = lane_id();
-    const double ek = k < ns ? E[k] : e0;
-    return exp(-(ek - e0) * dt);
-}
-
 // Thresholds outside which a state matrix is renormalised during a walk; in
 // between, the entries are left unscaled (rescaling by powers of two is exact,
 // so skipping it changes no rounding).
 constexpr double STATE_TINY = 0x1p-64, STATE_HUGE = 0x1p64;
-
-// Output element u of this lane in a (rows x no) row-major state: row rr[u],
-// column ii[u]; computed once per walk.
-template <int NM>
-struct LaneSlots {
-    static constexpr int PER = (NM * NM + WAVE - 1) / WAVE;
-    int rr[PER], ii[PER];
-    DEV explicit LaneSlots(int no)
-    {
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int idx = lane_id() + u * WAVE;
-            rr[u] = idx / no;
-            ii[u] = idx - rr[u] * no;
-        }
-    }
-};
-
-// One operator on blocks of at most 16 states: Kout (nt x no) = P * diag(d) *
-// Kin (ns x no), d broadcast from the lanes of prop_lane.  One barrier.
-template <int NM>
-DEV void apply_small(const double *P, const double *Kin, double *Kout, int nt, int ns, int no, double d,
-                     const LaneSlots<NM> &ls, double &lg)
-{
-    constexpr int PER = LaneSlots<NM>::PER;
-    // block and state entries first (independent of the propagator factors),
-    // for blocks up to 4 states held in registers
-    constexpr bool PRE = NM <= 4;
-    double pv[PRE ? PER : 1][PRE ? NM : 1], kv[PRE ? PER : 1][PRE ? NM : 1];
-    if constexpr (PRE) {
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int r = ls.rr[u] < nt ? ls.rr[u] : 0, i = ls.ii[u];
-#pragma unroll
-            for (int k = 0; k < NM; ++k) {
-                const int kk = k < ns ? k : 0;
-                pv[u][k] = P[r + kk * nt];
-                kv[u][k] = Kin[kk * no + i];
-            }
-        }
-    }
-    double dk[NM];
-#pragma unroll
-    for (int k = 0; k < NM; ++k) dk[k] = readlane_d(d, k);
-    // columns k >= ns contribute zero: their factor is zeroed and their
-    // addresses clamped, so the unrolled products run without branches
-#pragma unroll
-    for (int k = 0; k < NM; ++k) dk[k] = k < ns ? dk[k] : 0.0;
-    double v[PER];
-    double m = 0.0;
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-        double acc = 0.0;
-        const int r = ls.rr[u] < nt ? ls.rr[u] : 0, i = ls.ii[u];
-#pragma unroll
-        for (int k = 0; k < NM; ++k) {
-            const int kk = k < ns ? k : 0;
-            if constexpr (PRE)
-                acc = fma(pv[u][k] * dk[k], kv[u][k], acc);
-            else
-                acc = fma(P[r + kk * nt] * dk[k], Kin[kk * no + i], acc);
-        }
-        acc = ls.rr[u] < nt ? acc : 0.0;
-        v[u] = acc;
-        m = fmax(m, fabs(acc));
-    }
-    if (__ballot(m >= STATE_TINY) == 0ull || __ballot(m > STATE_HUGE) != 0ull) {
-        const double mm = wave_max(m);
-        if (mm > 0.0) {
-            const int e = ilogb(mm);
-            lg += (double)e * 0.69314718055994530942;
-#pragma unroll
-            for (int u = 0; u < PER; ++u) v[u] = ldexp(v[u], -e);
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < PER; ++u)
-        if (ls.rr[u] < nt) Kout[lane_id() + u * WAVE] = v[u];
-    wsync();
-}
-
-// Final propagation of a walk (rows scaled by lane r's factor d) and
-// normalisation to a maximum modulus of one.
-template <int NM>
-DEV void finish_small(double *K, int ns, int no, double d, const LaneSlots<NM> &ls, double &lg)
-{
-    constexpr int PER = LaneSlots<NM>::PER;
-    double v[PER];
-    double m = 0.0;
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-        const int r = ls.rr[u];
-        const double dr = __shfl(d, r < WAVE ? r : 0, WAVE);
-        v[u] = r < ns ? K[lane_id() + u * WAVE] * dr : 0.0;
-        m = fmax(m, fabs(v[u]));
-    }
-    m = wave_max(m);
-    if (m > 0.0) {
-        const double inv = 1.0 / m;
-        lg += log(m);
-#pragma unroll
-        for (int u = 0; u < PER; ++u) v[u] *= inv;
-    }
-#pragma unroll
-    for (int u = 0; u < PER; ++u)
-        if (ls.rr[u] < ns) K[lane_id() + u * WAVE] = v[u];
-    wsync();
-}
 
 // ---------------------------------------------------------------------------
 // Walks on blocks of at most 4 states, in registers.  The (ns x no) state is
@@ -797,67 +653,197 @@ struct NoAfter {
 };
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) double lds_d;
+typedef __attribute__((address_space(1))) double glb_d;
 
-// One operator on blocks above 16 states with the FP64 matrix cores:
-// Kout (nt x no, row-major) = P diag(dvec) (P: nt x ns, column-major) Kin
-// (ns x no, row-major), in 16 x 16 output tiles with k-steps of 4.  For
-// v_mfma_f64_16x16x4f64 lane l holds A(l%16, l/16), B(l/16, l%16) and the
-// outputs D(l/16 + 4e, l%16), e = 0..3.  Renormalised (by a power of two)
-// only when the largest entry leaves [2^-64, 2^64].  Blocks up to 128 states.
-DEV void apply_mfma(Ctx &c, const double *P, const double *Kin, double *Kout, int nt, int ns, int no,
-                    double &lg)
-{
-    // a 16-column strip of the output at a time, all its row tiles in
-    // registers: per k-step one B fragment serves every row tile
-    constexpr int RT = 8;                    // row tiles held (blocks up to 128 states)
-    const int l = lane_id();
-    const int lr = l & 15, lk = l >> 4;
-    const int ntr = (nt + 15) >> 4;
-    double m = 0.0;
-    for (int i0 = 0; i0 < no; i0 += 16) {
-        const int i = i0 + lr;
-        dbl4 acc[RT];
+// ---------------------------------------------------------------------------
+// Walks on blocks of 5 to 16 states, in registers, on the FP64 matrix cores.
+// The (ns x no) state is zero-padded to 16 x 16; lane l holds its entries
+// (4e + l/16, l%16), e = 0..3.  That is the output layout of
+// v_mfma_f64_16x16x4f64 and, register e taken as B(l/16, l%16), also the
+// operand layout of its k-step e: an operator is
+//   K' = sum_e A_e (d o K_e),  A_e(l%16, l/16) = P(l%16, 4e + l/16),
+// ceil(ns/4) chained matrix instructions, and the state never leaves its
+// registers.  Block entries come from the operator table in global memory (the
+// same 29 KB for every chain of the 3-orbital model: L1/L2 hits), two operators
+// ahead; the propagators of QCH operators are computed 64 at a time into LDS.
+// Bound by the latency of the operator chain (one wave per chain).  512 chains
+// of the 3-orbital model at beta = 100: 17.5 ms per 200 moves; per-lane dot
+// products with both matrices in LDS took 60 ms (9000 cycles per operator).
+// ---------------------------------------------------------------------------
+struct Hex {
+    int lr, lk;
+    DEV Hex() : lr(lane_id() & 15), lk(lane_id() >> 4) {}
+    DEV void load(const double *K, int ns, int no, double (&v)[4]) const
+    {
 #pragma unroll
-        for (int t = 0; t < RT; ++t) acc[t] = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 2
-        for (int k0 = 0; k0 < ns; k0 += 4) {
-            const int k = k0 + lk;
-            const bool kin = k < ns;
-            const double b = (kin && i < no) ? Kin[(long)k * no + i] : 0.0;
-            const double dk = kin ? c.dvec[k] : 0.0;
-#pragma unroll
-            for (int t = 0; t < RT; ++t) {
-                if (t < ntr) {
-                    const int r = t * 16 + lr;
-                    const double a = (r < nt && kin) ? P[r + (long)k * nt] * dk : 0.0;
-                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[t], 0, 0, 0);
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-            if (t < ntr) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int ro = t * 16 + lk + 4 * e;
-                    if (ro < nt && i < no) {
-                        Kout[(long)ro * no + i] = acc[t][e];
-                        m = fmax(m, fabs(acc[t][e]));
-                    }
-                }
-            }
+        for (int e = 0; e < 4; ++e) {
+            const int r = 4 * e + lk;
+            const bool in = r < ns && lr < no;
+            const double x = K[in ? r * no + lr : 0];
+            v[e] = in ? x : 0.0;
         }
     }
-    wsync();
+    DEV void store(double *K, int ns, int no, const double (&v)[4]) const
+    {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 4 * e + lk;
+            if (r < ns && lr < no) K[r * no + lr] = v[e];
+        }
+    }
+};
+
+// power-of-two renormalisation when the largest entry leaves [2^-64, 2^64]
+DEV void hex_renorm(double (&v)[4], double &lg)
+{
+    const double m = fmax(fmax(fabs(v[0]), fabs(v[1])), fmax(fabs(v[2]), fabs(v[3])));
     if (__ballot(m >= STATE_TINY) == 0ull || __ballot(m > STATE_HUGE) != 0ull) {
         const double mm = wave_max(m);
         if (mm > 0.0) {
-            const int e = ilogb(mm);
-            lg += (double)e * 0.69314718055994530942;
-            for (int idx = l; idx < nt * no; idx += WAVE) Kout[idx] = ldexp(Kout[idx], -e);
+            const int ex = ilogb(mm);
+            lg += (double)ex * 0.69314718055994530942;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ldexp(v[e], -ex);
+        }
+    }
+}
+
+// Walk over a list like quad_walk (same arguments and return value); dl[e] is
+// the propagation to tend of row 4e + l/16, its log factor already in lg.
+template <bool BRA, typename F>
+DEV bool hex_walk(Ctx &c, const Hex &q, double (&v)[4], int &s, double &lg, int no, double tstart,
+                  const double *otau, const int *ocode, int n, double tend, double (&dl)[4], Work &w, F &&after)
+{
+    const double egs = c.M.egs;
+    const int l = lane_id();
+    int ns = c.sz[s], eo = c.off[s];
+    const int nb4 = 4 * c.M.nb;
+    const glb_d *ops = (const glb_d *)c.M.ops;
+    double tlast = tstart;
+    for (int c0 = 0; c0 < n; c0 += QCH) {
+        const int nc = min(QCH, n - c0);
+        // (1) path: record {block offset, target size, source size, source
+        // energies offset}
+        int colv = 0;
+        if (l < nc) {
+            const int cd = ocode[BRA ? n - 1 - (c0 + l) : c0 + l];
+            const int ca = BRA ? 2 - op_ca(cd) : op_ca(cd) - 1;
+            colv = (op_orb(cd) * 2 + op_spin(cd)) * 2 + ca;
+        }
+        for (int kk = 0; kk < nc; ++kk) {
+            const int4 rec = c.tr[s * nb4 + __builtin_amdgcn_readlane(colv, kk)];
+            if (rec.x < 0) return false;
+            c.qrec[kk] = make_int4(rec.z, rec.y, ns, eo);
+            c.qsst[kk] = rec.x;
+            w.op(rec.y, ns, no);
+            s = rec.x;
+            ns = rec.y;
+            eo = rec.w;
         }
         wsync();
+        // (2) propagators: four operators per pass, one state per lane
+        for (int kb = 0; kb < nc; kb += 4) {
+            const int kk = kb + (l >> 4);
+            const bool act = kk < nc;
+            const int kq = act ? kk : kb;
+            const int4 rec = c.qrec[kq];
+            const int idx = BRA ? n - 1 - (c0 + kq) : c0 + kq;
+            const double tj = otau[idx];
+            const double tp = c0 + kq > 0 ? otau[BRA ? idx + 1 : idx - 1] : tstart;
+            const double dt = BRA ? tp - tj : tj - tp;
+            const double e0 = c.ev[rec.w];
+            const int k = l & 15;
+            const bool in = k < rec.z;
+            const double d = in ? exp(-(c.ev[rec.w + (in ? k : 0)] - e0) * dt) : 0.0;
+            if (act) {
+                c.qa[kk * 16 + k] = d;
+                c.qlc[kk] = -(e0 - egs) * dt;
+            }
+        }
+        wsync();
+        // (3) products; block entries are loaded two operators ahead
+        auto entries = [&](int kk, double (&a)[4]) {
+            const int4 rec = c.qrec[kk < nc ? kk : nc - 1];
+            const int off = __builtin_amdgcn_readfirstlane(rec.x), nt = __builtin_amdgcn_readfirstlane(rec.y),
+                      nsk = __builtin_amdgcn_readfirstlane(rec.z);
+            const glb_d *P = ops + off;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = 4 * e + q.lk;
+                if (4 * e < nsk) {
+                    const bool in = q.lr < nt && k < nsk;
+                    const double x = P[in ? q.lr + k * nt : 0];
+                    a[e] = in ? x : 0.0;
+                } else {
+                    a[e] = 0.0;
+                }
+            }
+        };
+        double a0[4], a1[4];
+        entries(0, a0);
+        entries(1, a1);
+        for (int kk = 0; kk < nc; ++kk) {
+            double a2[4];
+            entries(kk + 2, a2);
+            const int4 rec = c.qrec[kk];
+            const int nsk = __builtin_amdgcn_readfirstlane(rec.z);
+            const double *d = c.qa + kk * 16 + q.lk;
+            lg += c.qlc[kk];
+            dbl4 out{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (4 * e < nsk) out = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[e], v[e] * d[4 * e], out, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = out[e];
+                a0[e] = a1[e];
+                a1[e] = a2[e];
+            }
+            hex_renorm(v, lg);
+            after(c0 + kk, v, c.qsst[kk], rec.y, lg);
+        }
+        tlast = otau[BRA ? n - c0 - nc : c0 + nc - 1];
+        wsync();
     }
+    const double dt = BRA ? tlast - tend : tend - tlast;
+    const double e0 = c.ev[eo];
+    lg += -(e0 - egs) * dt;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int r = 4 * e + q.lk;
+        dl[e] = exp(-(c.ev[eo + (r < ns ? r : 0)] - e0) * dt);
+    }
+    return true;
+}
+
+struct HexNoAfter {
+    DEV void operator()(int, const double (&)[4], int, int, double) const {}
+};
+
+// Trace of a ket v (superstate s, log scale lg) against the row-major bra B at
+// the same time: part traces of the outer states to c.pl, the total in (tl, ts)
+DEV void hex_contract(Ctx &c, const Hex &q, const double (&v)[4], const double *B, int s, int no, double lg,
+                      double &tl, double &ts)
+{
+    double b[4];
+    q.load(B, c.sz[s], no, b);
+    double x = (v[0] * b[0] + v[1] * b[1]) + (v[2] * b[2] + v[3] * b[3]);
+    x += __shfl_xor(x, 16, WAVE);
+    x += __shfl_xor(x, 32, WAVE);
+    if (lane_id() < no) {
+        c.pl[2 * lane_id()] = lg + log(fabs(x));
+        c.pl[2 * lane_id() + 1] = copysign(1.0, x);
+    }
+    const double S = wave_sum(lane_id() < 16 ? x : 0.0);
+    if (S == 0.0) {
+        tl = -DBL_MAX;
+        ts = 0.0;
+    } else {
+        tl = lg + log(fabs(S));
+        ts = copysign(1.0, S);
+    }
+    wsync();
 }
 
 // What an operator walk over blocks above 16 states needs, by value (the walk
@@ -900,9 +886,6 @@ DEV void mfma_prop(const MfmaEnv &e, int s, double dt)
         e.dvec[k] = k < ns ? (ns > 1 ? exp(-(E[k] - e0) * dt) : 1.0) : 0.0;
     wsync();
 }
-
-typedef __attribute__((address_space(3))) double lds_d;
-typedef __attribute__((address_space(1))) double glb_d;
 
 // out[tp] (tp < NTP) += P diag(dvec) S over nkt groups of 16 k-steps: P the
 // zero-padded operator block (leading dimension ldp, global), S the LDS strip
@@ -1079,25 +1062,6 @@ __device__ __attribute__((noinline)) MfmaOut walk_mfma(const MfmaEnv e, const do
     return o;
 }
 
-// scale rows by dvec and renormalise (end-of-sweep propagation)
-DEV void scale_rows(Ctx &c, double *K, int ns, int no, double &lg)
-{
-    double m = 0.0;
-    for (int idx = lane_id(); idx < ns * no; idx += WAVE) {
-        double x = K[idx] * c.dvec[idx / no];
-        K[idx] = x;
-        m = fmax(m, fabs(x));
-    }
-    m = wave_max(m);
-    wsync();
-    if (m > 0.0) {
-        double inv = 1.0 / m;
-        lg += log(m);
-        for (int idx = lane_id(); idx < ns * no; idx += WAVE) K[idx] *= inv;
-    }
-    wsync();
-}
-
 DEV MfmaEnv mfma_env(const Ctx &c)
 {
     MfmaEnv e;
@@ -1137,38 +1101,21 @@ DEV bool ket_walk(Ctx &c, double *&K, double *&Kw, int &s, double &lg, int no, d
         wsync();
         return true;
     } else if constexpr (NM <= 16) {
-        // One LDS round trip per operator: the transition record of the next
-        // operator, its target block's energies, the current block entries and
-        // state are read together; operator codes and times two ahead.
-        const LaneSlots<NM> ls(no);
-        double tj = n > 0 ? otau[0] : t1;
-        int cj = n > 0 ? ocode[0] : 0;
-        double tn = n > 1 ? otau[1] : t1;
-        int cn = n > 1 ? ocode[1] : 0;
-        int ns = c.sz[s];
-        double d = prop_e(c, c.ev + c.off[s], ns, tj - t, lg);
-        int4 tr = n > 0 ? c.trans(s, cj, false) : make_int4(0, 0, 0, 0);
-        for (int j = 0; j < n; ++j) {
-            if (tr.x < 0) return w.commit(c), false;
-            const double tnn = j + 2 < n ? otau[j + 2] : t1;
-            const int cnn = j + 2 < n ? ocode[j + 2] : 0;
-            const int4 trn = j + 1 < n ? c.trans(tr.x, cn, false) : make_int4(0, 0, 0, 0);
-            const double dn = prop_e(c, c.ev + tr.w, tr.y, tn - tj, lg);
-            w.op(tr.y, ns, no);
-            apply_small<NM>(c.opsp + tr.z, K, Kw, tr.y, ns, no, d, ls, lg);
-            double *x = K;
-            K = Kw;
-            Kw = x;
-            s = tr.x;
-            ns = tr.y;
-            tr = trn;
-            d = dn;
-            tj = tn;
-            tn = tnn;
-            cj = cn;
-            cn = cnn;
-        }
-        finish_small<NM>(K, ns, no, d, ls, lg);
+        const Hex q;
+        double v[4], d[4];
+        q.load(K, c.sz[s], no, v);
+        const bool ok = hex_walk<false>(c, q, v, s, lg, no, t0, otau, ocode, n, t1, d, w, HexNoAfter());
+        w.commit(c);
+        if (!ok) return false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= d[e];
+        hex_renorm(v, lg);
+        q.store(Kw, c.sz[s], no, v);
+        double *x = K;
+        K = Kw;
+        Kw = x;
+        wsync();
+        return true;
     } else {
         const MfmaOut r = walk_mfma<false>(mfma_env(c), K, Kw, s, no, t, otau, ocode, n, t1);
         mfma_work(c, r, no);
@@ -1205,34 +1152,20 @@ DEV void bra_walk(Ctx &c, double *&B, double *&Bw, int &s, double &lg, int no, d
         wsync();
         return;
     } else if constexpr (NM <= 16) {
-        const LaneSlots<NM> ls(no);
-        double tj = n > 0 ? otau[n - 1] : t0;
-        int cj = n > 0 ? ocode[n - 1] : 0;
-        double tn = n > 1 ? otau[n - 2] : t0;
-        int cn = n > 1 ? ocode[n - 2] : 0;
-        int ns = c.sz[s];
-        double d = prop_e(c, c.ev + c.off[s], ns, t - tj, lg);
-        int4 tr = n > 0 ? c.trans(s, cj, true) : make_int4(0, 0, 0, 0);
-        for (int j = n - 1; j >= 0; --j) {
-            const double tnn = j >= 2 ? otau[j - 2] : t0;
-            const int cnn = j >= 2 ? ocode[j - 2] : 0;
-            const int4 trn = j >= 1 ? c.trans(tr.x, cn, true) : make_int4(0, 0, 0, 0);
-            const double dn = prop_e(c, c.ev + tr.w, tr.y, tj - tn, lg);
-            w.op(tr.y, ns, no);
-            apply_small<NM>(c.opsp + tr.z, B, Bw, tr.y, ns, no, d, ls, lg);
-            double *x = B;
-            B = Bw;
-            Bw = x;
-            s = tr.x;
-            ns = tr.y;
-            tr = trn;
-            d = dn;
-            tj = tn;
-            tn = tnn;
-            cj = cn;
-            cn = cnn;
-        }
-        finish_small<NM>(B, ns, no, d, ls, lg);
+        const Hex q;
+        double v[4], d[4];
+        q.load(B, c.sz[s], no, v);
+        hex_walk<true>(c, q, v, s, lg, no, t1, otau, ocode, n, t0, d, w, HexNoAfter());
+        w.commit(c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= d[e];
+        hex_renorm(v, lg);
+        q.store(Bw, c.sz[s], no, v);
+        double *x = B;
+        B = Bw;
+        Bw = x;
+        wsync();
+        return;
     } else {
         const MfmaOut r = walk_mfma<true>(mfma_env(c), B, Bw, s, no, t, otau, ocode, n, t0);
         mfma_work(c, r, no);
@@ -1470,6 +1403,18 @@ DEV bool window_trace(Ctx &c, int nl, double &tl, double &ts)
         w.commit(c);
         if (!ok || s != c.bndsst[top]) return false;
         quad_contract(c, q, v * d, c.bnd + (long)top * c.nm * c.nm, s, no, lg + c.bndlog[top], tl, ts);
+        return true;
+    } else if constexpr (NM <= 16) {
+        const Hex q;
+        double v[4], d[4];
+        q.load(c.kst, c.sz[s], no, v);
+        Work w;
+        const bool ok = hex_walk<false>(c, q, v, s, lg, no, ta, c.ttau, c.tcode, nl, tb, d, w, HexNoAfter());
+        w.commit(c);
+        if (!ok || s != c.bndsst[top]) return false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= d[e];
+        hex_contract(c, q, v, c.bnd + (long)top * c.nm * c.nm, s, no, lg + c.bndlog[top], tl, ts);
         return true;
     }
     double *K = c.K0, *Kw = c.K1;
@@ -3341,6 +3286,8 @@ DEV Ctx make_ctx(const DevModel &M, const ChainLayout &L, char *base, int chain,
         c.lbx = reinterpret_cast<double *>(lds + L.l_lbx);
         c.rks = reinterpret_cast<int *>(lds + L.l_rks);
         c.lbs = reinterpret_cast<int *>(lds + L.l_lbs);
+    }
+    if constexpr (NM <= 16) {
         c.qa = reinterpret_cast<double *>(lds + L.l_qa);
         c.qlc = reinterpret_cast<double *>(lds + L.l_qlc);
         c.qrec = reinterpret_cast<int4 *>(lds + L.l_qrec);
@@ -3389,10 +3336,6 @@ DEV Ctx make_ctx(const DevModel &M, const ChainLayout &L, char *base, int chain,
     // operator blocks: always LDS for blocks up to 4 states (known at compile
     // time, so the block reads are LDS instructions); LDS or HBM above
     if constexpr (NM <= 4) {
-        double *lops = reinterpret_cast<double *>(lds + L.l_ops);
-        for (long i = lane_id(); i < M.nops; i += WAVE) lops[i] = M.ops[i];
-        c.opsp = lops;
-    } else if (L.l_ops >= 0) {
         double *lops = reinterpret_cast<double *>(lds + L.l_ops);
         for (long i = lane_id(); i < M.nops; i += WAVE) lops[i] = M.ops[i];
         c.opsp = lops;
