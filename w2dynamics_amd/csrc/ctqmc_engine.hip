@@ -91,6 +91,7 @@ long align256(long x) { return (x + 255) / 256 * 256; }
 
 constexpr int KCAP_MAX = 4096;   // pairs per flavour a chain may grow to
 constexpr int ACCPAIR_BINS_MAX = 1024;   // accepted-pair histogram bins (NAccPair) at most, beyond Ntau
+constexpr int SEG_CACHE = 128;           // window operators the segment caches of blocks above 4 states cover
 constexpr int APT_CAP = 65536;           // accepted-pair distances a calibration list holds at most
 constexpr int GIW_NIW_MAX = 1 << 20;     // Matsubara frequencies of MeasGiw at most
 
@@ -218,6 +219,8 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     L.kwork = take(nm > 16 ? 2L * nm * nm * 8 : 8);
     const int nth = h->dm.ntheta;
     L.dwork = take(nth > 0 ? ((4L + 3L * nth) * nm * nm + nm) * 8 : 8);
+    L.grk = take(nm > 4 && nm <= 16 ? (SEG_CACHE + 1) * 2048L : 8);
+    L.glb = take(nm > 4 && nm <= 16 ? (SEG_CACHE + 1) * 2048L : 8);
     L.ltau = take((long)L.lcap * 8);
     L.lcode = take((long)L.lcap * 4);
     L.gtau = take((long)nf * h->ntau * 8);
@@ -261,14 +264,9 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     const int lc = (int)std::min<long>(std::min<long>(L.cap + 2, 1024),
                                        std::max<long>(64, 2L * L.cap / (nwin + 1) + 32));
     L.lcap_lds = lc;
-    L.l_hdr = lds(sizeof(ChainHdr));
     L.l_mt = lds(624 * 4);
     L.l_sz = lds((long)m.nsst * 4);
     L.l_off = lds((long)m.nsst * 4);
-    // Connect and operator-block offsets: LDS for blocks up to 16 states, HBM
-    // above (with them a chain of the 5-orbital model fits 20 KB, eight per CU)
-    L.l_cn = nm <= 16 ? lds((long)m.nsst * m.nbands * 4 * 4) : -1;
-    L.l_oo = nm <= 16 ? lds((long)m.nsst * m.nbands * 4 * 4) : -1;
     // transition records and energies: LDS for blocks up to 16 states, HBM
     // above (there the block products dominate and LDS buys chains per CU)
     L.l_tr = nm <= 16 ? lds((long)m.nsst * m.nbands * 4 * 16) : -1;
@@ -288,19 +286,19 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     L.l_k = nm <= 16 ? lds(2L * nm * nm * 8) : -1;
     L.l_strip = nm > 16 ? lds(128L * 16 * 8) : -1;
     L.l_legc = lds(2L * std::max(h->nleg, 1) * 8);
-    // chunk buffers of the register walks (16 operators)
-    if (nm <= 16) {
-        L.l_qa = lds(16L * 16 * 8);
-        L.l_qlc = lds(16L * 8);
-        L.l_qrec = lds(16L * 16);
-        L.l_qsst = lds(16L * 4);
-    } else {
-        L.l_qa = L.l_qlc = L.l_qrec = L.l_qsst = -1;
-    }
-    L.sc = nm <= 4 ? std::min(64, lc - 2) : 0;
+    // walks on blocks of up to 16 states: superstate keys and records;
+    // propagators of 16 operators
+    L.l_keys = nm <= 16 ? lds(512) : -1;
+    L.l_sinfo = nm <= 16 ? lds(16L * m.nsst) : -1;
+    L.l_qa = nm > 4 && nm <= 16 ? lds(16L * 16 * 8) : -1;
+    // window segment caches: state matrices in LDS for blocks of up to 4
+    // states, in the chain block above (2 KB each)
+    L.sc = nm <= 4 ? std::min(64, lc - 2) : nm <= 16 ? std::min(SEG_CACHE, lc - 2) : 0;
     if (L.sc > 0) {
-        L.l_rk = lds((long)(L.sc + 1) * nm * nm * 8);
-        L.l_lb = lds((long)(L.sc + 1) * nm * nm * 8);
+        if (nm <= 4) {
+            L.l_rk = lds((long)(L.sc + 1) * nm * nm * 8);
+            L.l_lb = lds((long)(L.sc + 1) * nm * nm * 8);
+        }
         L.l_rkx = lds((long)(L.sc + 1) * 8);
         L.l_lbx = lds((long)(L.sc + 1) * 8);
         L.l_rks = lds((long)(L.sc + 1) * 4);
@@ -711,6 +709,46 @@ int group_sums_into(w2d_ctqmc *h, int ngroups, void *work, double *gtau, double 
     return W2D_OK;
 }
 
+// Additive keys of the superstates, key = a N_0 + b N_1 + const with the
+// electron numbers of the two spins: then the superstate behind a string of
+// operators follows from a sum over its operators instead of one transition
+// after the other.  (a, b) = (16, 1) for blocks of both numbers, (1, 1) for
+// blocks of their sum, (1, -1) of their difference; checked against every
+// transition, and 0 is returned for blocks that none of them describes (or
+// refined blocks, several to a key).  keys: key of each superstate [256],
+// superstate of each key [256] (255: none).
+int superstate_keys(const w2d::LocalModel &m, std::vector<unsigned char> &keys)
+{
+    keys.assign(512, 255);
+    if (m.nsst > 255) return 0;
+    const int nb = m.nbands, ab[3][2] = {{16, 1}, {1, 1}, {1, -1}};
+    for (const auto &w : ab) {
+        std::vector<int> key(m.nsst), of(256, -1);
+        bool ok = true;
+        for (int s = 0; s < m.nsst && ok; ++s) {
+            int n0 = 0, n1 = 0;
+            for (int b = 0; b < nb; ++b) {
+                n0 += (m.states[m.offsets[s]] >> b) & 1;
+                n1 += (m.states[m.offsets[s]] >> (nb + b)) & 1;
+            }
+            key[s] = w[0] * n0 + w[1] * n1 + (w[1] < 0 ? nb : 0);
+            ok = key[s] >= 0 && key[s] < 256 && of[key[s]] < 0;
+            if (ok) of[key[s]] = s;
+        }
+        for (int s = 0; s < m.nsst && ok; ++s)
+            for (int o = 0; o < 4 * nb && ok; ++o) {
+                const int t = m.connect[(size_t)s * 4 * nb + o];
+                const int d = w[(o >> 1) & 1] * ((o & 1) ? -1 : 1);
+                ok = t < 0 || key[t] == key[s] + d;
+            }
+        if (!ok) continue;
+        for (int s = 0; s < m.nsst; ++s) keys[s] = (unsigned char)key[s];
+        for (int q = 0; q < 256; ++q) keys[256 + q] = of[q] < 0 ? 255 : (unsigned char)of[q];
+        return (w[0] & 255) | ((w[1] & 255) << 8);
+    }
+    return 0;
+}
+
 // Zero-padded copies of the operator blocks for the MFMA walks (engine for
 // blocks above 16 states): rows and columns padded to multiples of 16,
 // column-major with leading dimension 16 ceil(n_t / 16); offsets indexed like
@@ -902,6 +940,7 @@ int w2d_ctqmc_create(const char *params, int nbands, int nftau, const double *u_
     d.nstates = m.nstates;
     d.nftau = nftau;
     d.beta = h->beta;
+    d.rbeta = 1.0 / h->beta;
     d.egs = m.egs;
     std::vector<double> fdiag((size_t)nf * nftau);
     for (int b = 0; b < nbands; ++b)
@@ -926,9 +965,12 @@ int w2d_ctqmc_create(const char *params, int nbands, int nftau, const double *u_
         legc[2 * l] = (2.0 * l + 1.0) / (double)(l + 1);
         legc[2 * l + 1] = (double)l / (double)(l + 1);
     }
+    std::vector<unsigned char> keys;
+    d.dkey = superstate_keys(m, keys);
+    std::vector<double> opsz(m.ops);   // a zero behind the blocks (rows and columns beyond a block)
+    opsz.push_back(0.0);
     std::vector<int> first_state(m.nsst);
     for (int s = 0; s < m.nsst; ++s) first_state[s] = m.states[m.offsets[s]];
-    std::vector<int> opoff32(m.opoff.begin(), m.opoff.end());
     std::vector<int4> trans(m.connect.size());
     for (size_t i = 0; i < m.connect.size(); ++i) {
         const int ts = m.connect[i];
@@ -938,10 +980,10 @@ int w2d_ctqmc_create(const char *params, int nbands, int nftau, const double *u_
     if ((st = upload(h.get(), m.sizes, &d.sizes)) || (st = upload(h.get(), m.offsets, &d.offsets)) ||
         (st = upload(h.get(), m.connect, &d.connect)) || (st = upload(h.get(), first_state, &d.first_state)) ||
         (st = upload(h.get(), m.state_sst, &d.state_sst)) || (st = upload(h.get(), m.opoff, &d.opoff)) ||
-        (st = upload(h.get(), m.ops, &d.ops)) || (st = upload(h.get(), m.evals, &d.evals)) ||
+        (st = upload(h.get(), opsz, &d.ops)) || (st = upload(h.get(), m.evals, &d.evals)) ||
         (st = upload(h.get(), fdiag, &d.ftau)) || (st = upload(h.get(), dmoff, &d.dmoff)) ||
         (st = upload(h.get(), legc, &d.legc)) || (st = upload(h.get(), trans, &d.trans)) ||
-        (st = upload(h.get(), opoff32, &d.opoff32)) || (h->nm > 16 && (st = build_ops16(h.get()))))
+        (st = upload(h.get(), keys, &d.keys)) || (h->nm > 16 && (st = build_ops16(h.get()))))
         return st;
     // user symmetry moves (Trace.F90:471-478): SymMove01.. are 1-based
     // flavour permutations; their inverses follow in the table

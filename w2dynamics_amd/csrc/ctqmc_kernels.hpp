@@ -24,6 +24,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/w2dyn_ctqmc.h"
 #include "engine.hpp"
@@ -36,6 +37,19 @@ namespace w2d {
 // wave helpers (one wavefront per block)
 // ---------------------------------------------------------------------------
 DEV int lane_id() { return (int)threadIdx.x; }
+
+typedef __attribute__((address_space(3))) char lds_c;
+typedef __attribute__((address_space(3))) unsigned char lds_b;
+typedef __attribute__((address_space(3))) double lds_d;
+typedef __attribute__((address_space(3))) int lds_i;
+typedef __attribute__((address_space(3))) unsigned lds_u;
+
+DEV int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <typename T>
+DEV T *uni_lds(T *p)
+{
+    return (T *)(size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)p);
+}
 
 // Cross-lane reductions with DPP row operations (VALU, no LDS traffic): quad
 // permutes and row mirrors reduce each 16-lane row, readlane combines the four
@@ -101,15 +115,49 @@ DEV int wave_imax(int v)
 
 DEV int wave_imin(int v) { return -wave_imax(-v); }
 
-DEV int wave_excl_scan(int v, int *total)
+// Inclusive scans over the lanes: shifts by 1, 2, 4, 8 within the 16-lane
+// rows, then the rows' last lanes broadcast to the rows behind (six VALU steps,
+// no LDS traffic).
+template <int CTRL, int ROWS>
+DEV int dpp_mov_i(int old, int v)
 {
-    int x = v;
-    for (int o = 1; o < WAVE; o <<= 1) {
-        int y = __shfl_up(x, o, WAVE);
-        if (lane_id() >= o) x += y;
-    }
-    *total = __shfl(x, WAVE - 1, WAVE);
-    return x - v;
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+DEV double dpp_mov_d(double old, double v)
+{
+    return __hiloint2double(dpp_mov_i<CTRL, ROWS>(__double2hiint(old), __double2hiint(v)),
+                            dpp_mov_i<CTRL, ROWS>(__double2loint(old), __double2loint(v)));
+}
+DEV int wave_scan_i(int x)
+{
+    x += dpp_mov_i<0x111, 0xf>(0, x);
+    x += dpp_mov_i<0x112, 0xf>(0, x);
+    x += dpp_mov_i<0x114, 0xf>(0, x);
+    x += dpp_mov_i<0x118, 0xf>(0, x);
+    x += dpp_mov_i<0x142, 0xa>(0, x);
+    x += dpp_mov_i<0x143, 0xc>(0, x);
+    return x;
+}
+DEV double wave_scan_d(double x)
+{
+    x += dpp_mov_d<0x111, 0xf>(0.0, x);
+    x += dpp_mov_d<0x112, 0xf>(0.0, x);
+    x += dpp_mov_d<0x114, 0xf>(0.0, x);
+    x += dpp_mov_d<0x118, 0xf>(0.0, x);
+    x += dpp_mov_d<0x142, 0xa>(0.0, x);
+    x += dpp_mov_d<0x143, 0xc>(0.0, x);
+    return x;
+}
+DEV double wave_scan_mul(double x)
+{
+    x *= dpp_mov_d<0x111, 0xf>(1.0, x);
+    x *= dpp_mov_d<0x112, 0xf>(1.0, x);
+    x *= dpp_mov_d<0x114, 0xf>(1.0, x);
+    x *= dpp_mov_d<0x118, 0xf>(1.0, x);
+    x *= dpp_mov_d<0x142, 0xa>(1.0, x);
+    x *= dpp_mov_d<0x143, 0xc>(1.0, x);
+    return x;
 }
 
 // hardware FP64 add to device (global) memory, result unused
@@ -131,8 +179,10 @@ DEV void wsync() { __syncthreads(); }
 // shared in LDS; every lane draws the same numbers, the twist is lane-parallel.
 // ---------------------------------------------------------------------------
 struct Rng {
-    uint32_t *mt;   // LDS
-    int *idx;       // LDS (uniform)
+    lds_u *mt;      // LDS
+    int *idx;       // LDS (uniform): next word, kept there between open and close
+    uint32_t w;     // lane l: tempered word base + l
+    int pos, base, lim;
 };
 
 DEV uint32_t mt_twist_word(uint32_t a, uint32_t b, uint32_t c)
@@ -145,8 +195,9 @@ DEV uint32_t mt_twist_word(uint32_t a, uint32_t b, uint32_t c)
 
 // new mt[i] depends on mt[i+1] (old) and mt[i+397]: old for i < 227, new for
 // i >= 227 (from index i-227).  Phases [0,227) [227,454) [454,623) {623}.
-DEV void mt_regen(uint32_t *mt)
+__device__ __attribute__((noinline)) void mt_regen(lds_u *mt_)
 {
+    lds_u *mt = uni_lds(mt_);
     const int l = lane_id();
     uint32_t nv[4];
     int c = 0;
@@ -182,38 +233,53 @@ DEV uint32_t mt_temper(uint32_t y)
     return y;
 }
 
+DEV void rng_open(Rng &r)
+{
+    r.pos = uni(*r.idx);
+    r.base = r.lim = -1;
+}
+DEV void rng_close(Rng &r) { *r.idx = r.pos; }
+
+// The next word.  64 words at a time are tempered, one per lane, and handed out
+// by readlane: a draw is a few scalar instructions instead of an LDS round
+// trip for the position, one for the word and the tempering.
 DEV uint32_t mt_next(Rng &r)
 {
-    int i = *r.idx;
-    if (i >= 624) {
-        mt_regen(r.mt);
-        i = 0;
+    if (r.pos >= r.lim) {
+        if (r.pos >= 624) {
+            mt_regen(r.mt);
+            r.pos = 0;
+        }
+        r.base = r.pos;
+        r.lim = min(r.base + WAVE, 624);
+        r.w = mt_temper(r.mt[min(r.base + lane_id(), 623)]);
     }
-    const uint32_t y = r.mt[i];
-    *r.idx = i + 1;   // all lanes store the same value
-    return mt_temper(y);
+    return (uint32_t)__builtin_amdgcn_readlane((int)r.w, r.pos++ - r.base);
 }
 
-// generate_canonical<double,53>: (g1 + g2 2^32) / 2^64, clamped below 1.  The
-// two words are read together when both are left in the current block.
+// generate_canonical<double,53>: (g1 + g2 2^32) / 2^64, clamped below 1
 DEV double grnd(Rng &r)
 {
-    const int i = *r.idx;
-    uint32_t g1, g2;
-    if (i + 2 <= 624) {
-        g1 = mt_temper(r.mt[i]);
-        g2 = mt_temper(r.mt[i + 1]);
-        *r.idx = i + 2;
-    } else {
-        g1 = mt_next(r);
-        g2 = mt_next(r);
-    }
-    double sum = (double)g1;
+    const uint32_t g1 = mt_next(r), g2 = mt_next(r);
     const double tmp = 4294967296.0;
-    sum = __dadd_rn(sum, __dmul_rn((double)g2, tmp));
+    double sum = __dadd_rn((double)g1, __dmul_rn((double)g2, tmp));
     double ret = sum / (tmp * tmp);
     if (ret >= 1.0) ret = 0x1.fffffffffffffp-1;
     return ret;
+}
+
+// draws of a function: the position comes from and goes back to LDS
+struct RngScope {
+    Rng &r;
+    DEV explicit RngScope(Rng &x) : r(x) { rng_open(r); }
+    DEV ~RngScope() { rng_close(r); }
+};
+
+// a draw whose value is not used
+DEV void grnd_skip(Rng &r)
+{
+    (void)mt_next(r);
+    (void)mt_next(r);
 }
 
 DEV int randint(Rng &r, int a, int b)
@@ -242,15 +308,64 @@ DEV int mk_code(int orb, int spin, int ca) { return orb | (spin << 4) | ((ca - 1
 // ---------------------------------------------------------------------------
 // chain context: LDS views of the header, model tables and work buffers
 // ---------------------------------------------------------------------------
+// The kernels' model and layout arguments, read where they lie (constant
+// address space: scalar loads), also by functions that are not inlined.
+typedef const __attribute__((address_space(4))) DevModel CModel;
+typedef const __attribute__((address_space(4))) ChainLayout CLayout;
+typedef __attribute__((address_space(1))) char glb_c;
+typedef const __attribute__((address_space(4))) char *CArgs;   // a kernel's arguments: model, layout, ...
+typedef int iv4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) iv4 lds_i4;
+typedef __attribute__((address_space(1))) double glb_d;
+
+// What identifies a chain: the parts of a sweep that are rarely or seldom
+// taken (boundary caches, accepted moves, global moves, measurements) are
+// functions of their own, so that the loop over proposals stays small and has
+// its registers to itself; each rebuilds its view of the chain from this.
+struct ChainRef {
+    CModel *M;
+    CLayout *L;
+    char *base;
+};
+
+// What the out-of-line functions share of a chain, in LDS.
+struct WalkEnv {
+    double egs;
+    double flops, bytes;    // algorithmic work of this launch
+    const double *ops;      // operator blocks in global memory, a zero behind the last
+    const lds_i4 *tr;       // transition records
+    const lds_d *ev;        // energies
+    const lds_b *keys;      // key of each superstate, then the superstate of each key (255: none)
+    const lds_d *lops;      // operator blocks in LDS (blocks up to 4 states)
+    const lds_i4 *sinfo;    // per superstate: lowest energy, size | first energy << 8, width (float)
+    lds_d *qa;              // propagators of 16 operators (blocks of 5..16 states); scratch
+    lds_c *dyn;             // dynamic LDS
+    int ncol;               // operators per superstate (4 nb)
+    int dkey;               // key change by a creator of spin 0 | of spin 1 << 8; 0: no such keys
+    int np, full;           // removable pairs of the window; no room for another pair
+    int zero;               // offset of the zero behind the operator table
+    int nkmax;              // matrix-instruction steps of the largest block
+    int swapped;            // the trial list's buffer is the window list
+};
+__shared__ WalkEnv s_wenv;
+__shared__ ChainHdr s_hdr;
+
+DEV unsigned long long uni64(unsigned long long a)
+{
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)a),
+                   hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(a >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+DEV const glb_d *uni_glb(const double *p) { return (const glb_d *)uni64((unsigned long long)p); }
+
 struct Ctx {
-    const DevModel &M;
-    const ChainLayout &L;
+    CModel &M;
+    CLayout &L;
     char *base;          // chain block in global memory
-    ChainHdr *ghdr;      // the chain's header in the contiguous header array (HBM)
     ChainHdr &h;         // LDS copy
     Rng rng;
     // model tables (LDS)
-    const int *sz, *off, *cn, *oo;
+    const int *sz, *off;
     const int4 *tr;      // per (superstate, operator): target, target size, block offset, target energies offset
     const double *ev, *opsp;   // opsp: operator blocks (LDS or global)
     // chain arrays (global)
@@ -272,47 +387,114 @@ struct Ctx {
     // bras lb[m] (after the last m), with their logs and superstates (LDS)
     double *rk, *lb, *rkx, *lbx;
     int *rks, *lbs;
-    // quad-walk chunk buffers (LDS): entries, path records, targets, log factors
-    double *qa, *qlc;
-    int4 *qrec;
-    int *qsst;
     const double *legc;  // Legendre recursion coefficients (LDS)
     int nm;              // padded block size used for matrix strides
-    // algorithmic work of this launch, added to the header by save_ctx
-    double wflops = 0.0, wbytes = 0.0;
-    DEV Ctx(const DevModel &m, const ChainLayout &l, char *b, ChainHdr &hd) : M(m), L(l), base(b), h(hd) {}
+    DEV Ctx(CModel &m, CLayout &l, char *b) : M(m), L(l), base(b), h(s_hdr) {}
+    // algorithmic work, added to the header by save_ctx
+    DEV void work(double flops, double bytes)
+    {
+        s_wenv.flops += flops;
+        s_wenv.bytes += bytes;
+    }
+    DEV ChainRef ref() const { return ChainRef{&M, &L, base}; }
+    // window list and trial list of the chain (their buffers swap)
+    DEV void lists()
+    {
+        const bool sw = uni(s_wenv.swapped) != 0;
+        lds_c *lds = uni_lds(s_wenv.dyn);
+        wtau = (double *)(lds_d *)(lds + (sw ? L.l_ttau : L.l_wtau));
+        ttau = (double *)(lds_d *)(lds + (sw ? L.l_wtau : L.l_ttau));
+        wcode = (int *)(lds_i *)(lds + (sw ? L.l_tcode : L.l_wcode));
+        tcode = (int *)(lds_i *)(lds + (sw ? L.l_wcode : L.l_tcode));
+    }
     DEV double *mi(int f) { return minv + (long)f * L.kcap * L.kcap; }
     DEV int fl(int c) const { return op_orb(c) + M.nb * op_spin(c); }
     DEV int conn(int s, int c, bool adjoint) const
     {
         int ca = op_ca(c);
         if (adjoint) ca = 3 - ca;
-        return cn[((s * M.nb + op_orb(c)) * 2 + op_spin(c)) * 2 + (ca - 1)];
-    }
-    DEV int4 trans(int s, int c, bool adjoint) const
-    {
-        int ca = op_ca(c);
-        if (adjoint) ca = 3 - ca;
-        return tr[((s * M.nb + op_orb(c)) * 2 + op_spin(c)) * 2 + (ca - 1)];
-    }
-    DEV const double *opblock(int s, int c, bool adjoint) const
-    {
-        int ca = op_ca(c);
-        if (adjoint) ca = 3 - ca;
-        return opsp + oo[((s * M.nb + op_orb(c)) * 2 + op_spin(c)) * 2 + (ca - 1)];
+        return tr[((s * M.nb + op_orb(c)) * 2 + op_spin(c)) * 2 + (ca - 1)].x;
     }
 };
 
+// The chain's view: chain block in global memory and the dynamic LDS.
+template <int NM>
+DEV Ctx attach(ChainRef r)
+{
+    CModel &M = *(CModel *)uni64((unsigned long long)r.M);
+    CLayout &L = *(CLayout *)uni64((unsigned long long)r.L);
+    char *base = (char *)(glb_c *)uni64((unsigned long long)r.base);
+    Ctx c(M, L, base);
+    c.nm = NM;
+    c.tau = reinterpret_cast<double *>(base + L.tau);
+    c.code = reinterpret_cast<int *>(base + L.code);
+    c.fc = reinterpret_cast<double *>(base + L.fc);
+    c.fa = reinterpret_cast<double *>(base + L.fa);
+    c.fcs = reinterpret_cast<int *>(base + L.fcs);
+    c.fas = reinterpret_cast<int *>(base + L.fas);
+    c.minv = reinterpret_cast<double *>(base + L.minv);
+    c.scratch = reinterpret_cast<double *>(base + L.scratch);
+    c.kst = reinterpret_cast<double *>(base + L.kst);
+    c.bnd = reinterpret_cast<double *>(base + L.bnd);
+    c.bndlog = reinterpret_cast<double *>(base + L.bndlog);
+    c.bndsst = reinterpret_cast<int *>(base + L.bndsst);
+    c.part = reinterpret_cast<double *>(base + L.part);
+    lds_c *lds = uni_lds(s_wenv.dyn);
+    auto ld = [&](long o) { return (double *)(lds_d *)(lds + o); };
+    auto li = [&](long o) { return (int *)(lds_i *)(lds + o); };
+    c.lists();
+    c.pc = li(L.l_pc);
+    c.dvec = ld(L.l_dvec);
+    c.Q = ld(L.l_q);
+    c.R = ld(L.l_r);
+    c.colb = ld(L.l_col);
+    c.rowb = ld(L.l_row);
+    c.pl = ld(L.l_pl);
+    if constexpr (NM <= 16) {
+        c.rk = NM <= 4 ? ld(L.l_rk) : reinterpret_cast<double *>(base + L.grk);
+        c.lb = NM <= 4 ? ld(L.l_lb) : reinterpret_cast<double *>(base + L.glb);
+        c.rkx = ld(L.l_rkx);
+        c.lbx = ld(L.l_lbx);
+        c.rks = li(L.l_rks);
+        c.lbs = li(L.l_lbs);
+    }
+    c.legc = ld(L.l_legc);
+    // work matrices: LDS for blocks up to 16 states (decided at compile time so
+    // that their accesses are LDS instructions, not generic ones), HBM above
+    if constexpr (NM <= 16) c.K0 = ld(L.l_k);
+    else c.K0 = reinterpret_cast<double *>(base + L.kwork);
+    c.K1 = c.K0 + (long)NM * NM;
+    c.strip = NM > 16 ? ld(L.l_strip) : nullptr;
+    c.sz = li(L.l_sz);
+    c.off = li(L.l_off);
+    // transition records and energies: LDS for blocks up to 16 states
+    if constexpr (NM <= 16) {
+        c.tr = (const int4 *)(const void *)(lds_i4 *)(lds + L.l_tr);
+        c.ev = ld(L.l_ev);
+    } else {
+        c.tr = M.trans;
+        c.ev = M.evals;
+    }
+    // operator blocks: LDS for blocks up to 4 states
+    c.opsp = NM <= 4 ? ld(L.l_ops) : M.ops;
+    c.rng.mt = (lds_u *)(lds + L.l_mt);
+    c.rng.idx = &s_hdr.mti;
+    return c;
+}
+
 // get_HybrF (Trace.F90:1014-1033)
-DEV double hybr(const DevModel &M, double tau, int f)
+DEV double hybr(CModel &M, double tau, int f)
 {
     double sig = 1.0;
     if (tau < 0.0) {
         tau = tau + M.beta;
         sig = -1.0;
     }
-    double n = tau / M.beta * (double)(M.nftau - 1);
-    int i = (int)n;
+    // tau / beta by the reciprocal and one correction step
+    double q = tau * M.rbeta;
+    q = fma(fma(-q, M.beta, tau), M.rbeta, q);
+    const double n = q * (double)(M.nftau - 1);
+    const int i = (int)n;
     const double *F = M.ftau + (long)f * M.nftau;
     return sig * (F[i] + (n - (double)i) * (F[i + 1] - F[i]));
 }
@@ -393,36 +575,64 @@ DEV bool ensure_window(Ctx &c)
 // the trial list becomes the window list (after an accepted add / remove)
 DEV void swap_lists(Ctx &c)
 {
-    double *t = c.wtau;
-    c.wtau = c.ttau;
-    c.ttau = t;
-    int *k = c.wcode;
-    c.wcode = c.tcode;
-    c.tcode = k;
+    s_wenv.swapped ^= 1;
+    c.lists();
 }
 
 // ---------------------------------------------------------------------------
 // local trace
 // ---------------------------------------------------------------------------
-// algorithmic work of one operator application on `no` outer states: a
-// (nt x ns) block times an (ns x no) state matrix plus the diagonal propagator;
-// bytes = states in and out (the operator blocks are shared by all chains and
-// charged once per launch by the host).  Accumulated in registers during a
-// walk and added to the chain header once.
-struct Work {
-    long long ntns = 0, nss = 0, nts = 0;
-    int nout = 0;
-    DEV void op(int nt, int ns, int no)
+// ---------------------------------------------------------------------------
+// Walks on blocks of at most 16 states (trace engines 1, 4 and 16).
+//
+// A state matrix (rows: states of the current block, columns: outer states)
+// lives in registers in the layout that the FP64 matrix instructions both read
+// as operand B and write as D, so an operator K' = A (d o K) never moves data:
+//   blocks up to 4:  entry (l/16, l%4) in lane l, the four quads (l/4)%4 of a
+//     16-lane row being the four blocks of v_mfma_f64_4x4x4f64;
+//   blocks up to 16: entries (4e + l/16, l%16), e = 0..3, i.e. register e is
+//     operand B of k-step e of v_mfma_f64_16x16x4f64.
+// Rows and columns beyond the block are zero.
+// ---------------------------------------------------------------------------
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+constexpr int DPP_ROW_ROR4 = 0x124, DPP_ROW_ROR8 = 0x128;
+
+template <int NM>
+struct State {
+    static constexpr int NV = NM <= 4 ? 1 : 4;
+    double v[NV];
+    DEV static int row(int e) { return NM <= 4 ? lane_id() >> 4 : 4 * e + (lane_id() >> 4); }
+    DEV static int col() { return NM <= 4 ? lane_id() & 3 : lane_id() & 15; }
+    // row-major (ns x no) matrix
+    template <typename P>
+    DEV void load(P K, int ns, int no)
     {
-        ntns += nt * ns;
-        nss += ns;
-        nts += nt;
-        nout = no;
+#pragma unroll
+        for (int e = 0; e < NV; ++e) {
+            const bool in = row(e) < ns && col() < no;
+            const double x = K[in ? row(e) * no + col() : 0];
+            v[e] = in ? x : 0.0;
+        }
     }
-    DEV void commit(Ctx &c) const
+    template <typename P>
+    DEV void store(P K, int ns, int no) const
     {
-        c.wflops += (double)(nout * (2 * ntns + nss));
-        c.wbytes += (double)(8LL * nout * (nss + nts));
+#pragma unroll
+        for (int e = 0; e < NV; ++e)
+            if (row(e) < ns && col() < no && (NM > 4 || (lane_id() & 12) == 0)) K[row(e) * no + col()] = v[e];
+    }
+    DEV void identity(int no)
+    {
+#pragma unroll
+        for (int e = 0; e < NV; ++e) v[e] = row(e) == col() && col() < no ? 1.0 : 0.0;
+    }
+    // largest modulus; `on`: the lanes that count
+    DEV double maxabs() const
+    {
+        double m = fabs(v[0]);
+#pragma unroll
+        for (int e = 1; e < NV; ++e) m = fmax(m, fabs(v[e]));
+        return m;
     }
 };
 
@@ -431,419 +641,301 @@ struct Work {
 // so skipping it changes no rounding).
 constexpr double STATE_TINY = 0x1p-64, STATE_HUGE = 0x1p64;
 
-// ---------------------------------------------------------------------------
-// Walks on blocks of at most 4 states, in registers.  The (ns x no) state is
-// zero-padded to 4 x 4 and lane l holds its entry (r, i) = ((l / 4) % 4, l % 4);
-// the four 16-lane rows of the wave hold the same matrix.  An operator scales
-// row r by the propagator factor of state r (each lane its own), then forms
-// K'(r, i) = sum_k P(r, k) Kd(k, i): rotations of a 16-lane row by 4, 8 and 12
-// lanes (DPP) bring Kd(k, i) of the other three rows to lane (r, i).  Operator
-// entries and energies are each lane's own LDS reads, issued one operator
-// ahead; no state leaves registers and no barrier is taken per operator.
-// ---------------------------------------------------------------------------
-constexpr int DPP_ROW_ROR4 = 0x124, DPP_ROW_ROR8 = 0x128, DPP_ROW_ROR12 = 0x12C;
-
-struct Quad {
-    int r, i;    // entry held by this lane
-    int k[4];    // row of the entry that the rotation by 4m lanes brings here (k[0] = r)
-    DEV Quad()
-    {
-        const int l = lane_id() & 15;
-        r = l >> 2;
-        i = l & 3;
-        k[0] = r;
-        k[1] = dpp_i<DPP_ROW_ROR4>(r);
-        k[2] = dpp_i<DPP_ROW_ROR8>(r);
-        k[3] = dpp_i<DPP_ROW_ROR12>(r);
-    }
-    // entry of a row-major (ns x no) state, 0 outside
-    DEV double load(const double *K, int ns, int no) const
-    {
-        const bool in = r < ns && i < no;
-        const double x = K[in ? r * no + i : 0];
-        return in ? x : 0.0;
-    }
-    DEV void store(double *K, int ns, int no, double v) const
-    {
-        if (lane_id() < 16 && r < ns && i < no) K[r * no + i] = v;
-    }
-    // P(r, k[m]) of an (nt x ns) column-major block; zeros for a record
-    // without target
-    DEV void entries(const double *ops, int4 tr, int ns, double (&p)[4]) const
-    {
-        const double *P = ops + (tr.x >= 0 ? tr.z : 0);
-        const int nt = tr.x >= 0 ? tr.y : 0;
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const bool in = r < nt && k[m] < ns;
-            const double x = P[in ? r + k[m] * nt : 0];
-            p[m] = in ? x : 0.0;
-        }
-    }
-    // exp(-(E_r - E_0) dt) of this lane's row in a block of energies E (1
-    // beyond the block); the common log factor -(E_0 - Egs) dt is returned in lc
-    DEV double prop(const double *E, int ns, double dt, double egs, double &lc) const
-    {
-        const double e0 = E[0];
-        const double er = E[r < ns ? r : 0];
-        lc = -(e0 - egs) * dt;
-        return exp(-(er - e0) * dt);
-    }
-};
-
-// one operator on a quad state with this lane's entries p[m] = A(r, k[m]) of
-// A = P diag(d); power-of-two renormalisation when the largest entry leaves
-// [2^-64, 2^64]
-DEV double quad_apply(double v, const double (&p)[4], double &lg)
+// power-of-two renormalisation when the largest entry of the lanes in `mask`
+// leaves [2^-64, 2^64]
+template <int NM>
+DEV void renorm(State<NM> &k, unsigned long long mask, double &lg)
 {
-    const double x1 = dpp_d<DPP_ROW_ROR4>(v), x2 = dpp_d<DPP_ROW_ROR8>(v), x3 = dpp_d<DPP_ROW_ROR12>(v);
-    double w = fma(p[1], x1, p[0] * v) + fma(p[3], x3, p[2] * x2);
-    const double m = fabs(w);
-    if (__ballot(m >= STATE_TINY) == 0ull || __ballot(m > STATE_HUGE) != 0ull) {
-        const double mm = wave_max(m);
-        if (mm > 0.0) {
-            const int e = ilogb(mm);
-            lg += (double)e * 0.69314718055994530942;
-            w = ldexp(w, -e);
-        }
-    }
-    return w;
-}
-
-// final propagation (lane factor d); renormalised by a power of two only when
-// the largest entry leaves [2^-64, 2^64]
-DEV double quad_finish(double v, double d, double &lg)
-{
-    v *= d;
-    const double m = fabs(v);
-    if (__ballot(m >= STATE_TINY) == 0ull || __ballot(m > STATE_HUGE) != 0ull) {
-        const double mm = wave_max(m);
-        if (mm > 0.0) {
-            const int e = ilogb(mm);
-            lg += (double)e * 0.69314718055994530942;
-            v = ldexp(v, -e);
-        }
-    }
-    return v;
-}
-
-// Trace of a quad ket v (superstate s, log scale lg) against the row-major
-// bra B at the same time: column sums by row rotations, part traces of the
-// outer states to c.pl, the total in (tl, ts) (the plain sum of the columns:
-// every column carries the same scale exp(lg)).
-DEV void quad_contract(Ctx &c, const Quad &q, double v, const double *B, int s, int no, double lg, double &tl,
-                       double &ts)
-{
-    const double x = v * q.load(B, c.sz[s], no);
-    const double col = (x + dpp_d<DPP_ROW_ROR8>(x)) + (dpp_d<DPP_ROW_ROR4>(x) + dpp_d<DPP_ROW_ROR12>(x));
-    if (lane_id() < no) {
-        c.pl[2 * lane_id()] = lg + log(fabs(col));
-        c.pl[2 * lane_id() + 1] = copysign(1.0, col);
-    }
-    const double S = (readlane_d(col, 0) + readlane_d(col, 1)) + (readlane_d(col, 2) + readlane_d(col, 3));
-    if (S == 0.0) {
-        tl = -DBL_MAX;
-        ts = 0.0;
-    } else {
-        tl = lg + log(fabs(S));
-        ts = copysign(1.0, S);
-    }
-    wsync();
-}
-
-constexpr int QCH = 16;   // operators per chunk of a quad walk
-
-// Walk over the n operators of a list: ascending from entry 0 (ket, times
-// tstart < tau_0 < ... < tend) or, with BRA, descending from entry n-1 with the
-// adjoint blocks (tstart > tau_{n-1} > ... > tend).  In chunks of QCH
-// operators: (1) the superstate path, one transition record per operator
-// (uniform; stops at an operator without target block); (2) the entries
-// A(r, k) = P(r, k) exp(-(E_k - E_0) dt) of each operator's block with its
-// propagator, four operators per pass over the wave, one exp per lane, into
-// LDS; (3) the products in registers.  after(k, v, s, ns, lg) sees the state
-// after the k-th operator walked, at that operator's time.  Returns false at a
-// quantum-number violation; otherwise dlast holds the lane factor of the
-// propagation to tend (its log factor already in lg).
-template <bool BRA, typename F>
-DEV bool quad_walk(Ctx &c, const Quad &q, double &v, int &s, double &lg, int no, double tstart, const double *otau,
-                   const int *ocode, int n, double tend, double &dlast, Work &w, F &&after)
-{
-    const double egs = c.M.egs;
-    const int l = lane_id();
-    // pass (2): lane l computes entry (r, m) = (q.r, q.i), i.e. A(r, k[m])
-    const int km = q.i == 0 ? q.k[0] : q.i == 1 ? q.k[1] : q.i == 2 ? q.k[2] : q.k[3];
-    int ns = c.sz[s], eo = c.off[s];
-    const int nb4 = 4 * c.M.nb;
-    double tlast = tstart;
-    for (int c0 = 0; c0 < n; c0 += QCH) {
-        const int nc = min(QCH, n - c0);
-        // (1) path: record {block offset, target size, source size, source
-        // energies offset}; lane kk decodes the column of operator kk first
-        int colv = 0;
-        if (l < nc) {
-            const int cd = ocode[BRA ? n - 1 - (c0 + l) : c0 + l];
-            const int ca = BRA ? 2 - op_ca(cd) : op_ca(cd) - 1;
-            colv = (op_orb(cd) * 2 + op_spin(cd)) * 2 + ca;
-        }
-        for (int kk = 0; kk < nc; ++kk) {
-            const int4 rec = c.tr[s * nb4 + __builtin_amdgcn_readlane(colv, kk)];
-            if (rec.x < 0) return false;
-            c.qrec[kk] = make_int4(rec.z, rec.y, ns, eo);
-            c.qsst[kk] = rec.x;
-            w.op(rec.y, ns, no);
-            s = rec.x;
-            ns = rec.y;
-            eo = rec.w;
-        }
-        wsync();
-        // (2) entries of the chunk's operators
-        for (int kb = 0; kb < nc; kb += 4) {
-            const int kk = kb + (l >> 4);
-            const bool act = kk < nc;
-            const int kq = act ? kk : kb;
-            const int4 rec = c.qrec[kq];
-            const int j = c0 + kq;
-            const int idx = BRA ? n - 1 - j : j;
-            const double tj = otau[idx];
-            const double tp = j > 0 ? otau[BRA ? idx + 1 : idx - 1] : tstart;
-            const double dt = BRA ? tp - tj : tj - tp;
-            const double e0 = c.ev[rec.w];
-            const bool kin = km < rec.z;
-            const double ek = c.ev[rec.w + (kin ? km : 0)];
-            const bool in = kin && q.r < rec.y;
-            const double pv = c.opsp[in ? rec.x + q.r + km * rec.y : 0];
-            const double a = in ? pv * exp(-(ek - e0) * dt) : 0.0;
-            if (act) {
-                c.qa[kk * 16 + (l & 15)] = a;
-                c.qlc[kk] = -(e0 - egs) * dt;
-            }
-        }
-        wsync();
-        // (3) products; the next operator's entries, log factor and target
-        // are read one operator ahead
-        const double *pa = c.qa + q.r * 4;
-        double p[4] = {pa[0], pa[1], pa[2], pa[3]};
-        double lcv = c.qlc[0];
-        int sv = c.qsst[0], ntv = c.qrec[0].y;
-        for (int kk = 0; kk < nc; ++kk) {
-            const int kn = kk + 1 < nc ? kk + 1 : kk;
-            const double pn[4] = {pa[kn * 16], pa[kn * 16 + 1], pa[kn * 16 + 2], pa[kn * 16 + 3]};
-            const double lcn = c.qlc[kn];
-            const int svn = c.qsst[kn], ntn = c.qrec[kn].y;
-            lg += lcv;
-            v = quad_apply(v, p, lg);
-            after(c0 + kk, v, sv, ntv, lg);
-#pragma unroll
-            for (int m = 0; m < 4; ++m) p[m] = pn[m];
-            lcv = lcn;
-            sv = svn;
-            ntv = ntn;
-        }
-        tlast = otau[BRA ? n - c0 - nc : c0 + nc - 1];
-        wsync();
-    }
-    double lc;
-    dlast = q.prop(c.ev + eo, ns, BRA ? tlast - tend : tend - tlast, egs, lc);
-    lg += lc;
-    return true;
-}
-
-struct NoAfter {
-    DEV void operator()(int, double, int, int, double) const {}
-};
-
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) double lds_d;
-typedef __attribute__((address_space(1))) double glb_d;
-
-// ---------------------------------------------------------------------------
-// Walks on blocks of 5 to 16 states, in registers, on the FP64 matrix cores.
-// The (ns x no) state is zero-padded to 16 x 16; lane l holds its entries
-// (4e + l/16, l%16), e = 0..3.  That is the output layout of
-// v_mfma_f64_16x16x4f64 and, register e taken as B(l/16, l%16), also the
-// operand layout of its k-step e: an operator is
-//   K' = sum_e A_e (d o K_e),  A_e(l%16, l/16) = P(l%16, 4e + l/16),
-// ceil(ns/4) chained matrix instructions, and the state never leaves its
-// registers.  Block entries come from the operator table in global memory (the
-// same 29 KB for every chain of the 3-orbital model: L1/L2 hits), two operators
-// ahead; the propagators of QCH operators are computed 64 at a time into LDS.
-// Bound by the latency of the operator chain (one wave per chain).  512 chains
-// of the 3-orbital model at beta = 100: 17.5 ms per 200 moves; per-lane dot
-// products with both matrices in LDS took 60 ms (9000 cycles per operator).
-// ---------------------------------------------------------------------------
-struct Hex {
-    int lr, lk;
-    DEV Hex() : lr(lane_id() & 15), lk(lane_id() >> 4) {}
-    DEV void load(const double *K, int ns, int no, double (&v)[4]) const
-    {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int r = 4 * e + lk;
-            const bool in = r < ns && lr < no;
-            const double x = K[in ? r * no + lr : 0];
-            v[e] = in ? x : 0.0;
-        }
-    }
-    DEV void store(double *K, int ns, int no, const double (&v)[4]) const
-    {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int r = 4 * e + lk;
-            if (r < ns && lr < no) K[r * no + lr] = v[e];
-        }
-    }
-};
-
-// power-of-two renormalisation when the largest entry leaves [2^-64, 2^64]
-DEV void hex_renorm(double (&v)[4], double &lg)
-{
-    const double m = fmax(fmax(fabs(v[0]), fabs(v[1])), fmax(fabs(v[2]), fabs(v[3])));
-    if (__ballot(m >= STATE_TINY) == 0ull || __ballot(m > STATE_HUGE) != 0ull) {
-        const double mm = wave_max(m);
+    const double m = k.maxabs();
+    if ((__ballot(m >= STATE_TINY) & mask) == 0ull || (__ballot(m > STATE_HUGE) & mask) != 0ull) {
+        const double mm = wave_max((mask >> lane_id()) & 1ull ? m : 0.0);
         if (mm > 0.0) {
             const int ex = ilogb(mm);
             lg += (double)ex * 0.69314718055994530942;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = ldexp(v[e], -ex);
+            for (int e = 0; e < State<NM>::NV; ++e) k.v[e] = ldexp(k.v[e], -ex);
         }
     }
 }
 
-// Walk over a list like quad_walk (same arguments and return value); dl[e] is
-// the propagation to tend of row 4e + l/16, its log factor already in lg.
-template <bool BRA, typename F>
-DEV bool hex_walk(Ctx &c, const Hex &q, double (&v)[4], int &s, double &lg, int no, double tstart,
-                  const double *otau, const int *ocode, int n, double tend, double (&dl)[4], Work &w, F &&after)
-{
-    const double egs = c.M.egs;
-    const int l = lane_id();
-    int ns = c.sz[s], eo = c.off[s];
-    const int nb4 = 4 * c.M.nb;
-    const glb_d *ops = (const glb_d *)c.M.ops;
-    double tlast = tstart;
-    for (int c0 = 0; c0 < n; c0 += QCH) {
-        const int nc = min(QCH, n - c0);
-        // (1) path: record {block offset, target size, source size, source
-        // energies offset}
-        int colv = 0;
-        if (l < nc) {
-            const int cd = ocode[BRA ? n - 1 - (c0 + l) : c0 + l];
-            const int ca = BRA ? 2 - op_ca(cd) : op_ca(cd) - 1;
-            colv = (op_orb(cd) * 2 + op_spin(cd)) * 2 + ca;
-        }
-        for (int kk = 0; kk < nc; ++kk) {
-            const int4 rec = c.tr[s * nb4 + __builtin_amdgcn_readlane(colv, kk)];
-            if (rec.x < 0) return false;
-            c.qrec[kk] = make_int4(rec.z, rec.y, ns, eo);
-            c.qsst[kk] = rec.x;
-            w.op(rec.y, ns, no);
-            s = rec.x;
-            ns = rec.y;
-            eo = rec.w;
-        }
-        wsync();
-        // (2) propagators: four operators per pass, one state per lane
-        for (int kb = 0; kb < nc; kb += 4) {
-            const int kk = kb + (l >> 4);
-            const bool act = kk < nc;
-            const int kq = act ? kk : kb;
-            const int4 rec = c.qrec[kq];
-            const int idx = BRA ? n - 1 - (c0 + kq) : c0 + kq;
-            const double tj = otau[idx];
-            const double tp = c0 + kq > 0 ? otau[BRA ? idx + 1 : idx - 1] : tstart;
-            const double dt = BRA ? tp - tj : tj - tp;
-            const double e0 = c.ev[rec.w];
-            const int k = l & 15;
-            const bool in = k < rec.z;
-            const double d = in ? exp(-(c.ev[rec.w + (in ? k : 0)] - e0) * dt) : 0.0;
-            if (act) {
-                c.qa[kk * 16 + k] = d;
-                c.qlc[kk] = -(e0 - egs) * dt;
-            }
-        }
-        wsync();
-        // (3) products; block entries are loaded two operators ahead
-        auto entries = [&](int kk, double (&a)[4]) {
-            const int4 rec = c.qrec[kk < nc ? kk : nc - 1];
-            const int off = __builtin_amdgcn_readfirstlane(rec.x), nt = __builtin_amdgcn_readfirstlane(rec.y),
-                      nsk = __builtin_amdgcn_readfirstlane(rec.z);
-            const glb_d *P = ops + off;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int k = 4 * e + q.lk;
-                if (4 * e < nsk) {
-                    const bool in = q.lr < nt && k < nsk;
-                    const double x = P[in ? q.lr + k * nt : 0];
-                    a[e] = in ? x : 0.0;
-                } else {
-                    a[e] = 0.0;
-                }
-            }
-        };
-        double a0[4], a1[4];
-        entries(0, a0);
-        entries(1, a1);
-        for (int kk = 0; kk < nc; ++kk) {
-            double a2[4];
-            entries(kk + 2, a2);
-            const int4 rec = c.qrec[kk];
-            const int nsk = __builtin_amdgcn_readfirstlane(rec.z);
-            const double *d = c.qa + kk * 16 + q.lk;
-            lg += c.qlc[kk];
-            dbl4 out{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (4 * e < nsk) out = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[e], v[e] * d[4 * e], out, 0, 0, 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[e] = out[e];
-                a0[e] = a1[e];
-                a1[e] = a2[e];
-            }
-            hex_renorm(v, lg);
-            after(c0 + kk, v, c.qsst[kk], rec.y, lg);
-        }
-        tlast = otau[BRA ? n - c0 - nc : c0 + nc - 1];
-        wsync();
-    }
-    const double dt = BRA ? tlast - tend : tend - tlast;
-    const double e0 = c.ev[eo];
-    lg += -(e0 - egs) * dt;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int r = 4 * e + q.lk;
-        dl[e] = exp(-(c.ev[eo + (r < ns ? r : 0)] - e0) * dt);
-    }
-    return true;
-}
-
-struct HexNoAfter {
-    DEV void operator()(int, const double (&)[4], int, int, double) const {}
+// Where a walk leaves the state after each operator (at that operator's time):
+// state matrices, log scales (from the walk's start) and superstates.
+template <int NM>
+struct Prefix {
+    typedef typename std::conditional<(NM <= 4), lds_d *, glb_d *>::type mat;
+    mat k;
+    lds_d *lg;
+    lds_i *sst;
 };
 
-// Trace of a ket v (superstate s, log scale lg) against the row-major bra B at
-// the same time: part traces of the outer states to c.pl, the total in (tl, ts)
-DEV void hex_contract(Ctx &c, const Hex &q, const double (&v)[4], const double *B, int s, int no, double lg,
-                      double &tl, double &ts)
+template <int NM>
+struct WalkOut {
+    State<NM> k;
+    double lg;
+    int s;      // superstate after the walk; -1: an operator without target block
+};
+
+// Walk of a state over the n operators of an LDS list: a ket ascending from
+// entry 0 (tstart < tau_0 < ... < tend) or, with BRA, a bra descending from
+// entry n-1 with the adjoint blocks (tstart > tau_{n-1} > ... > tend):
+//   k <- exp(-H (t_end - t_n)) psi_n ... exp(-H (t_2 - t_1)) psi_1 exp(-H (t_1 - t_start)) k.
+// Up to 63 operators at a time (lane p holds operator p, the lane behind the
+// last one the propagation to tend):
+//  (1) the superstate before each operator: superstates carry additive keys
+//      (superstate_keys), so it is a scan over the lanes and one table read, and
+//      a quantum-number violation ends the walk before any arithmetic; blocks
+//      without such keys take one transition record after the other;
+//  (2) block offsets, sizes, energies and log factors, all lanes at once;
+//  (3) entries (blocks up to 4: block times propagator, four operators per
+//      pass, one exp per lane, kept in registers: quad b of pass p holds
+//      operator 4p + b) or propagators (blocks up to 16, into LDS);
+//  (4) the products.  Blocks up to 4: the state moves one quad on per operator
+//      (two DPP moves) to the quad that holds the operator's entries, one
+//      matrix instruction each; the other quads carry nothing.  Blocks up to
+//      16: ceil(ns/4) chained matrix instructions, block entries loaded from
+//      global memory (29 KB for the 3-orbital model, shared by all chains) one
+//      to two operators ahead.  Blocks of one state: a product over the lanes.
+// The renormalisation check runs per operator only if some propagation of the
+// group spans more than exp(-100), else every fourth operator: in between no
+// state can leave the FP64 range.
+// KEEP: the states after every operator go to px.
+template <int NM, bool BRA, bool KEEP>
+__device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_, double tstart, double tend,
+                                                            const lds_d *otau_, const lds_i *ocode_, int n_,
+                                                            int no_, Prefix<NM> px)
 {
-    double b[4];
-    q.load(B, c.sz[s], no, b);
-    double x = (v[0] * b[0] + v[1] * b[1]) + (v[2] * b[2] + v[3] * b[3]);
-    x += __shfl_xor(x, 16, WAVE);
-    x += __shfl_xor(x, 32, WAVE);
-    if (lane_id() < no) {
-        c.pl[2 * lane_id()] = lg + log(fabs(x));
-        c.pl[2 * lane_id() + 1] = copysign(1.0, x);
+    const int l = lane_id();
+    const int n = uni(n_), no = uni(no_);
+    const lds_d *otau = uni_lds(otau_);
+    const lds_i *ocode = uni_lds(ocode_);
+    // the environment (uniform)
+    const WalkEnv &E = s_wenv;
+    const double egs = E.egs;
+    const lds_i4 *tr = uni_lds(E.tr), *sinfo = uni_lds(E.sinfo);
+    const lds_d *ev = uni_lds(E.ev);
+    const lds_b *keys = uni_lds(E.keys);
+    const int ncol = uni(E.ncol), dkey = uni(E.dkey);
+    int s = uni(s_);
+    double lg = 0.0;
+    WalkOut<NM> out;
+    out.s = -1;
+    constexpr unsigned long long QUAD0 = 0x000F000F000F000Full;
+    int ntns = 0, nss = 0, nts = 0;
+    bool last = false;
+    for (int c0 = 0; !last; c0 += 63) {
+        const int nc = min(63, n - c0);
+        last = c0 + nc == n;
+        const int m = nc + (last ? 1 : 0);
+        // operator of this lane and the time before it
+        const int p = c0 + l;
+        int cd = 0;
+        double t = tend, tp = tstart;
+        if (l < nc) {
+            cd = ocode[BRA ? n - 1 - p : p];
+            t = otau[BRA ? n - 1 - p : p];
+        }
+        if (l < m && p > 0) tp = otau[BRA ? n - p : p - 1];
+        const double dt = l < m ? (BRA ? tp - t : t - tp) : 0.0;
+        const int ca = BRA ? 2 - op_ca(cd) : op_ca(cd) - 1;   // 0: creator
+        const int col = (op_orb(cd) * 2 + op_spin(cd)) * 2 + ca;
+        // (1) superstates before each operator, (2) this lane's blocks
+        int sb = s;
+        iv4 rec;
+        const int sfirst = s;
+        if (dkey) {
+            int d = (int)(signed char)(op_spin(cd) ? dkey >> 8 : dkey);
+            d = l < nc ? (ca ? -d : d) : 0;
+            const int key = (int)keys[s] + wave_scan_i(d) - d;
+            sb = keys[256 + (key & 255)];
+            const bool none = sb == 255;
+            sb = none ? 0 : sb;
+            rec = tr[sb * ncol + col];
+            // the first operator without a target has a valid superstate before it
+            if (__ballot(l < nc && (none || rec.x < 0)) != 0ull) return out;
+            if (nc > 0) s = __builtin_amdgcn_readlane(rec.x, nc - 1);
+            if (l >= nc) sb = s;
+        } else {
+            for (int kk = 0; kk < nc; ++kk) {
+                sb = l == kk ? s : sb;
+                s = uni(tr[s * ncol + __builtin_amdgcn_readlane(col, kk)].x);
+                if (s < 0) return out;
+            }
+            if (l >= nc) sb = s;
+            rec = tr[sb * ncol + col];
+        }
+        const iv4 si = sinfo[sb];
+        const double e0 = __hiloint2double(si.y, si.x), lc = -(e0 - egs) * dt;
+        const int ns = si.z & 255, eo = si.z >> 8;
+        if (l >= nc) rec = iv4{s, ns, -1, eo};
+        {
+            const int nn = l < nc ? rec.y * ns : 0, n1 = l < nc ? ns : 0;
+            const int both = wave_isum((nn << 12) | n1);   // at most 63 x 256 and 63 x 16
+            ntns += both >> 12;
+            nss += both & 0xfff;
+            // sum of nt: the sum of ns but for the ends
+            nts += (both & 0xfff) + (sinfo[s].z & 255) - (sinfo[sfirst].z & 255);
+        }
+        if constexpr (KEEP) {
+            if (l < nc) px.sst[p] = rec.x;
+        }
+        if constexpr (NM == 1) {
+            // every block is one number, every propagation a log factor only
+            const lds_d *lops = uni_lds(E.lops);
+            double a = l < nc ? lops[rec.z] : 1.0;
+            if constexpr (KEEP) {
+                a = wave_scan_mul(a);
+                const double sc = wave_scan_d(lc), k0 = readlane_d(k.v[0], 0);
+                if (l < nc) {
+                    px.k[p] = k0 * a;
+                    px.lg[p] = lg + sc;
+                }
+                k.v[0] *= readlane_d(a, m - 1);
+                lg += readlane_d(sc, m - 1);
+            } else {
+                k.v[0] *= readlane_d(wave_scan_mul(a), 63);
+                lg += wave_sum(lc);
+            }
+        } else if constexpr (NM <= 4) {
+            const unsigned chk = __ballot(__int_as_float(si.w) * (float)dt > 100.0f) ? 0u : 3u;
+            const lds_d *lops = uni_lds(E.lops);
+            const int blk = (l >> 2) & 3, i = l & 3, kr = l >> 4;
+            const double sc = KEEP ? wave_scan_d(lc) : wave_sum(lc);   // log factors so far / of the group
+            double lr = 0.0;                                           // renormalisations of the group
+            const int pack = (rec.z & 0xfffff) | (rec.y << 20) | (ns << 24) | (l >= nc ? 1 << 28 : 0);
+            for (int q0 = 0; q0 < m; q0 += 16) {
+                // (3) entries A(i, kr) of operators q0 + 4 pass + blk
+                double a[4];
+#pragma unroll
+                for (int ps = 0; ps < 4; ++ps) {
+                    a[ps] = 0.0;
+                    if (q0 + 4 * ps < m) {
+                        const int src = q0 + 4 * ps + blk;
+                        const int pk = __shfl(pack, src, WAVE), eq = __shfl(eo, src, WAVE);
+                        const double dq = __shfl(dt, src, WAVE);
+                        const int nt = (pk >> 20) & 15, nq = (pk >> 24) & 15;
+                        const bool in = i < nt && kr < nq, fin = (pk >> 28) != 0;   // fin: the propagation to tend
+                        const double pv = lops[in && !fin ? (pk & 0xfffff) + i + kr * nt : 0];
+                        const double d = exp(-(ev[eq + (kr < nq ? kr : 0)] - ev[eq]) * dq);
+                        a[ps] = in ? (fin ? (i == kr ? d : 0.0) : pv * d) : 0.0;
+                    }
+                }
+                // (4) products
+#pragma unroll
+                for (int ps = 0; ps < 4; ++ps) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const int t_ = 4 * ps + b;
+                        if (q0 + t_ < m) {
+                            const double r = dpp_d<DPP_ROW_ROR4>(k.v[0]);
+                            k.v[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[ps], r, 0.0, 0, 0, 0);
+                            if (b == 3 || chk == 0u) renorm(k, QUAD0 << (4 * b), lr);
+                            if constexpr (KEEP) {
+                                if (q0 + t_ < nc) {
+                                    const int j = c0 + q0 + t_, nt = __builtin_amdgcn_readlane(rec.y, q0 + t_);
+                                    if (blk == b && kr < nt && i < no) px.k[j * 16 + kr * no + i] = k.v[0];
+                                    px.lg[j] = lg + lr + readlane_d(sc, q0 + t_);
+                                }
+                            }
+                        }
+                    }
+                }
+            }
+            lg += lr + (KEEP ? readlane_d(sc, m - 1) : sc);
+            // the state to every quad
+            double x = blk == ((m - 1) & 3) ? k.v[0] : 0.0;
+            x += dpp_d<DPP_ROW_ROR4>(x);
+            k.v[0] = x + dpp_d<DPP_ROW_ROR8>(x);
+        } else {
+            const unsigned chk = __ballot(__int_as_float(si.w) * (float)dt > 100.0f) ? 0u : 3u;
+            lds_d *qa = uni_lds(E.qa);
+            const glb_d *ops = uni_glb(E.ops);
+            const int zero = uni(E.zero);
+            const int lr = l & 15, lk = l >> 4;
+            const double sc = KEEP ? wave_scan_d(lc) : wave_sum(lc);
+            double lren = 0.0;
+            for (int q0 = 0; q0 < m; q0 += 16) {
+                const int mq = min(16, m - q0);
+                // (3) propagators of operators q0 .. q0 + mq - 1, state l % 16
+                wsync();
+                for (int ps = 0; 4 * ps < mq; ++ps) {
+                    const int src = min(q0 + 4 * ps + lk, 63);
+                    const int nq = __shfl(ns, src, WAVE), eq = __shfl(eo, src, WAVE);
+                    const double dq = __shfl(dt, src, WAVE);
+                    const double d = exp(-(ev[eq + (lr < nq ? lr : 0)] - ev[eq]) * dq);
+                    qa[(4 * ps + lk) * 16 + lr] = lr < nq ? d : 0.0;
+                }
+                wsync();
+                // (4) products
+                const int mp = min(16, nc - q0);   // operators (the propagation to tend comes last)
+                auto load = [&](int t_, double (&a)[4]) {
+                    const int o = q0 + min(t_, max(mp - 1, 0));
+                    const int bo = __builtin_amdgcn_readlane(rec.z, o), nt = __builtin_amdgcn_readlane(rec.y, o),
+                              nq = __builtin_amdgcn_readlane(ns, o);
+                    int ad = bo + lr + lk * nt;
+                    const bool row = lr < nt && bo >= 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        a[e] = ops[row && 4 * e + lk < nq ? ad : zero];
+                        ad += 4 * nt;
+                    }
+                };
+                auto props = [&](int t_, double (&d)[4]) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) d[e] = qa[min(t_, 15) * 16 + 4 * e + lk];
+                };
+                auto step = [&](int t_, const double (&a)[4], const double (&d)[4]) {
+                    const int nq = __builtin_amdgcn_readlane(ns, q0 + t_);
+                    dbl4 r{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (4 * e < nq) r = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], k.v[e] * d[e], r, 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) k.v[e] = r[e];
+                };
+                auto after = [&](int t_) {
+                    if (((unsigned)t_ & chk) == chk) renorm(k, ~0ull, lren);
+                    if constexpr (KEEP) {
+                        const int j = c0 + q0 + t_;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) px.k[j * 256 + e * 64 + l] = k.v[e];
+                        px.lg[j] = lg + lren + readlane_d(sc, q0 + t_);
+                    }
+                };
+                double a0[4], a1[4], d0[4], d1[4];
+                load(0, a0);
+                load(1, a1);
+                props(0, d0);
+                for (int t_ = 0; t_ < mp; t_ += 2) {
+                    props(t_ + 1, d1);
+                    step(t_, a0, d0);
+                    load(t_ + 2, a0);
+                    after(t_);
+                    if (t_ + 1 < mp) {
+                        props(t_ + 2, d0);
+                        step(t_ + 1, a1, d1);
+                        load(t_ + 3, a1);
+                        after(t_ + 1);
+                    }
+                }
+                if (last && q0 + mq == m) {
+                    double d[4];
+                    props(mq - 1, d);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) k.v[e] *= d[e];
+                }
+            }
+            lg += lren + (KEEP ? readlane_d(sc, m - 1) : sc);
+        }
     }
-    const double S = wave_sum(lane_id() < 16 ? x : 0.0);
-    if (S == 0.0) {
-        tl = -DBL_MAX;
-        ts = 0.0;
-    } else {
-        tl = lg + log(fabs(S));
-        ts = copysign(1.0, S);
+    if constexpr (NM > 1) renorm(k, ~0ull, lg);
+    if (l == 0) {
+        __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.flops, (double)(no * (2 * ntns + nss)));
+        __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.bytes, (double)(8 * no * (nss + nts)));
     }
-    wsync();
+    out.k = k;
+    out.lg = lg;
+    out.s = s;
+    return out;
 }
 
 // What an operator walk over blocks above 16 states needs, by value (the walk
@@ -1074,110 +1166,38 @@ DEV MfmaEnv mfma_env(const Ctx &c)
 // algorithmic work of an MFMA walk (as Work::commit counts it)
 DEV void mfma_work(Ctx &c, const MfmaOut &r, int no)
 {
-    c.wflops += (double)no * (2.0 * r.ntns + r.nss);
-    c.wbytes += 8.0 * no * (r.nss + r.nts);
+    c.work((double)no * (2.0 * r.ntns + r.nss), 8.0 * no * (r.nss + r.nts));
 }
 
-// Ket sweep over a list (ascending tau) from t0 to t1.  Returns false if an
-// operator has no target block (quantum-number violation).
-template <int NM>
-DEV bool ket_walk(Ctx &c, double *&K, double *&Kw, int &s, double &lg, int no, double t0,
-                  const double *otau, const int *ocode, int n, double t1)
+
+// walk_small over a list of this chain (generic pointers into LDS)
+template <int NM, bool BRA>
+DEV bool walk_list(State<NM> &k, int &s, double &lg, int no, double t0, const double *otau, const int *ocode, int n,
+                   double t1)
 {
-    double t = t0;
-    Work w;
-    if constexpr (NM <= 4) {
-        const Quad q;
-        double v = q.load(K, c.sz[s], no);
-        double d;
-        const bool ok = quad_walk<false>(c, q, v, s, lg, no, t0, otau, ocode, n, t1, d, w, NoAfter());
-        w.commit(c);
-        if (!ok) return false;
-        v = quad_finish(v, d, lg);
-        q.store(Kw, c.sz[s], no, v);
-        double *x = K;
-        K = Kw;
-        Kw = x;
-        wsync();
-        return true;
-    } else if constexpr (NM <= 16) {
-        const Hex q;
-        double v[4], d[4];
-        q.load(K, c.sz[s], no, v);
-        const bool ok = hex_walk<false>(c, q, v, s, lg, no, t0, otau, ocode, n, t1, d, w, HexNoAfter());
-        w.commit(c);
-        if (!ok) return false;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] *= d[e];
-        hex_renorm(v, lg);
-        q.store(Kw, c.sz[s], no, v);
-        double *x = K;
-        K = Kw;
-        Kw = x;
-        wsync();
-        return true;
-    } else {
-        const MfmaOut r = walk_mfma<false>(mfma_env(c), K, Kw, s, no, t, otau, ocode, n, t1);
-        mfma_work(c, r, no);
-        if (r.s < 0) return false;
-        lg += r.lg;
-        s = r.s;
-        double *x = K;
-        K = Kw;
-        Kw = x;
-        return true;
-    }
-    w.commit(c);
+    const WalkOut<NM> o =
+        walk_small<NM, BRA, false>(k, s, t0, t1, (const lds_d *)otau, (const lds_i *)ocode, n, no, Prefix<NM>{});
+    if (o.s < 0) return false;
+    k = o.k;
+    s = o.s;
+    lg += o.lg;
     return true;
 }
 
-// Bra sweep downward from t1 over a list (taken in descending order) to t0.
-template <int NM>
-DEV void bra_walk(Ctx &c, double *&B, double *&Bw, int &s, double &lg, int no, double t1,
-                  const double *otau, const int *ocode, int n, double t0)
+// the same for blocks above 16 states: state matrices K / Kw in memory
+template <bool BRA>
+DEV bool walk_big(Ctx &c, double *&K, double *&Kw, int &s, double &lg, int no, double t0, const double *otau,
+                  const int *ocode, int n, double t1)
 {
-    double t = t1;
-    Work w;
-    if constexpr (NM <= 4) {
-        const Quad q;
-        double v = q.load(B, c.sz[s], no);
-        double d;
-        quad_walk<true>(c, q, v, s, lg, no, t1, otau, ocode, n, t0, d, w, NoAfter());
-        w.commit(c);
-        v = quad_finish(v, d, lg);
-        q.store(Bw, c.sz[s], no, v);
-        double *x = B;
-        B = Bw;
-        Bw = x;
-        wsync();
-        return;
-    } else if constexpr (NM <= 16) {
-        const Hex q;
-        double v[4], d[4];
-        q.load(B, c.sz[s], no, v);
-        hex_walk<true>(c, q, v, s, lg, no, t1, otau, ocode, n, t0, d, w, HexNoAfter());
-        w.commit(c);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] *= d[e];
-        hex_renorm(v, lg);
-        q.store(Bw, c.sz[s], no, v);
-        double *x = B;
-        B = Bw;
-        Bw = x;
-        wsync();
-        return;
-    } else {
-        const MfmaOut r = walk_mfma<true>(mfma_env(c), B, Bw, s, no, t, otau, ocode, n, t0);
-        mfma_work(c, r, no);
-        if (r.s < 0) return;
-        lg += r.lg;
-        s = r.s;
-        double *x = B;
-        B = Bw;
-        Bw = x;
-        return;
-    }
-    w.commit(c);
+    const MfmaOut r = walk_mfma<BRA>(mfma_env(c), K, Kw, s, no, t0, otau, ocode, n, t1);
+    mfma_work(c, r, no);
+    if (r.s < 0) return false;
+    lg += r.lg;
+    s = r.s;
+    double *x = K;
+    K = Kw;
+    Kw = x;
+    return true;
 }
 
 // stage global operators [j0, j1) into the LDS list (chunks of lcap)
@@ -1192,41 +1212,54 @@ DEV int stage_chunk(Ctx &c, int j0, int j1)
     return n;
 }
 
-// ket over global operators [j0, j1) in LDS-staged chunks
-template <int NM>
-DEV bool ket_walk_global(Ctx &c, double *&K, double *&Kw, int &s, double &lg, int no, double t0, int j0,
-                         int j1, double t1)
+// Walk over global operators [j0, j1) in LDS-staged chunks, ascending from t0
+// to t1 or (BRA) descending; walk(tstart, n, tend) takes the staged chunk.
+template <bool BRA, typename F>
+DEV bool walk_staged(Ctx &c, double tstart, int j0, int j1, double tend, F &&walk)
 {
     // one walk call site: an empty range is one chunk of no operators
-    double t = t0;
-    int b = j0;
-    do {
-        const int n = b < j1 ? stage_chunk(c, b, j1) : 0;
-        const double tend = (b + n < j1) ? c.ttau[n - 1] : t1;
-        // walk the chunk; the final propagation of a non-last chunk is zero
-        if (!ket_walk<NM>(c, K, Kw, s, lg, no, t, c.ttau, c.tcode, n, tend)) return false;
-        t = tend;
-        b += n;
-        wsync();
-    } while (b < j1);
+    double t = tstart;
+    if constexpr (!BRA) {
+        int b = j0;
+        do {
+            const int n = b < j1 ? stage_chunk(c, b, j1) : 0;
+            // the final propagation of a non-last chunk is zero
+            const double te = (b + n < j1) ? c.ttau[n - 1] : tend;
+            if (!walk(t, n, te)) return false;
+            t = te;
+            b += n;
+            wsync();
+        } while (b < j1);
+    } else {
+        int e = j1;
+        do {
+            const int b = max(j0, e - c.L.lcap_lds);
+            const int n = e > j0 ? stage_chunk(c, b, e) : 0;
+            const double te = (b > j0) ? c.ttau[0] : tend;
+            if (!walk(t, n, te)) return false;
+            t = te;
+            e = b;
+            wsync();
+        } while (e > j0);
+    }
     return true;
 }
 
-template <int NM>
-DEV void bra_walk_global(Ctx &c, double *&B, double *&Bw, int &s, double &lg, int no, double t1, int j0,
-                         int j1, double t0)
+template <int NM, bool BRA>
+DEV bool walk_global(Ctx &c, State<NM> &k, int &s, double &lg, int no, double t0, int j0, int j1, double t1)
 {
-    double t = t1;
-    int e = j1;
-    do {
-        const int b = max(j0, e - c.L.lcap_lds);
-        const int n = e > j0 ? stage_chunk(c, b, e) : 0;
-        const double tend = (b > j0) ? c.ttau[0] : t0;
-        bra_walk<NM>(c, B, Bw, s, lg, no, t, c.ttau, c.tcode, n, tend);
-        t = tend;
-        e = b;
-        wsync();
-    } while (e > j0);
+    return walk_staged<BRA>(c, t0, j0, j1, t1, [&](double ta, int n, double tb) {
+        return walk_list<NM, BRA>(k, s, lg, no, ta, c.ttau, c.tcode, n, tb);
+    });
+}
+
+template <bool BRA>
+DEV bool walk_global_big(Ctx &c, double *&K, double *&Kw, int &s, double &lg, int no, double t0, int j0, int j1,
+                         double t1)
+{
+    return walk_staged<BRA>(c, t0, j0, j1, t1, [&](double ta, int n, double tb) {
+        return walk_big<BRA>(c, K, Kw, s, lg, no, ta, c.ttau, c.tcode, n, tb);
+    });
 }
 
 DEV void set_identity(double *K, int no)
@@ -1241,25 +1274,40 @@ DEV void copy_mat(double *dst, const double *src, int n)
     wsync();
 }
 
-// signed log-sum (addLogTr, Trace.F90:286-298)
-DEV void log_add(double &al, double &as, double bl, double bs)
+// A local trace: S exp(lg).  x: this lane's part of the part traces of the
+// outer states (blocks up to 16 states; above, they are in c.pl and S is the
+// sign, lg the logarithm).  The logarithms are taken only where they are kept
+// (an accepted move): every column carries the same scale exp(lg), so the
+// total is the plain sum of the columns (the log-space sum of addLogTr,
+// Trace.F90:286-298, of the same numbers).
+struct TraceVal {
+    double S, lg, x;
+    DEV double log_abs() const { return S == 0.0 ? -DBL_MAX : lg + log(fabs(S)); }
+    DEV double sign() const { return S == 0.0 ? 0.0 : copysign(1.0, S); }
+};
+
+// from the lanes' products x (ket times bra, summed over the lane's own rows)
+template <int NM>
+DEV TraceVal trace_of(double x, double lg)
 {
-    if (al >= bl) {
-        al = al + log(1.0 + as * bs * exp(bl - al));
-    } else {
-        double nl = bl + log(1.0 + as * bs * exp(al - bl));
-        al = nl;
-        as = bs;
-    }
+    return TraceVal{wave_sum(NM > 4 || (lane_id() & 12) == 0 ? x : 0.0), lg, x};
+}
+
+template <int NM, typename P>
+DEV TraceVal contract_small(const State<NM> &k, P B, int ns, int no, double lg)
+{
+    State<NM> b;
+    b.load(B, ns, no);
+    double x = 0.0;
+#pragma unroll
+    for (int e = 0; e < State<NM>::NV; ++e) x = fma(k.v[e], b.v[e], x);
+    return trace_of<NM>(x, lg);
 }
 
 // Contract ket K and bra B (same superstate s, both at the same tau) column by
-// column; part traces to c.pl, total in (tl, ts).
-DEV void contract(Ctx &c, const double *K, const double *B, int s, int no, double lg, double &tl, double &ts)
+// column; part traces to c.pl (blocks above 16 states).
+DEV TraceVal contract(Ctx &c, const double *K, const double *B, int s, int no, double lg)
 {
-    // every column carries the same scale exp(lg), so the total is the plain
-    // sum of the columns (the log-space sum of addLogTr, Trace.F90:286-298, of
-    // the same numbers)
     const int ns = c.sz[s];
     double part = 0.0;
     for (int i = lane_id(); i < no; i += WAVE) {
@@ -1270,12 +1318,28 @@ DEV void contract(Ctx &c, const double *K, const double *B, int s, int no, doubl
         part += acc;
     }
     const double S = wave_sum(part);
-    if (S == 0.0) {
-        tl = -DBL_MAX;
-        ts = 0.0;
+    wsync();
+    if (S == 0.0) return TraceVal{0.0, -DBL_MAX, 0.0};
+    return TraceVal{copysign(1.0, S), lg + log(fabs(S)), 0.0};
+}
+
+// the trace becomes the chain's: its logarithm, sign and part traces
+template <int NM>
+DEV void keep_trace(Ctx &c, const TraceVal &T)
+{
+    const int no = c.sz[c.h.outer];
+    c.h.trace_log = T.log_abs();
+    c.h.trace_sign = T.sign();
+    if constexpr (NM <= 16) {
+        double x = T.x;   // columns: sum over the rows
+        x += __shfl_xor(x, 16, WAVE);
+        x += __shfl_xor(x, 32, WAVE);
+        if (lane_id() < no) {
+            c.part[2 * lane_id()] = T.lg + log(fabs(x));
+            c.part[2 * lane_id() + 1] = copysign(1.0, x);
+        }
     } else {
-        tl = lg + log(fabs(S));
-        ts = copysign(1.0, S);
+        for (int i = lane_id(); i < 2 * no; i += WAVE) c.part[i] = c.pl[i];
     }
     wsync();
 }
@@ -1284,24 +1348,33 @@ DEV void contract(Ctx &c, const double *K, const double *B, int s, int no, doubl
 // set_config, initial state): identity ket on the outer superstate at tau = 0
 // through every operator, contracted with the identity bra at beta.
 // A configuration that breaks the quantum numbers (an operator without a
-// target block) has a zero trace: returns false with tl = -DBL_MAX, ts = 0.
+// target block) has a zero trace.
 template <int NM>
-DEV bool full_trace(Ctx &c, int outer, double &tl, double &ts)
+DEV TraceVal full_trace(Ctx &c, int outer)
 {
     const int no = c.sz[outer];
-    double *K = c.K0, *Kw = c.K1;
-    set_identity(K, no);
     int s = outer;
     double lg = 0.0;
-    if (!ket_walk_global<NM>(c, K, Kw, s, lg, no, 0.0, 0, c.h.nop, c.M.beta) || s != outer) {
-        tl = -DBL_MAX;
-        ts = 0.0;
-        wsync();
-        return false;
+    if constexpr (NM <= 16) {
+        State<NM> k;
+        k.identity(no);
+        if (!walk_global<NM, false>(c, k, s, lg, no, 0.0, 0, c.h.nop, c.M.beta) || s != outer)
+            return TraceVal{0.0, -DBL_MAX, 0.0};
+        double x = 0.0;
+#pragma unroll
+        for (int e = 0; e < State<NM>::NV; ++e)
+            if (State<NM>::row(e) == State<NM>::col()) x = k.v[e];
+        return trace_of<NM>(x, lg);
+    } else {
+        double *K = c.K0, *Kw = c.K1;
+        set_identity(K, no);
+        if (!walk_global_big<false>(c, K, Kw, s, lg, no, 0.0, 0, c.h.nop, c.M.beta) || s != outer) {
+            wsync();
+            return TraceVal{0.0, -DBL_MAX, 0.0};
+        }
+        set_identity(Kw, no);
+        return contract(c, K, Kw, s, no, lg);
     }
-    set_identity(Kw, no);
-    contract(c, K, Kw, s, no, lg, tl, ts);
-    return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1315,13 +1388,19 @@ DEV void rebuild_cache(Ctx &c)
     const int nw = c.h.nwin;
     const int top = (nw > 1) ? nw + 1 : 2;
     const int stride = c.nm * c.nm;
+    State<NM <= 16 ? NM : 1> k;
     double *B = c.K0, *Bw = c.K1;
-    set_identity(B, no);
+    if constexpr (NM <= 16) {
+        k.identity(no);
+        k.store(c.bnd + (long)top * stride, no, no);
+    } else {
+        set_identity(B, no);
+        copy_mat(c.bnd + (long)top * stride, B, no * no);
+    }
     int s = outer;
     double lg = 0.0;
     double tb = c.M.beta;
     int hiidx = c.h.nop;
-    copy_mat(c.bnd + (long)top * stride, B, no * no);
     if (lane_id() == 0) {
         c.bndlog[top] = lg;
         c.bndsst[top] = s;
@@ -1329,8 +1408,13 @@ DEV void rebuild_cache(Ctx &c)
     for (int m = top - 1; m >= p + 2; --m) {
         const double tm = bound_tau(m, nw, c.M.beta);
         const int loidx = upper_bound_tau(c.tau, c.h.nop, tm);
-        bra_walk_global<NM>(c, B, Bw, s, lg, no, tb, loidx, hiidx, tm);
-        copy_mat(c.bnd + (long)m * stride, B, c.sz[s] * no);
+        if constexpr (NM <= 16) {
+            walk_global<NM, true>(c, k, s, lg, no, tb, loidx, hiidx, tm);
+            k.store(c.bnd + (long)m * stride, c.sz[s], no);
+        } else {
+            walk_global_big<true>(c, B, Bw, s, lg, no, tb, loidx, hiidx, tm);
+            copy_mat(c.bnd + (long)m * stride, B, c.sz[s] * no);
+        }
         if (lane_id() == 0) {
             c.bndlog[m] = lg;
             c.bndsst[m] = s;
@@ -1338,14 +1422,20 @@ DEV void rebuild_cache(Ctx &c)
         tb = tm;
         hiidx = loidx;
     }
-    double *K = c.K0, *Kw = c.K1;
-    set_identity(K, no);
     s = outer;
     lg = 0.0;
     const double tp = bound_tau(p, nw, c.M.beta);
     const int n0 = lower_bound_tau(c.tau, c.h.nop, tp);
-    ket_walk_global<NM>(c, K, Kw, s, lg, no, 0.0, 0, n0, tp);
-    copy_mat(c.kst, K, c.sz[s] * no);
+    if constexpr (NM <= 16) {
+        k.identity(no);
+        walk_global<NM, false>(c, k, s, lg, no, 0.0, 0, n0, tp);
+        k.store(c.kst, c.sz[s], no);
+    } else {
+        double *K = c.K0, *Kw = c.K1;
+        set_identity(K, no);
+        walk_global_big<false>(c, K, Kw, s, lg, no, 0.0, 0, n0, tp);
+        copy_mat(c.kst, K, c.sz[s] * no);
+    }
     c.h.kst_log = lg;
     c.h.kst_sst = s;
     c.h.cache_pos = p;
@@ -1355,10 +1445,10 @@ DEV void rebuild_cache(Ctx &c)
 // Bring the caches to the current window position: advance the ket across
 // passed half windows, or rebuild after a wrap / invalidation.
 template <int NM>
-DEV void ensure_cache(Ctx &c)
+__device__ __attribute__((noinline)) void move_cache(ChainRef r)
 {
+    Ctx c = attach<NM>(r);
     const int p = c.h.nwin > 1 ? c.h.wpos : 0;
-    if (c.h.cache_pos == p) return;
     c.h.rk_n = 0;
     c.h.lb_n = 0;
     if (c.h.cache_pos < 0 || c.h.cache_pos > p) {
@@ -1368,25 +1458,38 @@ DEV void ensure_cache(Ctx &c)
     const int no = c.sz[c.h.outer];
     int s = c.h.kst_sst;
     double lg = c.h.kst_log;
-    double *K = c.K0, *Kw = c.K1;
-    copy_mat(K, c.kst, c.sz[s] * no);
     const double ta = bound_tau(c.h.cache_pos, c.h.nwin, c.M.beta);
     const double tb = bound_tau(p, c.h.nwin, c.M.beta);
     const int ia = lower_bound_tau(c.tau, c.h.nop, ta);
     const int ib = lower_bound_tau(c.tau, c.h.nop, tb);
-    ket_walk_global<NM>(c, K, Kw, s, lg, no, ta, ia, ib, tb);
-    copy_mat(c.kst, K, c.sz[s] * no);
+    if constexpr (NM <= 16) {
+        State<NM> k;
+        k.load(c.kst, c.sz[s], no);
+        walk_global<NM, false>(c, k, s, lg, no, ta, ia, ib, tb);
+        k.store(c.kst, c.sz[s], no);
+    } else {
+        double *K = c.K0, *Kw = c.K1;
+        copy_mat(K, c.kst, c.sz[s] * no);
+        walk_global_big<false>(c, K, Kw, s, lg, no, ta, ia, ib, tb);
+        copy_mat(c.kst, K, c.sz[s] * no);
+    }
     c.h.kst_log = lg;
     c.h.kst_sst = s;
     c.h.cache_pos = p;
     wsync();
 }
 
+template <int NM>
+DEV void ensure_cache(Ctx &c)
+{
+    if (c.h.cache_pos != (c.h.nwin > 1 ? c.h.wpos : 0)) move_cache<NM>(c.ref());
+}
+
 // Trace of the LDS trial list between the cached ket and bra; returns false
 // on a quantum-number violation (check_sst_sequence, Trace.F90:1243-1302, on a
 // superset of the changed span).
 template <int NM>
-DEV bool window_trace(Ctx &c, int nl, double &tl, double &ts)
+DEV bool window_trace(Ctx &c, int nl, TraceVal &T)
 {
     const int no = c.sz[c.h.outer];
     const int p = c.h.nwin > 1 ? c.h.wpos : 0;
@@ -1394,39 +1497,24 @@ DEV bool window_trace(Ctx &c, int nl, double &tl, double &ts)
     const double ta = bound_tau(p, c.h.nwin, c.M.beta), tb = bound_tau(top, c.h.nwin, c.M.beta);
     int s = c.h.kst_sst;
     double lg = c.h.kst_log;
-    if constexpr (NM <= 4) {
-        const Quad q;
-        double v = q.load(c.kst, c.sz[s], no);
-        double d;
-        Work w;
-        const bool ok = quad_walk<false>(c, q, v, s, lg, no, ta, c.ttau, c.tcode, nl, tb, d, w, NoAfter());
-        w.commit(c);
-        if (!ok || s != c.bndsst[top]) return false;
-        quad_contract(c, q, v * d, c.bnd + (long)top * c.nm * c.nm, s, no, lg + c.bndlog[top], tl, ts);
-        return true;
-    } else if constexpr (NM <= 16) {
-        const Hex q;
-        double v[4], d[4];
-        q.load(c.kst, c.sz[s], no, v);
-        Work w;
-        const bool ok = hex_walk<false>(c, q, v, s, lg, no, ta, c.ttau, c.tcode, nl, tb, d, w, HexNoAfter());
-        w.commit(c);
-        if (!ok || s != c.bndsst[top]) return false;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] *= d[e];
-        hex_contract(c, q, v, c.bnd + (long)top * c.nm * c.nm, s, no, lg + c.bndlog[top], tl, ts);
-        return true;
+    const double *B = c.bnd + (long)top * c.nm * c.nm;
+    if constexpr (NM <= 16) {
+        State<NM> k;
+        k.load(c.kst, c.sz[s], no);
+        if (!walk_list<NM, false>(k, s, lg, no, ta, c.ttau, c.tcode, nl, tb) || s != c.bndsst[top]) return false;
+        T = contract_small<NM>(k, B, c.sz[s], no, lg + c.bndlog[top]);
+    } else {
+        double *K = c.K0, *Kw = c.K1;
+        copy_mat(K, c.kst, c.sz[s] * no);
+        if (!walk_big<false>(c, K, Kw, s, lg, no, ta, c.ttau, c.tcode, nl, tb)) return false;
+        if (s != c.bndsst[top]) return false;
+        T = contract(c, K, B, s, no, lg + c.bndlog[top]);
     }
-    double *K = c.K0, *Kw = c.K1;
-    copy_mat(K, c.kst, c.sz[s] * no);
-    if (!ket_walk<NM>(c, K, Kw, s, lg, no, ta, c.ttau, c.tcode, nl, tb)) return false;
-    if (s != c.bndsst[top]) return false;
-    contract(c, K, c.bnd + (long)top * c.nm * c.nm, s, no, lg + c.bndlog[top], tl, ts);
     return true;
 }
 
 // ---------------------------------------------------------------------------
-// Window segment caches (blocks of up to 4 states).  rk[j] is the ket after the
+// Window segment caches (blocks of up to 16 states).  rk[j] is the ket after the
 // window's first j operators, at the time of operator j-1 (rk[0] = the cached
 // ket at the window's lower edge); lb[m] is the bra after the window's last m
 // operators, at the time of operator nw-m (lb[0] = the cached bra at the upper
@@ -1435,74 +1523,75 @@ DEV bool window_trace(Ctx &c, int nl, double &tl, double &ts)
 // q2-q1 between them, a removal of w1 < w2 the w2-w1-1 between them.  The
 // caches are extended on demand and cut back to their unchanged parts after
 // an accepted move; both restart when the window list is reloaded or the
-// boundary caches change.
+// boundary caches change.  Their log scales and superstates are in LDS; the
+// matrices too for blocks up to 4 states (row-major, NM^2 apart), above they
+// are the lanes' registers as they are (2 KB, coalesced), in the chain block.
 // ---------------------------------------------------------------------------
 template <int NM>
-DEV void rk_extend(Ctx &c, int to)
+DEV State<NM> seg_load(const double *buf, int j, int ns, int no)
 {
-    constexpr int S2 = NM * NM;
-    const int no = c.sz[c.h.outer];
-    const double ta = bound_tau(c.h.nwin > 1 ? c.h.wpos : 0, c.h.nwin, c.M.beta);
-    int j = c.h.rk_n - 1;
-    if (j < 0) {
-        copy_mat(c.rk, c.kst, c.sz[c.h.kst_sst] * no);
-        c.rkx[0] = c.h.kst_log;
-        c.rks[0] = c.h.kst_sst;
-        j = 0;
+    State<NM> k;
+    if constexpr (NM <= 4) {
+        k.load(buf + j * NM * NM, ns, no);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) k.v[e] = buf[j * 256 + e * 64 + lane_id()];
     }
-    if (j < to) {
-        Work w;
-        int s = c.rks[j];
-        double lg = c.rkx[j];
-        const Quad q;
-        double v = q.load(c.rk + (long)j * S2, c.sz[s], no);
-        double d;
-        const int j0 = j;
-        quad_walk<false>(c, q, v, s, lg, no, j0 > 0 ? c.wtau[j0 - 1] : ta, c.wtau + j0, c.wcode + j0, to - j0,
-                         c.wtau[to - 1], d, w, [&](int k, double vk, int sk, int nsk, double lgk) {
-                             q.store(c.rk + (long)(j0 + k + 1) * S2, nsk, no, vk);
-                             c.rkx[j0 + k + 1] = lgk;
-                             c.rks[j0 + k + 1] = sk;
-                         });
-        w.commit(c);
+    return k;
+}
+template <int NM>
+DEV void seg_store(double *buf, int j, int ns, int no, const State<NM> &k)
+{
+    if constexpr (NM <= 4) {
+        k.store(buf + j * NM * NM, ns, no);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) buf[j * 256 + e * 64 + lane_id()] = k.v[e];
     }
-    c.h.rk_n = max(c.h.rk_n, to + 1);
-    wsync();
 }
 
-template <int NM>
-DEV void lb_extend(Ctx &c, int nw, int to)
+// extend rk to `to` operators (BRA = false) or lb (BRA = true); nw: window operators
+template <int NM, bool BRA>
+__device__ __attribute__((noinline)) void seg_extend(ChainRef ref, int nw_, int to_)
 {
-    constexpr int S2 = NM * NM;
+    Ctx c = attach<NM>(ref);
+    const int nw = uni(nw_), to = uni(to_);
+    constexpr int S = NM <= 4 ? NM * NM : 256;
+    double *buf = BRA ? c.lb : c.rk, *bx = BRA ? c.lbx : c.rkx;
+    int *bs = BRA ? c.lbs : c.rks;
     const int no = c.sz[c.h.outer];
-    const int top = (c.h.nwin > 1 ? c.h.wpos : 0) + 2;
-    const double tb = bound_tau(top, c.h.nwin, c.M.beta);
-    int m = c.h.lb_n - 1;
-    if (m < 0) {
-        copy_mat(c.lb, c.bnd + (long)top * c.nm * c.nm, c.sz[c.bndsst[top]] * no);
-        c.lbx[0] = c.bndlog[top];
-        c.lbs[0] = c.bndsst[top];
-        m = 0;
+    const int w = c.h.nwin > 1 ? c.h.wpos : 0;
+    int j = uni(BRA ? c.h.lb_n : c.h.rk_n) - 1;
+    State<NM> k;
+    int s;
+    double lg0;
+    if (j < 0) {
+        // the edge of the window
+        s = uni(BRA ? c.bndsst[w + 2] : c.h.kst_sst);
+        lg0 = BRA ? c.bndlog[w + 2] : c.h.kst_log;
+        k.load(BRA ? c.bnd + (long)(w + 2) * c.nm * c.nm : c.kst, c.sz[s], no);
+        seg_store<NM>(buf, 0, c.sz[s], no, k);
+        bx[0] = lg0;
+        bs[0] = s;
+        j = 0;
+    } else {
+        s = uni(bs[j]);
+        lg0 = bx[j];
+        k = seg_load<NM>(buf, j, c.sz[s], no);
     }
-    if (m < to) {
-        Work w;
-        int s = c.lbs[m];
-        double lg = c.lbx[m];
-        const Quad q;
-        double v = q.load(c.lb + (long)m * S2, c.sz[s], no);
-        double d;
-        const int m0 = m;
-        // the window operators nw-to .. nw-1-m0, walked downward
-        quad_walk<true>(c, q, v, s, lg, no, m0 > 0 ? c.wtau[nw - m0] : tb, c.wtau + (nw - to),
-                        c.wcode + (nw - to), to - m0, c.wtau[nw - to], d, w,
-                        [&](int k, double vk, int sk, int nsk, double lgk) {
-                            q.store(c.lb + (long)(m0 + k + 1) * S2, nsk, no, vk);
-                            c.lbx[m0 + k + 1] = lgk;
-                            c.lbs[m0 + k + 1] = sk;
-                        });
-        w.commit(c);
+    if (j < to) {
+        typedef typename Prefix<NM>::mat mat;
+        const Prefix<NM> px{(mat)(buf + (long)(j + 1) * S), (lds_d *)(bx + j + 1), (lds_i *)(bs + j + 1)};
+        // window operators j .. to-1 upward, or nw-1-j .. nw-to downward
+        const int a = BRA ? nw - to : j;
+        const double t0 = j > 0 ? c.wtau[BRA ? nw - j : j - 1] : bound_tau(BRA ? w + 2 : w, c.h.nwin, c.M.beta);
+        const double t1 = c.wtau[BRA ? nw - to : to - 1];
+        walk_small<NM, BRA, true>(k, s, t0, t1, (const lds_d *)(c.wtau + a), (const lds_i *)(c.wcode + a), to - j,
+                                  no, px);
+        // log scales of a walk count from its start
+        for (int i = j + 1 + lane_id(); i <= to; i += WAVE) bx[i] += lg0;
     }
-    c.h.lb_n = max(c.h.lb_n, to + 1);
+    (BRA ? c.h.lb_n : c.h.rk_n) = to + 1;
     wsync();
 }
 
@@ -1510,70 +1599,91 @@ DEV void lb_extend(Ctx &c, int nw, int to)
 // window's operators between rk[j0] and lb[m0]; t0 / t1 are the times of
 // those two states.  Returns false on a quantum-number violation.
 template <int NM>
-DEV bool segment_trace(Ctx &c, int nw, int j0, int m0, int a, int n, double t0, double t1, double &tl, double &ts)
+DEV bool segment_trace(Ctx &c, int nw, int j0, int m0, int a, int n, double t0, double t1, TraceVal &T)
 {
-    constexpr int S2 = NM * NM;
-    const int no = c.sz[c.h.outer];
-    if (c.h.rk_n <= j0) rk_extend<NM>(c, j0);
-    if (c.h.lb_n <= m0) lb_extend<NM>(c, nw, m0);
-    int s = c.rks[j0];
-    double lg = c.rkx[j0];
-    if constexpr (NM <= 4) {
-        const Quad q;
-        double v = q.load(c.rk + (long)j0 * S2, c.sz[s], no);
-        double d;
-        Work w;
-        const bool ok = quad_walk<false>(c, q, v, s, lg, no, t0, c.ttau + a, c.tcode + a, n, t1, d, w, NoAfter());
-        w.commit(c);
-        if (!ok || s != c.lbs[m0]) return false;
-        quad_contract(c, q, v * d, c.lb + (long)m0 * S2, s, no, lg + c.lbx[m0], tl, ts);
-        return true;
+    if constexpr (NM <= 16) {
+        const int no = c.sz[c.h.outer];
+        if (c.h.rk_n <= j0) seg_extend<NM, false>(c.ref(), nw, j0);
+        if (c.h.lb_n <= m0) seg_extend<NM, true>(c.ref(), nw, m0);
+        int s = c.rks[j0];
+        double lg = c.rkx[j0];
+        State<NM> k = seg_load<NM>(c.rk, j0, c.sz[s], no);
+        if (!walk_list<NM, false>(k, s, lg, no, t0, c.ttau + a, c.tcode + a, n, t1) || s != c.lbs[m0]) return false;
+        const State<NM> b = seg_load<NM>(c.lb, m0, c.sz[s], no);
+        double x = 0.0;
+#pragma unroll
+        for (int e = 0; e < State<NM>::NV; ++e) x = fma(k.v[e], b.v[e], x);
+        T = trace_of<NM>(x, lg + c.lbx[m0]);
     }
-    double *K = c.K0, *Kw = c.K1;
-    copy_mat(K, c.rk + (long)j0 * S2, c.sz[s] * no);
-    if (!ket_walk<NM>(c, K, Kw, s, lg, no, t0, c.ttau + a, c.tcode + a, n, t1)) return false;
-    if (s != c.lbs[m0]) return false;
-    contract(c, K, c.lb + (long)m0 * S2, s, no, lg + c.lbx[m0], tl, ts);
     return true;
 }
 
-// ---------------------------------------------------------------------------
-// removable pairs (ensure_valid_NPairs_diag, Trace.F90:1769-1810) in a list
-// ---------------------------------------------------------------------------
-DEV int pairs_from(const Ctx &c, const double *tau, const int *code, int n, int j)
+// Trace of a proposal: the window with its operators [j0, nw - m0) replaced by
+// the n entries of the trial list from a = j0 on; nl: length of the whole
+// trial list.  ok: no quantum-number violation.
+struct Proposal {
+    TraceVal T;
+    int ok;
+};
+template <int NM>
+__device__ __attribute__((noinline)) Proposal trace_proposal(ChainRef r, int nw_, int j0_, int m0_, int n_)
 {
-    const double te = tau[j];
-    if (te < c.h.tauwin_min || te > c.h.tauwin_max) return 0;
-    const int ce = code[j];
-    const int fe = c.fl(ce), ae = op_ca(ce);
-    // partners: later operators up to min(window end, te + taudiff_max); the
-    // list is read four entries at a time so that the LDS loads overlap
-    const double lim = fmin(c.h.tauwin_max, te + c.h.taudiff_max);
-    int cnt = 0;
-    for (int k = j + 1; k < n; k += 4) {
-        double tk[4];
-        int ck[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            tk[u] = k + u < n ? tau[k + u] : DBL_MAX;
-            ck[u] = k + u < n ? code[k + u] : 0;
-        }
-        bool stop = false;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            stop = stop || tk[u] > lim;
-            if (!stop && c.fl(ck[u]) == fe && op_ca(ck[u]) != ae) ++cnt;
-        }
-        if (stop) break;
+    Ctx c = attach<NM>(r);
+    const int nw = uni(nw_), j0 = uni(j0_), m0 = uni(m0_), n = uni(n_);
+    Proposal p;
+    p.T = TraceVal{0.0, 0.0, 0.0};
+    if (NM <= 16 && nw <= c.L.sc) {
+        const int w = c.h.nwin > 1 ? c.h.wpos : 0;
+        const double t0 = j0 > 0 ? c.wtau[j0 - 1] : bound_tau(w, c.h.nwin, c.M.beta);
+        const double t1 = m0 > 0 ? c.wtau[nw - m0] : bound_tau(w + 2, c.h.nwin, c.M.beta);
+        p.ok = segment_trace<NM>(c, nw, j0, m0, j0, n, t0, t1, p.T);
+    } else {
+        p.ok = window_trace<NM>(c, j0 + n + m0, p.T);
     }
-    return cnt;
+    return p;
 }
 
-DEV int npairs_list(const Ctx &c, const double *tau, const int *code, int n)
+// ---------------------------------------------------------------------------
+// removable pairs (ensure_valid_NPairs_diag, Trace.F90:1769-1810): for every
+// window operator the later operators of its flavour and the other type no
+// further than taudiff_max behind it.  pc[j] holds the counts of the first j+1
+// window operators together, so that the total is known and the pick of a
+// removal is one comparison per lane; kept until the window list changes.
+// ---------------------------------------------------------------------------
+template <int NM>
+__device__ __attribute__((noinline)) void count_pairs(ChainRef r)
 {
-    int cnt = 0;
-    for (int j = lane_id(); j < n; j += WAVE) cnt += pairs_from(c, tau, code, n, j);
-    return wave_isum(cnt);
+    Ctx c = attach<NM>(r);
+    const int nw = uni(c.h.wib - c.h.wia);
+    const double tdm = c.h.taudiff_max, wmax = c.h.tauwin_max;
+    int carry = 0;
+    for (int j0 = 0; j0 < nw; j0 += WAVE) {
+        const int j = j0 + lane_id();
+        int cnt = 0;
+        if (j < nw) {
+            const double lim = fmin(wmax, c.wtau[j] + tdm);
+            const int want = c.wcode[j] ^ 32;   // same flavour, other type
+            // the list is read four entries at a time so that the LDS loads overlap
+            for (int k = j + 1; k < nw; k += 4) {
+                double tk[4];
+                int ck[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    tk[u] = k + u < nw ? c.wtau[k + u] : DBL_MAX;
+                    ck[u] = k + u < nw ? c.wcode[k + u] : -1;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) cnt += tk[u] <= lim && ck[u] == want;
+                if (tk[3] > lim) break;
+            }
+        }
+        const int inc = wave_scan_i(cnt) + carry;
+        if (j < nw) c.pc[j] = inc;
+        carry = __builtin_amdgcn_readlane(inc, 63);
+    }
+    s_wenv.np = carry;
+    c.h.pc_valid = 1;
+    wsync();
 }
 
 // ---------------------------------------------------------------------------
@@ -1632,23 +1742,84 @@ DEV double config_sign(Ctx &c)
 // ---------------------------------------------------------------------------
 // hybridisation matrix algebra (MatrixUpdate.F90)
 // ---------------------------------------------------------------------------
-// S - R^T M Q for an order-k block (get_DetRatAdd)
-DEV double detrat_add(Ctx &c, const double *Mf, int k, double S)
-{
-    // lanes over the k^2 elements: every load of M is issued at once
-    const int ld = c.L.kcap;
-    double part = 0.0;
-    for (int idx = lane_id(); idx < k * k; idx += WAVE) {
-        const int i = idx % k, j = idx / k;
-        part = fma(c.R[i] * Mf[i + (long)j * ld], c.Q[j], part);
+// Lanes over the elements (i, j) of a k x k block without divisions: groups of
+// 16, 32 or 64 lanes hold a column each, so lane l keeps row i = l mod G and
+// takes the columns g, g + 64/G, ...
+struct MatLanes {
+    int i, g, step;
+    DEV explicit MatLanes(int k)
+    {
+        const int l = lane_id();
+        if (k <= 16) i = l & 15, g = l >> 4, step = 4;
+        else if (k <= 32) i = l & 31, g = l >> 5, step = 2;
+        else i = l, g = 0, step = 1;
     }
-    return S - wave_sum(part);
+    // sum over the lanes that hold the same row
+    DEV double rows(double v) const
+    {
+        if (step >= 2) v += __shfl_xor(v, 32, WAVE);
+        if (step == 4) v += __shfl_xor(v, 16, WAVE);
+        return v;
+    }
+};
+
+// M(i,j) += (a col(i)) row(j)
+DEV void rank1(Ctx &c, double *Mf, int k, const MatLanes &ml, double a, const double *col, const double *row)
+{
+    const int ld = c.L.kcap;
+    for (int i0 = 0; i0 < k; i0 += WAVE) {
+        const int i = i0 + ml.i;
+        const bool in = i < k;
+        double *Mi = Mf + (in ? i : 0);
+        const double ci = in ? a * col[i] : 0.0;
+        for (int j0 = ml.g; j0 < k; j0 += 8 * ml.step) {
+            double m[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) m[u] = Mi[(long)min(j0 + u * ml.step, k - 1) * ld];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int j = j0 + u * ml.step;
+                if (in && j < k) Mi[(long)j * ld] = fma(ci, row[j], m[u]);
+            }
+        }
+    }
+}
+
+// R^T M Q of an order-k block (get_DetRatAdd); leaves M Q in colb.  The loads
+// of eight columns are in flight together.
+DEV double detrat_add(Ctx &c, const double *Mf, int k)
+{
+    const int ld = c.L.kcap;
+    const MatLanes ml(k);
+    double part = 0.0;
+    for (int i0 = 0; i0 < k; i0 += WAVE) {
+        const int i = i0 + ml.i;
+        const bool in = i < k;
+        const double *col = Mf + (in ? i : 0);
+        double acc = 0.0;
+        for (int j0 = ml.g; j0 < k; j0 += 8 * ml.step) {
+            double m[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) m[u] = col[(long)min(j0 + u * ml.step, k - 1) * ld];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int j = j0 + u * ml.step;
+                acc = fma(m[u], j < k ? c.Q[j] : 0.0, acc);
+            }
+        }
+        acc = ml.rows(acc);
+        if (in && ml.g == 0) {
+            c.colb[i] = acc;
+            part = fma(c.R[i], acc, part);
+        }
+    }
+    return wave_sum(part);
 }
 
 // Bordering update to order k+1, get_MatAdd (MatrixUpdate.F90:410-442), on
 // physical storage: the new creator takes physical row k, the new annihilator
 // physical column k, so no entry moves.  c.Q holds Q by physical column, c.R
-// holds R by physical row.
+// holds R by physical row, c.colb M Q (detrat_add).
 //   col(i) = -(M Q)_i / dr,  row(j) = -(R M)_j / dr,
 //   M(i,j) += dr col(i) row(j),  M(i,k) = col(i),  M(k,j) = row(j),  M(k,k) = 1/dr
 DEV void mat_add_phys(Ctx &c, double *Mf, int k, double dr)
@@ -1656,24 +1827,28 @@ DEV void mat_add_phys(Ctx &c, double *Mf, int k, double dr)
     const int ld = c.L.kcap;
     const int l = lane_id();
     double *col = c.colb, *row = c.rowb;
-    for (int i = l; i < k; i += WAVE) {
+    // columns of M against R: the lane's column is contiguous
+    const MatLanes ml(k);
+    for (int j0 = 0; j0 < k; j0 += WAVE) {
+        const int j = j0 + ml.i;
+        const double *mc = Mf + (long)min(j, k - 1) * ld;
         double v = 0.0;
-#pragma unroll 8
-        for (int j = 0; j < k; ++j) v = fma(Mf[i + (long)j * ld], c.Q[j], v);
-        col[i] = -v / dr;
+        for (int i0 = ml.g; i0 < k; i0 += 8 * ml.step) {
+            double m[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) m[u] = mc[min(i0 + u * ml.step, k - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = i0 + u * ml.step;
+                v = fma(i < k ? c.R[i] : 0.0, m[u], v);
+            }
+        }
+        v = ml.rows(v);
+        if (j < k && ml.g == 0) row[j] = -v / dr;
     }
-    for (int j = l; j < k; j += WAVE) {
-        double v = 0.0;
-        const double *mc = Mf + (long)j * ld;
-#pragma unroll 8
-        for (int i = 0; i < k; ++i) v = fma(c.R[i], mc[i], v);
-        row[j] = -v / dr;
-    }
+    for (int i = l; i < k; i += WAVE) col[i] = -col[i] / dr;
     wsync();
-    for (int idx = l; idx < k * k; idx += WAVE) {
-        const int i = idx % k, j = idx / k;
-        Mf[i + (long)j * ld] = fma(dr * col[i], row[j], Mf[i + (long)j * ld]);
-    }
+    rank1(c, Mf, k, ml, dr, col, row);
     for (int i = l; i < k; i += WAVE) {
         Mf[i + (long)k * ld] = col[i];
         Mf[k + (long)i * ld] = row[i];
@@ -1696,11 +1871,7 @@ DEV void mat_rem_phys(Ctx &c, double *Mf, int k, int sc, int sa)
         rowp[i] = Mf[sc + (long)i * ld];
     }
     wsync();
-    const double inv = 1.0 / rowp[sa];
-    for (int idx = l; idx < k * k; idx += WAVE) {
-        const int i = idx % k, j = idx / k;
-        Mf[i + (long)j * ld] = fma(-colp[i] * inv, rowp[j], Mf[i + (long)j * ld]);
-    }
+    rank1(c, Mf, k, MatLanes(k), -(1.0 / rowp[sa]), colp, rowp);
     wsync();
     const int last = k - 1;
     if (sc != last) {
@@ -1810,31 +1981,73 @@ DEV void build_delta(Ctx &c, int f, int k, double *D, int ld, const double *fcl,
 // array edits (lane-parallel shifts; chunks ordered so nothing is overwritten
 // before it is read)
 // ---------------------------------------------------------------------------
-// Move arr[from, to) by `by` places (either sign).  Rounds of 8 elements per
-// lane: all loads of a round complete before its stores, and rounds run from
-// the end that is written into first, so nothing is overwritten unread.
-template <typename T>
-DEV void block_move(T *arr, int from, int to, int by)
+// Move the operators [from, to) by `by` places (either sign).  Rounds of 4
+// operators per lane: all loads of a round complete before its stores, and
+// rounds run from the end that is written into first, so nothing is
+// overwritten unread.
+DEV void move_ops(Ctx &c, int from, int to, int by)
 {
-    constexpr int U = 8, R = U * WAVE;
+    constexpr int U = 4, R = U * WAVE;
     const int l = lane_id();
     const int cnt = to - from;
     if (cnt <= 0 || by == 0) return;
     const int nr = (cnt + R - 1) / R;
     for (int q = 0; q < nr; ++q) {
-        const int r = by > 0 ? nr - 1 - q : q;
-        const int b = from + r * R;
-        T v[U];
+        const int b = from + (by > 0 ? nr - 1 - q : q) * R + l;
+        double t[U];
+        int cd[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = b + u * WAVE + l;
-            if (i < to) v[u] = arr[i];
-        }
+        for (int u = 0; u < U; ++u)
+            if (b + u * WAVE < to) t[u] = c.tau[b + u * WAVE], cd[u] = c.code[b + u * WAVE];
         wsync();
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = b + u * WAVE + l;
-            if (i < to) arr[i + by] = v[u];
+        for (int u = 0; u < U; ++u)
+            if (b + u * WAVE < to) c.tau[b + u * WAVE + by] = t[u], c.code[b + u * WAVE + by] = cd[u];
+        wsync();
+    }
+}
+
+// A pair joins the flavour lists (sorted times and their physical slots) of
+// length k: creator tc at rank pc, annihilator ta at rank pa, both in slot k.
+DEV void lists_insert(Ctx &c, long fo, int k, int pc, double tc, int pa, double ta)
+{
+    double *fc = c.fc + fo, *fa = c.fa + fo;
+    int *fcs = c.fcs + fo, *fas = c.fas + fo;
+    for (int b = k / WAVE * WAVE; b >= 0; b -= WAVE) {
+        const int j = b + lane_id();
+        const bool mc = j > pc && j <= k, ma = j > pa && j <= k;
+        double vc = tc, va = ta;
+        int sc = k, sa = k;
+        if (mc) vc = fc[j - 1], sc = fcs[j - 1];
+        if (ma) va = fa[j - 1], sa = fas[j - 1];
+        wsync();
+        if (mc || j == pc) fc[j] = vc, fcs[j] = sc;
+        if (ma || j == pa) fa[j] = va, fas[j] = sa;
+        wsync();
+    }
+}
+
+// The creator of rank pc (slot sc) and the annihilator of rank pa (slot sa)
+// leave the flavour lists of length k; the operators that owned the last slot
+// take the freed ones.
+DEV void lists_remove(Ctx &c, long fo, int k, int pc, int sc, int pa, int sa)
+{
+    double *fc = c.fc + fo, *fa = c.fa + fo;
+    int *fcs = c.fcs + fo, *fas = c.fas + fo;
+    for (int b = 0; b < k; b += WAVE) {
+        const int j = b + lane_id();
+        const bool in = j < k - 1;
+        double vc = 0.0, va = 0.0;
+        int xc = 0, xa = 0;
+        if (in) {
+            const int jc = j + (j >= pc), ja = j + (j >= pa);
+            vc = fc[jc], xc = fcs[jc];
+            va = fa[ja], xa = fas[ja];
+        }
+        wsync();
+        if (in) {
+            fc[j] = vc, fcs[j] = xc == k - 1 ? sc : xc;
+            fa[j] = va, fas[j] = xa == k - 1 ? sa : xa;
         }
         wsync();
     }
@@ -1854,10 +2067,12 @@ DEV int count_below_par(const double *arr, int n, double x)
 enum { OUT_REJ = 0, OUT_ACC = 1, OUT_QN = 2 };
 enum { ERR_CAP = 3, ERR_SING = 4, ERR_STATE_DEV = 6 };
 
-DEV void store_part(Ctx &c, int no)
+// Whether every flavour can take one more pair and the list two more operators
+DEV void room_left(Ctx &c)
 {
-    for (int i = lane_id(); i < 2 * no; i += WAVE) c.part[i] = c.pl[i];
-    wsync();
+    int km = 0;
+    for (int f = 0; f < c.M.nf; ++f) km = max(km, c.h.kf[f]);
+    s_wenv.full = km + 1 > c.L.kcap || c.h.nop + 2 > c.L.cap;
 }
 
 // write the LDS trial list into the global operator list at wia (its length
@@ -1866,8 +2081,7 @@ DEV void store_part(Ctx &c, int no)
 DEV void commit_window(Ctx &c, int nl)
 {
     const int nw = c.h.wib - c.h.wia;
-    block_move(c.tau, c.h.wib, c.h.nop, nl - nw);
-    block_move(c.code, c.h.wib, c.h.nop, nl - nw);
+    move_ops(c, c.h.wib, c.h.nop, nl - nw);
     for (int j = lane_id(); j < nl; j += WAVE) {
         c.tau[c.h.wia + j] = c.ttau[j];
         c.code[c.h.wia + j] = c.tcode[j];
@@ -1892,279 +2106,293 @@ DEV void record_pair(Ctx &c, int f, double dt)
     if (c.h.apt_index <= c.h.apt_n) c.h.apt_index++;
 }
 
-// StepAdd (CTQMC.F90:3353-3612), change_outer = false
+// an accepted insertion / removal: what the proposal found
+struct AddMove {
+    int f, k, nl, q1, q2, fp_c, fp_a;   // flavour, its order, length of the trial list, insertion points, FPos
+    double ta, tc, S, dr_sign;          // times, determinant ratio and its sign with the permutation's
+    double cfg_ratio;                   // change of the configuration sign but for the trace's
+    TraceVal T;
+};
+struct RemMove {
+    int f, k, nl, w1, w2, fp_c, fp_a, sc, sa;   // window indices of the pair, its physical slots
+    double dt, S, dr_sign, cfg_ratio;
+    TraceVal T;
+};
+
+// accept: M, operator list, flavour lists, weights, sign
 template <int NM>
-DEV int step_add(Ctx &c)
+__device__ __attribute__((noinline)) void accept_add(ChainRef ref, AddMove m)
 {
-    const DevModel &M = c.M;
-    c.h.try_add++;
-    const double width = c.h.tauwin_max - c.h.tauwin_min;
-    const double tref = c.h.tauwin_min + width * grnd(c.rng);
-    double tdf = width;
-    const int orb = randint(c.rng, 1, M.nb) - 1;
-    const int spin = randint(c.rng, 1, 2) - 1;
-    const double tmin = fmax(tref - c.h.taudiff_max, c.h.tauwin_min);
-    const double w2 = fmin(tref + c.h.taudiff_max, c.h.tauwin_max) - tmin;
-    const double t2 = tmin + w2 * grnd(c.rng);
-    tdf *= w2;
-    const int f = orb + M.nb * spin;
-    if (t2 == tref) return c.h.qn_rej++, OUT_QN;
-    const int k = c.h.kf[f];
-    // room_for_move checked these before the move's first draw; a failure here
-    // is a logic error, not a full chain
-    if (!ensure_window(c) || c.h.wib - c.h.wia + 2 > c.L.lcap_lds || k + 1 > c.L.kcap ||
-        c.h.nop + 2 > c.L.cap) {
-        c.h.err = ERR_STATE_DEV;
-        return OUT_REJ;
-    }
-    const int nw = c.h.wib - c.h.wia;
-    ensure_cache<NM>(c);
-    // equal times (process_OperAdd, Trace.F90:4287-4380) and insertion points
-    const double ta = tref, tc = t2;
-    const double t1 = fmin(ta, tc), t2o = fmax(ta, tc);
-    const int code_a = mk_code(orb, spin, 2), code_c = mk_code(orb, spin, 1);
-    const int code1 = ta < tc ? code_a : code_c, code2 = ta < tc ? code_c : code_a;
-    int eq = 0, q1 = 0, q2 = 0;
-    for (int j = lane_id(); j < nw; j += WAVE) {
-        const double x = c.wtau[j];
-        eq |= (x == t1) | (x == t2o);
-        q1 += x < t1;
-        q2 += x < t2o;
-    }
-    if (wave_isum(eq)) return c.h.qn_rej++, OUT_QN;
-    q1 = wave_isum(q1);
-    q2 = wave_isum(q2);
-    // trial list: the window with t1 before index q1 and t2o before index q2
-    for (int j = lane_id(); j < nw + 2; j += WAVE) {
-        double x;
-        int cd;
-        if (j < q1) x = c.wtau[j], cd = c.wcode[j];
-        else if (j == q1) x = t1, cd = code1;
-        else if (j <= q2) x = c.wtau[j - 1], cd = c.wcode[j - 1];
-        else if (j == q2 + 1) x = t2o, cd = code2;
-        else x = c.wtau[j - 2], cd = c.wcode[j - 2];
-        c.ttau[j] = x;
-        c.tcode[j] = cd;
-    }
-    wsync();
-    const int nl = nw + 2;
-    double tl, ts;
-    const bool seg = NM <= 4 && nw <= c.L.sc;
-    if (seg) {
-        const int p = c.h.nwin > 1 ? c.h.wpos : 0;
-        const double t0 = q1 > 0 ? c.wtau[q1 - 1] : bound_tau(p, c.h.nwin, c.M.beta);
-        const double t1e = q2 < nw ? c.wtau[q2] : bound_tau(p + 2, c.h.nwin, c.M.beta);
-        if (!segment_trace<NM>(c, nw, q1, nw - q2, q1, q2 - q1 + 2, t0, t1e, tl, ts))
-            return c.h.qn_rej++, OUT_QN;
-    } else if (!window_trace<NM>(c, nl, tl, ts)) {
-        return c.h.qn_rej++, OUT_QN;
-    }
-    // det ratio, get_LogDetRatPairAdd (Trace.F90:2775-2832): Q (annihilators) and
-    // R (creators) placed by physical slot; FPos = 1 + earlier operators of the type
+    Ctx c = attach<NM>(ref);
+    const int f = uni(m.f), k = uni(m.k), nl = uni(m.nl), q1 = uni(m.q1), q2 = uni(m.q2), fp_c = uni(m.fp_c),
+              fp_a = uni(m.fp_a), nw = nl - 2;
+    const double S = m.S, tc = m.tc, ta = m.ta;
     const long fo = (long)f * c.L.kcap;
-    const double *ctl = c.fc + fo, *atl = c.fa + fo;
-    const int *csl = c.fcs + fo, *asl = c.fas + fo;
-    int fpc = 0, fpa = 0;
-    for (int j = lane_id(); j < k; j += WAVE) {
-        const double xa = atl[j], xc = ctl[j];
-        c.Q[asl[j]] = hybr(M, xa - tc, f);
-        c.R[csl[j]] = hybr(M, ta - xc, f);
-        fpa += xa < ta;
-        fpc += xc < tc;
-    }
-    const int fp_c = wave_isum(fpc) + 1, fp_a = wave_isum(fpa) + 1;
-    wsync();
-    const double S = detrat_add(c, c.mi(f), k, hybr(M, ta - tc, f));
-    c.wflops += 2.0 * k * k;
-    c.wbytes += 8.0 * k * k;
-    const double sig = (abs(fp_c - fp_a) % 2) ? -1.0 : 1.0;
-    const double dr_log = log(fabs(S)), dr_sign = copysign(1.0, S) * sig;
-    const double rnd = grnd(c.rng);
-    // NPairs of the new configuration: pairs with both ends in the window all
-    // lie in the trial list
-    const int np = npairs_list(c, c.ttau, c.tcode, nl);
-    const double wr = exp((tl - c.h.trace_log) + dr_log);
-    const double prob = fabs(((1.0 * tdf) * (double)(2 * M.nb)) / (double)np * wr);
-    if (!(rnd < prob)) return OUT_REJ;
-    // accept: M, operator list, flavour lists, weights, sign
+    const bool seg = NM <= 16 && nw <= c.L.sc;
     mat_add_phys(c, c.mi(f), k, S);
-    c.wflops += 6.0 * k * k;
-    c.wbytes += 8.0 * k * k + 8.0 * (k + 1) * (k + 1);
+    c.work(6.0 * k * k, 8.0 * k * k + 8.0 * (k + 1) * (k + 1));
     commit_window(c, nl);
     c.h.pc_valid = 0;
     // segment caches: the first q1 and the last nw - q2 window operators are unchanged
     c.h.rk_n = seg ? min(c.h.rk_n, q1 + 1) : 0;
     c.h.lb_n = seg ? min(c.h.lb_n, nw - q2 + 1) : 0;
-    double *fcf = c.fc + fo, *faf = c.fa + fo;
-    int *fcsf = c.fcs + fo, *fasf = c.fas + fo;
-    block_move(fcf, fp_c - 1, k, 1);
-    block_move(fcsf, fp_c - 1, k, 1);
-    block_move(faf, fp_a - 1, k, 1);
-    block_move(fasf, fp_a - 1, k, 1);
-    if (lane_id() == 0) {
-        fcf[fp_c - 1] = tc;
-        fcsf[fp_c - 1] = k;
-        faf[fp_a - 1] = ta;
-        fasf[fp_a - 1] = k;
-    }
-    wsync();
+    lists_insert(c, fo, k, fp_c - 1, tc, fp_a - 1, ta);
     c.h.kf[f] = k + 1;
     c.h.kfmax[f] = max(c.h.kfmax[f], k + 1);
-    record_pair(c, f, t2o - t1);
-    c.h.det_log += dr_log;
-    c.h.det_sign *= dr_sign;
-    c.h.trace_log = tl;
-    c.h.trace_sign = ts;
-    store_part(c, c.sz[c.h.outer]);
-    c.h.cfgsign = -config_sign(c);
+    room_left(c);
+    record_pair(c, f, fabs(ta - tc));
+    c.h.det_log += log(fabs(S));
+    c.h.det_sign *= m.dr_sign;
+    c.h.cfgsign *= m.cfg_ratio * c.h.trace_sign;
+    keep_trace<NM>(c, m.T);
+    c.h.cfgsign *= c.h.trace_sign;
     c.h.acc_add++;
+}
+
+// |new weight / old weight| of a trace T and a determinant ratio S: one
+// exponential; through the logarithms where that could leave the FP64 range
+DEV double weight_ratio(const TraceVal &T, double S, double trace_log)
+{
+    const double d = T.lg - trace_log;
+    if (fabs(d) < 500.0) return fabs(T.S * S) * exp(d);
+    return exp((T.log_abs() - trace_log) + log(fabs(S)));
+}
+
+// StepAdd (CTQMC.F90:3353-3612), change_outer = false
+template <int NM>
+DEV int step_add(Ctx &c)
+{
+    CModel &M = c.M;
+    const double wmin = c.h.tauwin_min, wmax = c.h.tauwin_max, tdm = c.h.taudiff_max;
+    const int nw = uni(c.h.wib - c.h.wia);
+    const double width = wmax - wmin;
+    const double tref = wmin + width * grnd(c.rng);
+    double tdf = width;
+    const int orb = randint(c.rng, 1, M.nb) - 1;
+    const int spin = randint(c.rng, 1, 2) - 1;
+    const double tmin = fmax(tref - tdm, wmin);
+    const double w2 = fmin(tref + tdm, wmax) - tmin;
+    const double t2 = tmin + w2 * grnd(c.rng);
+    tdf *= w2;
+    const int f = orb + M.nb * spin;
+    if (t2 == tref) return OUT_QN;
+    const int k = uni(c.h.kf[f]);
+    if (!c.h.pc_valid) count_pairs<NM>(c.ref());
+    ensure_cache<NM>(c);
+    // equal times (process_OperAdd, Trace.F90:4287-4380), insertion points, the
+    // removable pairs that the two operators form with those of the window, and
+    // the trial list: the window with t1 before index q1 and t2o before index q2
+    const double ta = tref, tc = t2;
+    const double t1 = fmin(ta, tc), t2o = fmax(ta, tc);
+    const int code_a = mk_code(orb, spin, 2), code_c = mk_code(orb, spin, 1);
+    int q1 = 0, q2 = 0, np = uni(s_wenv.np) + (t2o <= t1 + tdm ? 1 : 0);
+    bool eq = false;
+    for (int j0 = 0; j0 < nw; j0 += WAVE) {
+        const int j = j0 + lane_id();
+        const bool in = j < nw;
+        const double x = in ? c.wtau[j] : DBL_MAX;
+        const int cd = in ? c.wcode[j] : 0;
+        const bool b1 = x < t1, b2 = x < t2o;
+        eq = eq || __ballot(x == t1 || x == t2o) != 0ull;
+        q1 += popc64(__ballot(b1));
+        q2 += popc64(__ballot(b2));
+        const double mate = cd == code_c ? ta : tc;
+        const bool pair = in && (cd == code_c || cd == code_a) && fmax(x, mate) <= fmin(x, mate) + tdm;
+        np += popc64(__ballot(pair));
+        if (in) {
+            const int d = j + !b1 + !b2;
+            c.ttau[d] = x;
+            c.tcode[d] = cd;
+        }
+    }
+    if (eq) return OUT_QN;
+    if (lane_id() < 2) {
+        const bool second = lane_id() == 1;
+        const int d = second ? q2 + 1 : q1;
+        c.ttau[d] = second ? t2o : t1;
+        c.tcode[d] = ((ta < tc) != second) ? code_a : code_c;
+    }
+    wsync();
+    const int nl = nw + 2;
+    const Proposal pr = trace_proposal<NM>(c.ref(), nw, q1, nw - q2, q2 - q1 + 2);
+    if (!pr.ok) return OUT_QN;
+    const TraceVal T = pr.T;
+    // det ratio, get_LogDetRatPairAdd (Trace.F90:2775-2832): Q (annihilators) and
+    // R (creators) placed by physical slot, the lane behind the last rank takes
+    // S0 = F(ta - tc); FPos = 1 + earlier operators of the type
+    const long fo = (long)f * c.L.kcap;
+    const double *ctl = c.fc + fo, *atl = c.fa + fo;
+    const int *csl = c.fcs + fo, *asl = c.fas + fo;
+    int fp_c = 1, fp_a = 1, sgn = q2 - q1 + (ta > tc) + 1;
+    double S0 = 0.0;
+    for (int j0 = 0; j0 <= k; j0 += WAVE) {
+        const int j = j0 + lane_id();
+        const bool in = j < k;
+        double xa = ta, xc = tc;
+        int sa = 0, sc = 0;
+        if (in) xa = atl[j], xc = ctl[j], sa = asl[j], sc = csl[j];
+        const double q = hybr(M, xa - tc, f), r = hybr(M, ta - xc, f);
+        if (in) {
+            c.Q[sa] = q;
+            c.R[sc] = r;
+        }
+        if (k - j0 < WAVE) S0 = readlane_d(q, k - j0);
+        const bool a_lt = in && xa < ta, c_lt = in && xc < tc;
+        fp_a += popc64(__ballot(a_lt));
+        fp_c += popc64(__ballot(c_lt));
+        // sign change of the operator order (config_sign): operators of other
+        // flavours between the pair, creators of its own between them, and
+        // operators of its own behind the new creator
+        const bool abet = in && xa > t1 && xa < t2o;
+        sgn += popc64(__ballot(abet)) + popc64(__ballot(in && xc > tc)) + popc64(__ballot(in && xa > tc));
+    }
+    wsync();
+    const double S = S0 - detrat_add(c, c.mi(f), k);
+    c.work(2.0 * k * k, 8.0 * k * k);
+    const double sig = ((fp_c - fp_a) & 1) ? -1.0 : 1.0;
+    const double dr_sign = copysign(1.0, S) * sig;
+    const double rnd = grnd(c.rng);
+    const double wr = weight_ratio(T, S, c.h.trace_log);
+    const double prob = fabs(((1.0 * tdf) * (double)(2 * M.nb)) / (double)np * wr);
+    if (!(rnd < prob)) return OUT_REJ;
+    accept_add<NM>(c.ref(), AddMove{f, k, nl, q1, q2, fp_c, fp_a, ta, tc, S, dr_sign,
+                                    (sgn & 1) ? -dr_sign : dr_sign, T});
+    c.lists();
     return OUT_ACC;
 }
 
-// rank whose slot equals `slot` in a slot list of length k (-1 if none)
-DEV int find_slot(const int *sl, int k, int slot)
+template <int NM>
+__device__ __attribute__((noinline)) void accept_rem(ChainRef ref, RemMove m)
 {
-    int r = -1;
-    for (int j = lane_id(); j < k; j += WAVE)
-        if (sl[j] == slot) r = j;
-    return wave_imax(r);
+    Ctx c = attach<NM>(ref);
+    const int f = uni(m.f), k = uni(m.k), nl = uni(m.nl), w1 = uni(m.w1), w2 = uni(m.w2), fp_c = uni(m.fp_c),
+              fp_a = uni(m.fp_a), sc = uni(m.sc), sa = uni(m.sa), nw = nl + 2;
+    const double S = m.S;
+    const long fo = (long)f * c.L.kcap;
+    const bool seg = NM <= 16 && nw <= c.L.sc;
+    mat_rem_phys(c, c.mi(f), k, sc, sa);
+    c.work(3.0 * k * k, 8.0 * k * k + 8.0 * (k - 1) * (k - 1));
+    commit_window(c, nl);
+    c.h.pc_valid = 0;
+    // segment caches: the first w1 and the last nw - 1 - w2 window operators are unchanged
+    c.h.rk_n = seg ? min(c.h.rk_n, w1 + 1) : 0;
+    c.h.lb_n = seg ? min(c.h.lb_n, nw - w2) : 0;
+    lists_remove(c, fo, k, fp_c - 1, sc, fp_a - 1, sa);
+    c.h.kf[f] = k - 1;
+    room_left(c);
+    record_pair(c, f, m.dt);
+    c.h.det_log += log(fabs(S));
+    c.h.det_sign *= m.dr_sign;
+    c.h.cfgsign *= m.cfg_ratio * c.h.trace_sign;
+    keep_trace<NM>(c, m.T);
+    c.h.cfgsign *= c.h.trace_sign;
+    c.h.acc_rem++;
 }
 
 // StepRem (CTQMC.F90:3892-4150) with gen_OperRemove (Trace.F90:4851-4977)
 template <int NM>
 DEV int step_rem(Ctx &c)
 {
-    const DevModel &M = c.M;
-    c.h.try_rem++;
-    if (!ensure_window(c)) {
-        c.h.err = ERR_STATE_DEV;
-        return OUT_REJ;
-    }
-    const int nw = c.h.wib - c.h.wia;
+    CModel &M = c.M;
+    const int nw = uni(c.h.wib - c.h.wia);
+    if (!c.h.pc_valid) count_pairs<NM>(c.ref());
     ensure_cache<NM>(c);
-    // pair counts per window operator (the window holds every removable pair)
-    // (kept in LDS until the window list changes)
-    if (!c.h.pc_valid) {
-        for (int j = lane_id(); j < nw; j += WAVE) c.pc[j] = pairs_from(c, c.wtau, c.wcode, nw, j);
-        c.h.pc_valid = 1;
-        wsync();
-    }
-    int np = 0;
-    for (int j0 = 0; j0 < nw; j0 += WAVE) {
-        const int j = j0 + lane_id();
-        np += wave_isum(j < nw ? c.pc[j] : 0);
-    }
-    if (np <= 0) return c.h.qn_rej++, OUT_QN;
+    const int np = uni(s_wenv.np);
+    if (np <= 0) return OUT_QN;
     int pick = randint(c.rng, 1, np);
-    int w1 = -1, w2 = -1;
-    {
-        int base = 0;
-        for (int j0 = 0; j0 < nw && w1 < 0; j0 += WAVE) {
-            const int j = j0 + lane_id();
-            const int cnt = j < nw ? c.pc[j] : 0;
-            int tot;
-            const int ex = wave_excl_scan(cnt, &tot);
-            int found = (pick > base + ex && pick <= base + ex + cnt) ? j : -1;
-            found = wave_imax(found);
-            if (found >= 0) {
-                int want = pick - base - __shfl(ex, found - j0, WAVE);
-                const int ce = c.wcode[found];
-                const int fe = c.fl(ce), ae = op_ca(ce);
-                int kk = found + 1;
-                for (; kk < nw; ++kk) {
-                    const int ck = c.wcode[kk];
-                    if (c.fl(ck) == fe && op_ca(ck) != ae)
-                        if (--want <= 0) break;
-                }
-                w1 = found;
-                w2 = kk;
-            }
-            base += tot;
-        }
+    // the pick-th pair: the operator w1 whose running count reaches it, and
+    // among the later operators of its flavour and the other type the one that
+    // the rest of the count names
+    int w1 = -1, w2 = -1, want = pick;
+    for (int j0 = 0; j0 < nw && w1 < 0; j0 += WAVE) {
+        const int j = j0 + lane_id();
+        const int pc = j < nw ? c.pc[j] : 0;
+        const unsigned long long at = __ballot(j < nw && pc >= pick);
+        const int b = at ? __builtin_ctzll(at) : WAVE;
+        if (b > 0) want = pick - __builtin_amdgcn_readlane(pc, b - 1);
+        if (at) w1 = j0 + b;
     }
-    if (w1 < 0 || w2 >= nw) {
+    if (w1 < 0) {
         c.h.err = ERR_STATE_DEV;
         return OUT_REJ;
     }
-    const int c1 = c.wcode[w1];
+    const int c1 = uni(c.wcode[w1]);
+    for (int j0 = w1 / WAVE * WAVE; j0 < nw && w2 < 0; j0 += WAVE) {
+        const int j = j0 + lane_id();
+        unsigned long long mate = __ballot(j > w1 && j < nw && c.wcode[j < nw ? j : 0] == (c1 ^ 32));
+        const int n = popc64(mate);
+        if (n < want) {
+            want -= n;
+            continue;
+        }
+        for (; want > 1; --want) mate &= mate - 1;
+        w2 = j0 + __builtin_ctzll(mate);
+    }
+    if (w2 < 0) {
+        c.h.err = ERR_STATE_DEV;
+        return OUT_REJ;
+    }
     const double t1 = c.wtau[w1], t2 = c.wtau[w2];
+    const double wmin = c.h.tauwin_min, wmax = c.h.tauwin_max, tdm = c.h.taudiff_max;
     const int f = c.fl(c1);
-    const int k = c.h.kf[f];
+    const int k = uni(c.h.kf[f]);
     const double tc = op_ca(c1) == 1 ? t1 : t2, ta = op_ca(c1) == 1 ? t2 : t1;
-    const double hprf = (double)np /
-                        ((c.h.tauwin_max - c.h.tauwin_min) *
-                         (fmin(ta + c.h.taudiff_max, c.h.tauwin_max) - fmax(ta - c.h.taudiff_max, c.h.tauwin_min)));
+    const double hprf = (double)np / ((wmax - wmin) * (fmin(ta + tdm, wmax) - fmax(ta - tdm, wmin)));
     // trial list: the window without entries w1 < w2
     const int nl = nw - 2;
-    for (int j = lane_id(); j < nl; j += WAVE) {
-        const int src = j < w1 ? j : (j < w2 - 1 ? j + 1 : j + 2);
-        c.ttau[j] = c.wtau[src];
-        c.tcode[j] = c.wcode[src];
+    for (int j = lane_id(); j < nw; j += WAVE) {
+        const double x = c.wtau[j];
+        const int cd = c.wcode[j];
+        if (j != w1 && j != w2) {
+            const int d = j - (j > w1) - (j > w2);
+            c.ttau[d] = x;
+            c.tcode[d] = cd;
+        }
     }
     wsync();
-    double tl, ts;
-    const bool seg = NM <= 4 && nw <= c.L.sc;
-    if (seg) {
-        const int p = c.h.nwin > 1 ? c.h.wpos : 0;
-        const double t0 = w1 > 0 ? c.wtau[w1 - 1] : bound_tau(p, c.h.nwin, c.M.beta);
-        const double t1e = w2 + 1 < nw ? c.wtau[w2 + 1] : bound_tau(p + 2, c.h.nwin, c.M.beta);
-        if (!segment_trace<NM>(c, nw, w1, nw - 1 - w2, w1, w2 - w1 - 1, t0, t1e, tl, ts))
-            return c.h.qn_rej++, OUT_QN;
-    } else if (!window_trace<NM>(c, nl, tl, ts)) {
-        return c.h.qn_rej++, OUT_QN;
-    }
+    const Proposal pr = trace_proposal<NM>(c.ref(), nw, w1, nw - 1 - w2, w2 - w1 - 1);
+    if (!pr.ok) return OUT_QN;
+    const TraceVal T = pr.T;
+    // ranks and slots of the pair; sign change as in step_add
     const long fo = (long)f * c.L.kcap;
-    const int fp_c = count_below_par(c.fc + fo, k, tc) + 1, fp_a = count_below_par(c.fa + fo, k, ta) + 1;
-    const int sc = c.fcs[fo + fp_c - 1], sa = c.fas[fo + fp_a - 1];
+    const double *ctl = c.fc + fo, *atl = c.fa + fo;
+    const int *csl = c.fcs + fo, *asl = c.fas + fo;
+    int fp_c = 1, fp_a = 1, sc = 0, sa = 0, sgn = w2 - w1 - 1 + 1;
+    for (int j0 = 0; j0 < k; j0 += WAVE) {
+        const int j = j0 + lane_id();
+        const bool in = j < k;
+        double xa = 0.0, xc = 0.0;
+        int xsa = 0, xsc = 0;
+        if (in) xa = atl[j], xc = ctl[j], xsa = asl[j], xsc = csl[j];
+        fp_a += popc64(__ballot(in && xa < ta));
+        fp_c += popc64(__ballot(in && xc < tc));
+        if (fp_a - 1 >= j0 && fp_a - 1 < j0 + WAVE) sa = __builtin_amdgcn_readlane(xsa, fp_a - 1 - j0);
+        if (fp_c - 1 >= j0 && fp_c - 1 < j0 + WAVE) sc = __builtin_amdgcn_readlane(xsc, fp_c - 1 - j0);
+        const bool abet = in && xa > t1 && xa < t2;
+        sgn += popc64(__ballot(abet)) + popc64(__ballot(in && xc > tc)) + popc64(__ballot(in && xa > tc));
+    }
     // get_LogDetRatPairRem (Trace.F90:2937-2963): M(FPos(1), FPos(2))
-    const int ld = c.L.kcap;
-    const double S = c.mi(f)[sc + (long)sa * ld];
-    const double sig = (abs(fp_c - fp_a) % 2) ? -1.0 : 1.0;
-    const double dr_log = log(fabs(S)), dr_sign = copysign(1.0, S) * sig;
-    const double wr = exp((tl - c.h.trace_log) + dr_log);
+    const double S = c.mi(f)[sc + (long)sa * c.L.kcap];
+    const double sig = ((fp_c - fp_a) & 1) ? -1.0 : 1.0;
+    const double dr_sign = copysign(1.0, S) * sig;
+    const double wr = weight_ratio(T, S, c.h.trace_log);
     const double prob = fabs(((1.0 * hprf) / (double)(2 * M.nb)) * wr);
     const double rnd = grnd(c.rng);
     if (!(rnd < prob)) return OUT_REJ;
-    if (fabs(dr_sign * exp(dr_log)) < 1e-12) {
+    if (fabs(S) < 1e-12) {
         c.h.err = ERR_SING;
         return OUT_REJ;
     }
-    mat_rem_phys(c, c.mi(f), k, sc, sa);
-    c.wflops += 3.0 * k * k;
-    c.wbytes += 8.0 * k * k + 8.0 * (k - 1) * (k - 1);
-    // the operators that owned the last physical row / column take the freed slots
-    int *fcsf = c.fcs + fo, *fasf = c.fas + fo;
-    const int rl = find_slot(fcsf, k, k - 1), al = find_slot(fasf, k, k - 1);
-    if (lane_id() == 0) {
-        fcsf[rl] = sc;
-        fasf[al] = sa;
-    }
-    wsync();
-    commit_window(c, nl);
-    c.h.pc_valid = 0;
-    // segment caches: the first w1 and the last nw - 1 - w2 window operators are unchanged
-    c.h.rk_n = seg ? min(c.h.rk_n, w1 + 1) : 0;
-    c.h.lb_n = seg ? min(c.h.lb_n, nw - w2) : 0;
-    block_move(c.fc + fo, fp_c, k, -1);
-    block_move(fcsf, fp_c, k, -1);
-    block_move(c.fa + fo, fp_a, k, -1);
-    block_move(fasf, fp_a, k, -1);
-    c.h.kf[f] = k - 1;
-    record_pair(c, f, t2 - t1);
-    c.h.det_log += dr_log;
-    c.h.det_sign *= dr_sign;
-    c.h.trace_log = tl;
-    c.h.trace_sign = ts;
-    store_part(c, c.sz[c.h.outer]);
-    c.h.cfgsign = -config_sign(c);
-    c.h.acc_rem++;
+    accept_rem<NM>(c.ref(), RemMove{f, k, nl, w1, w2, fp_c, fp_a, sc, sa, t2 - t1, S, dr_sign,
+                                    (sgn & 1) ? -dr_sign : dr_sign, T});
+    c.lists();
     return OUT_ACC;
 }
 
 // relabel flavours / swap c and c+ (globalUpdate, Trace.F90:2126-2188)
 DEV void global_update(Ctx &c, const int *gu)
 {
-    const DevModel &M = c.M;
+    CModel &M = c.M;
     for (int j = lane_id(); j < c.h.nop; j += WAVE) {
         const int cj = c.code[j];
         const int idx = op_orb(cj) + M.nb * op_spin(cj) + 1;
@@ -2181,7 +2409,7 @@ DEV void global_update(Ctx &c, const int *gu)
 // slot lists given, slots are reset to the identity (logical = physical order).
 DEV void rebuild_flavour_lists(Ctx &c, double *dfc, double *dfa, int *dkf, int *dfcs, int *dfas)
 {
-    const DevModel &M = c.M;
+    CModel &M = c.M;
     const long kc = c.L.kcap;
     for (int g = 0; g < M.nf; ++g) {
         int nc = 0, na = 0;
@@ -2243,9 +2471,11 @@ DEV int count_valid_outer(Ctx &c, unsigned long long *okmask)
 
 // StepGlob (CTQMC.F90:4433-4554)
 template <int NM>
-DEV int step_glob(Ctx &c)
+__device__ __attribute__((noinline)) int step_glob(ChainRef ref)
 {
-    const DevModel &M = c.M;
+    Ctx c = attach<NM>(ref);
+    const RngScope rs(c.rng);
+    CModel &M = c.M;
     c.h.try_glob++;
     if (c.h.nop == 0) return OUT_REJ;
     const int nf = M.nf, nb = M.nb;
@@ -2347,15 +2577,13 @@ DEV int step_glob(Ctx &c)
             dns *= s;
         }
         const double k3 = (double)k * k * k;
-        c.wflops += (2.0 / 3.0) * k3 * 2.0;
-        c.wbytes += 8.0 * (double)k * k;
+        c.work((2.0 / 3.0) * k3 * 2.0, 8.0 * (double)k * k);
     }
     // det(old M) = 1 / det(old Delta), which the chain carries
     dol = -c.h.det_log;
     dos = c.h.det_sign;
-    double tl, ts;
-    full_trace<NM>(c, c.h.outer, tl, ts);
-    const double wr = exp((tl - c.h.trace_log) + (dnl + dol));
+    const TraceVal T = full_trace<NM>(c, c.h.outer);
+    const double wr = exp((T.log_abs() - c.h.trace_log) + (dnl + dol));
     const double rr = grnd(c.rng);   // drawn even for a singular Delta (prob = 0)
     if (!sing && rr < fabs(wr * sst_factor)) {
         rebuild_flavour_lists(c, c.fc, c.fa, c.h.kf, c.fcs, c.fas);
@@ -2380,9 +2608,7 @@ DEV int step_glob(Ctx &c)
         }
         c.h.det_log = dnl;
         c.h.det_sign = dns;
-        c.h.trace_log = tl;
-        c.h.trace_sign = ts;
-        store_part(c, c.sz[c.h.outer]);
+        keep_trace<NM>(c, T);
         c.h.cfgsign = -config_sign(c);
         c.h.cache_pos = -1;
         c.h.wvalid = 0;   // relabelled codes: reload the window list
@@ -2400,9 +2626,8 @@ DEV double empty_weights(Ctx &c)
 {
     double sum = 0.0;
     for (int q = 0; q < c.M.nsst; ++q) {
-        double tl, ts;
-        full_trace<NM>(c, q, tl, ts);
-        const double v = ts * exp(tl);
+        const TraceVal T = full_trace<NM>(c, q);
+        const double v = T.sign() * exp(T.log_abs());
         if (lane_id() == 0) c.Q[q] = v;
         sum += v;
     }
@@ -2428,20 +2653,18 @@ DEV void choose_outer(Ctx &c)
         }
     }
     c.h.outer = pick;
-    double tl, ts;
-    full_trace<NM>(c, pick, tl, ts);
-    c.h.trace_log = tl;
-    c.h.trace_sign = ts;
-    store_part(c, c.sz[pick]);
+    keep_trace<NM>(c, full_trace<NM>(c, pick));
     c.h.cache_pos = -1;
 }
 
 // StepShiftTau_proper (CTQMC.F90:4641-4835) + update_InvFullHybrShiftTau_diag
 // (Trace.F90:2355-2457)
 template <int NM>
-DEV int step_shift(Ctx &c)
+__device__ __attribute__((noinline)) int step_shift(ChainRef ref)
 {
-    const DevModel &M = c.M;
+    Ctx c = attach<NM>(ref);
+    const RngScope rs(c.rng);
+    CModel &M = c.M;
     if (c.h.nop == 0) {
         choose_outer<NM>(c);
         c.h.cfgsign = -config_sign(c);
@@ -2484,13 +2707,10 @@ DEV int step_shift(Ctx &c)
         c.h.wpos = 0;
     }
     set_window(c);
-    double tl, ts;
-    full_trace<NM>(c, c.h.outer, tl, ts);
-    const double ratio = ts * c.h.trace_sign * exp(tl - c.h.trace_log);
+    const TraceVal T = full_trace<NM>(c, c.h.outer);
+    const double ratio = T.sign() * c.h.trace_sign * exp(T.log_abs() - c.h.trace_log);
     if (grnd(c.rng) < fabs(1.0 * ratio * 1.0)) {
-        c.h.trace_log = tl;
-        c.h.trace_sign = ts;
-        store_part(c, c.sz[c.h.outer]);
+        keep_trace<NM>(c, T);
         double detrat = 1.0;
         const int ld = c.L.kcap;
         const long kc = c.L.kcap;
@@ -2564,8 +2784,6 @@ DEV int step_shift(Ctx &c)
     return OUT_REJ;
 }
 
-// one Metropolis step with the dispatch of ctqmc_warmup / ctqmc_measure
-// (CTQMC.F90:8213-8254, 8432-8533) and the window-shift rule
 // Whether the next move fits the chain's memory whatever it proposes: every
 // flavour can take one more pair and the window plus a pair fits the LDS
 // lists.  Checked before the move's first random draw, so a chain that has no
@@ -2574,37 +2792,52 @@ DEV int step_shift(Ctx &c)
 // list (as the next insertion or removal would).
 DEV bool room_for_move(Ctx &c)
 {
-    int km = 0;
-    for (int f = 0; f < c.M.nf; ++f) km = max(km, c.h.kf[f]);
-    if (km + 1 > c.L.kcap || c.h.nop + 2 > c.L.cap) return false;
-    if (!ensure_window(c)) return false;
+    if (s_wenv.full || !ensure_window(c)) return false;
     return c.h.wib - c.h.wia + 2 <= c.L.lcap_lds;
 }
 
+// What a sweep counts in registers: insertion and removal attempts, proposals
+// rejected by quantum numbers, and the attempts since the last multiple of
+// nslide.
+struct Tally {
+    int add, rem, qn, slide;
+};
+
+// one Metropolis step with the dispatch of ctqmc_warmup / ctqmc_measure
+// (CTQMC.F90:8213-8254, 8432-8533) and the window-shift rule
 template <int NM>
-DEV void one_move(Ctx &c, int &kind, int &out)
+DEV void one_move(Ctx &c, Tally &ty, int &kind, int &out)
 {
-    const DevModel &M = c.M;
+    CModel &M = c.M;
     const double r = grnd(c.rng);
-    if (r < (1.0 - M.p_shift - M.p_glob) / 2.0) {
-        kind = 1;
-        (void)grnd(c.rng);               // Percentage4OperatorMove draw
-        (void)(grnd(c.rng) < M.p_outer); // PercentageOuterMove draw
-        out = step_add<NM>(c);
-    } else if (r <= 1.0 - M.p_shift - M.p_glob) {
-        kind = 2;
-        (void)grnd(c.rng);
-        (void)(grnd(c.rng) < M.p_outer);
-        out = step_rem<NM>(c);
-    } else if (r <= 1.0 - M.p_shift) {
-        kind = 3;
-        out = step_glob<NM>(c);
+    if (r <= 1.0 - M.p_shift - M.p_glob) {
+        grnd_skip(c.rng);   // Percentage4OperatorMove draw
+        grnd_skip(c.rng);   // PercentageOuterMove draw
+        if (r < (1.0 - M.p_shift - M.p_glob) / 2.0) {
+            kind = 1;
+            ty.add++;
+            out = step_add<NM>(c);
+        } else {
+            kind = 2;
+            ty.rem++;
+            out = step_rem<NM>(c);
+        }
+        ty.qn += out == OUT_QN;
+        if (++ty.slide == (int)M.nslide) ty.slide = 0;
     } else {
-        kind = 4;
-        out = step_shift<NM>(c);
+        rng_close(c.rng);
+        if (r <= 1.0 - M.p_shift) {
+            kind = 3;
+            out = step_glob<NM>(c.ref());
+        } else {
+            kind = 4;
+            out = step_shift<NM>(c.ref());
+        }
+        rng_open(c.rng);
     }
-    c.h.moves++;
-    if ((c.h.try_add + c.h.try_rem) % M.nslide == 0) shift_window(c);
+    // every nslide-th attempt; after a global move or shift the count, and with
+    // it this condition, stands
+    if (ty.slide == 0) shift_window(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -2797,7 +3030,7 @@ __device__ __attribute__((noinline)) double2 meas_gtau_narrow(const GtauArgs a) 
 // update; when the low bits of the count n are ones the finished bin of each
 // level (mean of its halves) rolls over to the next.  Lanes over components;
 // the roll-over depth depends on n only, so it is uniform.
-DEV void autocorr_add(const DevModel &M, double *gbuf, double *gacc, double *gtau, long long n0)
+DEV void autocorr_add(CModel &M, double *gbuf, double *gacc, double *gtau, long long n0)
 {
     const long nc = (long)M.nf * M.ntau;
     double *spill = gacc, *mean = gacc + nc * M.nlev, *sq = gacc + 2 * nc * M.nlev;
@@ -2831,23 +3064,37 @@ DEV void autocorr_add(const DevModel &M, double *gbuf, double *gacc, double *gta
 template <int NM>
 DEV void meas_dm(Ctx &c, double *dm)
 {
-    const DevModel &M = c.M;
+    CModel &M = c.M;
     const int outer = c.h.outer, no = c.sz[outer];
     if (c.h.nop != 0) {
         const double bh = M.beta / 2.0;
         const int nk = upper_bound_tau(c.tau, c.h.nop, bh);   // ops with tau <= beta/2
-        double *K = c.K0, *Kw = c.K1;
-        set_identity(K, no);
-        int s = outer;
-        double kl = 0.0;
-        ket_walk_global<NM>(c, K, Kw, s, kl, no, 0.0, 0, nk, bh);
-        double *Ks = c.scratch;
-        copy_mat(Ks, K, c.sz[s] * no);
-        double *B = c.K0, *Bw = c.K1;
-        set_identity(B, no);
-        int sb = outer;
-        double bl = 0.0;
-        bra_walk_global<NM>(c, B, Bw, sb, bl, no, M.beta, nk, c.h.nop, bh);
+        int s = outer, sb = outer;
+        double kl = 0.0, bl = 0.0;
+        double *Ks, *B;
+        if constexpr (NM <= 16) {
+            // both halves in registers, then to the work matrices
+            Ks = c.K0;
+            B = c.K1;
+            State<NM> k;
+            k.identity(no);
+            walk_global<NM, false>(c, k, s, kl, no, 0.0, 0, nk, bh);
+            k.store(Ks, c.sz[s], no);
+            k.identity(no);
+            walk_global<NM, true>(c, k, sb, bl, no, M.beta, nk, c.h.nop, bh);
+            k.store(B, c.sz[sb], no);
+            wsync();
+        } else {
+            double *K = c.K0, *Kw = c.K1;
+            set_identity(K, no);
+            walk_global_big<false>(c, K, Kw, s, kl, no, 0.0, 0, nk, bh);
+            Ks = c.scratch;
+            copy_mat(Ks, K, c.sz[s] * no);
+            B = c.K0;
+            double *Bw = c.K1;
+            set_identity(B, no);
+            walk_global_big<true>(c, B, Bw, sb, bl, no, M.beta, nk, c.h.nop, bh);
+        }
         const int n = c.sz[s];
         double *blk = dm + M.dmoff[s];
         const double fac = c.h.trace_sign * (-c.h.cfgsign) * exp(kl + bl - c.h.trace_log);
@@ -2888,7 +3135,7 @@ DEV void meas_dm(Ctx &c, double *dm)
 constexpr int MAXTHETA = 4;
 
 struct TanEnv {
-    const DevModel *M;
+    CModel *M;
     const int *sz, *off;
     const int4 *tr;
     const double *ev, *ops, *tau;
@@ -2923,7 +3170,7 @@ DEV int4 tan_trans(const TanEnv &e, int s, int code, bool adjoint)
 // segment of length dt in block s: dKw_t = P dK_t - (D_t o Phi) K, then K <- P K
 DEV void tan_prop(const TanEnv &e, int s, double dt, double *K, const double *dK, double *dKw, int no)
 {
-    const DevModel &M = *e.M;
+    CModel &M = *e.M;
     const int ns = e.sz[s];
     const long nm2 = (long)e.nm * e.nm;
     const double *E = e.ev + e.off[s];
@@ -2993,7 +3240,7 @@ template <bool BRA>
 DEV bool tan_walk(const TanEnv &e, double *&K, double *&Kw, double *&dK, double *&dKw, int &s, double &lg, int no,
                   double tstart, int j0, int j1, double tend)
 {
-    const DevModel &M = *e.M;
+    CModel &M = *e.M;
     double t = tstart;
     for (int jj = 0; jj < j1 - j0; ++jj) {
         const int j = BRA ? j1 - 1 - jj : j0 + jj;
@@ -3029,7 +3276,7 @@ struct HalfTangents {
 // ket from 0 and bra from beta to beta/2 with tangents
 DEV HalfTangents half_tangents(const TanEnv &e, int nop, int outer)
 {
-    const DevModel &M = *e.M;
+    CModel &M = *e.M;
     const long nm2 = (long)e.nm * e.nm;
     double *A0 = e.w + nm2, *A1 = A0 + nm2, *A2 = A1 + nm2;
     double *T0 = A2 + nm2, *T1 = T0 + e.nth * nm2, *T2 = T1 + e.nth * nm2;
@@ -3116,7 +3363,7 @@ DEV ScoreArgs score_args(const Ctx &c, double *gbuf, double *gtau)
 // d ln|det| / d theta = sum_f tr(Delta_f^{-1} dDelta_f)
 DEV void det_tangent(const ScoreArgs &a, double *dld)
 {
-    const DevModel &M = *a.e.M;
+    CModel &M = *a.e.M;
     const int ld = a.kcap;
     double acc[MAXTHETA] = {0.0, 0.0, 0.0, 0.0};
     for (int f = 0; f < M.nf; ++f) {
@@ -3152,7 +3399,7 @@ DEV void det_tangent(const ScoreArgs &a, double *dld)
 // configuration (the beta/2 sample depends on H explicitly).
 __device__ __attribute__((noinline)) void score_pass(const ScoreArgs a, double *out, bool accumulate)
 {
-    const DevModel &M = *a.e.M;
+    CModel &M = *a.e.M;
     const TanEnv &e = a.e;
     const long nm2 = (long)e.nm * e.nm;
     double dld[MAXTHETA], dlt[MAXTHETA], sc[MAXTHETA];
@@ -3207,7 +3454,7 @@ __device__ __attribute__((noinline)) void score_pass(const ScoreArgs a, double *
 // the order histogram
 DEV void meas_misc(Ctx &c, double *histo, double *outer_hist)
 {
-    const DevModel &M = c.M;
+    CModel &M = c.M;
     const int outer = c.h.outer, no = c.sz[outer], off = c.off[outer];
     double *ohst = reinterpret_cast<double *>(c.base + c.L.ohst);
     double *shss = reinterpret_cast<double *>(c.base + c.L.shss);
@@ -3241,130 +3488,135 @@ DEV void meas_misc(Ctx &c, double *histo, double *outer_hist)
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-// Map the chain block and carve the dynamic LDS; copies header, RNG state and
-// the model tables into LDS.
-template <int NM>
-DEV Ctx make_ctx(const DevModel &M, const ChainLayout &L, char *base, int chain, char *lds)
+// the chain a header pointer belongs to, in the header array behind the blocks
+DEV ChainHdr *global_hdr(CLayout &L, char *base, int chain)
 {
-    ChainHdr &hd = *reinterpret_cast<ChainHdr *>(lds + L.l_hdr);
-    Ctx c(M, L, base, hd);
-    c.nm = NM;
-    c.tau = reinterpret_cast<double *>(base + L.tau);
-    c.code = reinterpret_cast<int *>(base + L.code);
-    c.fc = reinterpret_cast<double *>(base + L.fc);
-    c.fa = reinterpret_cast<double *>(base + L.fa);
-    c.fcs = reinterpret_cast<int *>(base + L.fcs);
-    c.fas = reinterpret_cast<int *>(base + L.fas);
-    c.minv = reinterpret_cast<double *>(base + L.minv);
-    c.scratch = reinterpret_cast<double *>(base + L.scratch);
-    c.kst = reinterpret_cast<double *>(base + L.kst);
-    c.bnd = reinterpret_cast<double *>(base + L.bnd);
-    c.bndlog = reinterpret_cast<double *>(base + L.bndlog);
-    c.bndsst = reinterpret_cast<int *>(base + L.bndsst);
-    c.part = reinterpret_cast<double *>(base + L.part);
-    uint32_t *mt = reinterpret_cast<uint32_t *>(lds + L.l_mt);
-    int *sz = reinterpret_cast<int *>(lds + L.l_sz);
-    int *off = reinterpret_cast<int *>(lds + L.l_off);
-    int *cn = reinterpret_cast<int *>(lds + L.l_cn);
-    int *oo = reinterpret_cast<int *>(lds + L.l_oo);
-    double *ev = reinterpret_cast<double *>(lds + L.l_ev);
-    c.wtau = reinterpret_cast<double *>(lds + L.l_wtau);
-    c.wcode = reinterpret_cast<int *>(lds + L.l_wcode);
-    c.pc = reinterpret_cast<int *>(lds + L.l_pc);
-    c.ttau = reinterpret_cast<double *>(lds + L.l_ttau);
-    c.tcode = reinterpret_cast<int *>(lds + L.l_tcode);
-    c.dvec = reinterpret_cast<double *>(lds + L.l_dvec);
-    c.Q = reinterpret_cast<double *>(lds + L.l_q);
-    c.R = reinterpret_cast<double *>(lds + L.l_r);
-    c.colb = reinterpret_cast<double *>(lds + L.l_col);
-    c.rowb = reinterpret_cast<double *>(lds + L.l_row);
-    c.pl = reinterpret_cast<double *>(lds + L.l_pl);
-    if constexpr (NM <= 4) {
-        c.rk = reinterpret_cast<double *>(lds + L.l_rk);
-        c.lb = reinterpret_cast<double *>(lds + L.l_lb);
-        c.rkx = reinterpret_cast<double *>(lds + L.l_rkx);
-        c.lbx = reinterpret_cast<double *>(lds + L.l_lbx);
-        c.rks = reinterpret_cast<int *>(lds + L.l_rks);
-        c.lbs = reinterpret_cast<int *>(lds + L.l_lbs);
-    }
-    if constexpr (NM <= 16) {
-        c.qa = reinterpret_cast<double *>(lds + L.l_qa);
-        c.qlc = reinterpret_cast<double *>(lds + L.l_qlc);
-        c.qrec = reinterpret_cast<int4 *>(lds + L.l_qrec);
-        c.qsst = reinterpret_cast<int *>(lds + L.l_qsst);
-    }
-    {
-        double *lc = reinterpret_cast<double *>(lds + L.l_legc);
-        for (int i = lane_id(); i < 2 * M.nleg; i += WAVE) lc[i] = M.legc[i];
-        c.legc = lc;
-    }
-    // work matrices: LDS for blocks up to 16 states (decided at compile time so
-    // that their accesses are LDS instructions, not generic ones), HBM above
-    if constexpr (NM <= 16) {
-        c.K0 = reinterpret_cast<double *>(lds + L.l_k);
-    } else {
-        c.K0 = reinterpret_cast<double *>(base + L.kwork);
-    }
-    c.K1 = c.K0 + (long)NM * NM;
-    c.strip = L.l_strip >= 0 ? reinterpret_cast<double *>(lds + L.l_strip) : nullptr;
-    // header, RNG state and model tables into LDS
-    c.ghdr = reinterpret_cast<ChainHdr *>(base - (long)chain * L.stride + L.hdrs) + chain;
-    const int *gh = reinterpret_cast<const int *>(c.ghdr);
-    int *lh = reinterpret_cast<int *>(&hd);
+    return reinterpret_cast<ChainHdr *>(base - (long)chain * L.stride + L.hdrs) + chain;
+}
+
+// Start of a kernel: header, RNG state and model tables into LDS.
+template <int NM>
+DEV Ctx make_ctx(char *chains, int chain, CArgs args, char *lds)
+{
+    CModel &M = *(CModel *)args;
+    CLayout &L = *(CLayout *)(args + (sizeof(DevModel) + 7) / 8 * 8);
+    s_wenv.dyn = (lds_c *)lds;
+    s_wenv.swapped = 0;
+    wsync();
+    char *base = chains + (long)chain * L.stride;
+    Ctx c = attach<NM>(ChainRef{&M, &L, base});
+    const int *gh = reinterpret_cast<const int *>(global_hdr(L, base, chain));
+    int *lh = reinterpret_cast<int *>(&s_hdr);
     for (int i = lane_id(); i < (int)(sizeof(ChainHdr) / 4); i += WAVE) lh[i] = gh[i];
     const uint32_t *gmt = reinterpret_cast<const uint32_t *>(base + L.mt);
-    for (int i = lane_id(); i < 624; i += WAVE) mt[i] = gmt[i];
+    for (int i = lane_id(); i < 624; i += WAVE) c.rng.mt[i] = gmt[i];
     for (int i = lane_id(); i < M.nsst; i += WAVE) {
-        sz[i] = M.sizes[i];
-        off[i] = M.offsets[i];
+        const_cast<int *>(c.sz)[i] = M.sizes[i];
+        const_cast<int *>(c.off)[i] = M.offsets[i];
     }
+    for (int i = lane_id(); i < 2 * M.nleg; i += WAVE) const_cast<double *>(c.legc)[i] = M.legc[i];
     const int ncn = M.nsst * M.nb * 4;
     if constexpr (NM <= 16) {
-        for (int i = lane_id(); i < ncn; i += WAVE) {
-            cn[i] = M.connect[i];
-            oo[i] = (int)M.opoff[i];
+        for (int i = lane_id(); i < M.nstates; i += WAVE) const_cast<double *>(c.ev)[i] = M.evals[i];
+        for (int i = lane_id(); i < ncn; i += WAVE) const_cast<int4 *>(c.tr)[i] = M.trans[i];
+        // what the walks read
+        int *si = (int *)(lds_i *)(lds_c *)(lds + L.l_sinfo);
+        for (int q = lane_id(); q < M.nsst; q += WAVE) {
+            const int n = M.sizes[q], o = M.offsets[q];
+            const double e0 = M.evals[o];
+            si[4 * q] = __double2loint(e0);
+            si[4 * q + 1] = __double2hiint(e0);
+            si[4 * q + 2] = n | (o << 8);
+            si[4 * q + 3] = __float_as_int((float)(M.evals[o + n - 1] - e0));
         }
+        unsigned char *kb = (unsigned char *)(lds_b *)(lds_c *)(lds + L.l_keys);
+        for (int q = lane_id(); q < 512; q += WAVE) kb[q] = M.dkey ? M.keys[q] : 255;
+        WalkEnv &e = s_wenv;
+        e.ops = M.ops;
+        e.tr = (const lds_i4 *)c.tr;
+        e.ev = (const lds_d *)c.ev;
+        e.keys = (const lds_b *)kb;
+        e.sinfo = (const lds_i4 *)(const void *)si;
+        e.qa = NM > 4 ? (lds_d *)(lds_c *)(lds + L.l_qa) : nullptr;
+        e.lops = (const lds_d *)c.ev;
+        if constexpr (NM <= 4) {
+            for (long i = lane_id(); i < M.nops; i += WAVE) const_cast<double *>(c.opsp)[i] = M.ops[i];
+            e.lops = (const lds_d *)c.opsp;
+        }
+        e.ncol = 4 * M.nb;
+        e.dkey = M.dkey;
+        e.zero = (int)M.nops;
+        e.nkmax = (M.nmax + 3) / 4;
     }
-    if constexpr (NM <= 16) {
-        for (int i = lane_id(); i < M.nstates; i += WAVE) ev[i] = M.evals[i];
-        int4 *trt = reinterpret_cast<int4 *>(lds + L.l_tr);
-        for (int i = lane_id(); i < ncn; i += WAVE) trt[i] = M.trans[i];
-        c.tr = trt;
-    } else {
-        c.tr = M.trans;
-    }
-    // operator blocks: always LDS for blocks up to 4 states (known at compile
-    // time, so the block reads are LDS instructions); LDS or HBM above
-    if constexpr (NM <= 4) {
-        double *lops = reinterpret_cast<double *>(lds + L.l_ops);
-        for (long i = lane_id(); i < M.nops; i += WAVE) lops[i] = M.ops[i];
-        c.opsp = lops;
-    } else {
-        c.opsp = M.ops;
-    }
-    c.sz = sz, c.off = off;
-    if constexpr (NM <= 16) c.cn = cn, c.oo = oo;
-    else c.cn = M.connect, c.oo = M.opoff32;
-    if constexpr (NM <= 16) c.ev = ev;
-    else c.ev = M.evals;
-    c.rng.mt = mt;
-    c.rng.idx = &hd.mti;
-    hd.wvalid = 0;   // the LDS window list does not survive a launch
+    s_wenv.egs = M.egs;
+    s_wenv.flops = s_wenv.bytes = 0.0;
+    wsync();
+    s_hdr.wvalid = 0;   // the LDS window list does not survive a launch
     wsync();
     return c;
 }
 
-DEV void save_ctx(Ctx &c)
+DEV void save_ctx(Ctx &c, int chain)
 {
-    c.h.alg_flops += c.wflops;
-    c.h.alg_bytes += c.wbytes;
+    c.h.alg_flops += s_wenv.flops;
+    c.h.alg_bytes += s_wenv.bytes;
     uint32_t *gmt = reinterpret_cast<uint32_t *>(c.base + c.L.mt);
     for (int i = lane_id(); i < 624; i += WAVE) gmt[i] = c.rng.mt[i];
-    int *gh = reinterpret_cast<int *>(c.ghdr);
+    int *gh = reinterpret_cast<int *>(global_hdr(c.L, c.base, chain));
     const int *lh = reinterpret_cast<const int *>(&c.h);
     wsync();
     for (int i = lane_id(); i < (int)(sizeof(ChainHdr) / 4); i += WAVE) gh[i] = lh[i];
     wsync();
+}
+
+// Calibration: phase 1 ends once the distance list is full, phase 2 once every
+// flavour has calib.z accepted pairs (CTQMC.F90:8128-8175)
+template <int NM>
+__device__ __attribute__((noinline)) bool calib_done(ChainRef r, int3 calib)
+{
+    Ctx c = attach<NM>(r);
+    if (calib.x == 1) return c.h.apt_index > c.h.apt_n;
+    const double *ap = reinterpret_cast<const double *>(c.base + c.L.accpair);
+    int short_f = 0;
+    for (int f = 0; f < c.M.nf; ++f) {
+        double n = 0.0;
+        for (int b = lane_id(); b < c.h.naccpair; b += WAVE) n += ap[(long)f * c.L.naccpair_cap + b];
+        short_f += wave_sum(n) < (double)calib.z;
+    }
+    return short_f == 0;
+}
+
+// all measurements of the current configuration
+template <int NM, bool SCORE>
+__device__ __attribute__((noinline)) void measure(ChainRef r)
+{
+    Ctx c = attach<NM>(r);
+    CModel &M = c.M;
+    CLayout &L = c.L;
+    char *base = c.base;
+    double *gtau = reinterpret_cast<double *>(base + L.gtau);
+    double *gleg = reinterpret_cast<double *>(base + L.gleg);
+    double *gbuf = reinterpret_cast<double *>(base + L.gbuf);
+    c.h.cnt_meas++;
+    meas_misc(c, reinterpret_cast<double *>(base + L.histo), reinterpret_cast<double *>(base + L.outer));
+    if (M.meas_dm) meas_dm<NM>(c, reinterpret_cast<double *>(base + L.dm));
+    GtauArgs ga;
+    ga.nf = M.nf, ga.ntau = M.ntau, ga.nleg = M.nleg, ga.kcap = L.kcap;
+    ga.beta = M.beta, ga.cfgsign = c.h.cfgsign, ga.legc = c.legc;
+    ga.kf = c.h.kf, ga.fc = c.fc, ga.fa = c.fa, ga.minv = c.minv, ga.fcs = c.fcs, ga.fas = c.fas;
+    ga.gtau = (M.accum == 2 || SCORE) ? gbuf : gtau, ga.gleg = gleg;
+    const long long mi = c.h.cnt_meas - 1;   // g_inmeas - 1
+    const bool st = mi < M.nmstep;
+    ga.mstep = (st && M.step_mean) ? reinterpret_cast<double *>(base + L.gmstep) + mi * M.nf : nullptr;
+    ga.dstep = (st && M.step_mid) ? reinterpret_cast<double *>(base + L.gdstep) + mi * M.nf : nullptr;
+    // sign_step is set when the configuration has a pair (CTQMC.F90:2402)
+    if (st && M.step_sign && c.h.nop > 0 && lane_id() == 0)
+        reinterpret_cast<double *>(base + L.sstep)[mi] = c.h.cfgsign;
+    const double2 wk = NM == 1 ? meas_gtau_narrow(ga) : meas_gtau(ga);
+    c.work(wk.x, wk.y);
+    if constexpr (SCORE) score_pass(score_args(c, gbuf, gtau), nullptr, true);
+    if (M.accum == 2)
+        autocorr_add(M, gbuf, reinterpret_cast<double *>(base + L.gacc), gtau, c.h.cnt_meas - 1);
 }
 
 // Sweep kernel: each block advances chain blockIdx.x until it has done
@@ -3394,42 +3646,34 @@ __global__ void __launch_bounds__(WAVE) sweep_kernel(DevModel M, ChainLayout L, 
                             : (int)blockIdx.x;
     if (only >= 0 && chain != only) return;
     extern __shared__ __align__(16) char lds[];
-    char *base = chains + (long)chain * L.stride;
-    Ctx c = make_ctx<NM>(M, L, base, chain, lds);
-    double *gtau = reinterpret_cast<double *>(base + L.gtau);
-    double *gleg = reinterpret_cast<double *>(base + L.gleg);
-    double *dm = reinterpret_cast<double *>(base + L.dm);
-    double *histo = reinterpret_cast<double *>(base + L.histo);
-    double *ohist = reinterpret_cast<double *>(base + L.outer);
-    double *gbuf = reinterpret_cast<double *>(base + L.gbuf);
-    double *gacc = reinterpret_cast<double *>(base + L.gacc);
-    while (c.h.pos < target && c.h.err == 0 && c.h.halt == HALT_NONE) {
+    Ctx c = make_ctx<NM>(chains, chain, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
+    rng_open(c.rng);
+    room_left(c);
+    wsync();
+    const long long pos0 = c.h.pos;
+    const int todo = (int)min(target - pos0, (long long)0x7fffffff);   // moves of this launch
+    // moves until the next measurement, check of the calibration, look at the
+    // abort word (warm-up); counted down instead of divided
+    const int every = ncorr > 0 ? (int)min(ncorr, (long long)0x7fffffff) : 128;
+    int until = every - (int)(pos0 % every), ucal = calib.x ? calib.y - (int)(pos0 % calib.y) : 0;
+    Tally ty{0, 0, 0, (int)((c.h.try_add + c.h.try_rem) % c.M.nslide)};
+    int done = 0;
+    while (done < todo && (c.h.err | c.h.halt) == 0) {
         if (!room_for_move(c)) {
             c.h.halt = HALT_CAP;
             break;
         }
         int kind, out;
-        one_move<NM>(c, kind, out);
-        const long long m = c.h.pos++;
+        one_move<NM>(c, ty, kind, out);
         // ctqmc_calibrate (CTQMC.F90:8128-8175): every calib.y moves, phase 1
         // (calib.x = 1) ends once the distance list is full, phase 2
         // (calib.x = 2) once every flavour has calib.z accepted pairs
-        if (calib.x && (m + 1) % calib.y == 0) {
-            bool done = calib.x == 1 && c.h.apt_index > c.h.apt_n;
-            if (calib.x == 2) {
-                const double *ap = reinterpret_cast<const double *>(base + L.accpair);
-                int short_f = 0;
-                for (int f = 0; f < M.nf; ++f) {
-                    double n = 0.0;
-                    for (int b = lane_id(); b < c.h.naccpair; b += WAVE) n += ap[(long)f * L.naccpair_cap + b];
-                    short_f += wave_sum(n) < (double)calib.z;
-                }
-                done = short_f == 0;
-            }
-            if (done) c.h.halt = HALT_DONE;
+        if (calib.x && --ucal == 0) {
+            ucal = calib.y;
+            if (calib_done<NM>(c.ref(), calib)) c.h.halt = HALT_DONE;
         }
         if (rec && lane_id() == 0) {
-            w2d_move_record &r = rec[m - rec_base];
+            w2d_move_record &r = rec[pos0 + done - rec_base];
             r.kind = kind;
             r.outcome = out;
             r.noper = c.h.nop;
@@ -3441,35 +3685,21 @@ __global__ void __launch_bounds__(WAVE) sweep_kernel(DevModel M, ChainLayout L, 
             r.det_sign = c.h.det_sign;
             r.cfgsign = c.h.cfgsign;
         }
-        if (ncorr <= 0) {
-            if ((m + 1) % 128 == 0 && __hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))
-                c.h.halt = HALT_ABORT;
-        } else if ((m + 1) % ncorr == 0) {
-            c.h.cnt_meas++;
-            meas_misc(c, histo, ohist);
-            if (M.meas_dm) meas_dm<NM>(c, dm);
-            GtauArgs ga;
-            ga.nf = M.nf, ga.ntau = M.ntau, ga.nleg = M.nleg, ga.kcap = L.kcap;
-            ga.beta = M.beta, ga.cfgsign = c.h.cfgsign, ga.legc = c.legc;
-            ga.kf = c.h.kf, ga.fc = c.fc, ga.fa = c.fa, ga.minv = c.minv, ga.fcs = c.fcs, ga.fas = c.fas;
-            constexpr bool score = SCORE;
-            ga.gtau = (M.accum == 2 || score) ? gbuf : gtau, ga.gleg = gleg;
-            const long long mi = c.h.cnt_meas - 1;   // g_inmeas - 1
-            const bool st = mi < M.nmstep;
-            ga.mstep = (st && M.step_mean) ? reinterpret_cast<double *>(base + L.gmstep) + mi * M.nf : nullptr;
-            ga.dstep = (st && M.step_mid) ? reinterpret_cast<double *>(base + L.gdstep) + mi * M.nf : nullptr;
-            // sign_step is set when the configuration has a pair (CTQMC.F90:2402)
-            if (st && M.step_sign && c.h.nop > 0 && lane_id() == 0)
-                reinterpret_cast<double *>(base + L.sstep)[mi] = c.h.cfgsign;
-            const double2 wk = NM == 1 ? meas_gtau_narrow(ga) : meas_gtau(ga);
-            c.wflops += wk.x;
-            c.wbytes += wk.y;
-            if constexpr (SCORE) score_pass(score_args(c, gbuf, gtau), nullptr, true);
-            if (M.accum == 2) autocorr_add(M, gbuf, gacc, gtau, c.h.cnt_meas - 1);
+        ++done;
+        if (--until == 0) {
+            until = every;
+            if (ncorr > 0) measure<NM, SCORE>(c.ref());
             if (__hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) c.h.halt = HALT_ABORT;
         }
     }
-    save_ctx(c);
+    rng_close(c.rng);
+    c.h.pos += done;
+    c.h.moves += done;
+    c.h.try_add += ty.add;
+    c.h.try_rem += ty.rem;
+    c.h.qn_rej += ty.qn;
+    wsync();
+    save_ctx(c, chain);
 }
 
 // d ln|det| / d theta and d ln|Tr| / d theta of one chain's configuration:
@@ -3479,8 +3709,7 @@ __global__ void __launch_bounds__(WAVE) dlogw_kernel(DevModel M, ChainLayout L, 
                                                        double *out)
 {
     extern __shared__ __align__(16) char lds[];
-    char *base = chains + (long)chain * L.stride;
-    Ctx c = make_ctx<NM>(M, L, base, chain, lds);
+    Ctx c = make_ctx<NM>(chains, chain, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
     score_pass(score_args(c, nullptr, nullptr), out, false);
 }
 
@@ -3759,11 +3988,12 @@ template <int NM>
 __global__ void __launch_bounds__(WAVE) init_kernel(DevModel M, ChainLayout L, char *chains)
 {
     extern __shared__ __align__(16) char lds[];
-    char *base = chains + (long)blockIdx.x * L.stride;
-    Ctx c = make_ctx<NM>(M, L, base, (int)blockIdx.x, lds);
+    Ctx c = make_ctx<NM>(chains, (int)blockIdx.x, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
+    rng_open(c.rng);
     choose_outer<NM>(c);
+    rng_close(c.rng);
     if (!(c.h.trace_log > -DBL_MAX)) c.h.err = 5;
-    save_ctx(c);
+    save_ctx(c, (int)blockIdx.x);
 }
 
 // Adopt the configuration already written into tau/code/nop/outer: full trace,
@@ -3774,28 +4004,25 @@ __global__ void __launch_bounds__(WAVE) setconfig_kernel(DevModel M, ChainLayout
 {
     if ((int)blockIdx.x != only) return;
     extern __shared__ __align__(16) char lds[];
-    char *base = chains + (long)blockIdx.x * L.stride;
-    Ctx c = make_ctx<NM>(M, L, base, (int)blockIdx.x, lds);
+    Ctx c = make_ctx<NM>(chains, (int)blockIdx.x, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
     c.h.wpos = 0;
     set_window(c);
-    double tl, ts;
-    if (!full_trace<NM>(c, c.h.outer, tl, ts)) c.h.err = 5;   // W2D_ERR_ZERO_TRACE
-    c.h.trace_log = tl;
-    c.h.trace_sign = ts;
-    store_part(c, c.sz[c.h.outer]);
+    const TraceVal T = full_trace<NM>(c, c.h.outer);
+    if (T.S == 0.0 && !(T.lg > -DBL_MAX)) c.h.err = 5;   // W2D_ERR_ZERO_TRACE: broken quantum numbers
+    keep_trace<NM>(c, T);
     rebuild_flavour_lists(c, c.fc, c.fa, c.h.kf, c.fcs, c.fas);
     int *piv = reinterpret_cast<int *>(c.R);
     double dl = 0.0, dsg = 1.0;
-    for (int f = 0; f < M.nf; ++f) {
+    for (int f = 0; f < c.M.nf; ++f) {
         const int k = c.h.kf[f];
         if (k == 0) continue;
-        build_delta(c, f, k, c.scratch, L.kcap, c.fc, c.fa);
+        build_delta(c, f, k, c.scratch, c.L.kcap, c.fc, c.fa);
         double l, sg;
-        if (!lu_inplace(c.scratch, k, L.kcap, l, sg, piv)) {
+        if (!lu_inplace(c.scratch, k, c.L.kcap, l, sg, piv)) {
             c.h.err = ERR_SING;
             break;
         }
-        lu_inverse(c.scratch, k, L.kcap, piv, c.mi(f), L.kcap);
+        lu_inverse(c.scratch, k, c.L.kcap, piv, c.mi(f), c.L.kcap);
         dl += l;
         dsg *= sg;
     }
@@ -3803,7 +4030,7 @@ __global__ void __launch_bounds__(WAVE) setconfig_kernel(DevModel M, ChainLayout
     c.h.det_sign = dsg;
     c.h.cfgsign = -config_sign(c);
     c.h.cache_pos = -1;
-    save_ctx(c);
+    save_ctx(c, (int)blockIdx.x);
 }
 
 }  // namespace w2d

@@ -13,10 +13,14 @@ constexpr int MAXSST = 256;    // superstates (quantum-number blocks) a model ma
 // read-only model and parameters, passed by value to the kernels
 struct DevModel {
     int nb, nf, nsst, nmax, nstates, nftau;
-    double beta, egs;
+    double beta, rbeta, egs;     // rbeta = 1 / beta
+    // additive superstate keys (walk_small): key of each superstate [256], then
+    // superstate of each key [256] (255: none); dkey: key change by a creator of
+    // spin 0 | of spin 1 << 8, 0 if the blocks have no such keys
+    const unsigned char *keys;
+    int dkey;
     const int *sizes, *offsets, *connect, *first_state, *state_sst;
     const long *opoff;
-    const int *opoff32;                 // the same offsets as int (HBM operator-block table for blocks above 16 states)
     // blocks above 16 states: every operator block zero-padded to multiples of
     // 16 rows and columns (column-major, leading dimension 16 ceil(n_t / 16)),
     // offsets indexed like opoff; the MFMA walks read whole 16 x 4 fragments
@@ -104,12 +108,13 @@ struct ChainLayout {
     int cap, kcap, nbound, lcap;
     long kmat;            // max(kcap*kcap, nmax*nmax)
     // dynamic LDS carve-up (byte offsets; l_ops / l_k = -1: kept in global memory)
-    long l_hdr, l_mt, l_sz, l_off, l_cn, l_oo, l_ev, l_ops, l_wtau, l_wcode, l_ttau, l_tcode;
+    long l_mt, l_sz, l_off, l_ev, l_ops, l_wtau, l_wcode, l_ttau, l_tcode;
     long l_dvec, l_q, l_r, l_col, l_row, l_pl, l_k, l_legc, l_tr, l_pc, lds_bytes;
     int lcap_lds;         // operators each LDS list holds (window list, trial list)
-    // prefix kets / suffix bras of the window's operators (blocks up to 4 states)
+    // prefix kets / suffix bras of the window's operators (blocks up to 16 states)
     int sc;               // window operators they cover (0: not kept)
-    long l_rk, l_lb, l_rkx, l_lbx, l_rks, l_lbs, l_qa, l_qlc, l_qrec, l_qsst;
+    long l_rk, l_lb, l_rkx, l_lbx, l_rks, l_lbs, l_qa, l_keys, l_sinfo;
+    long grk, glb;        // the same for blocks of 5 to 16 states: in the chain block
     long l_strip;         // 16-column strip of the state for the MFMA walks (blocks above 16 states)
 };
 
