@@ -182,7 +182,7 @@ struct Rng {
     lds_u *mt;      // LDS
     int *idx;       // LDS (uniform): next word, kept there between open and close
     uint32_t w;     // lane l: tempered word base + l
-    int pos, base, lim;
+    int pos, base;
 };
 
 DEV uint32_t mt_twist_word(uint32_t a, uint32_t b, uint32_t c)
@@ -236,30 +236,44 @@ DEV uint32_t mt_temper(uint32_t y)
 DEV void rng_open(Rng &r)
 {
     r.pos = uni(*r.idx);
-    r.base = r.lim = -1;
+    r.base = -2 * WAVE;
 }
 DEV void rng_close(Rng &r) { *r.idx = r.pos; }
 
-// The next word.  64 words at a time are tempered, one per lane, and handed out
-// by readlane: a draw is a few scalar instructions instead of an LDS round
-// trip for the position, one for the word and the tempering.
-DEV uint32_t mt_next(Rng &r)
+// The next 64 words, tempered, one per lane: a draw is then a readlane and a
+// few scalar instructions instead of LDS round trips for position and word and
+// the tempering.  Words beyond the end of the state are those of the next
+// block, whose first 227 follow from this block's words alone; the block itself
+// is renewed once the position has passed its end.
+__device__ __attribute__((noinline)) uint32_t mt_words(lds_u *mt_, int pos_)
 {
-    if (r.pos >= r.lim) {
-        if (r.pos >= 624) {
-            mt_regen(r.mt);
-            r.pos = 0;
-        }
-        r.base = r.pos;
-        r.lim = min(r.base + WAVE, 624);
-        r.w = mt_temper(r.mt[min(r.base + lane_id(), 623)]);
-    }
-    return (uint32_t)__builtin_amdgcn_readlane((int)r.w, r.pos++ - r.base);
+    lds_u *mt = uni_lds(mt_);
+    const int i = uni(pos_) + lane_id();
+    uint32_t y = mt[min(i, 623)];
+    if (i >= 624) y = mt_twist_word(mt[i - 624], mt[i - 623], mt[i - 624 + 397]);
+    return mt_temper(y);
 }
 
+// at least n words at hand (n <= 64)
+DEV void rng_need(Rng &r, int n)
+{
+    if (r.pos - r.base > WAVE - n) {
+        if (r.pos >= 624) {
+            mt_regen(r.mt);
+            r.pos -= 624;
+        }
+        r.base = r.pos;
+        r.w = mt_words(r.mt, r.pos);
+    }
+}
+
+DEV uint32_t mt_next(Rng &r) { return (uint32_t)__builtin_amdgcn_readlane((int)r.w, r.pos++ - r.base); }
+
 // generate_canonical<double,53>: (g1 + g2 2^32) / 2^64, clamped below 1
+template <bool CHECK = true>
 DEV double grnd(Rng &r)
 {
+    if (CHECK) rng_need(r, 2);
     const uint32_t g1 = mt_next(r), g2 = mt_next(r);
     const double tmp = 4294967296.0;
     double sum = __dadd_rn((double)g1, __dmul_rn((double)g2, tmp));
@@ -275,21 +289,20 @@ struct RngScope {
     DEV ~RngScope() { rng_close(r); }
 };
 
-// a draw whose value is not used
-DEV void grnd_skip(Rng &r)
-{
-    (void)mt_next(r);
-    (void)mt_next(r);
-}
+// words a move draws before a look at what is at hand: an insertion takes 14
+constexpr int MOVE_WORDS = 24;
 
+template <bool CHECK = true>
 DEV int randint(Rng &r, int a, int b)
 {
+    if (CHECK) rng_need(r, 1);
     uint32_t range = (uint32_t)b - (uint32_t)a + 1u;
     uint64_t prod = (uint64_t)mt_next(r) * (uint64_t)range;
     uint32_t low = (uint32_t)prod;
     if (low < range) {
         uint32_t thr = (uint32_t)(0u - range) % range;
         while (low < thr) {
+            rng_need(r, 1);
             prod = (uint64_t)mt_next(r) * (uint64_t)range;
             low = (uint32_t)prod;
         }
@@ -342,7 +355,8 @@ struct WalkEnv {
     lds_c *dyn;             // dynamic LDS
     int ncol;               // operators per superstate (4 nb)
     int dkey;               // key change by a creator of spin 0 | of spin 1 << 8; 0: no such keys
-    int np, full;           // removable pairs of the window; no room for another pair
+    int np;                 // removable pairs of the window
+    int ready;              // window list valid and room for any move; cleared by whatever changes that
     int zero;               // offset of the zero behind the operator table
     int nkmax;              // matrix-instruction steps of the largest block
     int swapped;            // the trial list's buffer is the window list
@@ -511,56 +525,83 @@ DEV void set_window(Ctx &c)
     c.h.wvalid = 0;
 }
 
-DEV void shift_window(Ctx &c)
-{
-    if (c.h.nwin > 1) {
-        c.h.wpos++;
-        if (c.h.wpos == c.h.nwin) c.h.wpos = 0;
-        set_window(c);
-    } else {
-        c.h.wpos = 0;
-    }
-}
-
 DEV double bound_tau(int m, int nwin, double beta)
 {
     if (nwin <= 1) return m == 0 ? 0.0 : beta;
     return ((double)m / (double)(nwin + 1)) * beta;
 }
 
-DEV int lower_bound_tau(const double *tau, int n, double x)
+// Index of the first operator at or behind x (lower) / behind x (upper): the
+// sorted list is counted 256 entries at a time, one memory round trip instead
+// of one per bisection step.
+template <bool UPPER>
+DEV int bound_index(const double *tau, int n, double x)
 {
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (tau[mid] < x) lo = mid + 1; else hi = mid;
+    int cnt = 0;
+    for (int b = 0; b < n; b += 4 * WAVE) {
+        double t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = b + u * WAVE + lane_id();
+            t[u] = tau[min(j, n - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const bool in = b + u * WAVE + lane_id() < n;
+            cnt += popc64(__ballot(in && (UPPER ? t[u] <= x : t[u] < x)));
+        }
     }
-    return lo;
+    return cnt;
 }
-
-DEV int upper_bound_tau(const double *tau, int n, double x)
-{
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (tau[mid] <= x) lo = mid + 1; else hi = mid;
-    }
-    return lo;
-}
+DEV int lower_bound_tau(const double *tau, int n, double x) { return bound_index<false>(tau, n, x); }
+DEV int upper_bound_tau(const double *tau, int n, double x) { return bound_index<true>(tau, n, x); }
 
 // indices [wia, wib) of the operators inside [tauwin_min, tauwin_max] and
 // their copy in the LDS window list; kept across moves until the window
 // shifts or a global / tau-shift move rewrites the configuration.  Returns
-// false if the window does not fit the LDS list.
-DEV bool ensure_window(Ctx &c)
+// false if the window does not fit the LDS list.  Up to 512 operators are read
+// in one round trip.
+template <int NM>
+__device__ __attribute__((noinline)) bool load_window(ChainRef r)
 {
-    if (c.h.wvalid) return true;
-    const int ia = lower_bound_tau(c.tau, c.h.nop, c.h.tauwin_min);
-    const int ib = upper_bound_tau(c.tau, c.h.nop, c.h.tauwin_max);
+    Ctx c = attach<NM>(r);
+    constexpr int U = 8;
+    const int n = uni(c.h.nop), l = lane_id();
+    const double wmin = c.h.tauwin_min, wmax = c.h.tauwin_max;
+    int ia = 0, ib = 0;
+    double t[U];
+    int cd[U];
+    for (int b = 0; b < n; b += U * WAVE) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (b + u * WAVE < n) {
+                const int j = min(b + u * WAVE + l, n - 1);
+                t[u] = c.tau[j];
+                cd[u] = c.code[j];
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (b + u * WAVE < n) {
+                const bool in = b + u * WAVE + l < n;
+                ia += popc64(__ballot(in && t[u] < wmin));
+                ib += popc64(__ballot(in && t[u] <= wmax));
+            }
+    }
     if (ib - ia + 2 > c.L.lcap_lds) return false;
-    for (int j = lane_id(); j < ib - ia; j += WAVE) {
-        c.wtau[j] = c.tau[ia + j];
-        c.wcode[j] = c.code[ia + j];
+    if (n <= U * WAVE) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = u * WAVE + l;
+            if (u * WAVE < n && j >= ia && j < ib) {
+                c.wtau[j - ia] = t[u];
+                c.wcode[j - ia] = cd[u];
+            }
+        }
+    } else {
+        for (int j = l; j < ib - ia; j += WAVE) {
+            c.wtau[j] = c.tau[ia + j];
+            c.wcode[j] = c.code[ia + j];
+        }
     }
     c.h.wia = ia;
     c.h.wib = ib;
@@ -938,6 +979,175 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_,
     return out;
 }
 
+// sums and scans over the 16 lanes of a row
+DEV int row_sum_i(int x)
+{
+    x += dpp_i<DPP_QP_1032>(x);
+    x += dpp_i<DPP_QP_2301>(x);
+    x += dpp_i<DPP_ROW_HALF_MIRROR>(x);
+    return x + dpp_i<DPP_ROW_MIRROR>(x);
+}
+DEV double row_sum_d(double x)
+{
+    x += dpp_d<DPP_QP_1032>(x);
+    x += dpp_d<DPP_QP_2301>(x);
+    x += dpp_d<DPP_ROW_HALF_MIRROR>(x);
+    return x + dpp_d<DPP_ROW_MIRROR>(x);
+}
+DEV int row_scan_i(int x)
+{
+    x += dpp_mov_i<0x111, 0xf>(0, x);
+    x += dpp_mov_i<0x112, 0xf>(0, x);
+    x += dpp_mov_i<0x114, 0xf>(0, x);
+    return x + dpp_mov_i<0x118, 0xf>(0, x);
+}
+DEV double row_scan_d(double x)
+{
+    x += dpp_mov_d<0x111, 0xf>(0.0, x);
+    x += dpp_mov_d<0x112, 0xf>(0.0, x);
+    x += dpp_mov_d<0x114, 0xf>(0.0, x);
+    return x + dpp_mov_d<0x118, 0xf>(0.0, x);
+}
+DEV double row_scan_mul(double x)
+{
+    x *= dpp_mov_d<0x111, 0xf>(1.0, x);
+    x *= dpp_mov_d<0x112, 0xf>(1.0, x);
+    x *= dpp_mov_d<0x114, 0xf>(1.0, x);
+    return x * dpp_mov_d<0x118, 0xf>(1.0, x);
+}
+
+// walk_small for lists of up to 15 operators on blocks of up to 4 states whose
+// superstates have additive keys (most proposals: a 2-orbital window at
+// TaudiffMax = beta / 10 holds 22 operators, a proposal walks the 8 or so
+// between its changes).  Every row of 16 lanes holds the whole list (lane p of a
+// row operator p, the lane behind the last one the propagation to tend), so scans
+// and sums stay within a row; one exponential per lane gives the propagators of
+// all operators (lane (state r, operator p) = 16 r + p); operators come in
+// groups of four, filled up with identities, so that a group is four matrix
+// instructions in a row and one renormalisation check, and the state ends in
+// the last quad.
+// A chain alone on its SIMD issues an instruction about every five cycles, so
+// what counts is their number: about 350 here against 900 for the general walk.
+template <int NM, bool BRA, bool KEEP>
+__device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, double tstart, double tend,
+                                                          const lds_d *otau_, const lds_i *ocode_, int n_, int no_,
+                                                          Prefix<NM> px)
+{
+    const int l = lane_id(), p = l & 15;
+    const int n = uni(n_), no = uni(no_);
+    const lds_d *otau = uni_lds(otau_);
+    const lds_i *ocode = uni_lds(ocode_);
+    const WalkEnv &E = s_wenv;
+    const double egs = E.egs;
+    const lds_i4 *tr = uni_lds(E.tr), *sinfo = uni_lds(E.sinfo);
+    const lds_d *ev = uni_lds(E.ev), *lops = uni_lds(E.lops);
+    const lds_b *keys = uni_lds(E.keys);
+    const int ncol = uni(E.ncol), dkey = uni(E.dkey);
+    const int s0 = uni(s_);
+    WalkOut<NM> out;
+    out.s = -1;
+    // operator of this lane, the time before it, the superstate before it
+    const bool op = p < n;
+    const int j = op ? (BRA ? n - 1 - p : p) : 0;
+    const int cd = ocode[j];
+    const double tj = otau[j], tb = otau[p > 0 && p <= n ? (BRA ? n - p : p - 1) : 0];
+    const int key0 = (int)keys[s0];
+    const double t = op ? tj : tend, tp = p > 0 ? tb : tstart;
+    const double dt = p <= n ? (BRA ? tp - t : t - tp) : 0.0;
+    const int ca = BRA ? 2 - op_ca(cd) : op_ca(cd) - 1;   // 0: creator
+    const int col = (op_orb(cd) * 2 + op_spin(cd)) * 2 + ca;
+    int d = (int)(signed char)(op_spin(cd) ? dkey >> 8 : dkey);
+    d = op ? (ca ? -d : d) : 0;
+    const int key = key0 + row_scan_i(d) - d;
+    int sb = keys[256 + (key & 255)];
+    const bool none = sb == 255;
+    sb = none ? 0 : sb;
+    const iv4 rec = tr[sb * ncol + (op ? col : 0)], si = sinfo[sb];
+    if (__ballot((op && (none || rec.x < 0)) || (p == n && none)) != 0ull) return out;
+    out.s = __builtin_amdgcn_readlane(sb, n);
+    const double e0 = __hiloint2double(si.y, si.x), lc = -(e0 - egs) * dt;
+    const int ns = si.z & 255, eo = si.z >> 8;
+    {
+        const int both = __builtin_amdgcn_readlane(row_sum_i(op ? ((rec.y * ns) << 16) | (ns + rec.y) : 0), 0);
+        const int in = __builtin_amdgcn_readlane(row_sum_i(op ? ns : 0), 0);
+        if (l == 0) {
+            __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.flops, (double)(no * (2 * (both >> 16) + in)));
+            __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.bytes, (double)(8 * no * (both & 0xffff)));
+        }
+    }
+    if constexpr (KEEP) {
+        if (l < n) px.sst[p] = rec.x;
+    }
+    const double sc = KEEP ? row_scan_d(lc) : row_sum_d(lc);
+    double lg = 0.0;
+    if constexpr (NM == 1) {
+        // every block is one number, every propagation a log factor only
+        const double a = row_scan_mul(op ? lops[rec.z] : 1.0), k0 = readlane_d(k.v[0], 0);
+        if constexpr (KEEP) {
+            if (l < n) {
+                px.k[p] = k0 * a;
+                px.lg[p] = sc;
+            }
+        }
+        k.v[0] *= readlane_d(a, 15);   // zero in the lanes outside the block
+    } else {
+        const bool each = __ballot(__int_as_float(si.w) * (float)dt > 100.0f) != 0ull;
+        const int blk = (l >> 2) & 3, i = l & 3, r = l >> 4;
+        const double dr = exp(-(ev[eo + (r < ns ? r : 0)] - e0) * dt);
+        // block offset, sizes; 1 << 28: the propagation to tend, 1 << 29: beyond it
+        const int pack = op ? (rec.z & 0xfffff) | (rec.y << 20) | (ns << 24) : (ns << 20) | (ns << 24) | (p == n ? 1 << 28 : 1 << 29);
+        double a[4];
+#pragma unroll
+        for (int ps = 0; ps < 4; ++ps) {
+            if (4 * ps <= n) {
+                const int src = (l & 48) + 4 * ps + blk;
+                const int pk = __shfl(pack, src, WAVE);
+                const double dq = __shfl(dr, src, WAVE);
+                const int nt = (pk >> 20) & 15, nq = (pk >> 24) & 15, oth = pk >> 28;
+                const bool in = i < nt && r < nq;
+                const double pv = lops[in && !oth ? (pk & 0xfffff) + i + r * nt : 0];
+                a[ps] = oth ? (i == r ? (oth == 2 ? 1.0 : dq) : 0.0) : (in ? pv * dq : 0.0);
+            }
+        }
+#pragma unroll
+        for (int ps = 0; ps < 4; ++ps) {
+            if (4 * ps <= n) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const double x = dpp_d<DPP_ROW_ROR4>(k.v[0]);
+                    k.v[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[ps], x, 0.0, 0, 0, 0);
+                    if (b == 3 || each) renorm(k, 0x000F000F000F000Full << (4 * b), lg);
+                    if constexpr (KEEP) {
+                        const int t_ = 4 * ps + b;
+                        if (t_ < n) {
+                            const int nt = __builtin_amdgcn_readlane(rec.y, t_);
+                            if (blk == b && r < nt && i < no) px.k[t_ * 16 + r * no + i] = k.v[0];
+                            px.lg[t_] = lg + readlane_d(sc, t_);
+                        }
+                    }
+                }
+            }
+        }
+        // the state to every quad
+        double x = blk == 3 ? k.v[0] : 0.0;
+        x += dpp_d<DPP_ROW_ROR4>(x);
+        k.v[0] = x + dpp_d<DPP_ROW_ROR8>(x);
+    }
+    out.lg = lg + readlane_d(sc, KEEP ? n : 0);
+    out.k = k;
+    return out;
+}
+
+template <int NM, bool BRA, bool KEEP>
+DEV WalkOut<NM> walk_any(State<NM> k, int s, double tstart, double tend, const lds_d *otau, const lds_i *ocode, int n,
+                         int no, Prefix<NM> px)
+{
+    if constexpr (NM <= 4) {
+        if (n <= 15 && uni(s_wenv.dkey)) return walk_row<NM, BRA, KEEP>(k, s, tstart, tend, otau, ocode, n, no, px);
+    }
+    return walk_small<NM, BRA, KEEP>(k, s, tstart, tend, otau, ocode, n, no, px);
+}
+
 // What an operator walk over blocks above 16 states needs, by value (the walk
 // is out of line; a reference to the chain context would live in scratch).
 struct MfmaEnv {
@@ -1176,7 +1386,7 @@ DEV bool walk_list(State<NM> &k, int &s, double &lg, int no, double t0, const do
                    double t1)
 {
     const WalkOut<NM> o =
-        walk_small<NM, BRA, false>(k, s, t0, t1, (const lds_d *)otau, (const lds_i *)ocode, n, no, Prefix<NM>{});
+        walk_any<NM, BRA, false>(k, s, t0, t1, (const lds_d *)otau, (const lds_i *)ocode, n, no, Prefix<NM>{});
     if (o.s < 0) return false;
     k = o.k;
     s = o.s;
@@ -1204,9 +1414,19 @@ DEV bool walk_big(Ctx &c, double *&K, double *&Kw, int &s, double &lg, int no, d
 DEV int stage_chunk(Ctx &c, int j0, int j1)
 {
     const int n = min(j1 - j0, c.L.lcap_lds);
-    for (int j = lane_id(); j < n; j += WAVE) {
-        c.ttau[j] = c.tau[j0 + j];
-        c.tcode[j] = c.code[j0 + j];
+    for (int b = 0; b < n; b += 4 * WAVE) {
+        double t[4];
+        int cd[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = j0 + min(b + u * WAVE + lane_id(), n - 1);
+            t[u] = c.tau[j], cd[u] = c.code[j];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = b + u * WAVE + lane_id();
+            if (j < n) c.ttau[j] = t[u], c.tcode[j] = cd[u];
+        }
     }
     wsync();
     return n;
@@ -1405,11 +1625,15 @@ DEV void rebuild_cache(Ctx &c)
         c.bndlog[top] = lg;
         c.bndsst[top] = s;
     }
+    // the whole configuration in the trial list where it fits
+    const bool staged = NM <= 16 && c.h.nop <= c.L.lcap_lds;
+    if (staged) stage_chunk(c, 0, c.h.nop);
     for (int m = top - 1; m >= p + 2; --m) {
         const double tm = bound_tau(m, nw, c.M.beta);
-        const int loidx = upper_bound_tau(c.tau, c.h.nop, tm);
+        const int loidx = staged ? upper_bound_tau(c.ttau, hiidx, tm) : upper_bound_tau(c.tau, hiidx, tm);
         if constexpr (NM <= 16) {
-            walk_global<NM, true>(c, k, s, lg, no, tb, loidx, hiidx, tm);
+            if (staged) walk_list<NM, true>(k, s, lg, no, tb, c.ttau + loidx, c.tcode + loidx, hiidx - loidx, tm);
+            else walk_global<NM, true>(c, k, s, lg, no, tb, loidx, hiidx, tm);
             k.store(c.bnd + (long)m * stride, c.sz[s], no);
         } else {
             walk_global_big<true>(c, B, Bw, s, lg, no, tb, loidx, hiidx, tm);
@@ -1425,10 +1649,11 @@ DEV void rebuild_cache(Ctx &c)
     s = outer;
     lg = 0.0;
     const double tp = bound_tau(p, nw, c.M.beta);
-    const int n0 = lower_bound_tau(c.tau, c.h.nop, tp);
+    const int n0 = staged ? lower_bound_tau(c.ttau, hiidx, tp) : lower_bound_tau(c.tau, hiidx, tp);
     if constexpr (NM <= 16) {
         k.identity(no);
-        walk_global<NM, false>(c, k, s, lg, no, 0.0, 0, n0, tp);
+        if (staged) walk_list<NM, false>(k, s, lg, no, 0.0, c.ttau, c.tcode, n0, tp);
+        else walk_global<NM, false>(c, k, s, lg, no, 0.0, 0, n0, tp);
         k.store(c.kst, c.sz[s], no);
     } else {
         double *K = c.K0, *Kw = c.K1;
@@ -1586,7 +1811,7 @@ __device__ __attribute__((noinline)) void seg_extend(ChainRef ref, int nw_, int 
         const int a = BRA ? nw - to : j;
         const double t0 = j > 0 ? c.wtau[BRA ? nw - j : j - 1] : bound_tau(BRA ? w + 2 : w, c.h.nwin, c.M.beta);
         const double t1 = c.wtau[BRA ? nw - to : to - 1];
-        walk_small<NM, BRA, true>(k, s, t0, t1, (const lds_d *)(c.wtau + a), (const lds_i *)(c.wcode + a), to - j,
+        walk_any<NM, BRA, true>(k, s, t0, t1, (const lds_d *)(c.wtau + a), (const lds_i *)(c.wcode + a), to - j,
                                   no, px);
         // log scales of a walk count from its start
         for (int i = j + 1 + lane_id(); i <= to; i += WAVE) bx[i] += lg0;
@@ -1616,6 +1841,111 @@ DEV bool segment_trace(Ctx &c, int nw, int j0, int m0, int a, int n, double t0, 
         T = trace_of<NM>(x, lg + c.lbx[m0]);
     }
     return true;
+}
+
+// The window moves on by half its width (shift_window, Trace.F90:1652-1668).
+// While the list and the caches belong to the window left behind, they move
+// with it: the ket at the new lower edge is the prefix ket of the last operator
+// passed, propagated to the edge; the prefix kets of the upper half stay (LDS
+// caches); the list keeps its upper half and is continued from the
+// configuration.  Otherwise the next move reloads them.
+template <int NM>
+__device__ __attribute__((noinline)) void slide_window(ChainRef ref)
+{
+    Ctx c = attach<NM>(ref);
+    s_wenv.ready = 0;
+    const int p = uni(c.h.wpos), nw = uni(c.h.wib - c.h.wia), nwin = uni(c.h.nwin), nop = uni(c.h.nop);
+    if (nwin <= 1) {
+        c.h.wpos = 0;
+        return;
+    }
+    const bool follow = NM <= 16 && c.h.wvalid && c.h.cache_pos == p && p + 1 < nwin && nw <= c.L.sc;
+    c.h.wpos = p + 1 == nwin ? 0 : p + 1;
+    const double edge0 = bound_tau(p, nwin, c.M.beta);
+    set_window(c);
+    if constexpr (NM <= 16) {
+        if (!follow) return;
+        const double wmin = c.h.tauwin_min, wmax = c.h.tauwin_max, edge = bound_tau(p + 1, nwin, c.M.beta);
+        int low = 0;   // operators left behind
+        for (int j0 = 0; j0 < nw; j0 += WAVE) {
+            const int j = j0 + lane_id();
+            low += popc64(__ballot(j < nw && c.wtau[j < nw ? j : 0] < wmin));
+        }
+        // the operators that follow, one round trip
+        const int wib = uni(c.h.wib);
+        int more = 0;
+        for (int j0 = wib; j0 < nop; j0 += WAVE) {
+            const int j = min(j0 + lane_id(), nop - 1);
+            const double t = c.tau[j];
+            const int cd = c.code[j];
+            const bool in = j0 + lane_id() < nop && t <= wmax;
+            const int cnt = popc64(__ballot(in));
+            if (nw - low + more + cnt + 2 > c.L.lcap_lds) return;   // reported by the next move
+            if (in) {
+                c.ttau[nw - low + more + lane_id()] = t;
+                c.tcode[nw - low + more + lane_id()] = cd;
+            }
+            more += cnt;
+            if (cnt < WAVE) break;
+        }
+        // ket at the new edge
+        if (c.h.rk_n <= low) {
+            c.h.wpos = p;   // seg_extend starts from the window left behind
+            seg_extend<NM, false>(ref, nw, low);
+            c.h.wpos = p + 1;
+        }
+        const int s = uni(c.rks[low]), no = c.sz[c.h.outer], ns = c.sz[s];
+        State<NM> k = seg_load<NM>(c.rk, low, ns, no);
+        const double *E = c.ev + c.off[s];
+        const double dt = edge - (low > 0 ? c.wtau[low - 1] : edge0), e0 = E[0];
+        double lg = c.rkx[low] - (e0 - c.M.egs) * dt;
+#pragma unroll
+        for (int e = 0; e < State<NM>::NV; ++e) {
+            const int r = State<NM>::row(e);
+            k.v[e] *= exp(-(E[r < ns ? r : 0] - e0) * dt);
+        }
+        if constexpr (NM > 1) renorm(k, ~0ull, lg);
+        k.store(c.kst, ns, no);
+        c.h.kst_log = lg;
+        c.h.kst_sst = s;
+        c.h.cache_pos = p + 1;
+        // list
+        for (int j = low + lane_id(); j < nw; j += WAVE) {
+            c.ttau[j - low] = c.wtau[j];
+            c.tcode[j - low] = c.wcode[j];
+        }
+        c.h.wia += low;
+        c.h.wib = c.h.wia + nw - low + more;
+        c.h.wvalid = 1;
+        c.h.pc_valid = 0;
+        c.h.lb_n = 0;
+        if constexpr (NM <= 4) {
+            // prefix kets low + 1 .. rk_n - 1 become 1 .. rk_n - 1 - low
+            constexpr int S2 = NM * NM;
+            const int rn = uni(c.h.rk_n) - low;
+            for (int i = S2 + lane_id(); i - lane_id() < rn * S2; i += WAVE) {
+                const double x = i < rn * S2 ? c.rk[low * S2 + i] : 0.0;
+                wsync();
+                if (i < rn * S2) c.rk[i] = x;
+                wsync();
+            }
+            for (int i = 1 + lane_id(); i - lane_id() < rn; i += WAVE) {
+                const double x = i < rn ? c.rkx[low + i] : 0.0;
+                const int q = i < rn ? c.rks[low + i] : 0;
+                wsync();
+                if (i < rn) c.rkx[i] = x, c.rks[i] = q;
+                wsync();
+            }
+            k.store(c.rk, ns, no);
+            c.rkx[0] = lg;
+            c.rks[0] = s;
+            c.h.rk_n = rn;
+        } else {
+            c.h.rk_n = 0;
+        }
+        wsync();
+        swap_lists(c);
+    }
 }
 
 // Trace of a proposal: the window with its operators [j0, nw - m0) replaced by
@@ -1772,12 +2102,12 @@ DEV void rank1(Ctx &c, double *Mf, int k, const MatLanes &ml, double a, const do
         const bool in = i < k;
         double *Mi = Mf + (in ? i : 0);
         const double ci = in ? a * col[i] : 0.0;
-        for (int j0 = ml.g; j0 < k; j0 += 8 * ml.step) {
-            double m[8];
+        for (int j0 = ml.g; j0 < k; j0 += 16 * ml.step) {
+            double m[16];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) m[u] = Mi[(long)min(j0 + u * ml.step, k - 1) * ld];
+            for (int u = 0; u < 16; ++u) m[u] = Mi[(long)min(j0 + u * ml.step, k - 1) * ld];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < 16; ++u) {
                 const int j = j0 + u * ml.step;
                 if (in && j < k) Mi[(long)j * ld] = fma(ci, row[j], m[u]);
             }
@@ -1785,9 +2115,22 @@ DEV void rank1(Ctx &c, double *Mf, int k, const MatLanes &ml, double a, const do
     }
 }
 
+// The first columns of M for detrat_add, loaded ahead of the lists and the
+// hybridisation values that its product waits for (all of M up to order 32).
+struct MatHead {
+    double m[16];
+    DEV MatHead(const double *Mf, int k, int ld)
+    {
+        const MatLanes ml(k);
+        const double *col = Mf + (ml.i < k ? ml.i : 0);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) m[u] = col[(long)max(min(ml.g + u * ml.step, k - 1), 0) * ld];
+    }
+};
+
 // R^T M Q of an order-k block (get_DetRatAdd); leaves M Q in colb.  The loads
-// of eight columns are in flight together.
-DEV double detrat_add(Ctx &c, const double *Mf, int k)
+// of sixteen columns are in flight together.
+DEV double detrat_add(Ctx &c, const double *Mf, int k, const MatHead &head)
 {
     const int ld = c.L.kcap;
     const MatLanes ml(k);
@@ -1797,12 +2140,17 @@ DEV double detrat_add(Ctx &c, const double *Mf, int k)
         const bool in = i < k;
         const double *col = Mf + (in ? i : 0);
         double acc = 0.0;
-        for (int j0 = ml.g; j0 < k; j0 += 8 * ml.step) {
-            double m[8];
+        for (int j0 = ml.g; j0 < k; j0 += 16 * ml.step) {
+            double m[16];
+            if (i0 == 0 && j0 == ml.g) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) m[u] = col[(long)min(j0 + u * ml.step, k - 1) * ld];
+                for (int u = 0; u < 16; ++u) m[u] = head.m[u];
+            } else {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+                for (int u = 0; u < 16; ++u) m[u] = col[(long)min(j0 + u * ml.step, k - 1) * ld];
+            }
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
                 const int j = j0 + u * ml.step;
                 acc = fma(m[u], j < k ? c.Q[j] : 0.0, acc);
             }
@@ -1833,12 +2181,12 @@ DEV void mat_add_phys(Ctx &c, double *Mf, int k, double dr)
         const int j = j0 + ml.i;
         const double *mc = Mf + (long)min(j, k - 1) * ld;
         double v = 0.0;
-        for (int i0 = ml.g; i0 < k; i0 += 8 * ml.step) {
-            double m[8];
+        for (int i0 = ml.g; i0 < k; i0 += 16 * ml.step) {
+            double m[16];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) m[u] = mc[min(i0 + u * ml.step, k - 1)];
+            for (int u = 0; u < 16; ++u) m[u] = mc[min(i0 + u * ml.step, k - 1)];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < 16; ++u) {
                 const int i = i0 + u * ml.step;
                 v = fma(i < k ? c.R[i] : 0.0, m[u], v);
             }
@@ -2067,14 +2415,6 @@ DEV int count_below_par(const double *arr, int n, double x)
 enum { OUT_REJ = 0, OUT_ACC = 1, OUT_QN = 2 };
 enum { ERR_CAP = 3, ERR_SING = 4, ERR_STATE_DEV = 6 };
 
-// Whether every flavour can take one more pair and the list two more operators
-DEV void room_left(Ctx &c)
-{
-    int km = 0;
-    for (int f = 0; f < c.M.nf; ++f) km = max(km, c.h.kf[f]);
-    s_wenv.full = km + 1 > c.L.kcap || c.h.nop + 2 > c.L.cap;
-}
-
 // write the LDS trial list into the global operator list at wia (its length
 // nl replaces the window's nw operators: the tail [wib, nop) moves first); the
 // trial list then serves as the window list
@@ -2100,7 +2440,7 @@ DEV void record_pair(Ctx &c, int f, double dt)
     if (lane_id() == 0) {
         double *ap = reinterpret_cast<double *>(c.base + c.L.accpair) + (long)f * c.L.naccpair_cap;
         const int bin = min(c.h.naccpair, (int)floor(dt / c.h.accpair_max * (double)c.h.naccpair) + 1);
-        ap[bin - 1] += 1.0;
+        global_add(ap + bin - 1, 1.0);
         if (c.h.apt_index <= c.h.apt_n) reinterpret_cast<double *>(c.base + c.L.aptau)[c.h.apt_index - 1] = dt;
     }
     if (c.h.apt_index <= c.h.apt_n) c.h.apt_index++;
@@ -2131,6 +2471,7 @@ __device__ __attribute__((noinline)) void accept_add(ChainRef ref, AddMove m)
     const bool seg = NM <= 16 && nw <= c.L.sc;
     mat_add_phys(c, c.mi(f), k, S);
     c.work(6.0 * k * k, 8.0 * k * k + 8.0 * (k + 1) * (k + 1));
+    s_wenv.ready = 0;
     commit_window(c, nl);
     c.h.pc_valid = 0;
     // segment caches: the first q1 and the last nw - q2 window operators are unchanged
@@ -2139,7 +2480,6 @@ __device__ __attribute__((noinline)) void accept_add(ChainRef ref, AddMove m)
     lists_insert(c, fo, k, fp_c - 1, tc, fp_a - 1, ta);
     c.h.kf[f] = k + 1;
     c.h.kfmax[f] = max(c.h.kfmax[f], k + 1);
-    room_left(c);
     record_pair(c, f, fabs(ta - tc));
     c.h.det_log += log(fabs(S));
     c.h.det_sign *= m.dr_sign;
@@ -2166,13 +2506,13 @@ DEV int step_add(Ctx &c)
     const double wmin = c.h.tauwin_min, wmax = c.h.tauwin_max, tdm = c.h.taudiff_max;
     const int nw = uni(c.h.wib - c.h.wia);
     const double width = wmax - wmin;
-    const double tref = wmin + width * grnd(c.rng);
+    const double tref = wmin + width * grnd<false>(c.rng);
     double tdf = width;
-    const int orb = randint(c.rng, 1, M.nb) - 1;
-    const int spin = randint(c.rng, 1, 2) - 1;
+    const int orb = randint<false>(c.rng, 1, M.nb) - 1;
+    const int spin = randint<false>(c.rng, 1, 2) - 1;
     const double tmin = fmax(tref - tdm, wmin);
     const double w2 = fmin(tref + tdm, wmax) - tmin;
-    const double t2 = tmin + w2 * grnd(c.rng);
+    const double t2 = tmin + w2 * grnd<false>(c.rng);
     tdf *= w2;
     const int f = orb + M.nb * spin;
     if (t2 == tref) return OUT_QN;
@@ -2220,6 +2560,7 @@ DEV int step_add(Ctx &c)
     // det ratio, get_LogDetRatPairAdd (Trace.F90:2775-2832): Q (annihilators) and
     // R (creators) placed by physical slot, the lane behind the last rank takes
     // S0 = F(ta - tc); FPos = 1 + earlier operators of the type
+    const MatHead head(c.mi(f), k, c.L.kcap);
     const long fo = (long)f * c.L.kcap;
     const double *ctl = c.fc + fo, *atl = c.fa + fo;
     const int *csl = c.fcs + fo, *asl = c.fas + fo;
@@ -2247,11 +2588,11 @@ DEV int step_add(Ctx &c)
         sgn += popc64(__ballot(abet)) + popc64(__ballot(in && xc > tc)) + popc64(__ballot(in && xa > tc));
     }
     wsync();
-    const double S = S0 - detrat_add(c, c.mi(f), k);
+    const double S = S0 - detrat_add(c, c.mi(f), k, head);
     c.work(2.0 * k * k, 8.0 * k * k);
     const double sig = ((fp_c - fp_a) & 1) ? -1.0 : 1.0;
     const double dr_sign = copysign(1.0, S) * sig;
-    const double rnd = grnd(c.rng);
+    const double rnd = grnd<false>(c.rng);
     const double wr = weight_ratio(T, S, c.h.trace_log);
     const double prob = fabs(((1.0 * tdf) * (double)(2 * M.nb)) / (double)np * wr);
     if (!(rnd < prob)) return OUT_REJ;
@@ -2272,6 +2613,7 @@ __device__ __attribute__((noinline)) void accept_rem(ChainRef ref, RemMove m)
     const bool seg = NM <= 16 && nw <= c.L.sc;
     mat_rem_phys(c, c.mi(f), k, sc, sa);
     c.work(3.0 * k * k, 8.0 * k * k + 8.0 * (k - 1) * (k - 1));
+    s_wenv.ready = 0;
     commit_window(c, nl);
     c.h.pc_valid = 0;
     // segment caches: the first w1 and the last nw - 1 - w2 window operators are unchanged
@@ -2279,7 +2621,6 @@ __device__ __attribute__((noinline)) void accept_rem(ChainRef ref, RemMove m)
     c.h.lb_n = seg ? min(c.h.lb_n, nw - w2) : 0;
     lists_remove(c, fo, k, fp_c - 1, sc, fp_a - 1, sa);
     c.h.kf[f] = k - 1;
-    room_left(c);
     record_pair(c, f, m.dt);
     c.h.det_log += log(fabs(S));
     c.h.det_sign *= m.dr_sign;
@@ -2299,7 +2640,7 @@ DEV int step_rem(Ctx &c)
     ensure_cache<NM>(c);
     const int np = uni(s_wenv.np);
     if (np <= 0) return OUT_QN;
-    int pick = randint(c.rng, 1, np);
+    int pick = randint<false>(c.rng, 1, np);
     // the pick-th pair: the operator w1 whose running count reaches it, and
     // among the later operators of its flavour and the other type the one that
     // the rest of the count names
@@ -2313,7 +2654,7 @@ DEV int step_rem(Ctx &c)
         if (at) w1 = j0 + b;
     }
     if (w1 < 0) {
-        c.h.err = ERR_STATE_DEV;
+        c.h.err = ERR_STATE_DEV, s_wenv.ready = 0;
         return OUT_REJ;
     }
     const int c1 = uni(c.wcode[w1]);
@@ -2329,7 +2670,7 @@ DEV int step_rem(Ctx &c)
         w2 = j0 + __builtin_ctzll(mate);
     }
     if (w2 < 0) {
-        c.h.err = ERR_STATE_DEV;
+        c.h.err = ERR_STATE_DEV, s_wenv.ready = 0;
         return OUT_REJ;
     }
     const double t1 = c.wtau[w1], t2 = c.wtau[w2];
@@ -2377,10 +2718,10 @@ DEV int step_rem(Ctx &c)
     const double dr_sign = copysign(1.0, S) * sig;
     const double wr = weight_ratio(T, S, c.h.trace_log);
     const double prob = fabs(((1.0 * hprf) / (double)(2 * M.nb)) * wr);
-    const double rnd = grnd(c.rng);
+    const double rnd = grnd<false>(c.rng);
     if (!(rnd < prob)) return OUT_REJ;
     if (fabs(S) < 1e-12) {
-        c.h.err = ERR_SING;
+        c.h.err = ERR_SING, s_wenv.ready = 0;
         return OUT_REJ;
     }
     accept_rem<NM>(c.ref(), RemMove{f, k, nl, w1, w2, fp_c, fp_a, sc, sa, t2 - t1, S, dr_sign,
@@ -2474,6 +2815,7 @@ template <int NM>
 __device__ __attribute__((noinline)) int step_glob(ChainRef ref)
 {
     Ctx c = attach<NM>(ref);
+    s_wenv.ready = 0;
     const RngScope rs(c.rng);
     CModel &M = c.M;
     c.h.try_glob++;
@@ -2663,6 +3005,7 @@ template <int NM>
 __device__ __attribute__((noinline)) int step_shift(ChainRef ref)
 {
     Ctx c = attach<NM>(ref);
+    s_wenv.ready = 0;
     const RngScope rs(c.rng);
     CModel &M = c.M;
     if (c.h.nop == 0) {
@@ -2789,11 +3132,22 @@ __device__ __attribute__((noinline)) int step_shift(ChainRef ref)
 // lists.  Checked before the move's first random draw, so a chain that has no
 // room stops with its state and random stream intact and continues exactly
 // where it stopped once the host has enlarged its memory.  Loads the window
-// list (as the next insertion or removal would).
-DEV bool room_for_move(Ctx &c)
+// list (as the next insertion or removal would).  A chain that has stopped on
+// an error is not ready either.
+template <int NM>
+__device__ __attribute__((noinline)) bool make_ready(ChainRef r)
 {
-    if (s_wenv.full || !ensure_window(c)) return false;
-    return c.h.wib - c.h.wia + 2 <= c.L.lcap_lds;
+    Ctx c = attach<NM>(r);
+    if (c.h.err != 0 || c.h.halt != HALT_NONE) return false;
+    int km = 0;
+    for (int f = lane_id(); f < c.M.nf; f += WAVE) km = c.h.kf[f];
+    km = wave_imax(km);
+    const bool ok = km + 1 <= c.L.kcap && c.h.nop + 2 <= c.L.cap && (c.h.wvalid || load_window<NM>(r)) &&
+                    c.h.wib - c.h.wia + 2 <= c.L.lcap_lds;
+    if (!ok) c.h.halt = HALT_CAP;
+    s_wenv.ready = ok;
+    wsync();
+    return ok;
 }
 
 // What a sweep counts in registers: insertion and removal attempts, proposals
@@ -2809,10 +3163,10 @@ template <int NM>
 DEV void one_move(Ctx &c, Tally &ty, int &kind, int &out)
 {
     CModel &M = c.M;
-    const double r = grnd(c.rng);
+    rng_need(c.rng, MOVE_WORDS);
+    const double r = grnd<false>(c.rng);
     if (r <= 1.0 - M.p_shift - M.p_glob) {
-        grnd_skip(c.rng);   // Percentage4OperatorMove draw
-        grnd_skip(c.rng);   // PercentageOuterMove draw
+        c.rng.pos += 4;   // the draws of Percentage4OperatorMove and PercentageOuterMove
         if (r < (1.0 - M.p_shift - M.p_glob) / 2.0) {
             kind = 1;
             ty.add++;
@@ -2837,7 +3191,10 @@ DEV void one_move(Ctx &c, Tally &ty, int &kind, int &out)
     }
     // every nslide-th attempt; after a global move or shift the count, and with
     // it this condition, stands
-    if (ty.slide == 0) shift_window(c);
+    if (ty.slide == 0) {
+        slide_window<NM>(c.ref());
+        c.lists();
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -3501,6 +3858,7 @@ DEV Ctx make_ctx(char *chains, int chain, CArgs args, char *lds)
     CModel &M = *(CModel *)args;
     CLayout &L = *(CLayout *)(args + (sizeof(DevModel) + 7) / 8 * 8);
     s_wenv.dyn = (lds_c *)lds;
+    s_wenv.ready = 0;
     s_wenv.swapped = 0;
     wsync();
     char *base = chains + (long)chain * L.stride;
@@ -3580,7 +3938,9 @@ __device__ __attribute__((noinline)) bool calib_done(ChainRef r, int3 calib)
     int short_f = 0;
     for (int f = 0; f < c.M.nf; ++f) {
         double n = 0.0;
-        for (int b = lane_id(); b < c.h.naccpair; b += WAVE) n += ap[(long)f * c.L.naccpair_cap + b];
+        // the counts are written by atomics at L2: read past the vector L1
+        for (int b = lane_id(); b < c.h.naccpair; b += WAVE)
+            n += __hip_atomic_load(ap + (long)f * c.L.naccpair_cap + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         short_f += wave_sum(n) < (double)calib.z;
     }
     return short_f == 0;
@@ -3648,7 +4008,6 @@ __global__ void __launch_bounds__(WAVE) sweep_kernel(DevModel M, ChainLayout L, 
     extern __shared__ __align__(16) char lds[];
     Ctx c = make_ctx<NM>(chains, chain, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
     rng_open(c.rng);
-    room_left(c);
     wsync();
     const long long pos0 = c.h.pos;
     const int todo = (int)min(target - pos0, (long long)0x7fffffff);   // moves of this launch
@@ -3658,11 +4017,8 @@ __global__ void __launch_bounds__(WAVE) sweep_kernel(DevModel M, ChainLayout L, 
     int until = every - (int)(pos0 % every), ucal = calib.x ? calib.y - (int)(pos0 % calib.y) : 0;
     Tally ty{0, 0, 0, (int)((c.h.try_add + c.h.try_rem) % c.M.nslide)};
     int done = 0;
-    while (done < todo && (c.h.err | c.h.halt) == 0) {
-        if (!room_for_move(c)) {
-            c.h.halt = HALT_CAP;
-            break;
-        }
+    while (done < todo) {
+        if (!s_wenv.ready && !make_ready<NM>(c.ref())) break;
         int kind, out;
         one_move<NM>(c, ty, kind, out);
         // ctqmc_calibrate (CTQMC.F90:8128-8175): every calib.y moves, phase 1
@@ -3670,7 +4026,7 @@ __global__ void __launch_bounds__(WAVE) sweep_kernel(DevModel M, ChainLayout L, 
         // (calib.x = 2) once every flavour has calib.z accepted pairs
         if (calib.x && --ucal == 0) {
             ucal = calib.y;
-            if (calib_done<NM>(c.ref(), calib)) c.h.halt = HALT_DONE;
+            if (calib_done<NM>(c.ref(), calib)) c.h.halt = HALT_DONE, s_wenv.ready = 0;
         }
         if (rec && lane_id() == 0) {
             w2d_move_record &r = rec[pos0 + done - rec_base];
@@ -3689,7 +4045,8 @@ __global__ void __launch_bounds__(WAVE) sweep_kernel(DevModel M, ChainLayout L, 
         if (--until == 0) {
             until = every;
             if (ncorr > 0) measure<NM, SCORE>(c.ref());
-            if (__hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) c.h.halt = HALT_ABORT;
+            if (__hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))
+                c.h.halt = HALT_ABORT, s_wenv.ready = 0;
         }
     }
     rng_close(c.rng);
