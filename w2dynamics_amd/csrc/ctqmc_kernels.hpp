@@ -352,14 +352,17 @@ struct WalkEnv {
     const lds_d *lops;      // operator blocks in LDS (blocks up to 4 states)
     const lds_i4 *sinfo;    // per superstate: lowest energy, size | first energy << 8, width (float)
     lds_d *qa;              // propagators of 16 operators (blocks of 5..16 states); scratch
-    lds_c *dyn;             // dynamic LDS
     int ncol;               // operators per superstate (4 nb)
     int dkey;               // key change by a creator of spin 0 | of spin 1 << 8; 0: no such keys
     int np;                 // removable pairs of the window
     int ready;              // window list valid and room for any move; cleared by whatever changes that
     int zero;               // offset of the zero behind the operator table
     int nkmax;              // matrix-instruction steps of the largest block
-    int swapped;            // the trial list's buffer is the window list
+    int no;                 // states of the outer superstate (valid while ready)
+    // LDS addresses: window list and trial list (their buffers swap), pair
+    // counts, work vectors, segment caches, tables
+    unsigned wtau, wcode, ttau, tcode, pc, q, r, col, row, rk, lb, rkx, lbx, rks, lbs;
+    unsigned legc, k, sz, off, trt, evt, opst, mt, dvec, pl, strip;
 };
 __shared__ WalkEnv s_wenv;
 __shared__ ChainHdr s_hdr;
@@ -371,6 +374,14 @@ DEV unsigned long long uni64(unsigned long long a)
     return ((unsigned long long)hi << 32) | lo;
 }
 DEV const glb_d *uni_glb(const double *p) { return (const glb_d *)uni64((unsigned long long)p); }
+
+// generic pointer to the LDS address a (uniform)
+template <typename T>
+DEV T *lds_ptr(unsigned a)
+{
+    typedef __attribute__((address_space(3))) T lds_t;
+    return (T *)(lds_t *)(size_t)(unsigned)uni((int)a);
+}
 
 struct Ctx {
     CModel &M;
@@ -414,12 +425,10 @@ struct Ctx {
     // window list and trial list of the chain (their buffers swap)
     DEV void lists()
     {
-        const bool sw = uni(s_wenv.swapped) != 0;
-        lds_c *lds = uni_lds(s_wenv.dyn);
-        wtau = (double *)(lds_d *)(lds + (sw ? L.l_ttau : L.l_wtau));
-        ttau = (double *)(lds_d *)(lds + (sw ? L.l_wtau : L.l_ttau));
-        wcode = (int *)(lds_i *)(lds + (sw ? L.l_tcode : L.l_wcode));
-        tcode = (int *)(lds_i *)(lds + (sw ? L.l_wcode : L.l_tcode));
+        wtau = lds_ptr<double>(s_wenv.wtau);
+        wcode = lds_ptr<int>(s_wenv.wcode);
+        ttau = lds_ptr<double>(s_wenv.ttau);
+        tcode = lds_ptr<int>(s_wenv.tcode);
     }
     DEV double *mi(int f) { return minv + (long)f * L.kcap * L.kcap; }
     DEV int fl(int c) const { return op_orb(c) + M.nb * op_spin(c); }
@@ -453,45 +462,43 @@ DEV Ctx attach(ChainRef r)
     c.bndlog = reinterpret_cast<double *>(base + L.bndlog);
     c.bndsst = reinterpret_cast<int *>(base + L.bndsst);
     c.part = reinterpret_cast<double *>(base + L.part);
-    lds_c *lds = uni_lds(s_wenv.dyn);
-    auto ld = [&](long o) { return (double *)(lds_d *)(lds + o); };
-    auto li = [&](long o) { return (int *)(lds_i *)(lds + o); };
     c.lists();
-    c.pc = li(L.l_pc);
-    c.dvec = ld(L.l_dvec);
-    c.Q = ld(L.l_q);
-    c.R = ld(L.l_r);
-    c.colb = ld(L.l_col);
-    c.rowb = ld(L.l_row);
-    c.pl = ld(L.l_pl);
+    const WalkEnv &e = s_wenv;
+    c.pc = lds_ptr<int>(e.pc);
+    c.dvec = lds_ptr<double>(e.dvec);
+    c.Q = lds_ptr<double>(e.q);
+    c.R = lds_ptr<double>(e.r);
+    c.colb = lds_ptr<double>(e.col);
+    c.rowb = lds_ptr<double>(e.row);
+    c.pl = lds_ptr<double>(e.pl);
     if constexpr (NM <= 16) {
-        c.rk = NM <= 4 ? ld(L.l_rk) : reinterpret_cast<double *>(base + L.grk);
-        c.lb = NM <= 4 ? ld(L.l_lb) : reinterpret_cast<double *>(base + L.glb);
-        c.rkx = ld(L.l_rkx);
-        c.lbx = ld(L.l_lbx);
-        c.rks = li(L.l_rks);
-        c.lbs = li(L.l_lbs);
+        c.rk = NM <= 4 ? lds_ptr<double>(e.rk) : reinterpret_cast<double *>(base + L.grk);
+        c.lb = NM <= 4 ? lds_ptr<double>(e.lb) : reinterpret_cast<double *>(base + L.glb);
+        c.rkx = lds_ptr<double>(e.rkx);
+        c.lbx = lds_ptr<double>(e.lbx);
+        c.rks = lds_ptr<int>(e.rks);
+        c.lbs = lds_ptr<int>(e.lbs);
     }
-    c.legc = ld(L.l_legc);
+    c.legc = lds_ptr<double>(e.legc);
     // work matrices: LDS for blocks up to 16 states (decided at compile time so
     // that their accesses are LDS instructions, not generic ones), HBM above
-    if constexpr (NM <= 16) c.K0 = ld(L.l_k);
+    if constexpr (NM <= 16) c.K0 = lds_ptr<double>(e.k);
     else c.K0 = reinterpret_cast<double *>(base + L.kwork);
     c.K1 = c.K0 + (long)NM * NM;
-    c.strip = NM > 16 ? ld(L.l_strip) : nullptr;
-    c.sz = li(L.l_sz);
-    c.off = li(L.l_off);
+    c.strip = NM > 16 ? lds_ptr<double>(e.strip) : nullptr;
+    c.sz = lds_ptr<int>(e.sz);
+    c.off = lds_ptr<int>(e.off);
     // transition records and energies: LDS for blocks up to 16 states
     if constexpr (NM <= 16) {
-        c.tr = (const int4 *)(const void *)(lds_i4 *)(lds + L.l_tr);
-        c.ev = ld(L.l_ev);
+        c.tr = (const int4 *)(const void *)lds_ptr<iv4>(e.trt);
+        c.ev = lds_ptr<double>(e.evt);
     } else {
         c.tr = M.trans;
         c.ev = M.evals;
     }
     // operator blocks: LDS for blocks up to 4 states
-    c.opsp = NM <= 4 ? ld(L.l_ops) : M.ops;
-    c.rng.mt = (lds_u *)(lds + L.l_mt);
+    c.opsp = NM <= 4 ? lds_ptr<double>(e.opst) : M.ops;
+    c.rng.mt = (lds_u *)lds_ptr<unsigned>(e.mt);
     c.rng.idx = &s_hdr.mti;
     return c;
 }
@@ -616,7 +623,11 @@ __device__ __attribute__((noinline)) bool load_window(ChainRef r)
 // the trial list becomes the window list (after an accepted add / remove)
 DEV void swap_lists(Ctx &c)
 {
-    s_wenv.swapped ^= 1;
+    const unsigned t = s_wenv.wtau, k = s_wenv.wcode;
+    s_wenv.wtau = s_wenv.ttau;
+    s_wenv.wcode = s_wenv.tcode;
+    s_wenv.ttau = t;
+    s_wenv.tcode = k;
     c.lists();
 }
 
@@ -1067,14 +1078,6 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
     out.s = __builtin_amdgcn_readlane(sb, n);
     const double e0 = __hiloint2double(si.y, si.x), lc = -(e0 - egs) * dt;
     const int ns = si.z & 255, eo = si.z >> 8;
-    {
-        const int both = __builtin_amdgcn_readlane(row_sum_i(op ? ((rec.y * ns) << 16) | (ns + rec.y) : 0), 0);
-        const int in = __builtin_amdgcn_readlane(row_sum_i(op ? ns : 0), 0);
-        if (l == 0) {
-            __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.flops, (double)(no * (2 * (both >> 16) + in)));
-            __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.bytes, (double)(8 * no * (both & 0xffff)));
-        }
-    }
     if constexpr (KEEP) {
         if (l < n) px.sst[p] = rec.x;
     }
@@ -1091,7 +1094,9 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
         }
         k.v[0] *= readlane_d(a, 15);   // zero in the lanes outside the block
     } else {
-        const bool each = __ballot(__int_as_float(si.w) * (float)dt > 100.0f) != 0ull;
+        // long propagations: a check per operator
+        if (__ballot(__int_as_float(si.w) * (float)dt > 100.0f) != 0ull)
+            return walk_small<NM, BRA, KEEP>(k, s0, tstart, tend, otau, ocode, n, no, px);
         const int blk = (l >> 2) & 3, i = l & 3, r = l >> 4;
         const double dr = exp(-(ev[eo + (r < ns ? r : 0)] - e0) * dt);
         // block offset, sizes; 1 << 28: the propagation to tend, 1 << 29: beyond it
@@ -1116,7 +1121,7 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
                 for (int b = 0; b < 4; ++b) {
                     const double x = dpp_d<DPP_ROW_ROR4>(k.v[0]);
                     k.v[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[ps], x, 0.0, 0, 0, 0);
-                    if (b == 3 || each) renorm(k, 0x000F000F000F000Full << (4 * b), lg);
+                    if (b == 3) renorm(k, 0xF000F000F000F000ull, lg);
                     if constexpr (KEEP) {
                         const int t_ = 4 * ps + b;
                         if (t_ < n) {
@@ -1132,6 +1137,14 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
         double x = blk == 3 ? k.v[0] : 0.0;
         x += dpp_d<DPP_ROW_ROR4>(x);
         k.v[0] = x + dpp_d<DPP_ROW_ROR8>(x);
+    }
+    {
+        const int both = __builtin_amdgcn_readlane(row_sum_i(op ? ((rec.y * ns) << 16) | (ns + rec.y) : 0), 0);
+        const int in = __builtin_amdgcn_readlane(row_sum_i(op ? ns : 0), 0);
+        if (l == 0) {
+            __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.flops, (double)(no * (2 * (both >> 16) + in)));
+            __builtin_amdgcn_ds_atomic_fadd_f64((lds_d *)&s_wenv.bytes, (double)(8 * no * (both & 0xffff)));
+        }
     }
     out.lg = lg + readlane_d(sc, KEEP ? n : 0);
     out.k = k;
@@ -1784,7 +1797,7 @@ __device__ __attribute__((noinline)) void seg_extend(ChainRef ref, int nw_, int 
     constexpr int S = NM <= 4 ? NM * NM : 256;
     double *buf = BRA ? c.lb : c.rk, *bx = BRA ? c.lbx : c.rkx;
     int *bs = BRA ? c.lbs : c.rks;
-    const int no = c.sz[c.h.outer];
+    const int no = uni(s_wenv.no);
     const int w = c.h.nwin > 1 ? c.h.wpos : 0;
     int j = uni(BRA ? c.h.lb_n : c.h.rk_n) - 1;
     State<NM> k;
@@ -1827,7 +1840,7 @@ template <int NM>
 DEV bool segment_trace(Ctx &c, int nw, int j0, int m0, int a, int n, double t0, double t1, TraceVal &T)
 {
     if constexpr (NM <= 16) {
-        const int no = c.sz[c.h.outer];
+        const int no = uni(s_wenv.no);
         if (c.h.rk_n <= j0) seg_extend<NM, false>(c.ref(), nw, j0);
         if (c.h.lb_n <= m0) seg_extend<NM, true>(c.ref(), nw, m0);
         int s = c.rks[j0];
@@ -2093,67 +2106,90 @@ struct MatLanes {
     }
 };
 
+// In the block loops below, eight and then four columns (or rows) are loaded
+// together while every lane group has them; the last ones go one by one, masked.
 // M(i,j) += (a col(i)) row(j)
 DEV void rank1(Ctx &c, double *Mf, int k, const MatLanes &ml, double a, const double *col, const double *row)
 {
-    const int ld = c.L.kcap;
+    const int ld = c.L.kcap, full = k / ml.step;   // columns that every lane group has
     for (int i0 = 0; i0 < k; i0 += WAVE) {
         const int i = i0 + ml.i;
         const bool in = i < k;
-        double *Mi = Mf + (in ? i : 0);
         const double ci = in ? a * col[i] : 0.0;
-        for (int j0 = ml.g; j0 < k; j0 += 16 * ml.step) {
-            double m[16];
+        double *p = Mf + (in ? i : 0) + (long)ml.g * ld;
+        const double *q = row + ml.g;
+        int u = 0;
+        for (; u + 8 <= full; u += 8) {
+            double m[8], r[8];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) m[u] = Mi[(long)min(j0 + u * ml.step, k - 1) * ld];
+            for (int v = 0; v < 8; ++v) m[v] = p[(long)v * ml.step * ld];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int j = j0 + u * ml.step;
-                if (in && j < k) Mi[(long)j * ld] = fma(ci, row[j], m[u]);
+            for (int v = 0; v < 8; ++v) r[v] = q[v * ml.step];
+            if (in) {
+#pragma unroll
+                for (int v = 0; v < 8; ++v) p[(long)v * ml.step * ld] = fma(ci, r[v], m[v]);
             }
+            p += (long)8 * ml.step * ld;
+            q += 8 * ml.step;
+        }
+        if (u + 4 <= full) {
+            double m[4], r[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) m[v] = p[(long)v * ml.step * ld];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) r[v] = q[v * ml.step];
+            if (in) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) p[(long)v * ml.step * ld] = fma(ci, r[v], m[v]);
+            }
+            p += (long)4 * ml.step * ld;
+            q += 4 * ml.step;
+            u += 4;
+        }
+        for (; u <= full; ++u) {
+            if (in && u * ml.step + ml.g < k) *p = fma(ci, *q, *p);
+            p += (long)ml.step * ld;
+            q += ml.step;
         }
     }
 }
 
-// The first columns of M for detrat_add, loaded ahead of the lists and the
-// hybridisation values that its product waits for (all of M up to order 32).
-struct MatHead {
-    double m[16];
-    DEV MatHead(const double *Mf, int k, int ld)
-    {
-        const MatLanes ml(k);
-        const double *col = Mf + (ml.i < k ? ml.i : 0);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) m[u] = col[(long)max(min(ml.g + u * ml.step, k - 1), 0) * ld];
-    }
-};
-
-// R^T M Q of an order-k block (get_DetRatAdd); leaves M Q in colb.  The loads
-// of sixteen columns are in flight together.
-DEV double detrat_add(Ctx &c, const double *Mf, int k, const MatHead &head)
+// R^T M Q of an order-k block (get_DetRatAdd); leaves M Q in colb.
+DEV double detrat_add(Ctx &c, const double *Mf, int k)
 {
     const int ld = c.L.kcap;
     const MatLanes ml(k);
+    const int full = k / ml.step;
     double part = 0.0;
     for (int i0 = 0; i0 < k; i0 += WAVE) {
         const int i = i0 + ml.i;
         const bool in = i < k;
-        const double *col = Mf + (in ? i : 0);
+        const double *p = Mf + (in ? i : 0) + (long)ml.g * ld, *q = c.Q + ml.g;
         double acc = 0.0;
-        for (int j0 = ml.g; j0 < k; j0 += 16 * ml.step) {
-            double m[16];
-            if (i0 == 0 && j0 == ml.g) {
+        int u = 0;
+        for (; u + 8 <= full; u += 8) {
+            double m[8];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) m[u] = head.m[u];
-            } else {
+            for (int v = 0; v < 8; ++v) m[v] = p[(long)v * ml.step * ld];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) m[u] = col[(long)min(j0 + u * ml.step, k - 1) * ld];
-            }
+            for (int v = 0; v < 8; ++v) acc = fma(m[v], q[v * ml.step], acc);
+            p += (long)8 * ml.step * ld;
+            q += 8 * ml.step;
+        }
+        if (u + 4 <= full) {
+            double m[4];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int j = j0 + u * ml.step;
-                acc = fma(m[u], j < k ? c.Q[j] : 0.0, acc);
-            }
+            for (int v = 0; v < 4; ++v) m[v] = p[(long)v * ml.step * ld];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc = fma(m[v], q[v * ml.step], acc);
+            p += (long)4 * ml.step * ld;
+            q += 4 * ml.step;
+            u += 4;
+        }
+        for (; u <= full; ++u) {
+            if (u * ml.step + ml.g < k) acc = fma(*p, *q, acc);
+            p += (long)ml.step * ld;
+            q += ml.step;
         }
         acc = ml.rows(acc);
         if (in && ml.g == 0) {
@@ -2177,19 +2213,35 @@ DEV void mat_add_phys(Ctx &c, double *Mf, int k, double dr)
     double *col = c.colb, *row = c.rowb;
     // columns of M against R: the lane's column is contiguous
     const MatLanes ml(k);
+    const int full = k / ml.step;
     for (int j0 = 0; j0 < k; j0 += WAVE) {
         const int j = j0 + ml.i;
-        const double *mc = Mf + (long)min(j, k - 1) * ld;
+        const double *p = Mf + (long)min(j, k - 1) * ld + ml.g, *r = c.R + ml.g;
         double v = 0.0;
-        for (int i0 = ml.g; i0 < k; i0 += 16 * ml.step) {
-            double m[16];
+        int u = 0;
+        for (; u + 8 <= full; u += 8) {
+            double m[8];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) m[u] = mc[min(i0 + u * ml.step, k - 1)];
+            for (int w = 0; w < 8; ++w) m[w] = p[w * ml.step];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int i = i0 + u * ml.step;
-                v = fma(i < k ? c.R[i] : 0.0, m[u], v);
-            }
+            for (int w = 0; w < 8; ++w) v = fma(r[w * ml.step], m[w], v);
+            p += 8 * ml.step;
+            r += 8 * ml.step;
+        }
+        if (u + 4 <= full) {
+            double m[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) m[w] = p[w * ml.step];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v = fma(r[w * ml.step], m[w], v);
+            p += 4 * ml.step;
+            r += 4 * ml.step;
+            u += 4;
+        }
+        for (; u <= full; ++u) {
+            if (u * ml.step + ml.g < k) v = fma(*r, *p, v);
+            p += ml.step;
+            r += ml.step;
         }
         v = ml.rows(v);
         if (j < k && ml.g == 0) row[j] = -v / dr;
@@ -2560,7 +2612,6 @@ DEV int step_add(Ctx &c)
     // det ratio, get_LogDetRatPairAdd (Trace.F90:2775-2832): Q (annihilators) and
     // R (creators) placed by physical slot, the lane behind the last rank takes
     // S0 = F(ta - tc); FPos = 1 + earlier operators of the type
-    const MatHead head(c.mi(f), k, c.L.kcap);
     const long fo = (long)f * c.L.kcap;
     const double *ctl = c.fc + fo, *atl = c.fa + fo;
     const int *csl = c.fcs + fo, *asl = c.fas + fo;
@@ -2588,7 +2639,7 @@ DEV int step_add(Ctx &c)
         sgn += popc64(__ballot(abet)) + popc64(__ballot(in && xc > tc)) + popc64(__ballot(in && xa > tc));
     }
     wsync();
-    const double S = S0 - detrat_add(c, c.mi(f), k, head);
+    const double S = S0 - detrat_add(c, c.mi(f), k);
     c.work(2.0 * k * k, 8.0 * k * k);
     const double sig = ((fp_c - fp_a) & 1) ? -1.0 : 1.0;
     const double dr_sign = copysign(1.0, S) * sig;
@@ -3146,6 +3197,7 @@ __device__ __attribute__((noinline)) bool make_ready(ChainRef r)
                     c.h.wib - c.h.wia + 2 <= c.L.lcap_lds;
     if (!ok) c.h.halt = HALT_CAP;
     s_wenv.ready = ok;
+    s_wenv.no = c.sz[c.h.outer];
     wsync();
     return ok;
 }
@@ -3857,9 +3909,23 @@ DEV Ctx make_ctx(char *chains, int chain, CArgs args, char *lds)
 {
     CModel &M = *(CModel *)args;
     CLayout &L = *(CLayout *)(args + (sizeof(DevModel) + 7) / 8 * 8);
-    s_wenv.dyn = (lds_c *)lds;
-    s_wenv.ready = 0;
-    s_wenv.swapped = 0;
+    {
+        WalkEnv &e = s_wenv;
+        const unsigned d = (unsigned)(size_t)(lds_c *)lds;
+        e.wtau = d + (unsigned)L.l_wtau, e.wcode = d + (unsigned)L.l_wcode;
+        e.ttau = d + (unsigned)L.l_ttau, e.tcode = d + (unsigned)L.l_tcode;
+        e.pc = d + (unsigned)L.l_pc, e.dvec = d + (unsigned)L.l_dvec, e.pl = d + (unsigned)L.l_pl;
+        e.q = d + (unsigned)L.l_q, e.r = d + (unsigned)L.l_r;
+        e.col = d + (unsigned)L.l_col, e.row = d + (unsigned)L.l_row;
+        e.rk = d + (unsigned)L.l_rk, e.lb = d + (unsigned)L.l_lb;
+        e.rkx = d + (unsigned)L.l_rkx, e.lbx = d + (unsigned)L.l_lbx;
+        e.rks = d + (unsigned)L.l_rks, e.lbs = d + (unsigned)L.l_lbs;
+        e.legc = d + (unsigned)L.l_legc, e.k = d + (unsigned)L.l_k, e.strip = d + (unsigned)L.l_strip;
+        e.sz = d + (unsigned)L.l_sz, e.off = d + (unsigned)L.l_off;
+        e.trt = d + (unsigned)L.l_tr, e.evt = d + (unsigned)L.l_ev, e.opst = d + (unsigned)L.l_ops;
+        e.mt = d + (unsigned)L.l_mt;
+        e.ready = 0;
+    }
     wsync();
     char *base = chains + (long)chain * L.stride;
     Ctx c = attach<NM>(ChainRef{&M, &L, base});
