@@ -211,6 +211,13 @@ int w2d_ctqmc_get_config(w2d_ctqmc *h, int chain, int cap, int *n, double *tau, 
 int w2d_ctqmc_set_config(w2d_ctqmc *h, int chain, int n, const double *tau, const int *orb,
                          const int *spin, const int *ca, int outer_sst, double *weights);
 
+/* The same for chains 0 .. nconf - 1 at once (ReuseMCConfig for a batch,
+ * cthyb_solver.py:24-86, 328-332): configuration i holds the operators
+ * off[i] .. off[i+1] - 1 of the arrays; weights[nconf][5].  The configurations
+ * before the first that is refused are set; the first error is returned. */
+int w2d_ctqmc_set_configs(w2d_ctqmc *h, int nconf, const int64_t *off, const double *tau, const int *orb,
+                          const int *spin, const int *ca, const int *outer_sst, double *weights);
+
 /* Inverse hybridisation block of flavour f of one chain (column-major k x k,
  * rows creators, columns annihilators as Trace.F90:2279-2333); *k receives the
  * order, out may be NULL to query it. */

@@ -56,6 +56,11 @@ struct w2d_ctqmc {
     // MeasGiw: raw G(i w_n) sums [nchains][2N][niw][2] and the per (chain,
     // flavour) visit record of giw_kernel [nchains][2N][2]; niw = 0: off
     int niw = 0;
+    // device work area of the group sums, kept between calls (grown when a
+    // call needs more, freed with the handle), and pinned room for the headers
+    void *work = nullptr;
+    size_t work_bytes = 0;
+    w2d::ChainHdr *hdr_pinned = nullptr;
     double *giw = nullptr;
     long long *giw_seen = nullptr;
     ~w2d_ctqmc();
@@ -431,12 +436,18 @@ void launch_sweep(w2d_ctqmc *h, long long target, long long ncorr, int only, w2d
     }
 }
 
+// what setconfig_kernel reads, on the device
+struct DevConfigs {
+    const double *tau;
+    const int *code, *off, *outer;
+};
+
 template <int NM>
-void launch_setconfig(w2d_ctqmc *h, int chain)
+void launch_setconfig(w2d_ctqmc *h, int first, int count, const DevConfigs &d)
 {
     allow_lds(w2d::setconfig_kernel<NM>, h);
-    hipLaunchKernelGGL(w2d::setconfig_kernel<NM>, dim3(h->nchains), dim3(w2d::WAVE), (unsigned)h->L.lds_bytes, h->stream, h->dm,
-                       h->L, h->chains, chain);
+    hipLaunchKernelGGL(w2d::setconfig_kernel<NM>, dim3(count), dim3(w2d::WAVE), (unsigned)h->L.lds_bytes, h->stream, h->dm,
+                       h->L, h->chains, first, d.tau, d.code, d.off, d.outer);
 }
 
 template <int NM>
@@ -460,10 +471,10 @@ char *hdr_of(w2d_ctqmc *h, int c) { return h->chains + h->L.hdrs + (long)c * (lo
 
 int read_headers(w2d_ctqmc *h, std::vector<ChainHdr> &hd)
 {
-    hd.resize(h->nchains);
+    const size_t n = sizeof(ChainHdr) * (size_t)h->nchains;
+    HIPCHK(hipMemcpyAsync(h->hdr_pinned, h->chains + h->L.hdrs, n, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipMemcpy(hd.data(), h->chains + h->L.hdrs, sizeof(ChainHdr) * (size_t)h->nchains,
-                     hipMemcpyDeviceToHost));
+    hd.assign(h->hdr_pinned, h->hdr_pinned + h->nchains);
     return W2D_OK;
 }
 
@@ -667,46 +678,85 @@ int run_moves(w2d_ctqmc *h, long long nmoves, long long ncorr)
     return batch_status(hd);
 }
 
-// Device work area of the group sums: [ngroups][nel] partial sums, then
-// [ngroups][14] scalars, then [ngroups] chain counts.
+// Device work area of the group sums over all accumulators: [ngroups][nel]
+// partial sums, then [ngroups][14] scalars, then [ngroups] chain counts.
 size_t group_sums_bytes(const w2d_ctqmc *h, int ngroups)
 {
     const long nel = (h->L.stride - h->L.gtau) / 8;
     return (size_t)ngroups * ((size_t)nel * 8 + 14 * 8 + 8);
 }
 
-// Group sums into a caller-provided device work area; the results go straight
-// to the host arrays (strided copies), so nothing is allocated here.
+// at least `bytes` of device work area
+int need_work(w2d_ctqmc *h, size_t bytes)
+{
+    if (bytes <= h->work_bytes) return W2D_OK;
+    if (h->work) {
+        HIPCHK(hipStreamSynchronize(h->stream));
+        HIPCHK(hipFree(h->work));
+        h->work = nullptr;
+        h->work_bytes = 0;
+    }
+    HIPCHK(hipMalloc(&h->work, bytes));
+    h->work_bytes = bytes;
+    return W2D_OK;
+}
+
+// Sums over groups of chains of the accumulators in [from, to) of the chain
+// blocks into `work` ([ngroups][(to - from) / 8]); put() copies one array's
+// [ngroups][n] out of them.
+struct GroupSums {
+    w2d_ctqmc *h;
+    int ngroups;
+    long from, nel;
+    double *part;
+    int run(long to)
+    {
+        nel = (to - from) / 8;
+        const ChainHdr *hdrs = reinterpret_cast<const ChainHdr *>(h->chains + h->L.hdrs);
+        hipLaunchKernelGGL(w2d::group_sum_kernel, dim3((unsigned)((nel + 255) / 256), (unsigned)ngroups), dim3(256), 0,
+                           h->stream, (const char *)h->chains + from, h->L.stride, nel, h->nchains, ngroups, hdrs,
+                           part);
+        HIPCHK(hipGetLastError());
+        return W2D_OK;
+    }
+    int put(double *dst, long off, long n)
+    {
+        if (!dst || n <= 0) return W2D_OK;
+        HIPCHK(hipMemcpy2DAsync(dst, (size_t)n * 8, part + (off - from) / 8, (size_t)nel * 8, (size_t)n * 8,
+                                (size_t)ngroups, hipMemcpyDeviceToHost, h->stream));
+        return W2D_OK;
+    }
+    int done()
+    {
+        HIPCHK(hipStreamSynchronize(h->stream));
+        return W2D_OK;
+    }
+};
+
+// Group sums into a device work area; the results go straight to the host
+// arrays (strided copies), so nothing is allocated here.
 int group_sums_into(w2d_ctqmc *h, int ngroups, void *work, double *gtau, double *gleg, double *dm_blocks,
                     double *histo, double *outer, double *scalars, int32_t *nused)
 {
     const w2d::ChainLayout &L = h->L;
     const int nf = 2 * h->model.nbands, nc = h->nchains;
-    const long nel = (L.stride - L.gtau) / 8;
-    double *part = static_cast<double *>(work);
-    double *scal = part + (long)ngroups * nel;
+    GroupSums g{h, ngroups, L.gtau, 0, static_cast<double *>(work)};
+    int st = g.run(L.gbuf);
+    if (st) return st;
+    double *scal = g.part + (long)ngroups * g.nel;
     int *used = reinterpret_cast<int *>(scal + (long)ngroups * 14);
     const ChainHdr *hdrs = reinterpret_cast<const ChainHdr *>(h->chains + L.hdrs);
-    hipLaunchKernelGGL(w2d::group_sum_kernel, dim3((unsigned)((nel + 255) / 256), (unsigned)ngroups), dim3(256), 0,
-                       h->stream, (const char *)h->chains, L.stride, L.gtau, nel, nc, ngroups, hdrs, part);
     hipLaunchKernelGGL(w2d::group_scalars_kernel, dim3((unsigned)((ngroups + 63) / 64)), dim3(64), 0, h->stream, hdrs,
                        nc, ngroups, scal, used);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(h->stream));
-    auto put = [&](double *dst, long off, long n) -> int {
-        if (!dst || n <= 0) return W2D_OK;
-        HIPCHK(hipMemcpy2D(dst, (size_t)n * 8, part + (off - L.gtau) / 8, (size_t)nel * 8, (size_t)n * 8,
-                           (size_t)ngroups, hipMemcpyDeviceToHost));
-        return W2D_OK;
-    };
-    int st;
-    if ((st = put(gtau, L.gtau, (long)nf * h->ntau)) || (st = put(gleg, L.gleg, (long)nf * h->nleg)) ||
-        (st = put(dm_blocks, L.dm, h->dm.dmsize)) || (st = put(histo, L.histo, (long)nf * (h->maxhisto + 1))) ||
-        (st = put(outer, L.outer, h->model.nsst)))
+    if ((st = g.put(gtau, L.gtau, (long)nf * h->ntau)) || (st = g.put(gleg, L.gleg, (long)nf * h->nleg)) ||
+        (st = g.put(dm_blocks, L.dm, h->dm.dmsize)) || (st = g.put(histo, L.histo, (long)nf * (h->maxhisto + 1))) ||
+        (st = g.put(outer, L.outer, h->model.nsst)))
         return st;
-    if (scalars) HIPCHK(hipMemcpy(scalars, scal, (size_t)ngroups * 14 * 8, hipMemcpyDeviceToHost));
-    if (nused) HIPCHK(hipMemcpy(nused, used, (size_t)ngroups * 4, hipMemcpyDeviceToHost));
-    return W2D_OK;
+    if (scalars)
+        HIPCHK(hipMemcpyAsync(scalars, scal, (size_t)ngroups * 14 * 8, hipMemcpyDeviceToHost, h->stream));
+    if (nused) HIPCHK(hipMemcpyAsync(nused, used, (size_t)ngroups * 4, hipMemcpyDeviceToHost, h->stream));
+    return g.done();
 }
 
 // Additive keys of the superstates, key = a N_0 + b N_1 + const with the
@@ -825,6 +875,87 @@ int switch_engine(w2d_ctqmc *h, int nm)
     return write_headers(h, hd);
 }
 
+// Whether operators [a, b) form a configuration of this model: fills its codes
+// and the largest number of pairs of a flavour.
+bool valid_config(const w2d_ctqmc *h, int64_t a, int64_t b, const double *tau, const int *orb, const int *spin,
+                  const int *ca, int outer_sst, std::vector<int> &code, int &pairs)
+{
+    if (b < a || b - a > h->L.cap || outer_sst < 0 || outer_sst >= h->model.nsst) return false;
+    std::vector<int> cnt(2 * h->model.nbands * 2, 0);
+    for (int64_t i = a; i < b; ++i) {
+        if (orb[i] < 0 || orb[i] >= h->model.nbands || spin[i] < 0 || spin[i] > 1 || ca[i] < 1 || ca[i] > 2)
+            return false;
+        if (i > a && !(tau[i] > tau[i - 1])) return false;
+        if (tau[i] < 0.0 || tau[i] > h->beta) return false;
+        code[i] = orb[i] | (spin[i] << 4) | ((ca[i] - 1) << 5);
+        cnt[2 * (orb[i] + h->model.nbands * spin[i]) + ca[i] - 1]++;
+    }
+    for (int f = 0; f < 2 * h->model.nbands; ++f) {
+        if (cnt[2 * f] != cnt[2 * f + 1]) return false;
+        pairs = std::max(pairs, cnt[2 * f]);
+    }
+    return true;
+}
+
+// Configurations i = 0 .. nconf - 1 into chains first + i, all in one launch.
+// Like calls one after the other, the ones before the first that is refused are
+// set; returns the first error in order.
+int set_configs(w2d_ctqmc *h, int first, int nconf, const int64_t *off, const double *tau, const int *orb,
+                const int *spin, const int *ca, const int *outer_sst, double *weights)
+{
+    h->moved = true;
+    if (off[0] != 0) return W2D_ERR_ARG;
+    int status = W2D_OK, m = 0;
+    std::vector<int> code, o32(1, 0);
+    for (; m < nconf && status == W2D_OK; ++m) {
+        int pairs = 0;
+        if (off[m + 1] < off[m] || off[m + 1] > 0x7fffffff) {
+            status = W2D_ERR_ARG;
+            break;
+        }
+        code.resize((size_t)off[m + 1]);
+        if (!valid_config(h, off[m], off[m + 1], tau, orb, spin, ca, outer_sst[m], code, pairs)) {
+            status = W2D_ERR_ARG;
+            break;
+        }
+        // grow until every flavour's order fits
+        while (pairs > h->kcap && status == W2D_OK) status = regrow(h);
+        if (status) break;
+        o32.push_back((int)off[m + 1]);
+    }
+    if (m > 0) {
+        const size_t nops = (size_t)off[m];
+        const size_t btau = nops * 8, bcode = (nops * 4 + 7) / 8 * 8, boff = ((size_t)m + 1) * 4;
+        int st = need_work(h, btau + bcode + boff + (size_t)m * 4 + 64);
+        if (st) return st;
+        char *w = static_cast<char *>(h->work);
+        if (nops > 0) {
+            HIPCHK(hipMemcpyAsync(w, tau, btau, hipMemcpyHostToDevice, h->stream));
+            HIPCHK(hipMemcpyAsync(w + btau, code.data(), nops * 4, hipMemcpyHostToDevice, h->stream));
+        }
+        HIPCHK(hipMemcpyAsync(w + btau + bcode, o32.data(), boff, hipMemcpyHostToDevice, h->stream));
+        HIPCHK(hipMemcpyAsync(w + btau + bcode + boff, outer_sst, (size_t)m * 4, hipMemcpyHostToDevice, h->stream));
+        const DevConfigs d{reinterpret_cast<const double *>(w), reinterpret_cast<const int *>(w + btau),
+                           reinterpret_cast<const int *>(w + btau + bcode),
+                           reinterpret_cast<const int *>(w + btau + bcode + boff)};
+        DISPATCH(launch_setconfig, h, first, m, d);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(h->hdr_pinned, hdr_of(h, first), sizeof(ChainHdr) * (size_t)m, hipMemcpyDeviceToHost,
+                              h->stream));
+        HIPCHK(hipStreamSynchronize(h->stream));
+        for (int i = 0; i < m; ++i) {
+            const ChainHdr &x = h->hdr_pinned[i];
+            if (weights) {
+                double *v = weights + 5L * i;
+                v[0] = x.trace_log, v[1] = x.trace_sign, v[2] = x.det_log, v[3] = x.det_sign, v[4] = x.cfgsign;
+            }
+        }
+        for (int i = 0; i < m; ++i)
+            if (h->hdr_pinned[i].err) return map_err(h->hdr_pinned[i].err);
+    }
+    return status;
+}
+
 }  // namespace
 
 // every resource the handle holds (also on the error paths of create)
@@ -833,6 +964,8 @@ w2d_ctqmc::~w2d_ctqmc()
     if (stream) (void)hipStreamSynchronize(stream);
     for (void *p : dev_allocs) (void)hipFree(p);
     if (chains) (void)hipFree(chains);
+    if (work) (void)hipFree(work);
+    if (hdr_pinned) (void)hipHostFree(hdr_pinned);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);
@@ -921,6 +1054,7 @@ int w2d_ctqmc_create(const char *params, int nbands, int nftau, const double *u_
         h->dev_allocs.push_back(o);
         h->order = static_cast<int *>(o);
     }
+    HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&h->hdr_pinned), sizeof(ChainHdr) * (size_t)nchains, 0));
     HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&h->abort_host), sizeof(int),
                          hipHostMallocMapped | hipHostMallocCoherent));
     *h->abort_host = 0;
@@ -1096,42 +1230,24 @@ int w2d_ctqmc_set_taudiffmax(w2d_ctqmc *h, double tdm)
 int w2d_ctqmc_warmup(w2d_ctqmc *h, int64_t nwarmups)
 {
     if (!h || nwarmups < 0) return W2D_ERR_ARG;
-    std::vector<ChainHdr> hd;
-    int st = read_headers(h, hd);
-    if (st) return st;
-    // ctqmc_warmup: AccPair over NGtau bins of [0, beta], then init_counters
-    // (CTQMC.F90:8199-8206)
-    for (auto &x : hd) {
-        reset_counters(x);
-        x.naccpair = h->ntau;
-        x.accpair_max = h->beta;
-    }
-    if ((st = write_headers(h, hd)) || (st = clear_accpair(h))) return st;
+    hipLaunchKernelGGL(w2d::begin_kernel, dim3(h->nchains), dim3(256), 0, h->stream, h->L, h->chains,
+                       2 * h->model.nbands, 0, h->ntau, h->beta);
+    HIPCHK(hipGetLastError());
     return run_moves(h, nwarmups, 0);
 }
 
 int w2d_ctqmc_measure(w2d_ctqmc *h, int64_t nmeas)
 {
     if (!h || nmeas < 0) return W2D_ERR_ARG;
-    std::vector<ChainHdr> hd;
-    int st = read_headers(h, hd);
-    if (st) return st;
-    for (auto &x : hd) {
-        reset_counters(x);
-        x.meas_sign = 0.0;
-        x.cnt_meas = 0;
-    }
-    if ((st = write_headers(h, hd))) return st;
-    // clear the accumulators of every chain
-    const w2d::ChainLayout &L = h->L;
-    HIPCHK(hipMemset2DAsync(h->chains + L.gtau, (size_t)L.stride, 0, (size_t)(L.stride - L.gtau),
-                            (size_t)h->nchains, h->stream));
+    hipLaunchKernelGGL(w2d::begin_kernel, dim3(h->nchains), dim3(256), 0, h->stream, h->L, h->chains,
+                       2 * h->model.nbands, 1, h->ntau, h->beta);
+    HIPCHK(hipGetLastError());
     if (h->niw > 0) {
         const size_t nf = (size_t)h->dm.nf, nc = (size_t)h->nchains;
         HIPCHK(hipMemsetAsync(h->giw, 0, nc * nf * (size_t)h->niw * 2 * sizeof(double), h->stream));
         HIPCHK(hipMemsetAsync(h->giw_seen, 0, nc * nf * 2 * sizeof(long long), h->stream));
     }
-    st = run_moves(h, nmeas * h->ncorr, h->ncorr);
+    const int st = run_moves(h, nmeas * h->ncorr, h->ncorr);
     h->measured = (st == W2D_OK || st == W2D_ERR_PARTIAL);
     return st;
 }
@@ -1295,50 +1411,16 @@ int w2d_ctqmc_get_config(w2d_ctqmc *h, int chain, int cap, int *n, double *tau, 
 int w2d_ctqmc_set_config(w2d_ctqmc *h, int chain, int n, const double *tau, const int *orb, const int *spin,
                          const int *ca, int outer_sst, double *weights)
 {
-    if (!h || chain < 0 || chain >= h->nchains || n < 0 || n > h->L.cap || outer_sst < 0 ||
-        outer_sst >= h->model.nsst)
-        return W2D_ERR_ARG;
-    h->moved = true;
-    std::vector<int> cnt(2 * h->model.nbands * 2, 0);
-    std::vector<int> code(n);
-    for (int i = 0; i < n; ++i) {
-        if (orb[i] < 0 || orb[i] >= h->model.nbands || spin[i] < 0 || spin[i] > 1 || ca[i] < 1 || ca[i] > 2)
-            return W2D_ERR_ARG;
-        if (i > 0 && !(tau[i] > tau[i - 1])) return W2D_ERR_ARG;
-        if (tau[i] < 0.0 || tau[i] > h->beta) return W2D_ERR_ARG;
-        code[i] = orb[i] | (spin[i] << 4) | ((ca[i] - 1) << 5);
-        int f = orb[i] + h->model.nbands * spin[i];
-        cnt[2 * f + ca[i] - 1]++;
-    }
-    for (int f = 0; f < 2 * h->model.nbands; ++f)
-        if (cnt[2 * f] != cnt[2 * f + 1]) return W2D_ERR_ARG;
-    // grow until every flavour's order fits
-    for (int f = 0; f < 2 * h->model.nbands; ++f)
-        while (cnt[2 * f] > h->kcap) {
-            const int st = regrow(h);
-            if (st) return st;
-        }
-    char *base = h->chains + (long)chain * h->L.stride;
-    HIPCHK(hipStreamSynchronize(h->stream));
-    ChainHdr x;
-    HIPCHK(hipMemcpy(&x, hdr_of(h, chain), sizeof(x), hipMemcpyDeviceToHost));
-    x.nop = n;
-    x.outer = outer_sst;
-    x.err = 0;
-    HIPCHK(hipMemcpy(hdr_of(h, chain), &x, sizeof(x), hipMemcpyHostToDevice));
-    if (n > 0) {
-        HIPCHK(hipMemcpy(base + h->L.tau, tau, (size_t)n * 8, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(base + h->L.code, code.data(), (size_t)n * 4, hipMemcpyHostToDevice));
-    }
-    DISPATCH(launch_setconfig, h, chain);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipMemcpy(&x, hdr_of(h, chain), sizeof(x), hipMemcpyDeviceToHost));
-    if (weights) {
-        weights[0] = x.trace_log, weights[1] = x.trace_sign;
-        weights[2] = x.det_log, weights[3] = x.det_sign, weights[4] = x.cfgsign;
-    }
-    return map_err(x.err);
+    if (!h || chain < 0 || chain >= h->nchains || n < 0) return W2D_ERR_ARG;
+    const int64_t off[2] = {0, n};
+    return set_configs(h, chain, 1, off, tau, orb, spin, ca, &outer_sst, weights);
+}
+
+int w2d_ctqmc_set_configs(w2d_ctqmc *h, int nconf, const int64_t *off, const double *tau, const int *orb,
+                          const int *spin, const int *ca, const int *outer_sst, double *weights)
+{
+    if (!h || nconf < 0 || nconf > h->nchains || (nconf > 0 && (!off || !outer_sst))) return W2D_ERR_ARG;
+    return nconf > 0 ? set_configs(h, 0, nconf, off, tau, orb, spin, ca, outer_sst, weights) : W2D_OK;
 }
 
 int w2d_ctqmc_get_minv(w2d_ctqmc *h, int chain, int f, int *k, double *out)
@@ -1444,25 +1526,17 @@ int w2d_ctqmc_get_score_sums(w2d_ctqmc *h, int ngroups, double *ssum, double *gt
 {
     if (!h || ngroups < 1 || ngroups > h->nchains) return W2D_ERR_ARG;
     if (!h->measured || !h->dm.score || h->dm.ntheta < 1) return W2D_ERR_STATE;
-    void *work = nullptr;
-    HIPCHK(hipMalloc(&work, group_sums_bytes(h, ngroups)));
-    int st = group_sums_into(h, ngroups, work, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
     const w2d::ChainLayout &L = h->L;
-    const long nel = (L.stride - L.gtau) / 8;
-    const double *part = static_cast<const double *>(work);
-    auto put = [&](double *dst, long off, long n) -> int {
-        if (!dst || n <= 0) return W2D_OK;
-        HIPCHK(hipMemcpy2D(dst, (size_t)n * 8, part + (off - L.gtau) / 8, (size_t)nel * 8, (size_t)n * 8,
-                           (size_t)ngroups, hipMemcpyDeviceToHost));
-        return W2D_OK;
-    };
+    int st = need_work(h, (size_t)ngroups * (size_t)(L.stride - L.scsum));
+    if (st) return st;
+    GroupSums g{h, ngroups, L.scsum, 0, static_cast<double *>(h->work)};
+    st = g.run(L.stride);
     const long nt = h->dm.ntheta, nf = 2 * h->model.nbands;
-    if (!st) st = put(ssum, L.scsum, nt);
-    if (!st) st = put(gtau, L.scg, nt * nf * h->ntau);
-    if (!st) st = put(dm_blocks, L.scdm, nt * h->dm.dmsize);
-    if (!st) st = put(dm_explicit, L.scdmx, nt * h->dm.dmsize);
-    (void)hipFree(work);
-    return st;
+    if (!st) st = g.put(ssum, L.scsum, nt);
+    if (!st) st = g.put(gtau, L.scg, nt * nf * h->ntau);
+    if (!st) st = g.put(dm_blocks, L.scdm, nt * h->dm.dmsize);
+    if (!st) st = g.put(dm_explicit, L.scdmx, nt * h->dm.dmsize);
+    return st ? st : g.done();
 }
 
 int w2d_ctqmc_set_launch(w2d_ctqmc *h, int graphs, int order_chains, int64_t moves_per_launch)
@@ -1522,11 +1596,9 @@ int w2d_ctqmc_get_group_sums(w2d_ctqmc *h, int ngroups, double *gtau, double *gl
 {
     if (!h || ngroups < 1 || ngroups > h->nchains) return W2D_ERR_ARG;
     if (!h->measured) return W2D_ERR_STATE;
-    void *work = nullptr;
-    HIPCHK(hipMalloc(&work, group_sums_bytes(h, ngroups)));
-    const int st = group_sums_into(h, ngroups, work, gtau, gleg, dm_blocks, histo, outer, scalars, nused);
-    (void)hipFree(work);
-    return st;
+    const int st = need_work(h, (size_t)ngroups * (size_t)(h->L.gbuf - h->L.gtau + 14 * 8 + 8));
+    if (st) return st;
+    return group_sums_into(h, ngroups, h->work, gtau, gleg, dm_blocks, histo, outer, scalars, nused);
 }
 
 int w2d_ctqmc_get_group_sums_noalloc(w2d_ctqmc *h, int ngroups, double *gtau, double *gleg, double *dm_blocks,
@@ -1554,9 +1626,7 @@ int w2d_ctqmc_get_giw(w2d_ctqmc *h, int ngroups, int *niw, double *out)
     const int nf = h->dm.nf, nc = h->nchains;
     const size_t per = (size_t)nf * h->niw * 2;
     HIPCHK(hipStreamSynchronize(h->stream));
-    std::vector<double> all((size_t)nc * per);
     std::vector<long long> seen((size_t)nc * nf * 2);
-    HIPCHK(hipMemcpy(all.data(), h->giw, all.size() * sizeof(double), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(seen.data(), h->giw_seen, seen.size() * sizeof(long long), hipMemcpyDeviceToHost));
     std::vector<ChainHdr> hd;
     int st = read_headers(h, hd);
@@ -1572,20 +1642,20 @@ int w2d_ctqmc_get_giw(w2d_ctqmc *h, int ngroups, int *niw, double *out)
             }
     }
     if (ngroups == 0) {
-        std::copy(all.begin(), all.end(), out);
+        HIPCHK(hipMemcpy(out, h->giw, (size_t)nc * per * sizeof(double), hipMemcpyDeviceToHost));
         return W2D_OK;
     }
-    // groups of contiguous chains as in w2d_ctqmc_get_group_sums
-    std::fill(out, out + (size_t)ngroups * per, 0.0);
-    for (int g = 0; g < ngroups; ++g) {
-        const int c0 = (int)((long)g * nc / ngroups), c1 = (int)((long)(g + 1) * nc / ngroups);
-        double *o = out + (size_t)g * per;
-        for (int c = c0; c < c1; ++c) {
-            if (hd[c].err) continue;
-            const double *a = all.data() + (size_t)c * per;
-            for (size_t i = 0; i < per; ++i) o[i] += a[i];
-        }
-    }
+    // groups of contiguous chains as in w2d_ctqmc_get_group_sums, summed on the
+    // device (the sums of all chains are 64 MB for 512 chains of the 2-orbital
+    // model at 2000 frequencies)
+    if ((st = need_work(h, (size_t)ngroups * per * sizeof(double)))) return st;
+    const ChainHdr *hdrs = reinterpret_cast<const ChainHdr *>(h->chains + h->L.hdrs);
+    hipLaunchKernelGGL(w2d::group_sum_kernel, dim3((unsigned)((per + 255) / 256), (unsigned)ngroups), dim3(256), 0,
+                       h->stream, (const char *)h->giw, (long)(per * sizeof(double)), (long)per, nc, ngroups, hdrs,
+                       static_cast<double *>(h->work));
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(out, h->work, (size_t)ngroups * per * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
     return W2D_OK;
 }
 
@@ -1702,27 +1772,19 @@ int w2d_ctqmc_get_group_histograms(w2d_ctqmc *h, int ngroups, double *outer_stat
 {
     if (!h || ngroups < 1 || ngroups > h->nchains) return W2D_ERR_ARG;
     if (!h->measured) return W2D_ERR_STATE;
-    void *work = nullptr;
-    HIPCHK(hipMalloc(&work, group_sums_bytes(h, ngroups)));
-    int st = group_sums_into(h, ngroups, work, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
     const w2d::ChainLayout &L = h->L;
-    const long nel = (L.stride - L.gtau) / 8;
-    const double *part = static_cast<const double *>(work);
-    auto put = [&](double *dst, long off, long n) -> int {
-        if (!dst || n <= 0) return W2D_OK;
-        HIPCHK(hipMemcpy2D(dst, (size_t)n * 8, part + (off - L.gtau) / 8, (size_t)nel * 8, (size_t)n * 8,
-                           (size_t)ngroups, hipMemcpyDeviceToHost));
-        return W2D_OK;
-    };
+    int st = need_work(h, (size_t)ngroups * (size_t)(L.gmstep - L.ohst));
+    if (st) return st;
+    GroupSums g{h, ngroups, L.ohst, 0, static_cast<double *>(h->work)};
+    st = g.run(L.gmstep);
     const long nst = h->model.nstates, nss = h->model.nsst;
-    if (!st) st = put(outer_state, L.ohst, nst);
-    if (!st) st = put(sign_sst, L.shss, nss);
-    if (!st) st = put(sign_state, L.shst, nst);
-    if (!st) st = put(contrib_sst, L.tcss, nss);
-    if (!st) st = put(contrib_state, L.tcst, nst);
-    if (!st) st = put(accpair, L.accpair, 2L * h->model.nbands * L.naccpair_cap);
-    (void)hipFree(work);
-    return st;
+    if (!st) st = g.put(outer_state, L.ohst, nst);
+    if (!st) st = g.put(sign_sst, L.shss, nss);
+    if (!st) st = g.put(sign_state, L.shst, nst);
+    if (!st) st = g.put(contrib_sst, L.tcss, nss);
+    if (!st) st = g.put(contrib_state, L.tcst, nst);
+    if (!st) st = g.put(accpair, L.accpair, 2L * h->model.nbands * L.naccpair_cap);
+    return st ? st : g.done();
 }
 
 int w2d_ctqmc_get_steps(w2d_ctqmc *h, int chain, int *nmstep, double *gtau_mean_step, double *gtau_mid_step,

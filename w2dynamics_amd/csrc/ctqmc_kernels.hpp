@@ -4182,11 +4182,6 @@ __global__ void __launch_bounds__(WAVE) migrate_kernel(ChainLayout A, ChainLayou
     copy_words(d + B.gtau, s + A.gtau, accbytes);
 }
 
-// Accumulators (the contiguous tail [gtau, stride) of each chain block, as
-// doubles) summed over contiguous groups of chains: group g holds chains
-// [g*nc/ng, (g+1)*nc/ng) that have not stopped on an error (header err == 0).
-// Grid: x over elements, y over groups; consecutive threads read consecutive
-// doubles of one chain.
 // Launch order of the chains by expected cost: a counting sort of the chains
 // by expansion order (nop >> shift, clamped to 1023), largest first, in one
 // workgroup (LDS counters; order within a bucket is arbitrary: chains are
@@ -4360,20 +4355,76 @@ __global__ void __launch_bounds__(GIW_THREADS) giw_kernel(ChainLayout L, const c
     }
 }
 
-__global__ void __launch_bounds__(256) group_sum_kernel(const char *chains, long stride, long acc_off, long nel,
-                                                        int nc, int ng, const ChainHdr *hdrs, double *out)
+// Sum of the chains' arrays, element e of group g: group g holds chains
+// [g nc / ng, (g+1) nc / ng) that have not stopped on an error (header err ==
+// 0), chain c's array starts at `first` + c `stride` (bytes).  Grid: x over
+// elements, y over groups; consecutive threads read consecutive doubles of one
+// chain.  Bound by memory latency where groups are large: eight chains are in
+// flight per thread, added in order (so the sum is the plain one over chains).
+__global__ void __launch_bounds__(256) group_sum_kernel(const char *first, long stride, long nel, int nc, int ng,
+                                                        const ChainHdr *hdrs, double *out)
 {
     const long e = (long)blockIdx.x * 256 + threadIdx.x;
     const int g = blockIdx.y;
     if (e >= nel) return;
     const int c0 = (int)((long)g * nc / ng), c1 = (int)((long)(g + 1) * nc / ng);
     double acc = 0.0;
-    for (int c = c0; c < c1; ++c)
-        // the error flag is written by the sweep kernels: a device-coherent
-        // load (a uniform address would otherwise go through the scalar cache)
-        if (__hip_atomic_load(&hdrs[c].err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-            acc += reinterpret_cast<const double *>(chains + (long)c * stride + acc_off)[e];
+    for (int c = c0; c < c1; c += 8) {
+        double v[8];
+        int err[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int cc = min(c + u, c1 - 1);
+            // the error flag is written by the sweep kernels: a device-coherent
+            // load (a uniform address would otherwise go through the scalar cache)
+            err[u] = __hip_atomic_load(&hdrs[cc].err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v[u] = reinterpret_cast<const double *>(first + (long)cc * stride)[e];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (c + u < c1 && err[u] == 0) acc += v[u];
+    }
     out[(long)g * nel + e] = acc;
+}
+
+// Start of a warm-up or measurement call, one workgroup per chain: counters and
+// position of the header (init_counters, CTQMC.F90:847), and the arrays that the
+// call accumulates into.  measure: everything from gtau on but the unused part
+// of the calibration list; else AccPair, over the bins of [0, beta]
+// (CTQMC.F90:8199-8206).  On the device: reading and writing the headers from
+// the host cost more than a short call's sampling.
+__global__ void __launch_bounds__(256) begin_kernel(ChainLayout L, char *chains, int nf, int measure, int ntau,
+                                                    double beta)
+{
+    const int c = blockIdx.x;
+    char *base = chains + (long)c * L.stride;
+    ChainHdr *x = reinterpret_cast<ChainHdr *>(chains + L.hdrs) + c;
+    auto clear = [&](long from, long to) {
+        double *p = reinterpret_cast<double *>(base + from);
+        for (long i = threadIdx.x; i < (to - from) / 8; i += 256) p[i] = 0.0;
+    };
+    if (measure) {
+        clear(L.gtau, L.aptau);
+        clear(L.aptau, min(L.scsum, L.aptau + 8L * max(x->apt_n, 0)));
+        clear(L.scsum, L.stride);
+    } else {
+        clear(L.accpair, L.accpair + 8L * nf * L.naccpair_cap);
+    }
+    if (threadIdx.x != 0) return;
+    x->try_add = x->try_rem = x->try_glob = x->try_shift = 0;
+    x->acc_add = x->acc_rem = x->acc_glob = x->acc_shift = 0;
+    x->qn_rej = x->moves = 0;
+    x->alg_flops = x->alg_bytes = 0.0;
+    x->pos = 0;
+    x->halt = HALT_NONE;
+    x->apt_index = 1;
+    if (measure) {
+        x->meas_sign = 0.0;
+        x->cnt_meas = 0;
+    } else {
+        x->naccpair = ntau;
+        x->accpair_max = beta;
+    }
 }
 
 // The header scalars of the same groups: sum of signs, measurements,
@@ -4419,15 +4470,27 @@ __global__ void __launch_bounds__(WAVE) init_kernel(DevModel M, ChainLayout L, c
     save_ctx(c, (int)blockIdx.x);
 }
 
-// Adopt the configuration already written into tau/code/nop/outer: full trace,
+// Configurations for chains first, first + 1, ...: operators off[i] .. off[i+1]
+// of tau / code and outer superstate outer[i] for chain first + i; full trace,
 // flavour lists, full inverses, sign (set_mc_config_from_arrays,
-// Trace.F90:6872-7000).
+// Trace.F90:6872-7000).  One wave per chain, all chains at once.
 template <int NM>
-__global__ void __launch_bounds__(WAVE) setconfig_kernel(DevModel M, ChainLayout L, char *chains, int only)
+__global__ void __launch_bounds__(WAVE) setconfig_kernel(DevModel M, ChainLayout L, char *chains, int first,
+                                                         const double *tau, const int *code, const int *off,
+                                                         const int *outer)
 {
-    if ((int)blockIdx.x != only) return;
+    const int chain = first + (int)blockIdx.x;
     extern __shared__ __align__(16) char lds[];
-    Ctx c = make_ctx<NM>(chains, (int)blockIdx.x, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
+    Ctx c = make_ctx<NM>(chains, chain, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
+    const int o0 = off[blockIdx.x], n = off[blockIdx.x + 1] - o0;
+    for (int j = lane_id(); j < n; j += WAVE) {
+        c.tau[j] = tau[o0 + j];
+        c.code[j] = code[o0 + j];
+    }
+    c.h.nop = n;
+    c.h.outer = outer[blockIdx.x];
+    c.h.err = 0;
+    wsync();
     c.h.wpos = 0;
     set_window(c);
     const TraceVal T = full_trace<NM>(c, c.h.outer);
@@ -4453,7 +4516,7 @@ __global__ void __launch_bounds__(WAVE) setconfig_kernel(DevModel M, ChainLayout
     c.h.det_sign = dsg;
     c.h.cfgsign = -config_sign(c);
     c.h.cache_pos = -1;
-    save_ctx(c, (int)blockIdx.x);
+    save_ctx(c, chain);
 }
 
 }  // namespace w2d

@@ -75,6 +75,7 @@ def load_library(path: str | None = None):
     lib.w2d_ctqmc_moves_log.argtypes = [P, I, C.c_int64, P]
     lib.w2d_ctqmc_get_config.argtypes = [P, I, I, C.POINTER(I), P, P, P, P, C.POINTER(I), P]
     lib.w2d_ctqmc_set_config.argtypes = [P, I, I, P, P, P, P, I, P]
+    lib.w2d_ctqmc_set_configs.argtypes = [P, I, P, P, P, P, P, P, P]
     lib.w2d_ctqmc_get_minv.argtypes = [P, I, I, C.POINTER(I), P]
     lib.w2d_ctqmc_last_kernel_ms.argtypes = [P, C.POINTER(D), C.POINTER(C.c_int64)]
     lib.w2d_ctqmc_destroy.argtypes = [P]
@@ -307,15 +308,19 @@ class CtqmcGpu:
         """Set every chain to the configuration saved for it (chains beyond the
         saved ones keep theirs); returns the weights set_config computed."""
         with np.load(path) as z:
-            n, outer = z["n"], z["outer_sst"]
-            off = np.concatenate([[0], np.cumsum(n)])
-            arrs = {k: z[k] for k in ("taus", "orbs", "spins", "cas")}
-        out = []
-        for c in range(min(self.nchains, len(n))):
-            a, b = int(off[c]), int(off[c + 1])
-            out.append(self.set_config(c, arrs["taus"][a:b], arrs["orbs"][a:b], arrs["spins"][a:b],
-                                       arrs["cas"][a:b], int(outer[c])))
-        return out
+            n, outer = np.asarray(z["n"]), z["outer_sst"]
+            tau = np.ascontiguousarray(z["taus"], np.float64)
+            orb, spin, ca = (np.ascontiguousarray(z[k], np.int32) for k in ("orbs", "spins", "cas"))
+        m = min(self.nchains, len(n))
+        off = np.concatenate([[0], np.cumsum(n[:m])]).astype(np.int64)
+        outer = np.ascontiguousarray(outer[:m], np.int32)
+        if len(outer) < m or min(len(x) for x in (tau, orb, spin, ca)) < off[-1]:
+            raise CtqmcError(1, "load_configs (the file holds fewer operators than it announces)")
+        w = np.zeros((m, 5))
+        _check(self.lib.w2d_ctqmc_set_configs(self.h, m, _p(off), _p(tau), _p(orb), _p(spin), _p(ca), _p(outer),
+                                              _p(w)), "set_configs")
+        keys = ("trace_log", "trace_sign", "det_log", "det_sign", "cfgsign")
+        return [dict(zip(keys, x)) for x in w.tolist()]
 
     def get_minv(self, chain: int, f: int) -> np.ndarray:
         k = C.c_int()
