@@ -57,7 +57,8 @@ DEV T *uni_lds(T *p)
 template <int CTRL>
 DEV int dpp_i(int v)
 {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+    // permutations within a row: every lane has a source, so no old value
+    return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
 }
 
 template <int CTRL>
@@ -711,7 +712,7 @@ DEV void renorm(State<NM> &k, unsigned long long mask, double &lg)
 }
 
 // Where a walk leaves the state after each operator (at that operator's time):
-// state matrices, log scales (from the walk's start) and superstates.
+// state matrices, log scales (lg0 included) and superstates.
 template <int NM>
 struct Prefix {
     typedef typename std::conditional<(NM <= 4), lds_d *, glb_d *>::type mat;
@@ -754,7 +755,7 @@ struct WalkOut {
 template <int NM, bool BRA, bool KEEP>
 __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_, double tstart, double tend,
                                                             const lds_d *otau_, const lds_i *ocode_, int n_,
-                                                            int no_, Prefix<NM> px)
+                                                            int no_, double lg0, Prefix<NM> px)
 {
     const int l = lane_id();
     const int n = uni(n_), no = uni(no_);
@@ -768,7 +769,7 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_,
     const lds_b *keys = uni_lds(E.keys);
     const int ncol = uni(E.ncol), dkey = uni(E.dkey);
     int s = uni(s_);
-    double lg = 0.0;
+    double lg = lg0;
     WalkOut<NM> out;
     out.s = -1;
     constexpr unsigned long long QUAD0 = 0x000F000F000F000Full;
@@ -883,8 +884,8 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_,
                             if (b == 3 || chk == 0u) renorm(k, QUAD0 << (4 * b), lr);
                             if constexpr (KEEP) {
                                 if (q0 + t_ < nc) {
-                                    const int j = c0 + q0 + t_, nt = __builtin_amdgcn_readlane(rec.y, q0 + t_);
-                                    if (blk == b && kr < nt && i < no) px.k[j * 16 + kr * no + i] = k.v[0];
+                                    const int j = c0 + q0 + t_;
+                                    if (blk == b) px.k[j * 16 + kr * 4 + i] = k.v[0];
                                     px.lg[j] = lg + lr + readlane_d(sc, q0 + t_);
                                 }
                             }
@@ -1042,7 +1043,7 @@ DEV double row_scan_mul(double x)
 template <int NM, bool BRA, bool KEEP>
 __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, double tstart, double tend,
                                                           const lds_d *otau_, const lds_i *ocode_, int n_, int no_,
-                                                          Prefix<NM> px)
+                                                          double lg0, Prefix<NM> px)
 {
     const int l = lane_id(), p = l & 15;
     const int n = uni(n_), no = uni(no_);
@@ -1082,25 +1083,26 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
         if (l < n) px.sst[p] = rec.x;
     }
     const double sc = KEEP ? row_scan_d(lc) : row_sum_d(lc);
-    double lg = 0.0;
+    double lg = lg0;
     if constexpr (NM == 1) {
         // every block is one number, every propagation a log factor only
         const double a = row_scan_mul(op ? lops[rec.z] : 1.0), k0 = readlane_d(k.v[0], 0);
         if constexpr (KEEP) {
             if (l < n) {
                 px.k[p] = k0 * a;
-                px.lg[p] = sc;
+                px.lg[p] = lg + sc;
             }
         }
         k.v[0] *= readlane_d(a, 15);   // zero in the lanes outside the block
     } else {
         // long propagations: a check per operator
         if (__ballot(__int_as_float(si.w) * (float)dt > 100.0f) != 0ull)
-            return walk_small<NM, BRA, KEEP>(k, s0, tstart, tend, otau, ocode, n, no, px);
+            return walk_small<NM, BRA, KEEP>(k, s0, tstart, tend, otau, ocode, n, no, lg0, px);
         const int blk = (l >> 2) & 3, i = l & 3, r = l >> 4;
         const double dr = exp(-(ev[eo + (r < ns ? r : 0)] - e0) * dt);
         // block offset, sizes; 1 << 28: the propagation to tend, 1 << 29: beyond it
         const int pack = op ? (rec.z & 0xfffff) | (rec.y << 20) | (ns << 24) : (ns << 20) | (ns << 24) | (p == n ? 1 << 28 : 1 << 29);
+        double lgb = lg, lgp = lg;   // scales before this group; of this lane's operator
         double a[4];
 #pragma unroll
         for (int ps = 0; ps < 4; ++ps) {
@@ -1123,15 +1125,19 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
                     k.v[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[ps], x, 0.0, 0, 0, 0);
                     if (b == 3) renorm(k, 0xF000F000F000F000ull, lg);
                     if constexpr (KEEP) {
-                        const int t_ = 4 * ps + b;
-                        if (t_ < n) {
-                            const int nt = __builtin_amdgcn_readlane(rec.y, t_);
-                            if (blk == b && r < nt && i < no) px.k[t_ * 16 + r * no + i] = k.v[0];
-                            px.lg[t_] = lg + readlane_d(sc, t_);
-                        }
+                        // (entries behind the n-th are rewritten before they are read)
+                        if (blk == b && 4 * ps + b < n) px.k[(4 * ps + b) * 16 + r * 4 + i] = k.v[0];
                     }
                 }
+                if constexpr (KEEP) {
+                    // lanes 4 ps .. 4 ps + 2 of the list: scales before this group's check
+                    if (p >> 2 == ps) lgp = p == 4 * ps + 3 ? lg : lgb;
+                    lgb = lg;
+                }
             }
+        }
+        if constexpr (KEEP) {
+            if (l < n) px.lg[p] = lgp + sc;
         }
         // the state to every quad
         double x = blk == 3 ? k.v[0] : 0.0;
@@ -1153,12 +1159,12 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
 
 template <int NM, bool BRA, bool KEEP>
 DEV WalkOut<NM> walk_any(State<NM> k, int s, double tstart, double tend, const lds_d *otau, const lds_i *ocode, int n,
-                         int no, Prefix<NM> px)
+                         int no, double lg0, Prefix<NM> px)
 {
     if constexpr (NM <= 4) {
-        if (n <= 15 && uni(s_wenv.dkey)) return walk_row<NM, BRA, KEEP>(k, s, tstart, tend, otau, ocode, n, no, px);
+        if (n <= 15 && uni(s_wenv.dkey)) return walk_row<NM, BRA, KEEP>(k, s, tstart, tend, otau, ocode, n, no, lg0, px);
     }
-    return walk_small<NM, BRA, KEEP>(k, s, tstart, tend, otau, ocode, n, no, px);
+    return walk_small<NM, BRA, KEEP>(k, s, tstart, tend, otau, ocode, n, no, lg0, px);
 }
 
 // What an operator walk over blocks above 16 states needs, by value (the walk
@@ -1399,11 +1405,11 @@ DEV bool walk_list(State<NM> &k, int &s, double &lg, int no, double t0, const do
                    double t1)
 {
     const WalkOut<NM> o =
-        walk_any<NM, BRA, false>(k, s, t0, t1, (const lds_d *)otau, (const lds_i *)ocode, n, no, Prefix<NM>{});
+        walk_any<NM, BRA, false>(k, s, t0, t1, (const lds_d *)otau, (const lds_i *)ocode, n, no, lg, Prefix<NM>{});
     if (o.s < 0) return false;
     k = o.k;
     s = o.s;
-    lg += o.lg;
+    lg = o.lg;
     return true;
 }
 
@@ -1762,15 +1768,18 @@ DEV bool window_trace(Ctx &c, int nl, TraceVal &T)
 // caches are extended on demand and cut back to their unchanged parts after
 // an accepted move; both restart when the window list is reloaded or the
 // boundary caches change.  Their log scales and superstates are in LDS; the
-// matrices too for blocks up to 4 states (row-major, NM^2 apart), above they
-// are the lanes' registers as they are (2 KB, coalesced), in the chain block.
+// matrices too for blocks up to 4 states (4 x 4, zero beyond the block), above
+// they are the lanes' registers as they are (2 KB, coalesced), in the chain
+// block.
 // ---------------------------------------------------------------------------
 template <int NM>
 DEV State<NM> seg_load(const double *buf, int j, int ns, int no)
 {
     State<NM> k;
-    if constexpr (NM <= 4) {
-        k.load(buf + j * NM * NM, ns, no);
+    if constexpr (NM == 1) {
+        k.load(buf + j, ns, no);
+    } else if constexpr (NM <= 4) {
+        k.v[0] = buf[j * 16 + 4 * State<NM>::row(0) + State<NM>::col()];
     } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) k.v[e] = buf[j * 256 + e * 64 + lane_id()];
@@ -1780,8 +1789,10 @@ DEV State<NM> seg_load(const double *buf, int j, int ns, int no)
 template <int NM>
 DEV void seg_store(double *buf, int j, int ns, int no, const State<NM> &k)
 {
-    if constexpr (NM <= 4) {
-        k.store(buf + j * NM * NM, ns, no);
+    if constexpr (NM == 1) {
+        k.store(buf + j, ns, no);
+    } else if constexpr (NM <= 4) {
+        if ((lane_id() & 12) == 0) buf[j * 16 + 4 * State<NM>::row(0) + State<NM>::col()] = k.v[0];
     } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) buf[j * 256 + e * 64 + lane_id()] = k.v[e];
@@ -1825,9 +1836,7 @@ __device__ __attribute__((noinline)) void seg_extend(ChainRef ref, int nw_, int 
         const double t0 = j > 0 ? c.wtau[BRA ? nw - j : j - 1] : bound_tau(BRA ? w + 2 : w, c.h.nwin, c.M.beta);
         const double t1 = c.wtau[BRA ? nw - to : to - 1];
         walk_any<NM, BRA, true>(k, s, t0, t1, (const lds_d *)(c.wtau + a), (const lds_i *)(c.wcode + a), to - j,
-                                  no, px);
-        // log scales of a walk count from its start
-        for (int i = j + 1 + lane_id(); i <= to; i += WAVE) bx[i] += lg0;
+                                no, lg0, px);
     }
     (BRA ? c.h.lb_n : c.h.rk_n) = to + 1;
     wsync();
@@ -1949,7 +1958,7 @@ __device__ __attribute__((noinline)) void slide_window(ChainRef ref)
                 if (i < rn) c.rkx[i] = x, c.rks[i] = q;
                 wsync();
             }
-            k.store(c.rk, ns, no);
+            seg_store<NM>(c.rk, 0, ns, no, k);
             c.rkx[0] = lg;
             c.rks[0] = s;
             c.h.rk_n = rn;
