@@ -31,7 +31,8 @@ F2PY_EXT = os.path.join(HERE, "CTQMC" + (sysconfig.get_config_var("EXT_SUFFIX") 
 
 
 def build(verbose: bool = False) -> str:
-    cmd = ["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-fno-optimize-sibling-calls",
+    cmd = ["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-fno-optimize-sibling-calls", "-mllvm",
+           "-amdgpu-mfma-vgpr-form=1",
            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
            "-I" + os.path.join(ROOT, "include"), *SOURCES, "-o", TARGET + ".tmp"]
     if verbose:
