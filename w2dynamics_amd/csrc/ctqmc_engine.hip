@@ -1101,23 +1101,32 @@ int w2d_ctqmc_create(const char *params, int nbands, int nftau, const double *u_
     }
     std::vector<unsigned char> keys;
     d.dkey = superstate_keys(m, keys);
-    std::vector<double> opsz(m.ops);   // a zero behind the blocks (rows and columns beyond a block)
-    opsz.push_back(0.0);
+    std::vector<double> opsx;
     std::vector<int> first_state(m.nsst);
     for (int s = 0; s < m.nsst; ++s) first_state[s] = m.states[m.offsets[s]];
     std::vector<int4> trans(m.connect.size());
-    for (size_t i = 0; i < m.connect.size(); ++i) {
+    const int nk = std::max(3, (m.nmax + 3) / 4);
+    for (size_t i = 0, nblk = 0; i < m.connect.size(); ++i) {
         const int ts = m.connect[i];
-        trans[i] = make_int4(ts, ts >= 0 ? m.sizes[ts] : 0, (int)m.opoff[i], ts >= 0 ? m.offsets[ts] : 0);
+        trans[i] = make_int4(ts, ts >= 0 ? m.sizes[ts] : 0, (int)m.opoff[i], (int)nblk);
+        if (ts < 0 || m.nmax > 16) continue;
+        const int src = (int)(i / (4 * (size_t)nbands)), nt = m.sizes[ts], ns = m.sizes[src];
+        for (int e = 0; e < nk; ++e)
+            for (int l = 0; l < 64; ++l) {
+                const int r = l & 15, k = 4 * e + (l >> 4);
+                opsx.push_back(r < nt && k < ns ? m.ops[m.opoff[i] + r + (long)k * nt] : 0.0);
+            }
+        ++nblk;
     }
     int st = 0;
     if ((st = upload(h.get(), m.sizes, &d.sizes)) || (st = upload(h.get(), m.offsets, &d.offsets)) ||
         (st = upload(h.get(), m.connect, &d.connect)) || (st = upload(h.get(), first_state, &d.first_state)) ||
         (st = upload(h.get(), m.state_sst, &d.state_sst)) || (st = upload(h.get(), m.opoff, &d.opoff)) ||
-        (st = upload(h.get(), opsz, &d.ops)) || (st = upload(h.get(), m.evals, &d.evals)) ||
+        (st = upload(h.get(), m.ops, &d.ops)) || (st = upload(h.get(), m.evals, &d.evals)) ||
         (st = upload(h.get(), fdiag, &d.ftau)) || (st = upload(h.get(), dmoff, &d.dmoff)) ||
         (st = upload(h.get(), legc, &d.legc)) || (st = upload(h.get(), trans, &d.trans)) ||
-        (st = upload(h.get(), keys, &d.keys)) || (h->nm > 16 && (st = build_ops16(h.get()))))
+        (st = upload(h.get(), keys, &d.keys)) || (st = upload(h.get(), opsx, &d.opsx)) ||
+        (h->nm > 16 && (st = build_ops16(h.get()))))
         return st;
     // user symmetry moves (Trace.F90:471-478): SymMove01.. are 1-based
     // flavour permutations; their inverses follow in the table

@@ -346,7 +346,7 @@ struct ChainRef {
 struct WalkEnv {
     double egs;
     double flops, bytes;    // algorithmic work of this launch
-    const double *ops;      // operator blocks in global memory, a zero behind the last
+    const double *opsx;     // operator blocks in the order of the matrix instructions' lanes
     const lds_i4 *tr;       // transition records
     const lds_d *ev;        // energies
     const lds_b *keys;      // key of each superstate, then the superstate of each key (255: none)
@@ -357,7 +357,6 @@ struct WalkEnv {
     int dkey;               // key change by a creator of spin 0 | of spin 1 << 8; 0: no such keys
     int np;                 // removable pairs of the window
     int ready;              // window list valid and room for any move; cleared by whatever changes that
-    int zero;               // offset of the zero behind the operator table
     int nkmax;              // matrix-instruction steps of the largest block
     int no;                 // states of the outer superstate (valid while ready)
     // LDS addresses: window list and trial list (their buffers swap), pair
@@ -745,9 +744,10 @@ struct WalkOut {
 //  (4) the products.  Blocks up to 4: the state moves one quad on per operator
 //      (two DPP moves) to the quad that holds the operator's entries, one
 //      matrix instruction each; the other quads carry nothing.  Blocks up to
-//      16: ceil(ns/4) chained matrix instructions, block entries loaded from
-//      global memory (29 KB for the 3-orbital model, shared by all chains) one
-//      to two operators ahead.  Blocks of one state: a product over the lanes.
+//      16: ceil(ns/4) chained matrix instructions; the operator blocks lie in
+//      global memory in the lanes' own order (512 bytes per k-step, zero beyond
+//      the block; 216 KB for the 3-orbital model, shared by all chains), so an
+//      operator is three coalesced loads, issued two operators ahead.  Blocks of one state: a product over the lanes.
 // The renormalisation check runs per operator only if some propagation of the
 // group spans more than exp(-100), else every fourth operator: in between no
 // state can leave the FP64 range.
@@ -900,83 +900,90 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_,
             k.v[0] = x + dpp_d<DPP_ROW_ROR8>(x);
         } else {
             const unsigned chk = __ballot(__int_as_float(si.w) * (float)dt > 100.0f) ? 0u : 3u;
-            lds_d *qa = uni_lds(E.qa);
-            const glb_d *ops = uni_glb(E.ops);
-            const int zero = uni(E.zero);
-            const int lr = l & 15, lk = l >> 4;
             const double sc = KEEP ? wave_scan_d(lc) : wave_sum(lc);
             double lren = 0.0;
-            for (int q0 = 0; q0 < m; q0 += 16) {
-                const int mq = min(16, m - q0);
-                // (3) propagators of operators q0 .. q0 + mq - 1, state l % 16
-                wsync();
-                for (int ps = 0; 4 * ps < mq; ++ps) {
-                    const int src = min(q0 + 4 * ps + lk, 63);
-                    const int nq = __shfl(ns, src, WAVE), eq = __shfl(eo, src, WAVE);
-                    const double dq = __shfl(dt, src, WAVE);
-                    const double d = exp(-(ev[eq + (lr < nq ? lr : 0)] - ev[eq]) * dq);
-                    qa[(4 * ps + lk) * 16 + lr] = lr < nq ? d : 0.0;
-                }
-                wsync();
-                // (4) products
-                const int mp = min(16, nc - q0);   // operators (the propagation to tend comes last)
-                auto load = [&](int t_, double (&a)[4]) {
-                    const int o = q0 + min(t_, max(mp - 1, 0));
-                    const int bo = __builtin_amdgcn_readlane(rec.z, o), nt = __builtin_amdgcn_readlane(rec.y, o),
-                              nq = __builtin_amdgcn_readlane(ns, o);
-                    int ad = bo + lr + lk * nt;
-                    const bool row = lr < nt && bo >= 0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        a[e] = ops[row && 4 * e + lk < nq ? ad : zero];
-                        ad += 4 * nt;
+            auto products = [&](auto nk) {
+                constexpr int NK = decltype(nk)::value;
+                lds_d *qa = uni_lds(E.qa);
+                const glb_d *ops = uni_glb(E.opsx) + l;
+                const int lr = l & 15, lk = l >> 4;
+                for (int q0 = 0; q0 < m; q0 += 16) {
+                    const int mq = min(16, m - q0);
+                    // (3) propagators of operators q0 .. q0 + mq - 1, state l % 16
+                    wsync();
+                    for (int ps = 0; 4 * ps < mq; ++ps) {
+                        const int src = min(q0 + 4 * ps + lk, 63);
+                        const int nq = __shfl(ns, src, WAVE), eq = __shfl(eo, src, WAVE);
+                        const double dq = __shfl(dt, src, WAVE);
+                        const double d = exp(-(ev[eq + (lr < nq ? lr : 0)] - ev[eq]) * dq);
+                        qa[(4 * ps + lk) * 16 + lr] = lr < nq ? d : 0.0;
                     }
-                };
-                auto props = [&](int t_, double (&d)[4]) {
+                    wsync();
+                    // (4) products
+                    const int mp = min(16, nc - q0);   // operators (the propagation to tend comes last)
+                    auto load = [&](int t_, double (&a)[NK]) {
+                        const int b = __builtin_amdgcn_readlane(rec.w, q0 + min(t_, mp - 1));
+                        const glb_d *P = ops + (long)b * (NK * 64);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) d[e] = qa[min(t_, 15) * 16 + 4 * e + lk];
-                };
-                auto step = [&](int t_, const double (&a)[4], const double (&d)[4]) {
-                    const int nq = __builtin_amdgcn_readlane(ns, q0 + t_);
-                    dbl4 r{0.0, 0.0, 0.0, 0.0};
+                        for (int e = 0; e < NK; ++e) a[e] = P[e * 64];
+                    };
+                    auto props = [&](int t_, double (&d)[NK]) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (4 * e < nq) r = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], k.v[e] * d[e], r, 0, 0, 0);
+                        for (int e = 0; e < NK; ++e) d[e] = qa[min(t_, 15) * 16 + 4 * e + lk];
+                    };
+                    auto step = [&](int t_, const double (&a)[NK], const double (&d)[NK]) {
+                        const int nq = __builtin_amdgcn_readlane(ns, q0 + t_);
+                        dbl4 r = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], k.v[0] * d[0], dbl4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) k.v[e] = r[e];
-                };
-                auto after = [&](int t_) {
-                    if (((unsigned)t_ & chk) == chk) renorm(k, ~0ull, lren);
-                    if constexpr (KEEP) {
-                        const int j = c0 + q0 + t_;
+                        for (int e = 1; e < NK; ++e)
+                            if (4 * e < nq) r = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], k.v[e] * d[e], r, 0, 0, 0);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) px.k[j * 256 + e * 64 + l] = k.v[e];
-                        px.lg[j] = lg + lren + readlane_d(sc, q0 + t_);
+                        for (int e = 0; e < 4; ++e) k.v[e] = r[e];
+                    };
+                    auto after = [&](int t_) {
+                        if (((unsigned)t_ & chk) == chk) renorm(k, ~0ull, lren);
+                        if constexpr (KEEP) {
+                            const int j = c0 + q0 + t_;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) px.k[j * 256 + e * 64 + l] = k.v[e];
+                            px.lg[j] = lg + lren + readlane_d(sc, q0 + t_);
+                        }
+                    };
+                    if (mp > 0) {
+                        // an odd operator first, then pairs: every load has its
+                        // fixed place in the queue
+                        double a0[NK], a1[NK], d0[NK], d1[NK];
+                        load(0, a0);
+                        load(1, a1);
+                        int t_ = 0;
+                        if (mp & 1) {
+                            props(0, d0);
+                            step(0, a0, d0);
+                            load(1, a0);
+                            load(2, a1);
+                            after(0);
+                            t_ = 1;
+                        }
+                        props(t_, d0);
+                        for (; t_ < mp; t_ += 2) {
+                            props(t_ + 1, d1);
+                            step(t_, a0, d0);
+                            load(t_ + 2, a0);
+                            after(t_);
+                            props(t_ + 2, d0);
+                            step(t_ + 1, a1, d1);
+                            load(t_ + 3, a1);
+                            after(t_ + 1);
+                        }
                     }
-                };
-                double a0[4], a1[4], d0[4], d1[4];
-                load(0, a0);
-                load(1, a1);
-                props(0, d0);
-                for (int t_ = 0; t_ < mp; t_ += 2) {
-                    props(t_ + 1, d1);
-                    step(t_, a0, d0);
-                    load(t_ + 2, a0);
-                    after(t_);
-                    if (t_ + 1 < mp) {
-                        props(t_ + 2, d0);
-                        step(t_ + 1, a1, d1);
-                        load(t_ + 3, a1);
-                        after(t_ + 1);
+                    if (last && q0 + mq == m) {
+#pragma unroll
+                        for (int e = 0; e < NK; ++e) k.v[e] *= qa[(mq - 1) * 16 + 4 * e + lk];
                     }
                 }
-                if (last && q0 + mq == m) {
-                    double d[4];
-                    props(mq - 1, d);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) k.v[e] *= d[e];
-                }
-            }
+            };
+            if (uni(E.nkmax) <= 3) products(std::integral_constant<int, 3>());
+            else products(std::integral_constant<int, 4>());
             lg += lren + (KEEP ? readlane_d(sc, m - 1) : sc);
         }
     }
@@ -2293,97 +2300,207 @@ DEV void mat_rem_phys(Ctx &c, double *Mf, int k, int sc, int sa)
     }
 }
 
-// LU with partial pivoting of A (k x k, ld) in place; log|det| and sign as
-// get_LogDetFull (MatrixUpdate.F90:302-339).  Returns false if singular.
-DEV bool lu_inplace(double *A, int k, int ld, double &dl, double &ds, int *piv)
+// log|det| and sign from pivots: the product by mantissa and exponent, one
+// logarithm at the end
+struct PivotProduct {
+    double m = 1.0;
+    int e = 0;
+    DEV void mul(double d, bool swapped)
+    {
+        m *= swapped ? -d : d;
+        const int x = ilogb(m);
+        m = ldexp(m, -x);
+        e += x;
+    }
+    DEV double log_abs() const { return log(fabs(m)) + (double)e * 0.69314718055994530942; }
+    DEV double sign() const { return m >= 0.0 ? 1.0 : -1.0; }
+};
+
+// Pivot of column col among the rows col .. k-1 (largest modulus, lowest row
+// among ties), swapped into row col; false if the column is zero.
+template <typename P>
+DEV bool pivot_row(P A, int k, int ld, int col, int &bi)
 {
     const int l = lane_id();
-    dl = 0.0;
-    ds = 1.0;
-    for (int col = 0; col < k; ++col) {
-        double best = -1.0;
-        int bi = col;
-        for (int r = col + l; r < k; r += WAVE) {
-            double v = fabs(A[r + (long)col * ld]);
-            if (v > best) best = v, bi = r;
-        }
-        // largest modulus, lowest row among ties
-        const double wb = wave_max(best);
-        bi = wave_imin(best == wb ? bi : 0x7fffffff);
-        best = wb;
-        if (best == 0.0) return false;
-        if (l == 0) piv[col] = bi;
-        if (bi != col) {
-            for (int j = l; j < k; j += WAVE) {
-                double t = A[col + (long)j * ld];
-                A[col + (long)j * ld] = A[bi + (long)j * ld];
-                A[bi + (long)j * ld] = t;
-            }
-        }
-        wsync();
-        double d = A[col + (long)col * ld];
-        ds *= (bi != col ? -1.0 : 1.0) * (d >= 0 ? 1.0 : -1.0);
-        dl += log(fabs(d));
-        for (int r = col + 1 + l; r < k; r += WAVE) A[r + (long)col * ld] /= d;
-        wsync();
-        // trailing update, lanes over its elements
-        const int m = k - col - 1;
-        for (int idx = l; idx < m * m; idx += WAVE) {
-            const int r = col + 1 + idx % m, j = col + 1 + idx / m;
-            A[r + (long)j * ld] -= A[r + (long)col * ld] * A[col + (long)j * ld];
-        }
-        wsync();
+    double best = -1.0;
+    bi = 0x7fffffff;
+    for (int r = l; r < k; r += WAVE) {
+        const double v = r >= col ? fabs(A[r + (long)col * ld]) : -1.0;
+        if (v > best) best = v, bi = r;
     }
+    const double wb = wave_max(best);
+    bi = wave_imin(best == wb ? bi : 0x7fffffff);
+    if (!(wb > 0.0)) return false;
+    if (bi != col) {
+        for (int j = l; j < k; j += WAVE) {
+            const double t = A[col + (long)j * ld], u = A[bi + (long)j * ld];
+            A[col + (long)j * ld] = u;
+            A[bi + (long)j * ld] = t;
+        }
+    }
+    wsync();
     return true;
 }
 
-// Inverse from an in-place LU (row swaps piv) into out (k x k, leading
-// dimension ldo): out = U^-1 L^-1 P, by substitution on all columns at once,
-// lanes over the elements of each step.
-DEV void lu_inverse(const double *LU, int k, int ld, const int *piv, double *out, int ldo)
+// LU with partial pivoting of A (k x k, ld) in place; log|det| and sign as
+// get_LogDetFull (MatrixUpdate.F90:302-339).  Returns false if singular.
+template <typename P>
+DEV bool lu_inplace(P A, int k, int ld, double &dl, double &ds)
+{
+    const MatLanes ml(k);
+    PivotProduct det;
+    for (int col = 0; col < k; ++col) {
+        int bi;
+        if (!pivot_row(A, k, ld, col, bi)) {
+            dl = 0.0;
+            ds = 1.0;
+            return false;
+        }
+        const double d = A[col + (long)col * ld];
+        det.mul(d, bi != col);
+        const double rd = 1.0 / d;
+        for (int i0 = 0; i0 < k; i0 += WAVE) {
+            const int i = i0 + ml.i;
+            if (i > col && i < k) {
+                const double f = A[i + (long)col * ld] * rd;
+                for (int j = col + 1 + ml.g; j < k; j += ml.step) A[i + (long)j * ld] -= f * A[col + (long)j * ld];
+            }
+        }
+        wsync();
+    }
+    dl = det.log_abs();
+    ds = det.sign();
+    return true;
+}
+
+// Inverse of A (k x k, ld) in place by Gauss-Jordan elimination with partial
+// pivoting, and the determinant from its pivots; piv: k ints.
+template <typename P>
+DEV bool gj_inverse(P A, int k, int ld, int *piv, double &dl, double &ds)
 {
     const int l = lane_id();
-    for (int idx = l; idx < k * k; idx += WAVE) out[idx % k + (long)(idx / k) * ldo] = 0.0;
-    wsync();
-    // row r of the identity ends in row pos after the swaps
-    for (int r = l; r < k; r += WAVE) {
-        int pos = r;
-        for (int i = 0; i < k; ++i) {
-            const int p = piv[i];
-            pos = pos == i ? p : (pos == p ? i : pos);
+    const MatLanes ml(k);
+    PivotProduct det;
+    for (int col = 0; col < k; ++col) {
+        int bi;
+        if (!pivot_row(A, k, ld, col, bi)) {
+            dl = 0.0;
+            ds = 1.0;
+            return false;
         }
-        out[pos + (long)r * ldo] = 1.0;
-    }
-    wsync();
-    for (int i = 0; i + 1 < k; ++i) {
-        const int m = k - i - 1;
-        for (int idx = l; idx < m * k; idx += WAVE) {
-            const int r = i + 1 + idx % m, cc = idx / m;
-            out[r + (long)cc * ldo] -= LU[r + (long)i * ld] * out[i + (long)cc * ldo];
-        }
+        const double d = A[col + (long)col * ld], rd = 1.0 / d;
+        det.mul(d, bi != col);
+        if (l == 0) piv[col] = bi;
         wsync();
-    }
-    for (int i = k - 1; i >= 0; --i) {
-        for (int cc = l; cc < k; cc += WAVE) out[i + (long)cc * ldo] /= LU[i + (long)i * ld];
+        // the pivot row, with the pivot's place taken by the inverse's column
+        for (int j = l; j < k; j += WAVE) A[col + (long)j * ld] = j == col ? rd : A[col + (long)j * ld] * rd;
         wsync();
-        for (int idx = l; idx < i * k; idx += WAVE) {
-            const int r = idx % i, cc = idx / i;
-            out[r + (long)cc * ldo] -= LU[r + (long)i * ld] * out[i + (long)cc * ldo];
+        for (int i0 = 0; i0 < k; i0 += WAVE) {
+            const int i = i0 + ml.i;
+            const bool in = i < k && i != col;
+            const double f = in ? A[i + (long)col * ld] : 0.0;
+            wsync();
+            if (in)
+                for (int j = ml.g; j < k; j += ml.step)
+                    A[i + (long)j * ld] = fma(-f, A[col + (long)j * ld], j == col ? 0.0 : A[i + (long)j * ld]);
         }
         wsync();
     }
+    // undo the row swaps as column swaps
+    for (int col = k - 1; col >= 0; --col) {
+        const int b = uni(piv[col]);
+        if (b == col) continue;
+        for (int i = l; i < k; i += WAVE) {
+            const double t = A[i + (long)col * ld], u = A[i + (long)b * ld];
+            A[i + (long)col * ld] = u;
+            A[i + (long)b * ld] = t;
+        }
+        wsync();
+    }
+    dl = det.log_abs();
+    ds = det.sign();
+    return true;
 }
 
 // Delta_f(row = annihilator rank, col = creator rank) = F(tau_a - tau_c)
 // (get_InvFullHybr, Trace.F90:2279-2333) from the per-flavour lists
-DEV void build_delta(Ctx &c, int f, int k, double *D, int ld, const double *fcl, const double *fal)
+template <typename P>
+DEV void build_delta(Ctx &c, int f, int k, P D, int ld, const double *fcl, const double *fal)
 {
     const double *ct = fcl + (long)f * c.L.kcap, *at = fal + (long)f * c.L.kcap;
-    for (int idx = lane_id(); idx < k * k; idx += WAVE) {
-        int r = idx % k, col = idx / k;
-        D[r + (long)col * ld] = hybr(c.M, at[r] - ct[col], f);
+    const MatLanes ml(k);
+    for (int i0 = 0; i0 < k; i0 += WAVE) {
+        const int r = i0 + ml.i;
+        const double ta = at[min(r, k - 1)];
+        for (int j0 = ml.g; j0 < k; j0 += 4 * ml.step) {
+            double v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = hybr(c.M, ta - ct[min(j0 + u * ml.step, k - 1)], f);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (r < k && j0 + u * ml.step < k) D[r + (long)(j0 + u * ml.step) * ld] = v[u];
+        }
     }
     wsync();
+}
+
+// LDS work area for one k x k block: the window segment caches (blocks up to 4
+// states) or the trial list (blocks up to 16), both free during the moves that
+// need it; its size in doubles
+template <int NM>
+DEV lds_d *block_area(Ctx &c, long &cap)
+{
+    if constexpr (NM <= 4) {
+        cap = 2L * (c.L.sc + 1) * NM * NM;
+        c.h.rk_n = 0;
+        c.h.lb_n = 0;
+        return (lds_d *)c.rk;
+    } else if constexpr (NM <= 16) {
+        cap = 3L * (c.L.lcap_lds & ~1) / 2;   // times and codes lie behind each other
+        return (lds_d *)c.ttau;
+    } else {
+        cap = 0;
+        return nullptr;
+    }
+}
+
+// determinant of Delta_f of the given lists
+template <int NM>
+DEV bool delta_det(Ctx &c, int f, int k, const double *fcl, const double *fal, double &dl, double &ds)
+{
+    long cap;
+    lds_d *A = block_area<NM>(c, cap);
+    if ((long)k * k <= cap) {
+        build_delta(c, f, k, A, k, fcl, fal);
+        return lu_inplace(A, k, k, dl, ds);
+    }
+    build_delta(c, f, k, c.scratch, c.L.kcap, fcl, fal);
+    return lu_inplace(c.scratch, k, c.L.kcap, dl, ds);
+}
+
+// M_f = Delta_f^{-1} of the chain's lists (physical order = ranks), and det Delta_f
+template <int NM>
+DEV bool delta_inverse(Ctx &c, int f, int k, double &dl, double &ds)
+{
+    long cap;
+    lds_d *A = block_area<NM>(c, cap);
+    int *piv = reinterpret_cast<int *>(c.R);
+    double *Mf = c.mi(f);
+    const int ld = c.L.kcap;
+    if ((long)k * k <= cap) {
+        build_delta(c, f, k, A, k, c.fc, c.fa);
+        const bool ok = gj_inverse(A, k, k, piv, dl, ds);
+        const MatLanes ml(k);
+        for (int i0 = 0; i0 < k; i0 += WAVE) {
+            const int i = i0 + ml.i;
+            if (i < k)
+                for (int j = ml.g; j < k; j += ml.step) Mf[i + (long)j * ld] = A[i + (long)j * k];
+        }
+        wsync();
+        return ok;
+    }
+    build_delta(c, f, k, Mf, ld, c.fc, c.fa);
+    return gj_inverse(Mf, k, ld, piv, dl, ds);
 }
 
 // ---------------------------------------------------------------------------
@@ -2805,62 +2922,104 @@ DEV void global_update(Ctx &c, const int *gu)
     wsync();
 }
 
-// per-flavour tau lists and orders from the operator list: for every flavour,
-// ballot-compact the creators / annihilators of each 64-operator chunk.  With
-// slot lists given, slots are reset to the identity (logical = physical order).
+// per-flavour tau lists and orders from the operator list: ballot-compact the
+// creators / annihilators of every flavour in each 64-operator chunk (lane g of
+// the counts: creators of flavour g, lane 32 + g its annihilators).  With slot
+// lists given, slots are reset to the identity (logical = physical order).
 DEV void rebuild_flavour_lists(Ctx &c, double *dfc, double *dfa, int *dkf, int *dfcs, int *dfas)
 {
     CModel &M = c.M;
     const long kc = c.L.kcap;
-    for (int g = 0; g < M.nf; ++g) {
-        int nc = 0, na = 0;
-        for (int b0 = 0; b0 < c.h.nop; b0 += WAVE) {
-            const int j = b0 + lane_id();
-            int cj = 0;
-            double tj = 0.0;
-            if (j < c.h.nop) {
-                cj = c.code[j];
-                tj = c.tau[j];
-            }
-            const bool isc = j < c.h.nop && c.fl(cj) == g && op_ca(cj) == 1;
-            const bool isa = j < c.h.nop && c.fl(cj) == g && op_ca(cj) == 2;
+    const int n = uni(c.h.nop), l = lane_id(), nf = M.nf;
+    const unsigned long long below = l == 0 ? 0ull : (~0ull >> (64 - l));
+    int counts = 0;
+    for (int b0 = 0; b0 < n; b0 += WAVE) {
+        const int j = b0 + l;
+        const int cj = j < n ? c.code[j] : 0;
+        const double tj = j < n ? c.tau[j] : 0.0;
+        const int fj = j < n ? c.fl(cj) : -1;
+        const bool cre = op_ca(cj) == 1;
+        for (int g = 0; g < nf; ++g) {
+            const bool isc = fj == g && cre, isa = fj == g && !cre;
             const unsigned long long mc = __ballot(isc), ma = __ballot(isa);
-            const unsigned long long below = (lane_id() == 0) ? 0ull : (~0ull >> (64 - lane_id()));
+            const int nc = __builtin_amdgcn_readlane(counts, g), na = __builtin_amdgcn_readlane(counts, 32 + g);
             if (isc) dfc[g * kc + nc + popc64(mc & below)] = tj;
             if (isa) dfa[g * kc + na + popc64(ma & below)] = tj;
-            nc += popc64(mc);
-            na += popc64(ma);
+            counts += (l == g ? popc64(mc) : 0) + (l == 32 + g ? popc64(ma) : 0);
         }
+    }
+    for (int g = 0; g < nf; ++g) {
+        const int nc = __builtin_amdgcn_readlane(counts, g);
         if (dfcs)
-            for (int r = lane_id(); r < nc; r += WAVE) {
+            for (int r = l; r < nc; r += WAVE) {
                 dfcs[g * kc + r] = r;
                 dfas[g * kc + r] = r;
             }
-        if (lane_id() == 0) dkf[g] = nc;
-        wsync();
+        if (l == 0) dkf[g] = nc;
     }
     wsync();
 }
 
-DEV bool qn_cycle_global(Ctx &c, int s0)
+// change of a superstate's key by an operator (superstate_keys)
+DEV int key_delta(int dkey, int code)
 {
-    int s = s0;
-    for (int j = 0; j < c.h.nop && s >= 0; ++j) s = c.conn(s, c.code[j], false);
-    return s == s0;
+    const int d = (int)(signed char)(op_spin(code) ? dkey >> 8 : dkey);
+    return op_ca(code) == 1 ? d : -d;
 }
 
-// lane-parallel: which superstates give a valid cyclic sequence (lane = start
-// superstate, up to 64 per pass); bit s of the returned masks
-// okmask: one bit per superstate (at most MAXSST)
-DEV int count_valid_outer(Ctx &c, unsigned long long *okmask)
+DEV void all_outer(Ctx &c, unsigned long long *okmask)
 {
+    for (int w = 0; w < MAXSST / WAVE; ++w) {
+        const int left = c.M.nsst - w * WAVE;
+        okmask[w] = left <= 0 ? 0ull : left >= WAVE ? ~0ull : (1ull << left) - 1ull;
+    }
+}
+
+// Which of the superstates set in okmask (one bit each) give a valid cyclic
+// sequence of the configuration; the others' bits are cleared, the number of
+// the ones left returned.  With additive keys the lanes take 64 operators at a
+// time, else a superstate each.
+template <int NM>
+DEV int valid_outer(Ctx &c, unsigned long long *okmask)
+{
+    const int n = uni(c.h.nop), l = lane_id();
     int total = 0;
+    if constexpr (NM <= 16) {
+        const int dkey = uni(s_wenv.dkey), ncol = uni(s_wenv.ncol);
+        if (dkey) {
+            const lds_b *keys = uni_lds(s_wenv.keys);
+            int carry = 0;
+            for (int j0 = 0; j0 < n; j0 += WAVE) {
+                const bool in = j0 + l < n;
+                const int cd = in ? c.code[j0 + l] : 0;
+                const int d = in ? key_delta(dkey, cd) : 0;
+                const int sum = wave_scan_i(d), pre = carry + sum - d;
+                const int col = (op_orb(cd) * 2 + op_spin(cd)) * 2 + op_ca(cd) - 1;
+                carry += __builtin_amdgcn_readlane(sum, 63);
+                for (int w = 0; w * WAVE < c.M.nsst; ++w) {
+                    unsigned long long left = okmask[w], ok = left;
+                    for (; left; left &= left - 1) {
+                        const int b = __builtin_ctzll(left);
+                        const int sb = keys[256 + (((int)keys[w * WAVE + b] + pre) & 255)];
+                        const int t = c.tr[(sb == 255 ? 0 : sb) * ncol + col].x;
+                        if (__ballot(in && (sb == 255 || t < 0)) != 0ull) ok &= ~(1ull << b);
+                    }
+                    okmask[w] = ok;
+                }
+            }
+            for (int w = 0; w * WAVE < c.M.nsst; ++w) {
+                if ((carry & 255) != 0) okmask[w] = 0ull;
+                total += popc64(okmask[w]);
+            }
+            return total;
+        }
+    }
     for (int s0 = 0; s0 < c.M.nsst; s0 += WAVE) {
-        const int s = s0 + lane_id();
+        const int s = s0 + l;
         bool ok = false;
-        if (s < c.M.nsst) {
+        if (s < c.M.nsst && ((okmask[s0 / WAVE] >> l) & 1ull)) {
             int cur = s;
-            for (int j = 0; j < c.h.nop && cur >= 0; ++j) cur = c.conn(cur, c.code[j], false);
+            for (int j = 0; j < n && cur >= 0; ++j) cur = c.conn(cur, c.code[j], false);
             ok = (cur == s);
         }
         const unsigned long long m = __ballot(ok);
@@ -2868,6 +3027,24 @@ DEV int count_valid_outer(Ctx &c, unsigned long long *okmask)
         total += popc64(m);
     }
     return total;
+}
+
+// superstate before operator `first` of the configuration
+template <int NM>
+DEV int sst_before(Ctx &c, int first)
+{
+    int s = uni(c.h.outer);
+    if constexpr (NM <= 16) {
+        const int dkey = uni(s_wenv.dkey);
+        if (dkey) {
+            int sum = 0;
+            for (int j = lane_id(); j < first; j += WAVE) sum += key_delta(dkey, c.code[j]);
+            const lds_b *keys = uni_lds(s_wenv.keys);
+            return uni((int)keys[256 + (((int)keys[s] + wave_isum(sum)) & 255)]);
+        }
+    }
+    for (int i = 0; i < first; ++i) s = c.conn(s, c.code[i], false);
+    return s;
 }
 
 // StepGlob (CTQMC.F90:4433-4554)
@@ -2922,12 +3099,16 @@ __device__ __attribute__((noinline)) int step_glob(ChainRef ref)
         const int nst = up | (dn << nb);
         c.h.outer = M.state_sst[nst];
         global_update(c, gu);
-        sst_factor = qn_cycle_global(c, c.h.outer) ? 1.0 : 0.0;
+        okm[0] = okm[1] = okm[2] = okm[3] = 0;
+        okm[c.h.outer / WAVE] = 1ull << (c.h.outer % WAVE);
+        sst_factor = valid_outer<NM>(c, okm) ? 1.0 : 0.0;
     } else {
         // perform_global_check_qn (Trace.F90:1345-1383)
-        const int pold = count_valid_outer(c, okm);
+        all_outer(c, okm);
+        const int pold = valid_outer<NM>(c, okm);
         global_update(c, gu);
-        const int pnew = count_valid_outer(c, okm);
+        all_outer(c, okm);
+        const int pnew = valid_outer<NM>(c, okm);
         if (pnew <= 0) {
             sst_factor = 0.0;
         } else {
@@ -2950,31 +3131,14 @@ __device__ __attribute__((noinline)) int step_glob(ChainRef ref)
     double *tfc = c.scratch + c.L.kmat, *tfa = tfc + nf * kc;
     int *tkf = reinterpret_cast<int *>(tfa + nf * kc);
     rebuild_flavour_lists(c, tfc, tfa, tkf, nullptr, nullptr);
-    // det(new Delta) * det(old M) (get_InvFullHybr, get_FullLogDet); the old
-    // inverse is gathered into logical order first
-    int *piv = reinterpret_cast<int *>(c.R);
+    // det(new Delta) * det(old M) (get_InvFullHybr, get_FullLogDet)
     double dnl = 0.0, dns = 1.0, dol = 0.0, dos = 1.0;
-    const int ld = c.L.kcap;
-    // LDS work area for the k x k blocks (blocks up to 4 states: the window
-    // segment caches, restarted after this move); HBM scratch otherwise
-    double *wa = nullptr;
-    long wcap = 0;
-    if constexpr (NM <= 4) {
-        wa = c.rk;
-        wcap = 2L * (c.L.sc + 1) * NM * NM;
-        c.h.rk_n = 0;
-        c.h.lb_n = 0;
-    }
     bool sing = false;
     for (int f = 0; f < nf; ++f) {
         const int k = tkf[f];
         if (k > 0) {
-            const bool inl = (long)k * k <= wcap;
-            double *A = inl ? wa : c.scratch;
-            const int lda = inl ? k : ld;
-            build_delta(c, f, k, A, lda, tfc, tfa);
             double l, s;
-            if (!lu_inplace(A, k, lda, l, s, piv)) sing = true;
+            if (!delta_det<NM>(c, f, k, tfc, tfa, l, s)) sing = true;
             dnl += l;
             dns *= s;
         }
@@ -2993,20 +3157,7 @@ __device__ __attribute__((noinline)) int step_glob(ChainRef ref)
             const int k = c.h.kf[f];
             if (k == 0) continue;
             double l, s;
-            if (2L * k * k <= wcap) {
-                double *A = wa, *X = wa + (long)k * k;
-                build_delta(c, f, k, A, k, c.fc, c.fa);
-                lu_inplace(A, k, k, l, s, piv);
-                lu_inverse(A, k, k, piv, X, k);
-                double *Mf = c.mi(f);
-                for (int idx = lane_id(); idx < k * k; idx += WAVE)
-                    Mf[idx % k + (long)(idx / k) * ld] = X[idx];
-                wsync();
-            } else {
-                build_delta(c, f, k, c.scratch, ld, c.fc, c.fa);
-                lu_inplace(c.scratch, k, ld, l, s, piv);
-                lu_inverse(c.scratch, k, ld, piv, c.mi(f), ld);
-            }
+            delta_inverse<NM>(c, f, k, l, s);
         }
         c.h.det_log = dnl;
         c.h.det_sign = dns;
@@ -3079,8 +3230,7 @@ __device__ __attribute__((noinline)) int step_shift(ChainRef ref)
     const int n = c.h.nop, nf = M.nf;
     int first = lower_bound_tau(c.tau, n, dtau);
     if (first == n) first = 0;
-    int s = c.h.outer;
-    for (int i = 0; i < first; ++i) s = c.conn(s, c.code[i], false);
+    const int s = sst_before<NM>(c, first);
     // rotate through the operator scratch area behind the matrix scratch
     double *opscr = c.scratch + c.L.kmat;
     double *old_tau = opscr;
@@ -3300,13 +3450,14 @@ DEV double row_reduce_scatter16(double (&v)[16])
 
 // MeasGtauRem (CTQMC.F90:2252-2440): lanes over (annihilator, creator) pairs,
 // up to four pairs per lane.  G(tau) bins by atomic adds; the Legendre sums run
-// the Bonnet recursion per pair and fold 16 orders at a time with
-// row_reduce_scatter16 into per-lane accumulators (up to 128 orders per pass
-// over the pairs), combined across rows once per flavour.  Kept out of line: inlined into the sweep kernel, the
-// ROCm 7.2 backend emits an invalid V_CMP (src_shared_base operand) for it.
+// the Bonnet recursion of all pairs side by side, fold 16 orders at a time with
+// row_reduce_scatter16 and add them to the chain's sums.  Bound by instruction
+// issue of one wave; the orders are a loop of 16 at a time and not unrolled: the
+// unrolled form was 24 KB of code per flavour that every measurement fetched
+// anew (2-orbital model: 208 K cycles per measurement, 3-orbital 632 K).
 struct GtauArgs {
     int nf, ntau, nleg, kcap;
-    double beta, cfgsign;
+    double beta, rbeta, cfgsign;
     const double *legc;
     const int *kf;
     const double *fc, *fa, *minv;
@@ -3315,132 +3466,96 @@ struct GtauArgs {
     double *mstep, *dstep;   // this measurement's row of Gtau_mean_step / Gtau_mid_step (or null)
 };
 
-// One pass over the pairs of flavour f for the Legendre orders [l0, l0 + 128):
-// every lane takes PPL pairs (p = p0 + lane + 64u), runs their Bonnet
-// recursions side by side and folds the PPL products of each order before the
-// reduce-scatter, so one reduce-scatter serves 64 PPL pairs.
+// the pairs p0 .. p0 + 64 PPL - 1 of flavour f (k of them each way): lane l
+// takes p0 + l + 64 u
 template <int PPL>
-DEV void gtau_pass(const GtauArgs &a, int f, int l0, double (&acc)[8])
+DEV void gtau_pairs(const GtauArgs &a, int f, int k, int p0)
 {
-    constexpr int LPASS = 128, NCH = LPASS / 16;
-    const int ld = a.kcap;
-    const int k = a.kf[f];
+    const int ld = a.kcap, npair = k * k;
     const double *ctl = a.fc + (long)f * a.kcap, *atl = a.fa + (long)f * a.kcap;
     const int *csl = a.fcs + (long)f * a.kcap, *asl = a.fas + (long)f * a.kcap;
     const double *Mf = a.minv + (long)f * a.kcap * a.kcap;
-    const int npair = k * k;
-    const int lend = min(a.nleg, l0 + LPASS);
-    for (int p0 = 0; p0 < npair; p0 += WAVE * PPL) {
-        double Mv[PPL], x[PPL], pl[PPL], plm1[PPL];
+    const float rk = 1.0f / (float)k;
+    double Mv[PPL], x[PPL], pl[PPL], plm1[PPL], ta[PPL], tc[PPL], m[PPL];
 #pragma unroll
-        for (int u = 0; u < PPL; ++u) {
-            const int p = p0 + lane_id() + WAVE * u;
-            Mv[u] = 0.0;
-            x[u] = 0.0;
-            if (p < npair) {
-                const int ai = p / k, ci = p - ai * k;    // annihilator rank, creator rank
-                const double ta = atl[ai], tc = ctl[ci];
-                double m = Mf[csl[ci] + (long)asl[ai] * ld];
-                int idt;
-                if (ta - tc > 0.0) {
-                    idt = (int)((ta - tc) / a.beta * (double)a.ntau) + 1;
-                    x[u] = 2.0 / a.beta * (ta - tc) - 1.0;
-                } else {
-                    idt = (int)((a.beta + ta - tc) / a.beta * (double)a.ntau) + 1;
-                    x[u] = 2.0 / a.beta * (a.beta + ta - tc) - 1.0;
-                    m = -m;
-                }
-                Mv[u] = m * a.cfgsign;
-                if (idt > a.ntau) idt = a.ntau;
-                if (l0 == 0) {
-                    global_add(&a.gtau[(long)f * a.ntau + idt - 1], Mv[u]);
-                    // step-resolved sums (CTQMC.F90:2394-2401): M * cfgsign of
-                    // every pair, and of pairs with |ta - tc| / beta in [0.4, 0.6]
-                    if (a.mstep) global_add(&a.mstep[f], Mv[u] * a.cfgsign);
-                    if (a.dstep) {
-                        const double r = fabs(ta - tc) / a.beta;
-                        if (r >= 0.4 && r <= 0.6) global_add(&a.dstep[f], Mv[u] * a.cfgsign);
-                    }
-                }
+    for (int u = 0; u < PPL; ++u) {
+        const int p = min(p0 + lane_id() + WAVE * u, npair - 1);
+        int ai = (int)((float)p * rk);   // annihilator rank p / k (k <= 4096: off by one at most)
+        ai -= ai * k > p;
+        ai += (ai + 1) * k <= p;
+        const int ci = p - ai * k;       // creator rank
+        ta[u] = atl[ai];
+        tc[u] = ctl[ci];
+        m[u] = Mf[csl[ci] + (long)asl[ai] * ld];
+    }
+#pragma unroll
+    for (int u = 0; u < PPL; ++u) {
+        const bool in = p0 + lane_id() + WAVE * u < npair;
+        const double d = ta[u] - tc[u];
+        const bool fwd = d > 0.0;
+        const double dt = fwd ? d : a.beta + ta[u] - tc[u];
+        // dt / beta by the reciprocal and one correction step
+        double q = dt * a.rbeta;
+        q = fma(fma(-q, a.beta, dt), a.rbeta, q);
+        const int idt = min((int)(q * (double)a.ntau) + 1, a.ntau);
+        x[u] = in ? 2.0 / a.beta * dt - 1.0 : 0.0;
+        Mv[u] = in ? (fwd ? m[u] : -m[u]) * a.cfgsign : 0.0;
+        if (in) {
+            global_add(&a.gtau[(long)f * a.ntau + idt - 1], Mv[u]);
+            // step-resolved sums (CTQMC.F90:2394-2401): M * cfgsign of
+            // every pair, and of pairs with |ta - tc| / beta in [0.4, 0.6]
+            if (a.mstep) global_add(&a.mstep[f], Mv[u] * a.cfgsign);
+            if (a.dstep) {
+                const double r = fabs(d) / a.beta;
+                if (r >= 0.4 && r <= 0.6) global_add(&a.dstep[f], Mv[u] * a.cfgsign);
             }
-            pl[u] = 0.0;
-            plm1[u] = 0.0;
         }
-        // Bonnet recursion from order 0 up to the start of this pass
-        for (int l = 0; l < l0; ++l) {
+        pl[u] = 1.0;
+        plm1[u] = 0.0;
+    }
+    double *gl = a.gleg + (long)f * a.nleg;
+#pragma unroll 1
+    for (int lb = 0; lb < a.nleg; lb += 16) {
+        double v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            // order l = lb + j from pl, then the next: P_{l+1} = c1 x P_l - c2 P_{l-1}
+            const int l = min(lb + j, a.nleg - 1);
+            const double c1 = a.legc[2 * l], c2 = a.legc[2 * l + 1];
+            double sum = 0.0;
 #pragma unroll
             for (int u = 0; u < PPL; ++u) {
-                const double plp1 = l == 0 ? 1.0 : (l == 1 ? x[u] : a.legc[2 * (l - 1)] * x[u] * pl[u] - a.legc[2 * (l - 1) + 1] * plm1[u]);
+                sum = fma(Mv[u], pl[u], sum);
+                const double nx = c1 * x[u] * pl[u] - c2 * plm1[u];
                 plm1[u] = pl[u];
-                pl[u] = plp1;
+                pl[u] = nx;
             }
+            v[j] = sum;
         }
-#pragma unroll
-        for (int q = 0; q < NCH; ++q) {
-            const int lb = l0 + 16 * q;
-            if (lb >= lend) break;
-            double v[16];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int l = lb + j;
-                double sum = 0.0;
-                if (l < lend) {
-                    const double c1 = l >= 2 ? a.legc[2 * (l - 1)] : 0.0, c2 = l >= 2 ? a.legc[2 * (l - 1) + 1] : 0.0;
-#pragma unroll
-                    for (int u = 0; u < PPL; ++u) {
-                        const double plp1 = l == 0 ? 1.0 : (l == 1 ? x[u] : c1 * x[u] * pl[u] - c2 * plm1[u]);
-                        plm1[u] = pl[u];
-                        pl[u] = plp1;
-                        sum = fma(Mv[u], plp1, sum);
-                    }
-                }
-                v[j] = sum;
-            }
-            acc[q] += row_reduce_scatter16(v);
-        }
+        double r = row_reduce_scatter16(v);
+        r += __shfl_xor(r, 16, WAVE);
+        r += __shfl_xor(r, 32, WAVE);
+        if (lane_id() < 16 && lb + lane_id() < a.nleg) global_add(gl + lb + lane_id(), r);
     }
 }
 
-// all flavours; WIDE: flavours of more than 64 pairs take 2 or 4 pairs per lane
-template <bool WIDE>
-DEV double2 gtau_all(const GtauArgs &a)
+__device__ __attribute__((noinline)) double2 meas_gtau(const GtauArgs a)
 {
-    constexpr int LPASS = 128, NCH = LPASS / 16;
     double wflops = 0.0, wbytes = 0.0;
+#pragma unroll 1
     for (int f = 0; f < a.nf; ++f) {
-        const int k = a.kf[f];
+        const int k = uni(a.kf[f]), npair = k * k;
         wflops += (double)k * k * (5.0 * a.nleg + 4.0);
         wbytes += 8.0 * k * k;
-        const int npair = k * k;
-        for (int l0 = 0; l0 < a.nleg; l0 += LPASS) {
-            double acc[NCH];
-#pragma unroll
-            for (int q = 0; q < NCH; ++q) acc[q] = 0.0;
-            if (WIDE && npair > 2 * WAVE) gtau_pass<4>(a, f, l0, acc);
-            else if (WIDE && npair > WAVE) gtau_pass<2>(a, f, l0, acc);
-            else gtau_pass<1>(a, f, l0, acc);
-            // rows -> lanes 0..15, added to the chain's Legendre sums
-#pragma unroll
-            for (int q = 0; q < NCH; ++q) {
-                const int lb = l0 + 16 * q;
-                if (lb >= a.nleg) break;
-                double r = acc[q];
-                r += __shfl_xor(r, 16, WAVE);
-                r += __shfl_xor(r, 32, WAVE);
-                const int l = lb + lane_id();
-                if (lane_id() < 16 && l < a.nleg) a.gleg[(long)f * a.nleg + l] += r;
-            }
-        }
+        int p0 = 0;
+#pragma unroll 1
+        for (; npair - p0 > 2 * WAVE; p0 += 4 * WAVE) gtau_pairs<4>(a, f, k, p0);
+        if (npair - p0 > WAVE) gtau_pairs<2>(a, f, k, p0);
+        else if (npair - p0 > 0) gtau_pairs<1>(a, f, k, p0);
     }
     wsync();
     return make_double2(wflops, wbytes);
 }
-
-// Two out-of-line entry points: the caller's registers saved around the call
-// depend on the callee's footprint, so kernels whose chains stay at a few
-// pairs per flavour (one-state blocks) call the narrow one.
-__device__ __attribute__((noinline)) double2 meas_gtau(const GtauArgs a) { return gtau_all<true>(a); }
-__device__ __attribute__((noinline)) double2 meas_gtau_narrow(const GtauArgs a) { return gtau_all<false>(a); }
 
 // gtau_accum%add() of the binning accumulator (AccumGtau = 2,
 // autocorracc_add, Accumulators.F90:298-340): this measurement's G(tau) bins
@@ -3965,7 +4080,7 @@ DEV Ctx make_ctx(char *chains, int chain, CArgs args, char *lds)
         unsigned char *kb = (unsigned char *)(lds_b *)(lds_c *)(lds + L.l_keys);
         for (int q = lane_id(); q < 512; q += WAVE) kb[q] = M.dkey ? M.keys[q] : 255;
         WalkEnv &e = s_wenv;
-        e.ops = M.ops;
+        e.opsx = M.opsx;
         e.tr = (const lds_i4 *)c.tr;
         e.ev = (const lds_d *)c.ev;
         e.keys = (const lds_b *)kb;
@@ -3978,7 +4093,6 @@ DEV Ctx make_ctx(char *chains, int chain, CArgs args, char *lds)
         }
         e.ncol = 4 * M.nb;
         e.dkey = M.dkey;
-        e.zero = (int)M.nops;
         e.nkmax = (M.nmax + 3) / 4;
     }
     s_wenv.egs = M.egs;
@@ -4037,7 +4151,7 @@ __device__ __attribute__((noinline)) void measure(ChainRef r)
     if (M.meas_dm) meas_dm<NM>(c, reinterpret_cast<double *>(base + L.dm));
     GtauArgs ga;
     ga.nf = M.nf, ga.ntau = M.ntau, ga.nleg = M.nleg, ga.kcap = L.kcap;
-    ga.beta = M.beta, ga.cfgsign = c.h.cfgsign, ga.legc = c.legc;
+    ga.beta = M.beta, ga.rbeta = M.rbeta, ga.cfgsign = c.h.cfgsign, ga.legc = c.legc;
     ga.kf = c.h.kf, ga.fc = c.fc, ga.fa = c.fa, ga.minv = c.minv, ga.fcs = c.fcs, ga.fas = c.fas;
     ga.gtau = (M.accum == 2 || SCORE) ? gbuf : gtau, ga.gleg = gleg;
     const long long mi = c.h.cnt_meas - 1;   // g_inmeas - 1
@@ -4047,7 +4161,7 @@ __device__ __attribute__((noinline)) void measure(ChainRef r)
     // sign_step is set when the configuration has a pair (CTQMC.F90:2402)
     if (st && M.step_sign && c.h.nop > 0 && lane_id() == 0)
         reinterpret_cast<double *>(base + L.sstep)[mi] = c.h.cfgsign;
-    const double2 wk = NM == 1 ? meas_gtau_narrow(ga) : meas_gtau(ga);
+    const double2 wk = meas_gtau(ga);
     c.work(wk.x, wk.y);
     if constexpr (SCORE) score_pass(score_args(c, gbuf, gtau), nullptr, true);
     if (M.accum == 2)
@@ -4506,18 +4620,15 @@ __global__ void __launch_bounds__(WAVE) setconfig_kernel(DevModel M, ChainLayout
     if (T.S == 0.0 && !(T.lg > -DBL_MAX)) c.h.err = 5;   // W2D_ERR_ZERO_TRACE: broken quantum numbers
     keep_trace<NM>(c, T);
     rebuild_flavour_lists(c, c.fc, c.fa, c.h.kf, c.fcs, c.fas);
-    int *piv = reinterpret_cast<int *>(c.R);
     double dl = 0.0, dsg = 1.0;
     for (int f = 0; f < c.M.nf; ++f) {
         const int k = c.h.kf[f];
         if (k == 0) continue;
-        build_delta(c, f, k, c.scratch, c.L.kcap, c.fc, c.fa);
         double l, sg;
-        if (!lu_inplace(c.scratch, k, c.L.kcap, l, sg, piv)) {
+        if (!delta_inverse<NM>(c, f, k, l, sg)) {
             c.h.err = ERR_SING;
             break;
         }
-        lu_inverse(c.scratch, k, c.L.kcap, piv, c.mi(f), c.L.kcap);
         dl += l;
         dsg *= sg;
     }

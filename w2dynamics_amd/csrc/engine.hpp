@@ -28,9 +28,14 @@ struct DevModel {
     const double *ops16;
     const int *opoff16;
     const double *ops, *evals, *ftau;   // ftau[f][nftau]
+    // the blocks once more for the matrix-instruction walks on blocks of up to
+    // 16 states: max(3, ceil(nmax / 4)) k-steps of 64 doubles each, lane l of
+    // step e entry (l % 16, 4 e + l / 16), zero beyond the block; trans.w names
+    // the block
+    const double *opsx;
     const long *dmoff;                  // block-diagonal density-matrix offsets
     const double *legc;                 // Bonnet coefficients (2l+1)/(l+1), l/(l+1) per l
-    const int4 *trans;                  // per (superstate, operator): target, its size, block offset, its energies offset
+    const int4 *trans;                  // per (superstate, operator): target, its size, block offset, number of the block
     long dmsize;
     long nops;                          // size of ops
     double p_shift, p_glob, p_outer, p_4op;
