@@ -26,6 +26,9 @@ struct w2d_ctqmc {
     w2d::ChainLayout L{};
     int nchains = 0, nm = 0, device = 0, kcap = 0, ntau = 0, nleg = 0, maxhisto = 0;
     int lds_max = 64 * 1024;   // LDS bytes a workgroup may allocate on this device
+    int lds_cu = 64 * 1024;    // LDS bytes of a compute unit
+    int ncu = 1;               // compute units
+    bool full_lists = false;   // LDS operator lists at the window's full share (a chain outgrew shorter ones)
     bool moved = false;        // chains have taken steps since create
     int nwin_alloc = 0;
     uint32_t seed0 = 0;
@@ -96,6 +99,8 @@ long align256(long x) { return (x + 255) / 256 * 256; }
 
 constexpr int KCAP_MAX = 4096;   // pairs per flavour a chain may grow to
 constexpr int ACCPAIR_BINS_MAX = 1024;   // accepted-pair histogram bins (NAccPair) at most, beyond Ntau
+constexpr int SIMDS = 4;                 // per compute unit; a wave of the sweep kernel each
+constexpr long LDS_GRAIN = 1280;         // bytes LDS is handed out in
 constexpr int SEG_CACHE = 128;           // window operators the segment caches of blocks above 4 states cover
 constexpr int APT_CAP = 65536;           // accepted-pair distances a calibration list holds at most
 constexpr int GIW_NIW_MAX = 1 << 20;     // Matsubara frequencies of MeasGiw at most
@@ -221,7 +226,7 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     L.bndlog = take((long)nbound * 8);
     L.bndsst = take((long)nbound * 4);
     L.part = take(2L * nm * 8 + 16);
-    L.kwork = take(nm > 16 ? 2L * nm * nm * 8 : 8);
+    L.kwork = take(nm > 4 ? 2L * nm * nm * 8 : 8);
     const int nth = h->dm.ntheta;
     L.dwork = take(nth > 0 ? ((4L + 3L * nth) * nm * nm + nm) * 8 : 8);
     L.grk = take(nm > 4 && nm <= 16 ? (SEG_CACHE + 1) * 2048L : 8);
@@ -266,56 +271,80 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     };
     // list capacity: the window's share of the operator capacity with a margin
     const int nwin = std::max(nbound - 2, 1);
-    const int lc = (int)std::min<long>(std::min<long>(L.cap + 2, 1024),
-                                       std::max<long>(64, 2L * L.cap / (nwin + 1) + 32));
-    L.lcap_lds = lc;
-    L.l_mt = lds(624 * 4);
-    L.l_sz = lds((long)m.nsst * 4);
-    L.l_off = lds((long)m.nsst * 4);
-    // transition records and energies: LDS for blocks up to 16 states, HBM
-    // above (there the block products dominate and LDS buys chains per CU)
-    L.l_tr = nm <= 16 ? lds((long)m.nsst * m.nbands * 4 * 16) : -1;
-    L.l_ev = nm <= 16 ? lds((long)m.nstates * 8) : -1;
-    L.l_wtau = lds((long)lc * 8);
-    L.l_wcode = lds((long)lc * 4);
-    L.l_ttau = lds((long)lc * 8);
-    L.l_tcode = lds((long)lc * 4);
-    L.l_pc = lds((long)lc * 4);
-    L.l_dvec = lds((long)nm * 8);
-    const long qn = std::max<long>(kc + 2, m.nsst + 1);
-    L.l_q = lds(qn * 8);
-    L.l_r = lds(qn * 8);
-    L.l_col = lds((long)(kc + 2) * 8);
-    L.l_row = lds((long)(kc + 2) * 8);
-    L.l_pl = lds((long)(2 * nm + 2) * 8);
-    L.l_k = nm <= 16 ? lds(2L * nm * nm * 8) : -1;
-    L.l_strip = nm > 16 ? lds(128L * 16 * 8) : -1;
-    L.l_legc = lds(2L * std::max(h->nleg, 1) * 8);
-    // walks on blocks of up to 16 states: superstate keys and records;
-    // propagators of 16 operators
-    L.l_keys = nm <= 16 ? lds(512) : -1;
-    L.l_sinfo = nm <= 16 ? lds(16L * m.nsst) : -1;
-    L.l_qa = nm > 4 && nm <= 16 ? lds(16L * 16 * 8) : -1;
-    // window segment caches: state matrices in LDS for blocks of up to 4
-    // states, in the chain block above (2 KB each)
-    L.sc = nm <= 4 ? std::min(64, lc - 2) : nm <= 16 ? std::min(SEG_CACHE, lc - 2) : 0;
-    if (L.sc > 0) {
-        if (nm <= 4) {
-            L.l_rk = lds((long)(L.sc + 1) * nm * nm * 8);
-            L.l_lb = lds((long)(L.sc + 1) * nm * nm * 8);
+    const int lfull = (int)std::min<long>(std::min<long>(L.cap + 2, 1024),
+                                          std::max<long>(64, 2L * L.cap / (nwin + 1) + 32));
+    auto carve = [&](int lc) {
+        q = 0;
+        L.lcap_lds = lc;
+        L.l_mt = lds(624 * 4);
+        L.l_sz = lds((long)m.nsst * 4);
+        L.l_off = lds((long)m.nsst * 4);
+        // transition records and energies: LDS for blocks up to 16 states, HBM
+        // above (there the block products dominate and LDS buys chains per CU)
+        L.l_tr = nm <= 16 ? lds((long)m.nsst * m.nbands * 4 * 16) : -1;
+        L.l_ev = nm <= 16 ? lds((long)m.nstates * 8) : -1;
+        L.l_wtau = lds((long)lc * 8);
+        L.l_wcode = lds((long)lc * 4);
+        L.l_ttau = lds((long)lc * 8);
+        L.l_tcode = lds((long)lc * 4);
+        L.l_pc = lds((long)lc * 4);
+        L.l_dvec = lds((long)nm * 8);
+        const long qn = std::max<long>(kc + 2, m.nsst + 1);
+        L.l_q = lds(qn * 8);
+        L.l_r = lds(qn * 8);
+        L.l_col = lds((long)(kc + 2) * 8);
+        L.l_row = lds((long)(kc + 2) * 8);
+        L.l_pl = lds((long)(2 * nm + 2) * 8);
+        L.l_k = nm <= 4 ? lds(2L * nm * nm * 8) : -1;
+        L.l_strip = nm > 16 ? lds(128L * 16 * 8) : -1;
+        L.l_legc = lds(2L * std::max(h->nleg, 1) * 8);
+        // walks on blocks of up to 16 states: superstate keys and records;
+        // propagators of 16 operators
+        L.l_keys = nm <= 16 ? lds(512) : -1;
+        L.l_sinfo = nm <= 16 ? lds(16L * m.nsst) : -1;
+        L.l_qa = nm > 4 && nm <= 16 ? lds(16L * 16 * 8) : -1;
+        // window segment caches: state matrices in LDS for blocks of up to 4
+        // states, in the chain block above (2 KB each)
+        L.sc = nm <= 4 ? std::min(64, lc - 2) : nm <= 16 ? std::min(SEG_CACHE, lc - 2) : 0;
+        if (L.sc > 0) {
+            if (nm <= 4) {
+                L.l_rk = lds((long)(L.sc + 1) * nm * nm * 8);
+                L.l_lb = lds((long)(L.sc + 1) * nm * nm * 8);
+            }
+            L.l_rkx = lds((long)(L.sc + 1) * 8);
+            L.l_lbx = lds((long)(L.sc + 1) * 8);
+            L.l_rks = lds((long)(L.sc + 1) * 4);
+            L.l_lbs = lds((long)(L.sc + 1) * 4);
+        } else {
+            L.l_rk = L.l_lb = L.l_rkx = L.l_lbx = L.l_rks = L.l_lbs = -1;
         }
-        L.l_rkx = lds((long)(L.sc + 1) * 8);
-        L.l_lbx = lds((long)(L.sc + 1) * 8);
-        L.l_rks = lds((long)(L.sc + 1) * 4);
-        L.l_lbs = lds((long)(L.sc + 1) * 4);
-    } else {
-        L.l_rk = L.l_lb = L.l_rkx = L.l_lbx = L.l_rks = L.l_lbs = -1;
+        // operator blocks: in LDS for blocks of up to 4 states; above, the matrix-
+        // core walks read them from global memory (the table is shared by all
+        // chains and prefetched, and LDS buys chains per CU)
+        L.l_ops = nm <= 4 ? lds((long)m.ops.size() * 8) : -1;
+        L.lds_bytes = q;
+    };
+    carve(lfull);
+    // The lists are the LDS that grows with the capacity, and a chain's window
+    // rarely holds more than a third of its share.  Where the full lists keep
+    // chains of the batch from being resident (a wave per SIMD), they are cut as
+    // far as that takes, down to a third; a chain that outgrows them halts and
+    // the lists are laid out in full.  3-orbital model, capacity 384: 800 -> 488
+    // operators, 51 -> 39 KB, four chains per compute unit instead of three;
+    // 1024 chains, 2 sweeps 10.9 -> 6.2 ms.
+    if (nm <= 16 && !h->full_lists) {
+        const int lmin = std::max(64, (lfull - 32) / 3 + 32);
+        const int want = std::min((h->nchains + h->ncu - 1) / h->ncu, SIMDS);
+        const long fixed = sizeof(w2d::WalkEnv) + sizeof(w2d::ChainHdr) + 64;
+        auto room = [&](int n) { return h->lds_cu / n / LDS_GRAIN * LDS_GRAIN - fixed; };
+        for (int n = want; n > 1 && q > room(n); --n) {
+            const int lc = std::min<long>(lfull, lfull - (q - room(n) + 27) / 28 - 4);
+            if (lc < lmin) continue;
+            carve(lc);
+            L.lcap_short = lc < lfull;
+            break;
+        }
     }
-    // operator blocks: in LDS for blocks of up to 4 states; above, the matrix-
-    // core walks read them from global memory (the table is shared by all
-    // chains and prefetched, and LDS buys chains per CU)
-    L.l_ops = nm <= 4 ? lds((long)m.ops.size() * 8) : -1;
-    L.lds_bytes = q;
     if (L.lds_bytes > h->lds_max) return W2D_ERR_CAPACITY;
     L.hdrs = L.stride * h->nchains;
     return W2D_OK;
@@ -573,23 +602,34 @@ void launch_range(w2d_ctqmc *h, long long from, long long target, long long ncor
     }
 }
 
+// whether the chain's orders fit one more pair (its window may not fit the LDS lists)
+bool has_room(const w2d_ctqmc *h, const ChainHdr &x)
+{
+    for (int f = 0; f < 2 * h->model.nbands; ++f)
+        if (x.kf[f] + 1 > h->L.kcap) return false;
+    return x.nop + 2 <= h->L.cap;
+}
+
 // After a pass: chains halted for room get a larger capacity and continue;
 // returns whether another pass is needed.  Chains that cannot grow further
 // are stopped with W2D_ERR_CAPACITY (their results are left out).
 int resume_halted(w2d_ctqmc *h, std::vector<ChainHdr> &hd, long long &from, bool &again)
 {
     again = false;
-    bool cap = false;
+    bool cap = false, lists = h->L.lcap_short != 0;
     from = -1;
     for (const auto &x : hd) {
         if (x.halt == w2d::HALT_ABORT) h->aborted = 1;
         if (x.halt == w2d::HALT_CAP && x.err == 0) {
             cap = true;
+            lists = lists && has_room(h, x);
             from = from < 0 ? x.pos : std::min(from, x.pos);
         }
     }
     if (!cap || h->aborted) return W2D_OK;
-    const int st = regrow(h);
+    // where only shortened lists ran out: their full share first
+    if (lists) h->full_lists = true;
+    const int st = lists ? relayout(h, h->kcap, h->L.nbound) : regrow(h);
     if (st && st != W2D_ERR_CAPACITY) return st;
     for (auto &x : hd)
         if (x.halt == w2d::HALT_CAP) {
@@ -1045,6 +1085,8 @@ int w2d_ctqmc_create(const char *params, int nbands, int nftau, const double *u_
     h->nm_min = h->nm;
     HIPCHK(hipSetDevice(device));
     HIPCHK(hipDeviceGetAttribute(&h->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+    HIPCHK(hipDeviceGetAttribute(&h->lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device));
+    HIPCHK(hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, device));
     HIPCHK(hipStreamCreate(&h->stream));
     HIPCHK(hipEventCreate(&h->ev0));
     HIPCHK(hipEventCreate(&h->ev1));

@@ -482,7 +482,7 @@ DEV Ctx attach(ChainRef r)
     c.legc = lds_ptr<double>(e.legc);
     // work matrices: LDS for blocks up to 16 states (decided at compile time so
     // that their accesses are LDS instructions, not generic ones), HBM above
-    if constexpr (NM <= 16) c.K0 = lds_ptr<double>(e.k);
+    if constexpr (NM <= 4) c.K0 = lds_ptr<double>(e.k);
     else c.K0 = reinterpret_cast<double *>(base + L.kwork);
     c.K1 = c.K0 + (long)NM * NM;
     c.strip = NM > 16 ? lds_ptr<double>(e.strip) : nullptr;

@@ -95,7 +95,7 @@ struct ChainLayout {
     long bnd;             // double[nbound][nmax*nmax]: bras at window boundaries
     long bndlog, bndsst;  // double[nbound], int[nbound]
     long part;            // double[2*nmax]: part traces (log, sign)
-    long kwork;           // double[2][nmax*nmax]: work matrices (large blocks)
+    long kwork;           // double[2][nmax*nmax]: work matrices (blocks above 4 states)
     long ltau, lcode;     // trial operator list (double[lcap], int[lcap])
     long gtau, gleg, dm, histo, outer; // accumulators
     long gbuf, gacc;      // AccumGtau = 2: one measurement's G(tau); binning levels [3][nlev][nf*ntau]
@@ -116,6 +116,7 @@ struct ChainLayout {
     long l_mt, l_sz, l_off, l_ev, l_ops, l_wtau, l_wcode, l_ttau, l_tcode;
     long l_dvec, l_q, l_r, l_col, l_row, l_pl, l_k, l_legc, l_tr, l_pc, lds_bytes;
     int lcap_lds;         // operators each LDS list holds (window list, trial list)
+    int lcap_short;       // fewer than the window's full share (more chains resident)
     // prefix kets / suffix bras of the window's operators (blocks up to 16 states)
     int sc;               // window operators they cover (0: not kept)
     long l_rk, l_lb, l_rkx, l_lbx, l_rks, l_lbs, l_qa, l_keys, l_sinfo;
