@@ -2122,51 +2122,70 @@ struct MatLanes {
     }
 };
 
-// In the block loops below, eight and then four columns (or rows) are loaded
-// together while every lane group has them; the last ones go one by one, masked.
-// M(i,j) += (a col(i)) row(j)
-DEV void rank1(Ctx &c, double *Mf, int k, const MatLanes &ml, double a, const double *col, const double *row)
+// The block loops below are chains of memory round trips (the inverses of a
+// batch lie in HBM or the last-level cache): f(c) steps of `step` columns each,
+// N at a time with all their loads ahead of their arithmetic, as long as every
+// lane group has them; the last ones, at most four, go together, their column
+// clamped to the last one and masked.
+template <int N, typename Body>
+DEV int batches(int u, int full, const Body &body)
 {
-    const int ld = c.L.kcap, full = k / ml.step;   // columns that every lane group has
+    for (; u + N <= full; u += N) body(std::integral_constant<int, N>(), u);
+    return u;
+}
+
+template <typename Body, typename Tail>
+DEV void in_batches(int k, const MatLanes &ml, const Body &body, const Tail &tail)
+{
+    const int full = k / ml.step;   // steps that every lane group has
+    int u = 0;
+    if (ml.step == 1) u = batches<16>(u, full, body);
+    u = batches<8>(u, full, body);
+    u = batches<4>(u, full, body);
+    if (u * ml.step < k) tail(u);
+}
+
+// M(i,j) += (a col(i)) row(j)
+DEV void rank1(Ctx &c, double *Mf, int k, double a, const double *col, const double *row)
+{
+    const int ld = c.L.kcap;
     for (int i0 = 0; i0 < k; i0 += WAVE) {
+        const MatLanes ml(k - i0);
         const int i = i0 + ml.i;
         const bool in = i < k;
         const double ci = in ? a * col[i] : 0.0;
         double *p = Mf + (in ? i : 0) + (long)ml.g * ld;
         const double *q = row + ml.g;
-        int u = 0;
-        for (; u + 8 <= full; u += 8) {
-            double m[8], r[8];
+        const long ps = (long)ml.step * ld;
+        in_batches(
+            k, ml,
+            [&](auto n, int) {
+                constexpr int N = decltype(n)::value;
+                double m[N], r[N];
 #pragma unroll
-            for (int v = 0; v < 8; ++v) m[v] = p[(long)v * ml.step * ld];
+                for (int v = 0; v < N; ++v) m[v] = p[v * ps];
 #pragma unroll
-            for (int v = 0; v < 8; ++v) r[v] = q[v * ml.step];
-            if (in) {
+                for (int v = 0; v < N; ++v) r[v] = q[v * ml.step];
+                if (in) {
 #pragma unroll
-                for (int v = 0; v < 8; ++v) p[(long)v * ml.step * ld] = fma(ci, r[v], m[v]);
-            }
-            p += (long)8 * ml.step * ld;
-            q += 8 * ml.step;
-        }
-        if (u + 4 <= full) {
-            double m[4], r[4];
+                    for (int v = 0; v < N; ++v) p[v * ps] = fma(ci, r[v], m[v]);
+                }
+                p += N * ps;
+                q += N * ml.step;
+            },
+            [&](int u) {
+                const int left = k - 1 - (u * ml.step + ml.g);   // columns behind this one
+                double m[4], r[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) m[v] = p[(long)v * ml.step * ld];
+                for (int v = 0; v < 4; ++v) {
+                    const int d = min(v * ml.step, left);
+                    m[v] = p[(long)d * ld];
+                    r[v] = q[d];
+                }
 #pragma unroll
-            for (int v = 0; v < 4; ++v) r[v] = q[v * ml.step];
-            if (in) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) p[(long)v * ml.step * ld] = fma(ci, r[v], m[v]);
-            }
-            p += (long)4 * ml.step * ld;
-            q += 4 * ml.step;
-            u += 4;
-        }
-        for (; u <= full; ++u) {
-            if (in && u * ml.step + ml.g < k) *p = fma(ci, *q, *p);
-            p += (long)ml.step * ld;
-            q += ml.step;
-        }
+                for (int v = 0; v < 4; ++v)
+                    if (in && v * ml.step <= left) p[v * ps] = fma(ci, r[v], m[v]);
+            });
     }
 }
 
@@ -2174,39 +2193,38 @@ DEV void rank1(Ctx &c, double *Mf, int k, const MatLanes &ml, double a, const do
 DEV double detrat_add(Ctx &c, const double *Mf, int k)
 {
     const int ld = c.L.kcap;
-    const MatLanes ml(k);
-    const int full = k / ml.step;
     double part = 0.0;
     for (int i0 = 0; i0 < k; i0 += WAVE) {
+        const MatLanes ml(k - i0);
         const int i = i0 + ml.i;
         const bool in = i < k;
         const double *p = Mf + (in ? i : 0) + (long)ml.g * ld, *q = c.Q + ml.g;
+        const long ps = (long)ml.step * ld;
         double acc = 0.0;
-        int u = 0;
-        for (; u + 8 <= full; u += 8) {
-            double m[8];
+        in_batches(
+            k, ml,
+            [&](auto n, int) {
+                constexpr int N = decltype(n)::value;
+                double m[N];
 #pragma unroll
-            for (int v = 0; v < 8; ++v) m[v] = p[(long)v * ml.step * ld];
+                for (int v = 0; v < N; ++v) m[v] = p[v * ps];
 #pragma unroll
-            for (int v = 0; v < 8; ++v) acc = fma(m[v], q[v * ml.step], acc);
-            p += (long)8 * ml.step * ld;
-            q += 8 * ml.step;
-        }
-        if (u + 4 <= full) {
-            double m[4];
+                for (int v = 0; v < N; ++v) acc = fma(m[v], q[v * ml.step], acc);
+                p += N * ps;
+                q += N * ml.step;
+            },
+            [&](int u) {
+                const int left = k - 1 - (u * ml.step + ml.g);
+                double m[4], r[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) m[v] = p[(long)v * ml.step * ld];
+                for (int v = 0; v < 4; ++v) {
+                    const int d = min(v * ml.step, left);
+                    m[v] = p[(long)d * ld];
+                    r[v] = v * ml.step <= left ? q[d] : 0.0;
+                }
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc = fma(m[v], q[v * ml.step], acc);
-            p += (long)4 * ml.step * ld;
-            q += 4 * ml.step;
-            u += 4;
-        }
-        for (; u <= full; ++u) {
-            if (u * ml.step + ml.g < k) acc = fma(*p, *q, acc);
-            p += (long)ml.step * ld;
-            q += ml.step;
-        }
+                for (int v = 0; v < 4; ++v) acc = fma(m[v], r[v], acc);
+            });
         acc = ml.rows(acc);
         if (in && ml.g == 0) {
             c.colb[i] = acc;
@@ -2228,43 +2246,41 @@ DEV void mat_add_phys(Ctx &c, double *Mf, int k, double dr)
     const int l = lane_id();
     double *col = c.colb, *row = c.rowb;
     // columns of M against R: the lane's column is contiguous
-    const MatLanes ml(k);
-    const int full = k / ml.step;
     for (int j0 = 0; j0 < k; j0 += WAVE) {
+        const MatLanes ml(k - j0);
         const int j = j0 + ml.i;
         const double *p = Mf + (long)min(j, k - 1) * ld + ml.g, *r = c.R + ml.g;
         double v = 0.0;
-        int u = 0;
-        for (; u + 8 <= full; u += 8) {
-            double m[8];
+        in_batches(
+            k, ml,
+            [&](auto n, int) {
+                constexpr int N = decltype(n)::value;
+                double m[N];
 #pragma unroll
-            for (int w = 0; w < 8; ++w) m[w] = p[w * ml.step];
+                for (int w = 0; w < N; ++w) m[w] = p[w * ml.step];
 #pragma unroll
-            for (int w = 0; w < 8; ++w) v = fma(r[w * ml.step], m[w], v);
-            p += 8 * ml.step;
-            r += 8 * ml.step;
-        }
-        if (u + 4 <= full) {
-            double m[4];
+                for (int w = 0; w < N; ++w) v = fma(r[w * ml.step], m[w], v);
+                p += N * ml.step;
+                r += N * ml.step;
+            },
+            [&](int u) {
+                const int left = k - 1 - (u * ml.step + ml.g);
+                double m[4], q[4];
 #pragma unroll
-            for (int w = 0; w < 4; ++w) m[w] = p[w * ml.step];
+                for (int w = 0; w < 4; ++w) {
+                    const int d = min(w * ml.step, left);
+                    m[w] = p[d];
+                    q[w] = w * ml.step <= left ? r[d] : 0.0;
+                }
 #pragma unroll
-            for (int w = 0; w < 4; ++w) v = fma(r[w * ml.step], m[w], v);
-            p += 4 * ml.step;
-            r += 4 * ml.step;
-            u += 4;
-        }
-        for (; u <= full; ++u) {
-            if (u * ml.step + ml.g < k) v = fma(*r, *p, v);
-            p += ml.step;
-            r += ml.step;
-        }
+                for (int w = 0; w < 4; ++w) v = fma(q[w], m[w], v);
+            });
         v = ml.rows(v);
         if (j < k && ml.g == 0) row[j] = -v / dr;
     }
     for (int i = l; i < k; i += WAVE) col[i] = -col[i] / dr;
     wsync();
-    rank1(c, Mf, k, ml, dr, col, row);
+    rank1(c, Mf, k, dr, col, row);
     for (int i = l; i < k; i += WAVE) {
         Mf[i + (long)k * ld] = col[i];
         Mf[k + (long)i * ld] = row[i];
@@ -2287,7 +2303,7 @@ DEV void mat_rem_phys(Ctx &c, double *Mf, int k, int sc, int sa)
         rowp[i] = Mf[sc + (long)i * ld];
     }
     wsync();
-    rank1(c, Mf, k, MatLanes(k), -(1.0 / rowp[sa]), colp, rowp);
+    rank1(c, Mf, k, -(1.0 / rowp[sa]), colp, rowp);
     wsync();
     const int last = k - 1;
     if (sc != last) {
