@@ -161,12 +161,6 @@ extern "C" void w2d_signal_handler(int)
     }
 }
 
-void seed_mt(uint32_t *mt, uint32_t s)
-{
-    mt[0] = s;
-    for (int i = 1; i < 624; ++i) mt[i] = 1812433253u * (mt[i - 1] ^ (mt[i - 1] >> 30)) + (uint32_t)i;
-}
-
 // init_window (Trace.F90:1608-1646) on a host copy of the header
 void init_window(ChainHdr &hd, double tdm, double beta)
 {
@@ -423,7 +417,7 @@ void launch_init(w2d_ctqmc *h)
 {
     allow_lds(w2d::init_kernel<NM>, h);
     hipLaunchKernelGGL(w2d::init_kernel<NM>, dim3(h->nchains), dim3(w2d::WAVE), (unsigned)h->L.lds_bytes, h->stream, h->dm, h->L,
-                       h->chains);
+                       h->chains, h->seed0);
 }
 
 // LDS attribute of the sweep kernels (set outside any stream capture)
@@ -509,8 +503,10 @@ int read_headers(w2d_ctqmc *h, std::vector<ChainHdr> &hd)
 
 int write_headers(w2d_ctqmc *h, const std::vector<ChainHdr> &hd)
 {
-    HIPCHK(hipMemcpy(h->chains + h->L.hdrs, hd.data(), sizeof(ChainHdr) * (size_t)h->nchains,
-                     hipMemcpyHostToDevice));
+    const size_t n = sizeof(ChainHdr) * (size_t)h->nchains;
+    std::memcpy(h->hdr_pinned, hd.data(), n);
+    HIPCHK(hipMemcpyAsync(h->chains + h->L.hdrs, h->hdr_pinned, n, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
     return W2D_OK;
 }
 
@@ -521,12 +517,11 @@ int first_error(const std::vector<ChainHdr> &hd)
     return W2D_OK;
 }
 
-// (re)initialise every chain: seeded MT state, empty configuration, window from
-// the TaudiffMax parameter, then the initial outer-superstate draw on the GPU
+// (re)initialise every chain: empty configuration, window from the TaudiffMax
+// parameter; random stream and initial outer superstate on the GPU
 int init_chains(w2d_ctqmc *h)
 {
     std::vector<ChainHdr> hds(h->nchains);
-    std::vector<uint32_t> mt(624L * h->nchains);
     for (int c = 0; c < h->nchains; ++c) {
         ChainHdr &hd = hds[c];
         std::memset(&hd, 0, sizeof(hd));
@@ -540,12 +535,9 @@ int init_chains(w2d_ctqmc *h)
         hd.apt_index = 1;
         hd.apt_n = 0;
         init_window(hd, h->taudiff_param, h->beta);
-        seed_mt(mt.data() + 624L * c, h->seed0 + (uint32_t)c);
     }
     int st0 = write_headers(h, hds);
     if (st0) return st0;
-    HIPCHK(hipMemcpy2D(h->chains + h->L.mt, (size_t)h->L.stride, mt.data(), 624 * 4, 624 * 4,
-                       (size_t)h->nchains, hipMemcpyHostToDevice));
     DISPATCH(launch_init, h);
     HIPCHK(hipGetLastError());
     std::vector<ChainHdr> hd;

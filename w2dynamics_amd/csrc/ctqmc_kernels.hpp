@@ -4595,13 +4595,23 @@ __global__ void __launch_bounds__(64) group_scalars_kernel(const ChainHdr *hdrs,
     used[g] = n;
 }
 
-// Initial state of every chain: empty configuration, initial outer superstate
-// drawn proportional to the empty traces (init_Trace, Trace.F90:640-670).
+// Initial state of every chain: random stream of seed seed0 + chain, empty
+// configuration, initial outer superstate drawn proportional to the empty traces
+// (init_Trace, Trace.F90:640-670).  The stream is seeded here (mt19937's initial
+// recurrence, uniform over the wave: 623 steps of four scalar instructions, 8 us
+// for all chains at once): drawn up on the host, its upload as a strided copy
+// from pageable memory cost 2 ms of a create of 256 chains.
 template <int NM>
-__global__ void __launch_bounds__(WAVE) init_kernel(DevModel M, ChainLayout L, char *chains)
+__global__ void __launch_bounds__(WAVE) init_kernel(DevModel M, ChainLayout L, char *chains, uint32_t seed0)
 {
     extern __shared__ __align__(16) char lds[];
     Ctx c = make_ctx<NM>(chains, (int)blockIdx.x, (CArgs)__builtin_amdgcn_kernarg_segment_ptr(), lds);
+    uint32_t x = seed0 + blockIdx.x;
+    for (int i = 0; i < 624; ++i) {
+        if (i > 0) x = 1812433253u * (x ^ (x >> 30)) + (uint32_t)i;
+        if (lane_id() == 0) c.rng.mt[i] = x;
+    }
+    wsync();
     rng_open(c.rng);
     choose_outer<NM>(c);
     rng_close(c.rng);
