@@ -595,14 +595,10 @@ def pooled_estimate(sums: dict, nb: int, beta: float, ntau: int, nleg: int, mode
         for k in est:
             out[k + "_err"] = np.full_like(out[k], np.nan, dtype=float)
         return out
-    jk = {k: [] for k in est}
-    for i in range(n):
-        part = {k: tot[k] - np.asarray(sums[k], dtype=float)[i][None] for k in keys}
-        r = normalise(part, nb, beta, ntau, nleg, model)
-        for k in est:
-            jk[k].append(np.asarray(r[k])[0])
-    for k in est:
-        a = np.array(jk[k])
+    # every leave-one-out sample in one normalisation
+    parts = {k: tot[k] - np.asarray(sums[k], dtype=float) for k in keys}
+    for k, a in normalise(parts, nb, beta, ntau, nleg, model).items():
+        a = np.asarray(a)
         out[k + "_err"] = np.sqrt((n - 1) / n * (np.abs(a - a.mean(0)) ** 2).sum(0))
     out["nchains_groups"] = n
     return out
