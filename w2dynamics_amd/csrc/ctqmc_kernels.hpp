@@ -356,6 +356,7 @@ struct WalkEnv {
     int ncol;               // operators per superstate (4 nb)
     int dkey;               // key change by a creator of spin 0 | of spin 1 << 8; 0: no such keys
     int np;                 // removable pairs of the window
+    int k0;                 // key of the superstate at the window's lower edge (with the pair counts)
     int ready;              // window list valid and room for any move; cleared by whatever changes that
     int nkmax;              // matrix-instruction steps of the largest block
     int no;                 // states of the outer superstate (valid while ready)
@@ -2002,20 +2003,76 @@ __device__ __attribute__((noinline)) Proposal trace_proposal(ChainRef r, int nw_
     return p;
 }
 
+// change of a superstate's key by an operator (superstate_keys)
+DEV int key_delta(int dkey, int code)
+{
+    const int d = (int)(signed char)(op_spin(code) ? dkey >> 8 : dkey);
+    return op_ca(code) == 1 ? d : -d;
+}
+
 // ---------------------------------------------------------------------------
 // removable pairs (ensure_valid_NPairs_diag, Trace.F90:1769-1810): for every
 // window operator the later operators of its flavour and the other type no
 // further than taudiff_max behind it.  pc[j] holds the counts of the first j+1
 // window operators together, so that the total is known and the pick of a
 // removal is one comparison per lane; kept until the window list changes.
+//
+// The upper 8 bits of pc[j] are the key of the superstate behind operator j (at
+// most 2^19 pairs in a list of 1024): an operator pair put in or taken out
+// shifts the keys between its two places by its first operator's change and
+// leaves the others, so whether a proposal breaks quantum numbers is a look-up
+// per operator between them, before any walk (blocked).  Three to five proposals in
+// ten end there; the walk found out only after the segment caches were extended
+// for it (2-orbital model 7 K cycles; the look-up is three LDS round trips).
+// 1024 chains: 2-orbital, 40 sweeps 42.8 -> 40.2 ms; 1-orbital 24.2 -> 23.3 ms;
+// 2-orbital in one window, 256 chains, 10 sweeps 6.8 -> 6.2 ms.
 // ---------------------------------------------------------------------------
+constexpr int PC_PAIRS = 0xffffff;
+struct Keys {
+    const lds_b *keys;    // key of each superstate, superstate of each key
+    const lds_i4 *tr;
+    int ncol, dkey;       // dkey 0: no such keys
+    int k0;               // key at the window's lower edge
+};
+template <int NM>
+DEV Keys window_keys()
+{
+    Keys q{nullptr, nullptr, 0, 0, 0};
+    if constexpr (NM <= 16) {
+        const WalkEnv &E = s_wenv;
+        q.keys = uni_lds(E.keys);
+        q.tr = uni_lds(E.tr);
+        q.ncol = uni(E.ncol);
+        q.dkey = uni(E.dkey);
+        q.k0 = uni(E.k0);
+    }
+    return q;
+}
+// Whether quantum numbers stop one of n operators: operator i in front of window
+// position q + max(i - lead, 0), the keys from i = lead on shifted.
+DEV bool blocked(const Keys &ks, const int *pc, const int *code, int q, int n, int lead, int shift)
+{
+    bool bad = false;
+    for (int i0 = 0; i0 < n; i0 += WAVE) {
+        const bool in = i0 + lane_id() < n;
+        const int i = in ? i0 + lane_id() : 0, a = q + max(i - lead, 0), cd = code[i];
+        const int key = (a > 0 ? pc[max(a - 1, 0)] >> 24 : ks.k0) + (i >= lead ? shift : 0);
+        const int s = ks.keys[256 + (key & 255)];
+        const int col = (op_orb(cd) * 2 + op_spin(cd)) * 2 + op_ca(cd) - 1;
+        const iv4 rec = ks.tr[(s == 255 ? 0 : s) * ks.ncol + col];
+        bad |= in & ((s == 255) | (rec.x < 0));
+    }
+    return __ballot(bad) != 0ull;
+}
 template <int NM>
 __device__ __attribute__((noinline)) void count_pairs(ChainRef r)
 {
     Ctx c = attach<NM>(r);
     const int nw = uni(c.h.wib - c.h.wia);
     const double tdm = c.h.taudiff_max, wmax = c.h.tauwin_max;
-    int carry = 0;
+    Keys ks = window_keys<NM>();
+    if (ks.dkey) s_wenv.k0 = ks.k0 = ks.keys[uni(c.h.kst_sst)];
+    int carry = (int)((unsigned)ks.k0 << 24);
     for (int j0 = 0; j0 < nw; j0 += WAVE) {
         const int j = j0 + lane_id();
         int cnt = 0;
@@ -2036,11 +2093,12 @@ __device__ __attribute__((noinline)) void count_pairs(ChainRef r)
                 if (tk[3] > lim) break;
             }
         }
+        if (ks.dkey && j < nw) cnt += (int)((unsigned)key_delta(ks.dkey, c.wcode[j]) << 24);
         const int inc = wave_scan_i(cnt) + carry;
         if (j < nw) c.pc[j] = inc;
         carry = __builtin_amdgcn_readlane(inc, 63);
     }
-    s_wenv.np = carry;
+    s_wenv.np = carry & PC_PAIRS;
     c.h.pc_valid = 1;
     wsync();
 }
@@ -2711,8 +2769,8 @@ DEV int step_add(Ctx &c)
     const int f = orb + M.nb * spin;
     if (t2 == tref) return OUT_QN;
     const int k = uni(c.h.kf[f]);
-    if (!c.h.pc_valid) count_pairs<NM>(c.ref());
     ensure_cache<NM>(c);
+    if (!c.h.pc_valid) count_pairs<NM>(c.ref());
     // equal times (process_OperAdd, Trace.F90:4287-4380), insertion points, the
     // removable pairs that the two operators form with those of the window, and
     // the trial list: the window with t1 before index q1 and t2o before index q2
@@ -2747,6 +2805,9 @@ DEV int step_add(Ctx &c)
         c.tcode[d] = ((ta < tc) != second) ? code_a : code_c;
     }
     wsync();
+    const Keys ks = window_keys<NM>();
+    if (ks.dkey && blocked(ks, c.pc, c.tcode + q1, q1, q2 - q1 + 2, 1, key_delta(ks.dkey, ta < tc ? code_a : code_c)))
+        return OUT_QN;
     const int nl = nw + 2;
     const Proposal pr = trace_proposal<NM>(c.ref(), nw, q1, nw - q2, q2 - q1 + 2);
     if (!pr.ok) return OUT_QN;
@@ -2829,8 +2890,8 @@ DEV int step_rem(Ctx &c)
 {
     CModel &M = c.M;
     const int nw = uni(c.h.wib - c.h.wia);
-    if (!c.h.pc_valid) count_pairs<NM>(c.ref());
     ensure_cache<NM>(c);
+    if (!c.h.pc_valid) count_pairs<NM>(c.ref());
     const int np = uni(s_wenv.np);
     if (np <= 0) return OUT_QN;
     int pick = randint<false>(c.rng, 1, np);
@@ -2840,7 +2901,7 @@ DEV int step_rem(Ctx &c)
     int w1 = -1, w2 = -1, want = pick;
     for (int j0 = 0; j0 < nw && w1 < 0; j0 += WAVE) {
         const int j = j0 + lane_id();
-        const int pc = j < nw ? c.pc[j] : 0;
+        const int pc = j < nw ? c.pc[j] & PC_PAIRS : 0;
         const unsigned long long at = __ballot(j < nw && pc >= pick);
         const int b = at ? __builtin_ctzll(at) : WAVE;
         if (b > 0) want = pick - __builtin_amdgcn_readlane(pc, b - 1);
@@ -2866,6 +2927,10 @@ DEV int step_rem(Ctx &c)
         c.h.err = ERR_STATE_DEV, s_wenv.ready = 0;
         return OUT_REJ;
     }
+    const Keys ks = window_keys<NM>();
+    if (ks.dkey && w2 > w1 + 1 &&
+        blocked(ks, c.pc, c.wcode + w1 + 1, w1 + 1, w2 - w1 - 1, 0, -key_delta(ks.dkey, c1)))
+        return OUT_QN;
     const double t1 = c.wtau[w1], t2 = c.wtau[w2];
     const double wmin = c.h.tauwin_min, wmax = c.h.tauwin_max, tdm = c.h.taudiff_max;
     const int f = c.fl(c1);
@@ -2974,13 +3039,6 @@ DEV void rebuild_flavour_lists(Ctx &c, double *dfc, double *dfa, int *dkf, int *
         if (l == 0) dkf[g] = nc;
     }
     wsync();
-}
-
-// change of a superstate's key by an operator (superstate_keys)
-DEV int key_delta(int dkey, int code)
-{
-    const int d = (int)(signed char)(op_spin(code) ? dkey >> 8 : dkey);
-    return op_ca(code) == 1 ? d : -d;
 }
 
 DEV void all_outer(Ctx &c, unsigned long long *okmask)
@@ -3224,6 +3282,7 @@ DEV void choose_outer(Ctx &c)
     c.h.outer = pick;
     keep_trace<NM>(c, full_trace<NM>(c, pick));
     c.h.cache_pos = -1;
+    c.h.pc_valid = 0;   // the key at the window's lower edge
 }
 
 // StepShiftTau_proper (CTQMC.F90:4641-4835) + update_InvFullHybrShiftTau_diag
