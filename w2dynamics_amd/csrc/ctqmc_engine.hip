@@ -329,7 +329,7 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     if (nm <= 16 && !h->full_lists) {
         const int lmin = std::max(64, (lfull - 32) / 3 + 32);
         const int want = std::min((h->nchains + h->ncu - 1) / h->ncu, SIMDS);
-        const long fixed = sizeof(w2d::WalkEnv) + sizeof(w2d::ChainHdr) + 64;
+        const long fixed = sizeof(w2d::WalkEnv) + 64;
         auto room = [&](int n) { return h->lds_cu / n / LDS_GRAIN * LDS_GRAIN - fixed; };
         for (int n = want; n > 1 && q > room(n); --n) {
             const int lc = std::min<long>(lfull, lfull - (q - room(n) + 27) / 28 - 4);
