@@ -3647,31 +3647,53 @@ __device__ __attribute__((noinline)) double2 meas_gtau(const GtauArgs a)
 // (gbuf, filled by atomics) go into the sum and into level 0 by the Welford
 // update; when the low bits of the count n are ones the finished bin of each
 // level (mean of its halves) rolls over to the next.  Lanes over components;
-// the roll-over depth depends on n only, so it is uniform.
+// the roll-over depth depends on n only, so it is uniform.  Bound by round trips
+// to memory: eight components a lane go together, level by level, all their loads
+// ahead of their arithmetic (4 flavours of 1000 bins: one by one 176 K cycles a
+// measurement; one chain, 16 measurements 13.3 -> 12.5 ms).
 DEV void autocorr_add(CModel &M, double *gbuf, double *gacc, double *gtau, long long n0)
 {
+    constexpr int U = 8;
     const long nc = (long)M.nf * M.ntau;
     double *spill = gacc, *mean = gacc + nc * M.nlev, *sq = gacc + 2 * nc * M.nlev;
     wsync();
-    for (long i = lane_id(); i < nc; i += WAVE) {
-        // the bins were written by atomics at L2: read past the vector L1
-        double v = __hip_atomic_load(gbuf + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        gbuf[i] = 0.0;
-        gtau[i] += v;
+    for (long i0 = lane_id(); i0 - lane_id() < nc; i0 += U * WAVE) {
+        // v: this level's value; s, m, q: its half-filled bin, mean and squares
+        double v[U], g[U], s[U], m[U], q[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long i = min(i0 + u * WAVE, nc - 1);
+            // the bins were written by atomics at L2: read past the vector L1
+            v[u] = __hip_atomic_load(gbuf + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            g[u] = gtau[i], s[u] = spill[i], m[u] = mean[i], q[u] = sq[i];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long i = i0 + u * WAVE;
+            if (i < nc) gbuf[i] = 0.0, gtau[i] = g[u] + v[u];
+        }
         long long n = n0;
-        spill[i] += v;
-        double d1 = v - mean[i];
-        mean[i] += d1 / (double)(n + 1);
-        sq[i] += d1 * (v - mean[i]);
-        for (int lvl = 1; (n & 1) != 0 && lvl < M.nlev; ++lvl) {
+        for (int lvl = 0;; ++lvl) {
+            const bool roll = (n & 1) != 0 && lvl + 1 < M.nlev;
+            const long at = (long)lvl * nc;
+            const double cnt = (double)(n + 1);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long i = i0 + u * WAVE;
+                s[u] += v[u];
+                const double d1 = v[u] - m[u];
+                m[u] += d1 / cnt;
+                q[u] += d1 * (v[u] - m[u]);
+                if (i < nc) spill[at + i] = roll ? 0.0 : s[u], mean[at + i] = m[u], sq[at + i] = q[u];
+                v[u] = s[u] / 2.0;
+            }
+            if (!roll) break;
             n >>= 1;
-            const long lo = (long)(lvl - 1) * nc + i, hi = (long)lvl * nc + i;
-            const double u = spill[lo] / 2.0;
-            spill[lo] = 0.0;
-            spill[hi] += u;
-            const double e1 = u - mean[hi];
-            mean[hi] += e1 / (double)(n + 1);
-            sq[hi] += e1 * (u - mean[hi]);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long i = at + nc + min(i0 + u * WAVE, nc - 1);
+                s[u] = spill[i], m[u] = mean[i], q[u] = sq[i];
+            }
         }
     }
     wsync();
