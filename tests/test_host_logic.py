@@ -1,0 +1,84 @@
+"""Decisions of the library's host code, on machines without a GPU: the host
+code is built over a stand-in for the HIP runtime (tests/native/host_library.cpp:
+device memory is host memory, kernels do nothing)."""
+
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+from w2dynamics_amd import ctqmc
+from w2dynamics_amd import problems as P
+
+
+@pytest.fixture(scope="module")
+def host_so(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "libhost.so")
+    subprocess.run(["hipcc", "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-shared",
+                    "-Wl,-Bsymbolic", "-I" + os.path.join(ROOT, "include"),
+                    os.path.join(ROOT, "tests", "native", "host_library.cpp"),
+                    os.path.join(ROOT, "w2dynamics_amd", "csrc", "model.cpp"), "-o", so], check=True)
+    return so
+
+
+@pytest.fixture
+def host(host_so, monkeypatch):
+    """CtqmcGpu drives the stand-in; its library."""
+    monkeypatch.setattr(ctqmc, "_lib", None)
+    lib = ctqmc.load_library(host_so)
+    for f in ("host_layout", "host_halt", "host_resume", "host_chain"):
+        getattr(lib, f).argtypes = None
+    yield lib
+    monkeypatch.setattr(ctqmc, "_lib", None)
+
+
+def _layout(lib, g):
+    v = (C.c_longlong * 7)()
+    lib.host_layout(g.h, v)
+    return dict(zip(("lists", "short", "lds", "lds_total", "lds_max", "cap", "full_lists"), v))
+
+
+def _memory(lib):
+    a, b = C.c_longlong(), C.c_longlong()
+    lib.host_memory(C.byref(a), C.byref(b))
+    return a.value, b.value
+
+
+def _chain(lib, g, c):
+    halt, err = C.c_int(), C.c_int()
+    lib.host_chain(g.h, c, C.byref(halt), C.byref(err))
+    return halt.value, err.value
+
+
+def _resume(lib, g):
+    again = C.c_int()
+    st = lib.host_resume(g.h, C.byref(again))
+    return st, again.value
+
+
+def _short_lists(lib, capacity):
+    """Four chains on the stand-in's one compute unit: their lists are cut."""
+    g = ctqmc.CtqmcGpu.from_problem(P.kanamori_3orb(beta=100.0, TaudiffMax=8.0), nchains=4, seed=1, capacity=capacity)
+    g.set_taudiffmax(8.0)
+    assert _layout(lib, g)["short"] == 1
+    return g
+
+
+@pytest.mark.parametrize("capacity", [384, -384])
+def test_full_lists_return_in_place(host, capacity):
+    """A chain that outgrew its shortened list goes on with full ones: only
+    offsets in LDS change, so no memory is allocated, not even where none is left."""
+    g = _short_lists(host, capacity)
+    before = _layout(host, g), _memory(host)
+    host.host_halt(g.h, 2, 40)
+    host.host_memory_full(1)
+    st, again = _resume(host, g)
+    host.host_memory_full(0)
+    assert (st, again) == (0, 1)
+    after = _layout(host, g)
+    assert after["short"] == 0 and after["lists"] > before[0]["lists"] and after["cap"] == before[0]["cap"]
+    assert _memory(host) == before[1]
+    assert _chain(host, g, 2) == (0, 0)
+    g.close()

@@ -602,6 +602,21 @@ bool has_room(const w2d_ctqmc *h, const ChainHdr &x)
     return x.nop + 2 <= h->L.cap;
 }
 
+// The LDS operator lists at their full share: offsets in LDS only, the chain
+// blocks stay where and as they are.
+int lengthen_lists(w2d_ctqmc *h)
+{
+    w2d::ChainLayout B;
+    h->full_lists = true;
+    const int st = compute_layout(h, h->L.nbound, h->kcap, B);
+    if (st) {
+        h->full_lists = false;
+        return st;
+    }
+    h->L = B;
+    return W2D_OK;
+}
+
 // After a pass: chains halted for room get a larger capacity and continue;
 // returns whether another pass is needed.  Chains that cannot grow further
 // are stopped with W2D_ERR_CAPACITY (their results are left out).
@@ -620,8 +635,7 @@ int resume_halted(w2d_ctqmc *h, std::vector<ChainHdr> &hd, long long &from, bool
     }
     if (!cap || h->aborted) return W2D_OK;
     // where only shortened lists ran out: their full share first
-    if (lists) h->full_lists = true;
-    const int st = lists ? relayout(h, h->kcap, h->L.nbound) : regrow(h);
+    const int st = lists ? lengthen_lists(h) : regrow(h);
     if (st && st != W2D_ERR_CAPACITY) return st;
     for (auto &x : hd)
         if (x.halt == w2d::HALT_CAP) {
@@ -1394,9 +1408,9 @@ int w2d_ctqmc_moves_log(w2d_ctqmc *h, int chain, int64_t n, w2d_move_record *rec
     if ((st = write_headers(h, hd))) return st;
     w2d_move_record *d = nullptr;
     HIPCHK(hipMalloc(&d, sizeof(w2d_move_record) * per));
-    DISPATCH(prepare_sweep, h);
     for (long long done = 0; done < n && st == W2D_OK;) {
         const long long k = std::min<long long>(per, n - done);
+        DISPATCH(prepare_sweep, h);   // the LDS may have grown
         DISPATCH(launch_sweep, h, done + k, 0, chain, d, done);
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(h->stream) != hipSuccess) {
             st = W2D_ERR_HIP;
@@ -1765,8 +1779,8 @@ int w2d_ctqmc_calibrate(w2d_ctqmc *h, int list, int phase1pairnum, int phase2tau
     const long long per = 4000;
     long long from = 0;
     h->last_launches = 0;
-    DISPATCH(prepare_sweep, h);
     for (;;) {
+        DISPATCH(prepare_sweep, h);   // the LDS may have grown
         launch_range(h, from, from + per, 0, per, -1, nullptr, 0);
         if (hipGetLastError() != hipSuccess) {
             h->calib = make_int3(0, 1, 0);
