@@ -82,3 +82,31 @@ def test_full_lists_return_in_place(host, capacity):
     assert _memory(host) == before[1]
     assert _chain(host, g, 2) == (0, 0)
     g.close()
+
+
+def test_only_chains_without_room_stop(host):
+    """One chain is at its fixed capacity, another only outgrew its shortened
+    list: the second goes on with full ones."""
+    g = _short_lists(host, -384)
+    host.host_halt(g.h, 1, 384)
+    host.host_halt(g.h, 2, 40)
+    assert _resume(host, g) == (0, 1)
+    assert _chain(host, g, 1) == (0, 3)
+    assert _chain(host, g, 2) == (0, 0)
+    assert _layout(host, g)["short"] == 0
+    # with full lists a chain halted for room has none left
+    host.host_halt(g.h, 2, 40)
+    assert _resume(host, g) == (0, 0)
+    assert _chain(host, g, 2) == (0, 3)
+    g.close()
+
+
+def test_both_kinds_resume_where_memory_grows(host):
+    g = _short_lists(host, 384)
+    cap = _layout(host, g)["cap"]
+    host.host_halt(g.h, 1, 384)
+    host.host_halt(g.h, 2, 40)
+    assert _resume(host, g) == (0, 1)
+    lay = _layout(host, g)
+    assert lay["cap"] == 2 * cap and lay["short"] == 0
+    g.close()

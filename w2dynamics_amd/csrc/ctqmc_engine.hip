@@ -617,35 +617,42 @@ int lengthen_lists(w2d_ctqmc *h)
     return W2D_OK;
 }
 
-// After a pass: chains halted for room get a larger capacity and continue;
-// returns whether another pass is needed.  Chains that cannot grow further
-// are stopped with W2D_ERR_CAPACITY (their results are left out).
+// After a pass: chains halted for room continue, those that only outgrew a
+// shortened list with full ones, the others with a larger capacity; `again`:
+// another pass is needed.  Chains that cannot grow further are stopped with
+// W2D_ERR_CAPACITY (their results are left out).
 int resume_halted(w2d_ctqmc *h, std::vector<ChainHdr> &hd, long long &from, bool &again)
 {
     again = false;
-    bool cap = false, lists = h->L.lcap_short != 0;
     from = -1;
-    for (const auto &x : hd) {
-        if (x.halt == w2d::HALT_ABORT) h->aborted = 1;
-        if (x.halt == w2d::HALT_CAP && x.err == 0) {
-            cap = true;
-            lists = lists && has_room(h, x);
-            from = from < 0 ? x.pos : std::min(from, x.pos);
-        }
+    bool lists = false, grow = false;
+    auto halted = [](const ChainHdr &x) { return x.halt == w2d::HALT_CAP && x.err == 0; };
+    const bool lcap_short = h->L.lcap_short != 0;
+    std::vector<char> outgrew(hd.size(), 0);   // its shortened list only
+    for (size_t c = 0; c < hd.size(); ++c) {
+        if (hd[c].halt == w2d::HALT_ABORT) h->aborted = 1;
+        if (!halted(hd[c])) continue;
+        outgrew[c] = lcap_short && has_room(h, hd[c]);
+        (outgrew[c] ? lists : grow) = true;
     }
-    if (!cap || h->aborted) return W2D_OK;
-    // where only shortened lists ran out: their full share first
-    const int st = lists ? lengthen_lists(h) : regrow(h);
+    if (!(lists || grow) || h->aborted) return W2D_OK;
+    int st;
+    if (lists && (st = lengthen_lists(h))) return st;
+    st = grow ? regrow(h) : W2D_OK;
     if (st && st != W2D_ERR_CAPACITY) return st;
-    for (auto &x : hd)
-        if (x.halt == w2d::HALT_CAP) {
-            x.halt = w2d::HALT_NONE;
-            if (st == W2D_ERR_CAPACITY) x.err = W2D_ERR_CAPACITY;
+    for (size_t c = 0; c < hd.size(); ++c) {
+        ChainHdr &x = hd[c];
+        if (x.halt != w2d::HALT_CAP) continue;
+        x.halt = w2d::HALT_NONE;
+        if (x.err) continue;
+        if (st && !outgrew[c]) {
+            x.err = W2D_ERR_CAPACITY;
+            continue;
         }
-    int wst = write_headers(h, hd);
-    if (wst) return wst;
-    again = (st == W2D_OK);
-    return W2D_OK;
+        again = true;
+        from = from < 0 ? x.pos : std::min(from, x.pos);
+    }
+    return write_headers(h, hd);
 }
 
 // W2D_OK if every chain is fine, W2D_ERR_PARTIAL if some chains stopped on an
