@@ -110,3 +110,24 @@ def test_both_kinds_resume_where_memory_grows(host):
     lay = _layout(host, g)
     assert lay["cap"] == 2 * cap and lay["short"] == 0
     g.close()
+
+
+def _fits(lib, nleg, capacity=3000):
+    """LDS of a single chain's handle, None where it is refused for capacity."""
+    try:
+        g = ctqmc.CtqmcGpu.from_problem(P.anderson_1orb(NLegMax=nleg), nchains=1, seed=1, capacity=capacity)
+    except ctqmc.CtqmcError as e:
+        assert e.code == 3
+        return None
+    lay = _layout(lib, g)
+    g.close()
+    return lay
+
+
+def test_lds_limit_counts_the_kernels_own_variables(host):
+    """Every order of the Legendre sums takes 16 bytes of LDS: up to the last one
+    that fits with the kernels' static variables a handle is made, then refused."""
+    lay = _fits(host, 100)
+    last = 100 + (lay["lds_max"] - lay["lds_total"]) // 16
+    assert _fits(host, last)["lds_total"] <= lay["lds_max"] < lay["lds_total"] + 16 * (last + 1 - 100)
+    assert _fits(host, last + 1) is None

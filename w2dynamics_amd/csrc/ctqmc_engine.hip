@@ -101,6 +101,9 @@ constexpr int KCAP_MAX = 4096;   // pairs per flavour a chain may grow to
 constexpr int ACCPAIR_BINS_MAX = 1024;   // accepted-pair histogram bins (NAccPair) at most, beyond Ntau
 constexpr int SIMDS = 4;                 // per compute unit; a wave of the sweep kernel each
 constexpr long LDS_GRAIN = 1280;         // bytes LDS is handed out in
+// LDS of the chain kernels beside the dynamic part: their one variable, and what
+// the dynamic part may start behind it
+constexpr long LDS_STATIC = (sizeof(w2d::WalkEnv) + 15) / 16 * 16;
 constexpr int SEG_CACHE = 128;           // window operators the segment caches of blocks above 4 states cover
 constexpr int APT_CAP = 65536;           // accepted-pair distances a calibration list holds at most
 constexpr int GIW_NIW_MAX = 1 << 20;     // Matsubara frequencies of MeasGiw at most
@@ -329,7 +332,7 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
     if (nm <= 16 && !h->full_lists) {
         const int lmin = std::max(64, (lfull - 32) / 3 + 32);
         const int want = std::min((h->nchains + h->ncu - 1) / h->ncu, SIMDS);
-        const long fixed = sizeof(w2d::WalkEnv) + 64;
+        const long fixed = LDS_STATIC + 64;
         auto room = [&](int n) { return h->lds_cu / n / LDS_GRAIN * LDS_GRAIN - fixed; };
         for (int n = want; n > 1 && q > room(n); --n) {
             const int lc = std::min<long>(lfull, lfull - (q - room(n) + 27) / 28 - 4);
@@ -339,7 +342,7 @@ int compute_layout(const w2d_ctqmc *h, int nbound, int kc, w2d::ChainLayout &L)
             break;
         }
     }
-    if (L.lds_bytes > h->lds_max) return W2D_ERR_CAPACITY;
+    if (L.lds_bytes + LDS_STATIC > h->lds_max) return W2D_ERR_CAPACITY;
     L.hdrs = L.stride * h->nchains;
     return W2D_OK;
 }
@@ -403,11 +406,11 @@ int regrow(w2d_ctqmc *h)
     return st;
 }
 
-// allow the dynamic LDS of this handle (above 64 KB on devices that have it)
+// allow the LDS of this handle (above 64 KB on devices that have it)
 template <typename K>
 void allow_lds(K kernel, const w2d_ctqmc *h)
 {
-    if (h->L.lds_bytes > 64 * 1024)
+    if (h->L.lds_bytes + LDS_STATIC > 64 * 1024)
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->L.lds_bytes);
 }
