@@ -2708,6 +2708,15 @@ DEV void record_pair(Ctx &c, int f, double dt)
     if (c.h.apt_index <= c.h.apt_n) c.h.apt_index++;
 }
 
+// Sign of the whole configuration.  Accepted insertions and removals carry the
+// sign on from move to move; behind a zero trace there is none to carry.
+template <int NM>
+__device__ __attribute__((noinline)) void sign_anew(ChainRef r)
+{
+    Ctx c = attach<NM>(r);
+    c.h.cfgsign = -config_sign(c);
+}
+
 // an accepted insertion / removal: what the proposal found
 struct AddMove {
     int f, k, nl, q1, q2, fp_c, fp_a;   // flavour, its order, length of the trial list, insertion points, FPos
@@ -2863,6 +2872,7 @@ DEV int step_add(Ctx &c)
     accept_add<NM>(c.ref(), AddMove{f, k, nl, q1, q2, fp_c, fp_a, ta, tc, S, dr_sign,
                                     (sgn & 1) ? -dr_sign : dr_sign, T});
     c.lists();
+    if (c.h.cfgsign == 0.0) sign_anew<NM>(c.ref());
     return OUT_ACC;
 }
 
@@ -2995,6 +3005,7 @@ DEV int step_rem(Ctx &c)
     accept_rem<NM>(c.ref(), RemMove{f, k, nl, w1, w2, fp_c, fp_a, sc, sa, t2 - t1, S, dr_sign,
                                     (sgn & 1) ? -dr_sign : dr_sign, T});
     c.lists();
+    if (c.h.cfgsign == 0.0) sign_anew<NM>(c.ref());
     return OUT_ACC;
 }
 
