@@ -696,6 +696,13 @@ struct State {
 // between, the entries are left unscaled (rescaling by powers of two is exact,
 // so skipping it changes no rounding).
 constexpr double STATE_TINY = 0x1p-64, STATE_HUGE = 0x1p64;
+// A walk looks every fourth operator whether its state needs renormalisation,
+// unless a propagation of its group spans more than exp(-WALK_DECAY).  A walk
+// that starts on a cached state has up to ten propagations between two looks:
+// three that the cache holds, three at the end of a group of 63, four more.  They
+// keep exp(-500) of the FP64 range, and a product with a cached bra exp(-150) of
+// what is left.
+constexpr float WALK_DECAY = 50.0f;
 
 // power-of-two renormalisation when the largest entry of the lanes in `mask`
 // leaves [2^-64, 2^64]
@@ -753,8 +760,7 @@ struct WalkOut {
 //      the block; 216 KB for the 3-orbital model, shared by all chains), so an
 //      operator is three coalesced loads, issued two operators ahead.  Blocks of one state: a product over the lanes.
 // The renormalisation check runs per operator only if some propagation of the
-// group spans more than exp(-100), else every fourth operator: in between no
-// state can leave the FP64 range.
+// group spans more than exp(-WALK_DECAY), else every fourth operator.
 // KEEP: the states after every operator go to px.
 template <int NM, bool BRA, bool KEEP>
 __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_, double tstart, double tend,
@@ -853,7 +859,7 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_,
                 lg += wave_sum(lc);
             }
         } else if constexpr (NM <= 4) {
-            const unsigned chk = __ballot(__int_as_float(si.w) * (float)dt > 100.0f) ? 0u : 3u;
+            const unsigned chk = __ballot(__int_as_float(si.w) * (float)dt > WALK_DECAY) ? 0u : 3u;
             const lds_d *lops = uni_lds(E.lops);
             const int blk = (l >> 2) & 3, i = l & 3, kr = l >> 4;
             const double sc = KEEP ? wave_scan_d(lc) : wave_sum(lc);   // log factors so far / of the group
@@ -903,7 +909,7 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_small(State<NM> k, int s_,
             x += dpp_d<DPP_ROW_ROR4>(x);
             k.v[0] = x + dpp_d<DPP_ROW_ROR8>(x);
         } else {
-            const unsigned chk = __ballot(__int_as_float(si.w) * (float)dt > 100.0f) ? 0u : 3u;
+            const unsigned chk = __ballot(__int_as_float(si.w) * (float)dt > WALK_DECAY) ? 0u : 3u;
             const double sc = KEEP ? wave_scan_d(lc) : wave_sum(lc);
             double lren = 0.0;
             auto products = [&](auto nk) {
@@ -1111,7 +1117,7 @@ __device__ __attribute__((noinline)) WalkOut<NM> walk_row(State<NM> k, int s_, d
         // caller (a function that calls none saves no registers to memory; with
         // the segment caches extended in line, 2-orbital, 1024 chains, 40 sweeps
         // 39.8 -> 38.6 ms)
-        if (__ballot(__int_as_float(si.w) * (float)dt > 100.0f) != 0ull) {
+        if (__ballot(__int_as_float(si.w) * (float)dt > WALK_DECAY) != 0ull) {
             out.s = WALK_LONG;
             return out;
         }
@@ -1845,6 +1851,9 @@ DEV void seg_extend(Ctx &c, int nw, int to)
         s = uni(bs[j]);
         lg0 = bx[j];
         k = seg_load<NM>(buf, j, c.sz[s], no);
+        // cached as it was between two looks: a cache that grows by one to three
+        // operators at a time would never see one
+        if constexpr (NM > 1) renorm(k, ~0ull, lg0);
     }
     if (j < to) {
         typedef typename Prefix<NM>::mat mat;
@@ -1939,6 +1948,7 @@ __device__ __attribute__((noinline)) void slide_window(ChainRef ref)
         const double *E = c.ev + c.off[s];
         const double dt = edge - (low > 0 ? c.wtau[low - 1] : edge0), e0 = E[0];
         double lg = c.rkx[low] - (e0 - c.M.egs) * dt;
+        if constexpr (NM > 1) renorm(k, ~0ull, lg);
 #pragma unroll
         for (int e = 0; e < State<NM>::NV; ++e) {
             const int r = State<NM>::row(e);
