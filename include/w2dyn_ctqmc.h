@@ -214,7 +214,8 @@ int w2d_ctqmc_set_config(w2d_ctqmc *h, int chain, int n, const double *tau, cons
 /* The same for chains 0 .. nconf - 1 at once (ReuseMCConfig for a batch,
  * cthyb_solver.py:24-86, 328-332): configuration i holds the operators
  * off[i] .. off[i+1] - 1 of the arrays; weights[nconf][5].  The configurations
- * before the first that is refused are set; the first error is returned. */
+ * before the first that is refused are set, the chains behind it keep theirs;
+ * its error is returned. */
 int w2d_ctqmc_set_configs(w2d_ctqmc *h, int nconf, const int64_t *off, const double *tau, const int *orb,
                           const int *spin, const int *ca, const int *outer_sst, double *weights);
 

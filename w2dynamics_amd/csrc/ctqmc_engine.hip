@@ -105,6 +105,7 @@ constexpr long LDS_GRAIN = 1280;         // bytes LDS is handed out in
 // the dynamic part may start behind it
 constexpr long LDS_STATIC = (sizeof(w2d::WalkEnv) + 15) / 16 * 16;
 constexpr int SEG_CACHE = 128;           // window operators the segment caches of blocks above 4 states cover
+constexpr long HOLD_BYTES = 64L << 20;   // chain states that one launch of set_configs may have to put back
 constexpr int APT_CAP = 65536;           // accepted-pair distances a calibration list holds at most
 constexpr int GIW_NIW_MAX = 1 << 20;     // Matsubara frequencies of MeasGiw at most
 
@@ -468,12 +469,13 @@ struct DevConfigs {
     const int *code, *off, *outer;
 };
 
+// configurations from, from + 1, ... into chains first, first + 1, ...
 template <int NM>
-void launch_setconfig(w2d_ctqmc *h, int first, int count, const DevConfigs &d)
+void launch_setconfig(w2d_ctqmc *h, int first, int count, const DevConfigs &d, int from)
 {
     allow_lds(w2d::setconfig_kernel<NM>, h);
     hipLaunchKernelGGL(w2d::setconfig_kernel<NM>, dim3(count), dim3(w2d::WAVE), (unsigned)h->L.lds_bytes, h->stream, h->dm,
-                       h->L, h->chains, first, d.tau, d.code, d.off, d.outer);
+                       h->L, h->chains, first, d.tau, d.code, d.off + from, d.outer + from);
 }
 
 template <int NM>
@@ -953,16 +955,23 @@ bool valid_config(const w2d_ctqmc *h, int64_t a, int64_t b, const double *tau, c
     return true;
 }
 
-// Configurations i = 0 .. nconf - 1 into chains first + i, all in one launch.
-// Like calls one after the other, the ones before the first that is refused are
-// set; returns the first error in order.
+// Configurations i = 0 .. nconf - 1 into chains first + i, as many in one launch
+// as the replaced states take up to HOLD_BYTES.  Like calls one after the other
+// that stop at the first error: the chains behind a configuration that is refused
+// keep theirs (the chain of one with a zero trace or a singular matrix, which
+// shows on the device only, takes it and has stopped); returns that error.
 int set_configs(w2d_ctqmc *h, int first, int nconf, const int64_t *off, const double *tau, const int *orb,
                 const int *spin, const int *ca, const int *outer_sst, double *weights)
 {
     h->moved = true;
     if (off[0] != 0) return W2D_ERR_ARG;
     int status = W2D_OK, m = 0;
-    std::vector<int> code, o32(1, 0);
+    std::vector<int> code, ints(1, 0);
+    // the states that will be replaced: their headers arrive while the
+    // configurations are looked over
+    if (nconf > 1)
+        HIPCHK(hipMemcpyAsync(h->hdr_pinned, hdr_of(h, first), sizeof(ChainHdr) * (size_t)nconf, hipMemcpyDeviceToHost,
+                              h->stream));
     for (; m < nconf && status == W2D_OK; ++m) {
         int pairs = 0;
         if (off[m + 1] < off[m] || off[m + 1] > 0x7fffffff) {
@@ -977,37 +986,69 @@ int set_configs(w2d_ctqmc *h, int first, int nconf, const int64_t *off, const do
         // grow until every flavour's order fits
         while (pairs > h->kcap && status == W2D_OK) status = regrow(h);
         if (status) break;
-        o32.push_back((int)off[m + 1]);
+        ints.push_back((int)off[m + 1]);
     }
-    if (m > 0) {
-        const size_t nops = (size_t)off[m];
-        const size_t btau = nops * 8, bcode = (nops * 4 + 7) / 8 * 8, boff = ((size_t)m + 1) * 4;
-        int st = need_work(h, btau + bcode + boff + (size_t)m * 4 + 64);
-        if (st) return st;
-        char *w = static_cast<char *>(h->work);
-        if (nops > 0) {
-            HIPCHK(hipMemcpyAsync(w, tau, btau, hipMemcpyHostToDevice, h->stream));
-            HIPCHK(hipMemcpyAsync(w + btau, code.data(), nops * 4, hipMemcpyHostToDevice, h->stream));
+    if (nconf > 1) HIPCHK(hipStreamSynchronize(h->stream));
+    if (m == 0) return status;
+    // launches: configurations [cut[p], cut[p + 1]); the first of a launch has
+    // none before it that could be refused, so the state it replaces is not held
+    const int nf = 2 * h->model.nbands;
+    std::vector<long> at((size_t)m, 0);
+    std::vector<int> cut(1, 0);
+    long held = 0, most = 0;
+    for (int i = 1; i < m; ++i) {
+        const long n = w2d::held_bytes(h->hdr_pinned[i], nf, h->nm);
+        if (held + n > HOLD_BYTES) {
+            cut.push_back(i);
+            held = 0;
+            continue;
         }
-        HIPCHK(hipMemcpyAsync(w + btau + bcode, o32.data(), boff, hipMemcpyHostToDevice, h->stream));
-        HIPCHK(hipMemcpyAsync(w + btau + bcode + boff, outer_sst, (size_t)m * 4, hipMemcpyHostToDevice, h->stream));
-        const DevConfigs d{reinterpret_cast<const double *>(w), reinterpret_cast<const int *>(w + btau),
-                           reinterpret_cast<const int *>(w + btau + bcode),
-                           reinterpret_cast<const int *>(w + btau + bcode + boff)};
-        DISPATCH(launch_setconfig, h, first, m, d);
+        at[i] = held;
+        held += n;
+        most = std::max(most, held);
+    }
+    cut.push_back(m);
+    const size_t nops = (size_t)off[m], btau = nops * 8, bat = (size_t)m * 8, bcode = nops * 4;
+    ints.insert(ints.end(), outer_sst, outer_sst + m);
+    int st = need_work(h, (size_t)most + btau + bat + bcode + ints.size() * 4);
+    if (st) return st;
+    char *hold = static_cast<char *>(h->work), *wtau = hold + most, *wat = wtau + btau, *wcode = wat + bat,
+         *wints = wcode + bcode;
+    if (nops > 0) {
+        HIPCHK(hipMemcpyAsync(wtau, tau, btau, hipMemcpyHostToDevice, h->stream));
+        HIPCHK(hipMemcpyAsync(wcode, code.data(), bcode, hipMemcpyHostToDevice, h->stream));
+    }
+    if (m > 1) HIPCHK(hipMemcpyAsync(wat, at.data(), bat, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(hipMemcpyAsync(wints, ints.data(), ints.size() * 4, hipMemcpyHostToDevice, h->stream));
+    const DevConfigs d{reinterpret_cast<const double *>(wtau), reinterpret_cast<const int *>(wcode),
+                       reinterpret_cast<const int *>(wints), reinterpret_cast<const int *>(wints) + m + 1};
+    const long *dat = reinterpret_cast<const long *>(wat);
+    for (size_t p = 0; p + 1 < cut.size(); ++p) {
+        const int i0 = cut[p], i1 = cut[p + 1];
+        if (i1 > i0 + 1)
+            hipLaunchKernelGGL(w2d::hold_kernel<false>, dim3(i1 - i0 - 1, nf + 1), dim3(256), 0, h->stream, h->L,
+                               h->chains, first + i0 + 1, nf, h->nm, hold, dat + i0 + 1);
+        DISPATCH(launch_setconfig, h, first + i0, i1 - i0, d, i0);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(h->hdr_pinned, hdr_of(h, first), sizeof(ChainHdr) * (size_t)m, hipMemcpyDeviceToHost,
-                              h->stream));
+        HIPCHK(hipMemcpyAsync(h->hdr_pinned, hdr_of(h, first + i0), sizeof(ChainHdr) * (size_t)(i1 - i0),
+                              hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
-        for (int i = 0; i < m; ++i) {
-            const ChainHdr &x = h->hdr_pinned[i];
+        for (int i = i0; i < i1; ++i) {
+            const ChainHdr &x = h->hdr_pinned[i - i0];
             if (weights) {
                 double *v = weights + 5L * i;
                 v[0] = x.trace_log, v[1] = x.trace_sign, v[2] = x.det_log, v[3] = x.det_sign, v[4] = x.cfgsign;
             }
+            if (!x.err) continue;
+            status = map_err(x.err);
+            if (i + 1 < i1) {
+                hipLaunchKernelGGL(w2d::hold_kernel<true>, dim3(i1 - i - 1, nf + 1), dim3(256), 0, h->stream, h->L,
+                                   h->chains, first + i + 1, nf, h->nm, hold, dat + i + 1);
+                HIPCHK(hipGetLastError());
+                HIPCHK(hipStreamSynchronize(h->stream));
+            }
+            return status;
         }
-        for (int i = 0; i < m; ++i)
-            if (h->hdr_pinned[i].err) return map_err(h->hdr_pinned[i].err);
     }
     return status;
 }

@@ -4732,6 +4732,56 @@ __global__ void __launch_bounds__(WAVE) init_kernel(DevModel M, ChainLayout L, c
     save_ctx(c, (int)blockIdx.x);
 }
 
+// Bytes of a chain's state that setconfig_kernel replaces: header, part traces,
+// operators, flavour lists and the used corner of the inverses.
+__host__ __device__ inline long held_bytes(const ChainHdr &x, int nf, int nm)
+{
+    long n = (long)sizeof(ChainHdr) + 16L * nm + 12L * x.nop;
+    for (int f = 0; f < nf; ++f) n += (24L + 8L * x.kf[f]) * x.kf[f];
+    return (n + 7) / 8 * 8;
+}
+
+// That state of the chains first, first + 1, ... to buf + at[i] (each held_bytes
+// long), or (BACK) from there.  Grid: x over chains, y over flavours and, last,
+// what belongs to none; a workgroup's copies are one to five round trips.
+template <bool BACK>
+__global__ void __launch_bounds__(256) hold_kernel(ChainLayout L, char *chains, int first, int nf, int nm, char *buf,
+                                                   const long *at)
+{
+    const int chain = first + (int)blockIdx.x, f = blockIdx.y, t = threadIdx.x;
+    char *base = chains + (long)chain * L.stride, *hdr = chains + L.hdrs + (long)chain * (long)sizeof(ChainHdr);
+    char *b = buf + at[blockIdx.x];
+    const ChainHdr &x = *reinterpret_cast<const ChainHdr *>(BACK ? b : hdr);
+    // n words between the chain and the buffer
+    auto move = [&](char *p, long n) {
+        int *c = reinterpret_cast<int *>(p), *q = reinterpret_cast<int *>(b);
+        for (long i = t; i < n; i += 256) (BACK ? c : q)[i] = (BACK ? q : c)[i];
+        b += 4 * n;
+    };
+    if (f == nf) {
+        move(hdr, sizeof(ChainHdr) / 4);
+        move(base + L.part, 4L * nm);
+        move(base + L.tau, 2L * x.nop);
+        move(base + L.code, x.nop);
+        return;
+    }
+    b += (long)sizeof(ChainHdr) + 16L * nm + 12L * x.nop;
+    for (int g = 0; g < f; ++g) b += (24L + 8L * x.kf[g]) * x.kf[g];
+    const int k = x.kf[f];
+    const long fo = (long)f * L.kcap;
+    move(base + L.fc + 8 * fo, 2L * k);
+    move(base + L.fa + 8 * fo, 2L * k);
+    move(base + L.fcs + 4 * fo, k);
+    move(base + L.fas + 4 * fo, k);
+    // columns of the inverse (in words: the buffer is aligned to four bytes here)
+    int *M = reinterpret_cast<int *>(base + L.minv) + 2 * fo * L.kcap, *q = reinterpret_cast<int *>(b);
+    for (int j = t / WAVE; j < k; j += 256 / WAVE)
+        for (int i = t % WAVE; i < 2 * k; i += WAVE) {
+            int &c = M[2L * j * L.kcap + i], &h = q[2L * j * k + i];
+            (BACK ? c : h) = BACK ? h : c;
+        }
+}
+
 // Configurations for chains first, first + 1, ...: operators off[i] .. off[i+1]
 // of tau / code and outer superstate outer[i] for chain first + i; full trace,
 // flavour lists, full inverses, sign (set_mc_config_from_arrays,
