@@ -5,6 +5,7 @@ device memory is host memory, kernels do nothing)."""
 import ctypes as C
 import os
 import subprocess
+import sys
 
 import pytest
 
@@ -131,3 +132,27 @@ def test_lds_limit_counts_the_kernels_own_variables(host):
     last = 100 + (lay["lds_max"] - lay["lds_total"]) // 16
     assert _fits(host, last)["lds_total"] <= lay["lds_max"] < lay["lds_total"] + 16 * (last + 1 - 100)
     assert _fits(host, last + 1) is None
+
+
+def test_refused_configuration_allocates_nothing(host_so):
+    """A configuration longer than any the handle can hold is refused before the
+    host makes room for its operators (a C++ exception must not reach the C
+    caller); run in a process of its own with little memory left."""
+    code = """
+import resource, sys
+import numpy as np
+sys.path.insert(0, %r)
+from w2dynamics_amd import ctqmc, problems as P
+lib = ctqmc.load_library(%r)
+g = ctqmc.CtqmcGpu.from_problem(P.anderson_1orb(), nchains=2, seed=1, capacity=8)
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (1 << 30),) * 2)
+p = ctqmc._p
+tau, i4, off = np.zeros(4), np.zeros(4, np.int32), np.array([0, 0, 2**31 - 1], np.int64)
+a = lib.w2d_ctqmc_set_config(g.h, 0, 2**31 - 1, p(tau), p(i4), p(i4), p(i4), 0, None)
+b = lib.w2d_ctqmc_set_configs(g.h, 2, p(off), p(tau), p(i4), p(i4), p(i4), p(i4), None)
+print(a, b)
+""" % (ROOT, host_so)
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr[-400:]
+    assert out.stdout.split() == ["1", "1"]

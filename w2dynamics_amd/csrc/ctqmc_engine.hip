@@ -938,7 +938,7 @@ int switch_engine(w2d_ctqmc *h, int nm)
 bool valid_config(const w2d_ctqmc *h, int64_t a, int64_t b, const double *tau, const int *orb, const int *spin,
                   const int *ca, int outer_sst, std::vector<int> &code, int &pairs)
 {
-    if (b < a || b - a > h->L.cap || outer_sst < 0 || outer_sst >= h->model.nsst) return false;
+    if (outer_sst < 0 || outer_sst >= h->model.nsst) return false;
     std::vector<int> cnt(2 * h->model.nbands * 2, 0);
     for (int64_t i = a; i < b; ++i) {
         if (orb[i] < 0 || orb[i] >= h->model.nbands || spin[i] < 0 || spin[i] > 1 || ca[i] < 1 || ca[i] > 2)
@@ -963,7 +963,6 @@ bool valid_config(const w2d_ctqmc *h, int64_t a, int64_t b, const double *tau, c
 int set_configs(w2d_ctqmc *h, int first, int nconf, const int64_t *off, const double *tau, const int *orb,
                 const int *spin, const int *ca, const int *outer_sst, double *weights)
 {
-    h->moved = true;
     if (off[0] != 0) return W2D_ERR_ARG;
     int status = W2D_OK, m = 0;
     std::vector<int> code, ints(1, 0);
@@ -974,7 +973,8 @@ int set_configs(w2d_ctqmc *h, int first, int nconf, const int64_t *off, const do
                               h->stream));
     for (; m < nconf && status == W2D_OK; ++m) {
         int pairs = 0;
-        if (off[m + 1] < off[m] || off[m + 1] > 0x7fffffff) {
+        // (before there is room for its operators)
+        if (off[m + 1] < off[m] || off[m + 1] - off[m] > h->L.cap || off[m + 1] > 0x7fffffff) {
             status = W2D_ERR_ARG;
             break;
         }
@@ -990,6 +990,7 @@ int set_configs(w2d_ctqmc *h, int first, int nconf, const int64_t *off, const do
     }
     if (nconf > 1) HIPCHK(hipStreamSynchronize(h->stream));
     if (m == 0) return status;
+    h->moved = true;
     // launches: configurations [cut[p], cut[p + 1]); the first of a launch has
     // none before it that could be refused, so the state it replaces is not held
     const int nf = 2 * h->model.nbands;
