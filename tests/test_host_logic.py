@@ -156,3 +156,17 @@ print(a, b)
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
     assert out.returncode == 0, out.stderr[-400:]
     assert out.stdout.split() == ["1", "1"]
+
+
+@pytest.mark.parametrize("ncorr,per_launch,launches", [(100, 2**33, 9), (100, 2**28, 33), (2**32, 0, 8)])
+def test_launches_stay_within_the_kernels_counters(host, ncorr, per_launch, launches):
+    """The sweep kernel counts a launch's moves in 32 bits: longer passes than
+    2^30 moves take several launches, whatever the caller asks for."""
+    g = ctqmc.CtqmcGpu.from_problem(P.anderson_1orb(NCorr=ncorr), nchains=1, seed=1, capacity=8)
+    assert host.w2d_ctqmc_set_launch(g.h, 0, 0, C.c_int64(per_launch)) == 0
+    if per_launch:
+        g.warmup(2**33 + 1)
+    else:
+        g.measure(2)
+    assert g.last_kernel_ms()[1] == launches
+    g.close()

@@ -584,7 +584,8 @@ int map_err(int e)
 }
 
 // Bring every chain to `target` moves of the current call in launches of at
-// most `per` moves (whole measurement intervals), starting from position
+// most `per` moves (whole measurement intervals where those take no more than
+// LAUNCH_MOVES), starting from position
 // `from`.  Asynchronous: the caller synchronises.
 void launch_range(w2d_ctqmc *h, long long from, long long target, long long ncorr, long long per, int only,
                   w2d_move_record *rec, long long rec_base)
@@ -593,7 +594,7 @@ void launch_range(w2d_ctqmc *h, long long from, long long target, long long ncor
     // ncorr, also when a resumed pass starts between two of them
     const bool giw = h->niw > 0 && ncorr > 0;
     for (long long t = from; t < target;) {
-        t = std::min(target, giw ? (t / ncorr + 1) * ncorr : t + per);
+        t = std::min({target, giw ? (t / ncorr + 1) * ncorr : t + per, t + w2d::LAUNCH_MOVES});
         DISPATCH(launch_sweep, h, t, ncorr, only, rec, rec_base);
         ++h->last_launches;
     }

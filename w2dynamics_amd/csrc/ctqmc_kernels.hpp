@@ -3467,9 +3467,14 @@ __device__ __attribute__((noinline)) bool make_ready(ChainRef r)
     return ok;
 }
 
+// A count of moves in 32 bits: a launch has at most LAUNCH_MOVES moves, so what
+// lies further ahead is as good as never.
+DEV int near(long long n) { return (int)min(n, (long long)0x7fffffff); }
+
 // What a sweep counts in registers: insertion and removal attempts, proposals
 // rejected by quantum numbers, and the attempts since the last multiple of
-// nslide.
+// nslide (where nslide exceeds 32 bits: such that the next multiple comes up at
+// near(nslide), 0 only at a multiple).
 struct Tally {
     int add, rem, qn, slide;
 };
@@ -3494,7 +3499,7 @@ DEV void one_move(Ctx &c, Tally &ty, int &kind, int &out)
             out = step_rem<NM>(c);
         }
         ty.qn += out == OUT_QN;
-        if (++ty.slide == (int)M.nslide) ty.slide = 0;
+        if (++ty.slide == near(M.nslide)) ty.slide = 0;
     } else {
         rng_close(c.rng);
         if (r <= 1.0 - M.p_shift) {
@@ -4327,12 +4332,14 @@ __global__ void __launch_bounds__(WAVE) sweep_kernel(DevModel M, ChainLayout L, 
     rng_open(c.rng);
     wsync();
     const long long pos0 = c.h.pos;
-    const int todo = (int)min(target - pos0, (long long)0x7fffffff);   // moves of this launch
+    const int todo = near(target - pos0);   // moves of this launch
     // moves until the next measurement, check of the calibration, look at the
     // abort word (warm-up); counted down instead of divided
-    const int every = ncorr > 0 ? (int)min(ncorr, (long long)0x7fffffff) : 128;
-    int until = every - (int)(pos0 % every), ucal = calib.x ? calib.y - (int)(pos0 % calib.y) : 0;
-    Tally ty{0, 0, 0, (int)((c.h.try_add + c.h.try_rem) % c.M.nslide)};
+    const long long step = ncorr > 0 ? ncorr : 128;
+    const int every = near(step);
+    int until = near(step - pos0 % step), ucal = calib.x ? calib.y - (int)(pos0 % calib.y) : 0;
+    const long long past = (c.h.try_add + c.h.try_rem) % c.M.nslide;
+    Tally ty{0, 0, 0, past == 0 ? 0 : max(near(c.M.nslide) - near(c.M.nslide - past), 1)};
     int done = 0;
     while (done < todo) {
         if (!s_wenv.ready && !make_ready<NM>(c.ref())) break;

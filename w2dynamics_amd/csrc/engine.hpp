@@ -78,6 +78,9 @@ struct ChainHdr {
     int kfmax[MAXF];               // largest order each flavour has reached
 };
 
+// moves of one launch at most (the sweep kernel counts them in 32 bits)
+constexpr long long LAUNCH_MOVES = 1LL << 30;
+
 // reasons a chain stops before the launch's target position (chain state intact)
 enum { HALT_NONE = 0, HALT_CAP = 1, HALT_ABORT = 2, HALT_DONE = 3 };
 
