@@ -7,6 +7,7 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 from conftest import ROOT
@@ -169,4 +170,42 @@ def test_launches_stay_within_the_kernels_counters(host, ncorr, per_launch, laun
     else:
         g.measure(2)
     assert g.last_kernel_ms()[1] == launches
+    g.close()
+
+
+@pytest.mark.parametrize("call", ["group_sums", "group_histograms", "giw", "score_sums", "load_configs"])
+def test_large_work_areas_are_given_back(host, call, tmp_path):
+    """The device memory that a call works in stays with the handle up to 64 MB;
+    what takes more is gone when the call returns."""
+    kw = dict(Ntau=400000) if call in ("group_sums", "group_histograms") else {}
+    if call == "giw":
+        kw = dict(MeasGiw=1, Niw=300000)
+    nch = 16
+    if call == "score_sums":
+        prob, deriv = P.kanamori_3orb_theta(beta=4.0, Ntau=30000)
+        g = ctqmc.CtqmcGpu.from_problem(prob, nchains=nch, seed=1, capacity=4)
+        g.set_derivatives(deriv)
+    else:
+        g = ctqmc.CtqmcGpu.from_problem(P.anderson_1orb(**kw), nchains=nch, seed=1, capacity=4)
+    g.measure(1)
+    if call == "load_configs":
+        # 16 chains of 2 x 1000 pairs: 16 MB each to hold
+        g.close()
+        g = ctqmc.CtqmcGpu.from_problem(P.anderson_1orb(), nchains=nch, seed=1, capacity=1100)
+        for c in range(nch):
+            host.host_halt(g.h, c, 1000)
+        path = str(tmp_path / "empty.npz")
+        np.savez(path, n=np.zeros(nch, np.int64), outer_sst=np.zeros(nch, np.int32), taus=np.zeros(0),
+                 orbs=np.zeros(0, np.int32), spins=np.zeros(0, np.int32), cas=np.zeros(0, np.int32))
+    before = _memory(host)[1]
+    run = dict(group_sums=lambda: g.group_sums(nch), giw=lambda: g.giw_sums(nch), score_sums=lambda: g.score_sums(nch),
+               group_histograms=lambda: g.group_histograms(nch),
+               load_configs=lambda: g.load_configs(path))[call]
+    run()
+    assert _memory(host)[1] - before <= 64 << 20
+    small = _memory(host)
+    if call == "group_sums":
+        g.group_sums(1)
+        g.group_sums(1)
+        assert _memory(host)[0] == small[0] + 1      # allocated once, then kept
     g.close()

@@ -59,8 +59,8 @@ struct w2d_ctqmc {
     // MeasGiw: raw G(i w_n) sums [nchains][2N][niw][2] and the per (chain,
     // flavour) visit record of giw_kernel [nchains][2N][2]; niw = 0: off
     int niw = 0;
-    // device work area of the group sums, kept between calls (grown when a
-    // call needs more, freed with the handle), and pinned room for the headers
+    // device work area of the group sums and stored configurations (WorkArea),
+    // and pinned room for the headers
     void *work = nullptr;
     size_t work_bytes = 0;
     w2d::ChainHdr *hdr_pinned = nullptr;
@@ -105,6 +105,7 @@ constexpr long LDS_GRAIN = 1280;         // bytes LDS is handed out in
 // the dynamic part may start behind it
 constexpr long LDS_STATIC = (sizeof(w2d::WalkEnv) + 15) / 16 * 16;
 constexpr int SEG_CACHE = 128;           // window operators the segment caches of blocks above 4 states cover
+constexpr size_t WORK_KEEP = (size_t)64 << 20;   // device work area a handle keeps between calls
 constexpr long HOLD_BYTES = 64L << 20;   // chain states that one launch of set_configs may have to put back
 constexpr int APT_CAP = 65536;           // accepted-pair distances a calibration list holds at most
 constexpr int GIW_NIW_MAX = 1 << 20;     // Matsubara frequencies of MeasGiw at most
@@ -745,20 +746,34 @@ size_t group_sums_bytes(const w2d_ctqmc *h, int ngroups)
     return (size_t)ngroups * ((size_t)nel * 8 + 14 * 8 + 8);
 }
 
-// at least `bytes` of device work area
-int need_work(w2d_ctqmc *h, size_t bytes)
-{
-    if (bytes <= h->work_bytes) return W2D_OK;
-    if (h->work) {
+// The device work area for the length of a call: what stays with the handle is
+// at most WORK_KEEP bytes, more is given back when the call ends.
+struct WorkArea {
+    w2d_ctqmc *h;
+    // at least `bytes`
+    int need(size_t bytes)
+    {
+        if (bytes <= h->work_bytes) return W2D_OK;
+        const int st = release();
+        if (st) return st;
+        HIPCHK(hipMalloc(&h->work, bytes));
+        h->work_bytes = bytes;
+        return W2D_OK;
+    }
+    int release()
+    {
+        if (!h->work) return W2D_OK;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipFree(h->work));
         h->work = nullptr;
         h->work_bytes = 0;
+        return W2D_OK;
     }
-    HIPCHK(hipMalloc(&h->work, bytes));
-    h->work_bytes = bytes;
-    return W2D_OK;
-}
+    ~WorkArea()
+    {
+        if (h->work_bytes > WORK_KEEP) (void)release();
+    }
+};
 
 // Sums over groups of chains of the accumulators in [from, to) of the chain
 // blocks into `work` ([ngroups][(to - from) / 8]); put() copies one array's
@@ -1012,7 +1027,8 @@ int set_configs(w2d_ctqmc *h, int first, int nconf, const int64_t *off, const do
     cut.push_back(m);
     const size_t nops = (size_t)off[m], btau = nops * 8, bat = (size_t)m * 8, bcode = nops * 4;
     ints.insert(ints.end(), outer_sst, outer_sst + m);
-    int st = need_work(h, (size_t)most + btau + bat + bcode + ints.size() * 4);
+    WorkArea area{h};
+    int st = area.need((size_t)most + btau + bat + bcode + ints.size() * 4);
     if (st) return st;
     char *hold = static_cast<char *>(h->work), *wtau = hold + most, *wat = wtau + btau, *wcode = wat + bat,
          *wints = wcode + bcode;
@@ -1637,7 +1653,8 @@ int w2d_ctqmc_get_score_sums(w2d_ctqmc *h, int ngroups, double *ssum, double *gt
     if (!h || ngroups < 1 || ngroups > h->nchains) return W2D_ERR_ARG;
     if (!h->measured || !h->dm.score || h->dm.ntheta < 1) return W2D_ERR_STATE;
     const w2d::ChainLayout &L = h->L;
-    int st = need_work(h, (size_t)ngroups * (size_t)(L.stride - L.scsum));
+    WorkArea area{h};
+    int st = area.need((size_t)ngroups * (size_t)(L.stride - L.scsum));
     if (st) return st;
     GroupSums g{h, ngroups, L.scsum, 0, static_cast<double *>(h->work)};
     st = g.run(L.stride);
@@ -1706,7 +1723,8 @@ int w2d_ctqmc_get_group_sums(w2d_ctqmc *h, int ngroups, double *gtau, double *gl
 {
     if (!h || ngroups < 1 || ngroups > h->nchains) return W2D_ERR_ARG;
     if (!h->measured) return W2D_ERR_STATE;
-    const int st = need_work(h, (size_t)ngroups * (size_t)(h->L.gbuf - h->L.gtau + 14 * 8 + 8));
+    WorkArea area{h};
+    const int st = area.need((size_t)ngroups * (size_t)(h->L.gbuf - h->L.gtau + 14 * 8 + 8));
     if (st) return st;
     return group_sums_into(h, ngroups, h->work, gtau, gleg, dm_blocks, histo, outer, scalars, nused);
 }
@@ -1758,7 +1776,8 @@ int w2d_ctqmc_get_giw(w2d_ctqmc *h, int ngroups, int *niw, double *out)
     // groups of contiguous chains as in w2d_ctqmc_get_group_sums, summed on the
     // device (the sums of all chains are 64 MB for 512 chains of the 2-orbital
     // model at 2000 frequencies)
-    if ((st = need_work(h, (size_t)ngroups * per * sizeof(double)))) return st;
+    WorkArea area{h};
+    if ((st = area.need((size_t)ngroups * per * sizeof(double)))) return st;
     const ChainHdr *hdrs = reinterpret_cast<const ChainHdr *>(h->chains + h->L.hdrs);
     hipLaunchKernelGGL(w2d::group_sum_kernel, dim3((unsigned)((per + 255) / 256), (unsigned)ngroups), dim3(256), 0,
                        h->stream, (const char *)h->giw, (long)(per * sizeof(double)), (long)per, nc, ngroups, hdrs,
@@ -1883,7 +1902,8 @@ int w2d_ctqmc_get_group_histograms(w2d_ctqmc *h, int ngroups, double *outer_stat
     if (!h || ngroups < 1 || ngroups > h->nchains) return W2D_ERR_ARG;
     if (!h->measured) return W2D_ERR_STATE;
     const w2d::ChainLayout &L = h->L;
-    int st = need_work(h, (size_t)ngroups * (size_t)(L.gmstep - L.ohst));
+    WorkArea area{h};
+    int st = area.need((size_t)ngroups * (size_t)(L.gmstep - L.ohst));
     if (st) return st;
     GroupSums g{h, ngroups, L.ohst, 0, static_cast<double *>(h->work)};
     st = g.run(L.gmstep);
