@@ -3237,7 +3237,7 @@ __device__ __attribute__((noinline)) int step_glob(ChainRef ref)
     int *tkf = reinterpret_cast<int *>(tfa + nf * kc);
     rebuild_flavour_lists(c, tfc, tfa, tkf, nullptr, nullptr);
     // det(new Delta) * det(old M) (get_InvFullHybr, get_FullLogDet)
-    double dnl = 0.0, dns = 1.0, dol = 0.0, dos = 1.0;
+    double dnl = 0.0, dns = 1.0;
     bool sing = false;
     for (int f = 0; f < nf; ++f) {
         const int k = tkf[f];
@@ -3247,12 +3247,10 @@ __device__ __attribute__((noinline)) int step_glob(ChainRef ref)
             dnl += l;
             dns *= s;
         }
-        const double k3 = (double)k * k * k;
-        c.work((2.0 / 3.0) * k3 * 2.0, 8.0 * (double)k * k);
+        c.work((2.0 / 3.0) * k * k * k, 8.0 * k * k);
     }
     // det(old M) = 1 / det(old Delta), which the chain carries
-    dol = -c.h.det_log;
-    dos = c.h.det_sign;
+    const double dol = -c.h.det_log;
     const TraceVal T = full_trace<NM>(c, c.h.outer);
     const double wr = exp((T.log_abs() - c.h.trace_log) + (dnl + dol));
     const double rr = grnd(c.rng);   // drawn even for a singular Delta (prob = 0)
@@ -3263,6 +3261,7 @@ __device__ __attribute__((noinline)) int step_glob(ChainRef ref)
             if (k == 0) continue;
             double l, s;
             delta_inverse<NM>(c, f, k, l, s);
+            c.work(2.0 * k * k * k, 8.0 * k * k);
         }
         c.h.det_log = dnl;
         c.h.det_sign = dns;
