@@ -30,6 +30,12 @@ F2PY_MAP = os.path.join(HERE, "fortran", "f2cmap")
 F2PY_EXT = os.path.join(HERE, "CTQMC" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 
+# -amdgpu-mfma-vgpr-form lets matrix instructions write vector registers, not
+# accumulation registers that every result is then copied out of.  It is an option
+# of LLVM's AMDGPU backend and not of the driver: the hipcc of ROCm 7.2.0, with
+# which everything here is built and measured, knows it; one that does not stops
+# with "Unknown command line argument".  It changes register allocation only, so it
+# can be left out there.
 def build(verbose: bool = False) -> str:
     cmd = ["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-fno-optimize-sibling-calls", "-mllvm",
            "-amdgpu-mfma-vgpr-form=1",

@@ -738,8 +738,10 @@ int run_moves(w2d_ctqmc *h, long long nmoves, long long ncorr)
     return batch_status(hd);
 }
 
-// Device work area of the group sums over all accumulators: [ngroups][nel]
-// partial sums, then [ngroups][14] scalars, then [ngroups] chain counts.
+// What the allocation-free group sums set aside in the static scratch: room for
+// sums over all accumulators, [ngroups][14] scalars and [ngroups] chain counts.
+// (They take less, the accumulators up to gbuf; the limit is kept, so that the
+// calls it refuses stay the same.)
 size_t group_sums_bytes(const w2d_ctqmc *h, int ngroups)
 {
     const long nel = (h->L.stride - h->L.gtau) / 8;
@@ -1237,8 +1239,7 @@ int w2d_ctqmc_create(const char *params, int nbands, int nftau, const double *u_
     }
     int st = 0;
     if ((st = upload(h.get(), m.sizes, &d.sizes)) || (st = upload(h.get(), m.offsets, &d.offsets)) ||
-        (st = upload(h.get(), m.connect, &d.connect)) || (st = upload(h.get(), first_state, &d.first_state)) ||
-        (st = upload(h.get(), m.state_sst, &d.state_sst)) || (st = upload(h.get(), m.opoff, &d.opoff)) ||
+        (st = upload(h.get(), first_state, &d.first_state)) || (st = upload(h.get(), m.state_sst, &d.state_sst)) ||
         (st = upload(h.get(), m.ops, &d.ops)) || (st = upload(h.get(), m.evals, &d.evals)) ||
         (st = upload(h.get(), fdiag, &d.ftau)) || (st = upload(h.get(), dmoff, &d.dmoff)) ||
         (st = upload(h.get(), legc, &d.legc)) || (st = upload(h.get(), trans, &d.trans)) ||

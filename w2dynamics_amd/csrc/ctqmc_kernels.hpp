@@ -484,7 +484,7 @@ DEV Ctx attach(ChainRef r)
         c.lbs = lds_ptr<int>(e.lbs);
     }
     c.legc = lds_ptr<double>(e.legc);
-    // work matrices: LDS for blocks up to 16 states (decided at compile time so
+    // work matrices: LDS for blocks up to 4 states (decided at compile time so
     // that their accesses are LDS instructions, not generic ones), HBM above
     if constexpr (NM <= 4) c.K0 = lds_ptr<double>(e.k);
     else c.K0 = reinterpret_cast<double *>(base + L.kwork);
@@ -682,7 +682,7 @@ struct State {
 #pragma unroll
         for (int e = 0; e < NV; ++e) v[e] = row(e) == col() && col() < no ? 1.0 : 0.0;
     }
-    // largest modulus; `on`: the lanes that count
+    // largest modulus of this lane's entries
     DEV double maxabs() const
     {
         double m = fabs(v[0]);
@@ -758,7 +758,8 @@ struct WalkOut {
 //      16: ceil(ns/4) chained matrix instructions; the operator blocks lie in
 //      global memory in the lanes' own order (512 bytes per k-step, zero beyond
 //      the block; 216 KB for the 3-orbital model, shared by all chains), so an
-//      operator is three coalesced loads, issued two operators ahead.  Blocks of one state: a product over the lanes.
+//      operator is three coalesced loads, issued two operators ahead.  Blocks of
+//      one state: a product over the lanes.
 // The renormalisation check runs per operator only if some propagation of the
 // group spans more than exp(-WALK_DECAY), else every fourth operator.
 // KEEP: the states after every operator go to px.
@@ -1418,7 +1419,7 @@ DEV MfmaEnv mfma_env(const Ctx &c)
     return e;
 }
 
-// algorithmic work of an MFMA walk (as Work::commit counts it)
+// algorithmic work of an MFMA walk (states in and out, block products)
 DEV void mfma_work(Ctx &c, const MfmaOut &r, int no)
 {
     c.work((double)no * (2.0 * r.ntns + r.nss), 8.0 * no * (r.nss + r.nts));

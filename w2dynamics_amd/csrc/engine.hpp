@@ -19,11 +19,10 @@ struct DevModel {
     // spin 0 | of spin 1 << 8, 0 if the blocks have no such keys
     const unsigned char *keys;
     int dkey;
-    const int *sizes, *offsets, *connect, *first_state, *state_sst;
-    const long *opoff;
+    const int *sizes, *offsets, *first_state, *state_sst;
     // blocks above 16 states: every operator block zero-padded to multiples of
     // 16 rows and columns (column-major, leading dimension 16 ceil(n_t / 16)),
-    // offsets indexed like opoff; the MFMA walks read whole 16 x 4 fragments
+    // offsets indexed like trans; the MFMA walks read whole 16 x 4 fragments
     // without bounds checks
     const double *ops16;
     const int *opoff16;
