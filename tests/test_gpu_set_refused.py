@@ -81,7 +81,8 @@ def test_chains_behind_a_refused_one_keep_theirs(case, where, tmp_path):
             continue
         for f in range(2 * nb):
             assert np.array_equal(a.get_minv(c, f), b.get_minv(c, f)), (c, f)
-        assert np.array_equal(a.moves_log(c, 150), b.moves_log(c, 150)), c
+        x, y = a.moves_log(c, 150), b.moves_log(c, 150)
+        assert all(np.array_equal(x[k], y[k]) for k in x.dtype.names if k != "pad"), c
     for g in (a, b, src):
         g.close()
 
